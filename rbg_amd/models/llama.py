@@ -374,7 +374,7 @@ class LlamaForCausalLM(nn.Module):
                gather_idx: Optional[torch.Tensor] = None) -> torch.Tensor:
         if gather_idx is not None:
             hidden = hidden[gather_idx.long()]
-        return torch.nn.functional.linear(hidden, self.lm_head).float()
+        return ops.linear(hidden, self.lm_head).float()
 
     def reload_weights(self, seed: int) -> None:
         """In-place weight refresh — the live-update path (SURVEY §2.3

@@ -94,24 +94,30 @@ def _on_gpu(t: torch.Tensor) -> bool:
 SKINNY_GEMM = int(__import__("os").environ.get("RBG_SKINNY_GEMM", "1"))
 
 
+def _skinny(rows: int, n: int, k: int) -> bool:
+    """Does the hand-written decode GEMM (hip/skinny_gemm.hip) take a [rows, k]
+    x [n, k] product, rather than hipBLASLt?  Measured with cold weights (us,
+    own against library): narrow matrices at any decode batch (4096 x 14336:
+    1 row 22 against 24, 64 rows 28 against 38, 128 rows 38 against 73; 10240 x
+    8192: 39 against 41 and 50 against 55), but the short ones only up to 64
+    (3072 x 2048: 16 rows 7.6 against 8.6, 64 rows 9.5 against 9.2, 128 rows
+    12.5 against 12.0).  Wide
+    ones up to 64 rows (28672 x 4096: 1 row 40 against 57, 64 rows 46 against
+    49, 128 rows 58 against 53), where rows are a multiple of 4 KB apart
+    (51200 x 5120: 1 row 94 against 89, 64 rows 122 against 98)."""
+    if rows < 1 or n % 32 or k % 512:
+        return False
+    if n <= 12288:
+        return rows <= (128 if k > 2048 else 64)
+    return rows <= 64 and k % 2048 == 0
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """Projection GEMM with decode-shape dispatch: for M <= 128 rows the
-    hand-written split-K streaming kernel (hip/skinny_gemm.hip) replaces
-    hipBLASLt, which leaves 2-5x on narrow-N skinny shapes
-    (profiles/gemm_ab_b128.json).  Prefill-sized M goes to the library."""
-    # measured policy (profiles/sg_micro7_b*.json): the custom kernel wins
-    # on narrow-N shapes (o/down, N<=4096) at any decode batch, on mid-N
-    # (qkv, 6144) only up to M=64, and never on wide-N (gate_up 28672,
-    # where hipBLASLt already streams at ~6 TB/s).  Between them, for a few
-    # rows, hipBLASLt takes up to 2.7 times as long (18432 x 2048: 58 us
-    # against 22) and is nowhere ahead by more than a tenth
+    """Projection GEMM: decode shapes take the hand-written kernel,
+    prefill-sized ones the library."""
     if (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and
-            x.dtype == torch.bfloat16 and x.shape[0] <= 128 and
-            w.shape[0] % 32 == 0 and x.shape[1] % 512 == 0 and
-            (w.shape[0] <= 4608 or
-             (x.shape[0] <= 64 and w.shape[0] <= 8192) or
-             (x.shape[0] <= 16 and w.shape[0] <= 24576 and
-              x.shape[1] <= 4096))):
+            x.dtype == torch.bfloat16 and
+            _skinny(x.shape[0], w.shape[0], x.shape[1])):
         # one of these is there whatever the model
         return require("_hip_ops", "_hip_mix", "_hip_gated", "_hip_moe",
                        "_hip_hyper").skinny_gemm(

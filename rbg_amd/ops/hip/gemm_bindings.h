@@ -6,9 +6,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 extern "C" {
 void launch_skinny_gemm(void*, void*, const void*, const void*, int, int,
-                        int, int, hipStream_t);
+                        int, int, int, int, hipStream_t);
 void launch_reduce_splits(void*, const void*, int, long, hipStream_t);
 }
 
@@ -16,47 +18,63 @@ inline hipStream_t gemm_stream() {
   return at::hip::getCurrentHIPStream().stream();
 }
 
-inline int pick_gemm_splits(int N, int K) {
-  // fill the chip with 16-wave workgroups (>= ~256 WGs); each split's K
-  // range divides into 8 x 32-k wave slices (K % (splits*256) == 0)
-  const int n_groups = N >> 5;
-  for (int s : {8, 4, 2})
-    if (n_groups * s <= 512 && n_groups * s >= 192 && K % (s * 256) == 0)
-      return s;
-  for (int s : {4, 2})
-    if (n_groups * s >= 128 && K % (s * 256) == 0) return s;
-  return 1;
+// Which kernel a shape takes: waves per workgroup (0: the kernel of a few
+// rows) and the parts that K is split into.
+struct SkinnyPlan {
+  int waves, splits;
+};
+
+inline SkinnyPlan pick_skinny(int M, int N, int K) {
+  // a few rows; where rows of W are no multiple of 4 KB apart the kernel falls
+  // behind (5120 x 25600: 66 us against 50, 4096 x 14336: 22.4 against 24.3)
+  if (M <= 4 && K % 2048 == 0) return {0, 1};
+  // up to 32 rows of a narrow matrix: workgroups of half the size, half again
+  // as many as fit at once (6144 x 4096, one row: 13.2 us against 14.2; above
+  // 32 rows A's copies cost more, 14336 x 4096, 64 rows: 30.1 against 26.7)
+  if (M <= 32 && N <= 8192) {
+    const int tiles = (N + 63) / 64;
+    return {4, std::max(1, std::min({768 / tiles, K / 256, 8}))};
+  }
+  // one workgroup of 8 waves per CU, all of them at once: the last of 1.5 or
+  // 2.5 rounds is lost (10240 x 8192, 64 rows: 3 splits = 240 workgroups 38 us,
+  // 4 splits 48, 6 splits 40)
+  const int tiles = (N + 127) / 128;
+  return {8, std::max(1, std::min({256 / tiles, K / 256, 16}))};
 }
 
 inline bool skinny_gemm_supported(int64_t M, int64_t N, int64_t K) {
-  // M <= 256: the cross-slice LDS reduce holds 4 waves x M_TILES x 1 KB
-  // (64 KB at M_TILES=16); larger batches fall back to hipBLASLt
   return M >= 1 && M <= 256 && (N % 32) == 0 && (K % 256) == 0;
 }
 
-inline torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor w,
-                          int64_t force_splits = 0) {
+inline void check_skinny(const torch::Tensor& a, const torch::Tensor& w) {
   for (const auto& t : {a, w})
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
                 t.is_contiguous() && t.dim() == 2,
                 "operands must be contiguous bf16 matrices on GPU");
+  TORCH_CHECK(w.size(1) == a.size(1), "K mismatch");
+  TORCH_CHECK(skinny_gemm_supported(a.size(0), w.size(0), a.size(1)),
+              "unsupported skinny shape");
+}
+
+inline torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor w,
+                          int64_t force_splits = 0) {
+  check_skinny(a, w);
   const int64_t M = a.size(0), K = a.size(1), N = w.size(0);
-  TORCH_CHECK(w.size(1) == K, "K mismatch");
-  TORCH_CHECK(skinny_gemm_supported(M, N, K), "unsupported skinny shape");
   auto c = torch::empty({M, N}, a.options());
-  int splits = force_splits > 0 ? (int)force_splits
-                                : pick_gemm_splits((int)N, (int)K);
-  if (K % (splits * 256) != 0) splits = pick_gemm_splits((int)N, (int)K);
+  SkinnyPlan plan = pick_skinny((int)M, (int)N, (int)K);
+  if (force_splits > 0 && K % (force_splits * 256) == 0)
+    plan = {plan.waves ? plan.waves : 8, (int)force_splits};
   torch::Tensor ws;
   void* wsp = nullptr;
-  if (splits > 1) {
-    ws = torch::empty({splits, M, N}, a.options().dtype(torch::kFloat32));
+  if (plan.splits > 1) {
+    ws = torch::empty({plan.splits, M, N}, a.options().dtype(torch::kFloat32));
     wsp = ws.data_ptr();
   }
   launch_skinny_gemm(c.data_ptr(), wsp, a.data_ptr(), w.data_ptr(), (int)M,
-                     (int)N, (int)K, splits, gemm_stream());
-  if (splits > 1)
-    launch_reduce_splits(c.data_ptr(), wsp, splits, (long)(M * N),
+                     (int)N, (int)K, plan.waves, plan.splits, 0,
+                     gemm_stream());
+  if (plan.splits > 1)
+    launch_reduce_splits(c.data_ptr(), wsp, plan.splits, (long)(M * N),
                          gemm_stream());
   return c;
 }

@@ -1,287 +1,342 @@
-// Skinny GEMM for decode-shape projections: C[M,N] = A[M,K] x W[N,K]^T,
-// bf16 in / f32 accumulate / bf16 out, M <= 256 (a decode batch).
+// Decode-shape GEMM: C[M,N] = A[M,K] x W[N,K]^T, bf16 in, f32 accumulators,
+// bf16 out, M <= 256 rows.  Optionally W's two halves are a gate and an up
+// matrix and C[M,N/2] = silu(A Wg^T) * (A Wu^T).
 //
-// Why hand-written: at M=128 the layer projections are pure weight streams
-// (ideal time = W bytes / HBM bandwidth), yet every library backend leaves
-// 2-5x on the narrow-N shapes (profiles/gemm_ab_b128.json: hipBLASLt and
-// rocBLAS both ~1.7-2.4 TB/s on o/qkv/down vs ~6 TB/s on the wide gate_up;
-// composable-kernel far worse).  Library tilings are built for big M; a
-// skinny GEMM wants every CU streaming DISTINCT weight rows with the whole
-// A operand riding in L2.
+// Bound: the weights, read once from HBM.  A plain read reaches 6.1-6.3 TB/s
+// here, so 28672 x 4096 takes 38 us at best; up to 16 rows take 40 of them,
+// 64 take 46 and 128 take 58, whose A panels pass the L2s as often as the
+// weights do.
 //
-// Kernel shape (CDNA4, 64-lane waves, v_mfma_f32_16x16x32_bf16):
-//   grid  = (N/32) * SPLITS workgroups of 4 waves: (k_slice 0..1) x
-//           (n_tile 0..1) over a 32-column C panel, 64 k per step
-//   stage = W[32 x 64] + A[M x 64] through LDS via coalesced 16-lane row
-//           pieces (direct per-lane fragment gathers measured 3-5x slow)
-//   pipe  = DOUBLE-buffered LDS + TWO register load-sets issuing 2-3
-//           steps ahead, ONE barrier per step.  Earlier cuts of this
-//           kernel staged 1 step ahead behind 2 barriers: every step then
-//           serialized on full HBM latency (rocprof: SQ_WAIT_ANY = 90%
-//           of cycles, 42 us for a 33 MB weight stream).  Small WGs
-//           (23 KB stage + 32 KB reduce scratch) keep ~3 WGs resident
-//           per CU so stalled WGs are covered by runnable ones.
-//   math  = per step each wave reads 1 W + M_TILES A fragments from LDS
-//           (contiguous-8 per-lane MFMA layout) and issues M_TILES MFMAs
-//   end   = the 2 k-slices of each n-tile fold through the LDS reduce
-//           scratch, one bf16 store; SPLITS>1 writes f32 partials +
-//           reduce_splits() folds them
-//
-// A-traffic note: a 32-column panel reads all of A (M x K, ~1 MB at
-// M=128/K=4096) — L2-resident after the first panel per XCD, so HBM sees
-// ~W + 8 x A bytes.
+// Weights go from global memory straight into MFMA operand registers: a lane
+// of v_mfma_f32_16x16x32_bf16 holds 8 consecutive k of one row, so a wave's
+// load covers 64 bytes of 16 rows, the next one the other half of the lines.
+// What made the difference, at 28672 x 4096:
+//  * plain loads, not non-temporal ones, which send both halves of a line to
+//    L2 and back as requests of their own (16 rows: 48 -> 42 us),
+//  * loads pinned where they are issued: the compiler otherwise moves A's to
+//    their use, behind the MFMAs, and every chunk pays their latency (128
+//    rows: 75 -> 64 us),
+//  * two lines of a row at a time, not one (57344 x 8192, 1 row: 189 -> 169),
+//  * workgroups begin at different places of K.  All rows of A and W are K
+//    apart, so workgroups in step ask the same few L2 channels (128 rows: 78
+//    -> 75 us).
 #include "common.h"
 
-typedef __attribute__((ext_vector_type(8))) __bf16 gg_bf8;
+namespace {
 
-DEV_INLINE gg_bf8 lds_frag(const __hip_bfloat16* p) {
-  union { uint4 u; gg_bf8 v; } cvt;
-  cvt.u = *reinterpret_cast<const uint4*>(p);
-  return cvt.v;
+constexpr int KC = 128;           // k per chunk
+constexpr int DEPTH = 2;          // chunks of weights in flight per wave
+constexpr int ROWS_KC = 64, ROWS_DEPTH = 4;     // of skinny_rows_kernel
+
+typedef __attribute__((ext_vector_type(4))) unsigned int sg_u4;
+
+DEV_INLINE sg_u4 sg_load(const __hip_bfloat16* p) {
+  return *reinterpret_cast<const sg_u4*>(p);
 }
 
-#define SG_KSTEP 64                   // k consumed per WG step
-#define SG_LDS_PITCH (SG_KSTEP + 8)   // +8 bf16: bank-conflict pad
-#define SG_NT 256                     // threads (4 waves)
+DEV_INLINE bf16x8 sg_frag(sg_u4 u) {
+  union { sg_u4 u; bf16x8 v; } c;
+  c.u = u;
+  return c.v;
+}
 
-template <int M_TILES, int SPLITS>
-__global__ __launch_bounds__(SG_NT, 3) void skinny_gemm_kernel(
+DEV_INLINE float silu(float g) { return g / (1.f + __expf(-g)); }
+
+// The chunk that a workgroup takes as its c-th.
+DEV_INLINE int sg_turn(int c, int first, int n) {
+  c += first;
+  return c >= n ? c - n : c;
+}
+
+// A few rows: 8 waves share one 16-row tile of W and take its K in turns,
+// without a barrier until their sums meet in LDS, and without splits whose
+// sums a second launch would add.  4096 x 4096, one row: 8.5 us against 10.5 of
+// the kernel below with its reduction.  Its time grows with the rows, since
+// every workgroup reads all of A (28672 x 4096: 4 rows 40 us, 16 rows 56).
+// GLU: the tile is 8 rows of the gate and the same 8 of the up matrix.
+template <bool GLU>
+__global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
     const __hip_bfloat16* __restrict__ a,   // [M, K]
     const __hip_bfloat16* __restrict__ w,   // [N, K]
-    __hip_bfloat16* __restrict__ c,         // [M, N]   (SPLITS == 1)
-    float* __restrict__ ws,                 // [SPLITS, M, N] (SPLITS > 1)
+    __hip_bfloat16* __restrict__ c,         // [M, N], GLU: [M, N / 2]
     const int M, const int N, const int K) {
-  const int n_groups = N >> 5;
-  const int n_group = blockIdx.x % n_groups;
-  const int split = blockIdx.x / n_groups;
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int lane = tid & 63;
-  const int gl = lane & 15;        // fragment row lane
-  const int gslice = lane >> 4;    // fragment k sub-chunk
+  constexpr int WAVES = 8;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int row = GLU ? blockIdx.x * 8 + (r & 7) + (r >> 3) * (N / 2)
+                      : blockIdx.x * 16 + r;
+  const __hip_bfloat16* wp = w + (size_t)row * K + wave * ROWS_KC + g * 8;
+  const __hip_bfloat16* ap = a + (size_t)min(r, M - 1) * K + wave * ROWS_KC + g * 8;
+  const int n = (K / ROWS_KC - wave + WAVES - 1) / WAVES;
+  const int first = n ? ((blockIdx.x >> 3) + (blockIdx.x & 7) * (n >> 3)) % n
+                      : 0;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  sg_u4 wr[ROWS_DEPTH][2], ar[ROWS_DEPTH][2];
+#define SR_LOAD(s, at)                                                     \
+  do {                                                                     \
+    const int off = sg_turn(at, first, n) * (ROWS_KC * WAVES);                  \
+    wr[s][0] = sg_load(wp + off);                                          \
+    wr[s][1] = sg_load(wp + off + 32);                                     \
+    ar[s][0] = sg_load(ap + off);                                          \
+    ar[s][1] = sg_load(ap + off + 32);                                     \
+  } while (0)
+#define SR_MATH(s)                                                         \
+  do {                                                                     \
+    _Pragma("unroll") for (int h = 0; h < 2; ++h)                          \
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(                     \
+            sg_frag(ar[s][h]), sg_frag(wr[s][h]), acc, 0, 0, 0);           \
+  } while (0)
+  if (n > 0) {
+#pragma unroll
+    for (int s = 0; s < ROWS_DEPTH; ++s) SR_LOAD(s, min(s, n - 1));
+    int at = 0;
+    for (; at + ROWS_DEPTH < n; at += ROWS_DEPTH) {
+#pragma unroll
+      for (int s = 0; s < ROWS_DEPTH; ++s) {
+        SR_MATH(s);
+        SR_LOAD(s, min(at + ROWS_DEPTH + s, n - 1));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < ROWS_DEPTH; ++s)
+      if (at + s < n) SR_MATH(s);
+  }
+#undef SR_LOAD
+#undef SR_MATH
 
-  const int n_tile = wave & 1;               // 0..1 within the 32-col panel
-  const int k_slice = wave >> 1;             // 0..1, 32 k each per step
-  const int k_wg = K / SPLITS;               // this WG's k span
-  const int k0 = split * k_wg;
-  const int nsteps = k_wg / SG_KSTEP;
+  // lane l, register q: row 4 * (l >> 4) + q of A, row l & 15 of the tile
+  __shared__ float red[WAVES][256];
+  *reinterpret_cast<f32x4*>(&red[wave][lane * 4]) = acc;
+  __syncthreads();
+  const int e = threadIdx.x;
+  if (e < 256) {
+    const int col = (e >> 2) & 15, m = (e >> 6) * 4 + (e & 3);
+    float v = 0.f;
+#pragma unroll
+    for (int k = 0; k < WAVES; ++k) v += red[k][e];
+    if (GLU) {
+      if (m < M && col < 8) {
+        float up = 0.f;
+#pragma unroll
+        for (int k = 0; k < WAVES; ++k) up += red[k][e + 8 * 4];
+        c[(size_t)m * (N / 2) + blockIdx.x * 8 + col] = f2bf(silu(v) * up);
+      }
+    } else if (m < M) {
+      c[(size_t)m * N + blockIdx.x * 16 + col] = f2bf(v);
+    }
+  }
+}
 
-  constexpr int A_ROWS = M_TILES * 16;
-  constexpr int BUF = (32 + A_ROWS) * SG_LDS_PITCH;
-  __shared__ union {
-    __hip_bfloat16 stage[2][BUF];
-    float red[4][M_TILES * 256];
-  } lds;
+// NW waves of 16 rows of W each share MT * 16 rows of A through LDS, a chunk
+// at a time, two buffers, one barrier a chunk.  blockIdx.y: a part of K, whose
+// sums go to ws in f32.  GLU: half of the waves hold the gate's rows, the
+// others the same rows of the up matrix, and meet in LDS.
+template <int MT, int NW, bool GLU>
+__global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
+    const __hip_bfloat16* __restrict__ a,   // [M, K]
+    const __hip_bfloat16* __restrict__ w,   // [N, K]
+    __hip_bfloat16* __restrict__ c,         // [M, N], GLU: [M, N / 2]
+    float* __restrict__ ws,                 // [gridDim.y, M, N] if > 1
+    const int M, const int N, const int K) {
+  constexpr int THREADS = 64 * NW, PITCH = KC + 8;   // + 8: no bank conflicts
+  constexpr int PER = THREADS * 8 / KC;     // rows of A that one load covers
+  constexpr int PIECES = (MT * 16 + PER - 1) / PER, ROWS = PIECES * PER;
+  constexpr int STAGE = 2 * ROWS * PITCH * 2, MEET = GLU ? NW * MT * 1024 : 0;
+  __shared__ __align__(16) char lds[STAGE > MEET ? STAGE : MEET];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  // columns of this wave; beyond the last it reads the last ones again
+  const int half = GLU ? N / 2 : N;
+  constexpr int SIDE = GLU ? NW / 2 : NW;
+  const int col0 = (blockIdx.x * SIDE + wave % SIDE) * 16;
+  const int row = min(col0, half - 16) + r + (wave / SIDE) * half;
+  const int chunks = K / KC;
+  const int c0 = chunks * blockIdx.y / gridDim.y;
+  const int n = chunks * (blockIdx.y + 1) / gridDim.y - c0;
+  const int first = ((blockIdx.x >> 3) + (blockIdx.x & 7) * (n >> 3)) % n;
+  const __hip_bfloat16* wp = w + (size_t)row * K + c0 * KC + g * 8;
+  const __hip_bfloat16* ap[PIECES];
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p)
+    ap[p] = a + (size_t)min((tid / (KC / 8)) + p * PER, M - 1) * K + c0 * KC +
+            (tid % (KC / 8)) * 8;
+  __hip_bfloat16* buf[2];
+  buf[0] = (__hip_bfloat16*)lds;
+  buf[1] = buf[0] + ROWS * PITCH;
+  const int put = (tid / (KC / 8)) * PITCH + (tid % (KC / 8)) * 8;
 
-  // staging pieces, 16 B per (row, chunk): a 64-k row is 8 chunks, so
-  // W = 32 x 8 = 256 pieces (one per thread) and A = A_ROWS x 8 pieces
-  // (up to 4 per thread); 8 lanes x 16 B = 128 B contiguous per row.
-  // The two in-flight load sets are NAMED variables and the loop is
-  // unrolled by 2: a runtime-indexed set[2] array was demoted to scratch
-  // memory and every prefetch round-tripped through HBM (seen in the ISA
-  // as scratch_load/store_dwordx4 in the hot loop — 5x slowdown)
-  const int wrow_st = tid >> 3, wchk = (tid & 7) * 8;
-  constexpr int A_PIECES = (A_ROWS * 8 + SG_NT - 1) / SG_NT;
-  // the two in-flight load sets are SEPARATE named arrays: a struct array
-  // passed through lambda references was demoted to scratch memory and
-  // every prefetch round-tripped through HBM (ISA: scratch_*_dwordx4 in
-  // the hot loop)
-  // fully scalar load sets (a0..a3 per set): any array or struct here,
-  // even with unrolled constant indices, was demoted to scratch memory by
-  // the compiler and every prefetch round-tripped through HBM
-  uint4 wreg0, wreg1;
-  uint4 a00 = {}, a01 = {}, a02 = {}, a03 = {};
-  uint4 a04 = {}, a05 = {}, a06 = {}, a07 = {};
-  uint4 a10 = {}, a11 = {}, a12 = {}, a13 = {};
-  uint4 a14 = {}, a15 = {}, a16 = {}, a17 = {};
-  const __hip_bfloat16* wbase =
-      w + (size_t)((n_group << 5) + wrow_st) * K + wchk;
-  const __hip_bfloat16* ab0 = nullptr;
-  const __hip_bfloat16* ab1 = nullptr;
-  const __hip_bfloat16* ab2 = nullptr;
-  const __hip_bfloat16* ab3 = nullptr;
-  const __hip_bfloat16* ab4 = nullptr;
-  const __hip_bfloat16* ab5 = nullptr;
-  const __hip_bfloat16* ab6 = nullptr;
-  const __hip_bfloat16* ab7 = nullptr;
-#define SG_ABASE(s) (a + (size_t)min((tid + (s) * SG_NT) >> 3, M - 1) * K + \
-                     ((tid + (s) * SG_NT) & 7) * 8)
-  ab0 = SG_ABASE(0);
-  if (A_PIECES > 1) ab1 = SG_ABASE(1);
-  if (A_PIECES > 2) ab2 = SG_ABASE(2);
-  if (A_PIECES > 3) ab3 = SG_ABASE(3);
-  if (A_PIECES > 4) ab4 = SG_ABASE(4);
-  if (A_PIECES > 5) ab5 = SG_ABASE(5);
-  if (A_PIECES > 6) ab6 = SG_ABASE(6);
-  if (A_PIECES > 7) ab7 = SG_ABASE(7);
-  static_assert(A_PIECES <= 8, "A_PIECES grew past the scalar sets");
-
-#define SG_LD(p, kb) (*reinterpret_cast<const uint4*>((p) + (kb)))
-#define SG_ISSUE(step, wreg, a0, a1, a2, a3, a4, a5, a6, a7)                \
-  do {                                                                      \
-    const int kb = k0 + min(step, nsteps - 1) * SG_KSTEP;                   \
-    wreg = SG_LD(wbase, kb);                                                \
-    a0 = SG_LD(ab0, kb);                                                    \
-    if (A_PIECES > 1) a1 = SG_LD(ab1, kb);                                  \
-    if (A_PIECES > 2) a2 = SG_LD(ab2, kb);                                  \
-    if (A_PIECES > 3) a3 = SG_LD(ab3, kb);                                  \
-    if (A_PIECES > 4) a4 = SG_LD(ab4, kb);                                  \
-    if (A_PIECES > 5) a5 = SG_LD(ab5, kb);                                  \
-    if (A_PIECES > 6) a6 = SG_LD(ab6, kb);                                  \
-    if (A_PIECES > 7) a7 = SG_LD(ab7, kb);                                  \
+  f32x4 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = {0.f, 0.f, 0.f, 0.f};
+  sg_u4 wr[DEPTH][KC / 32], ar[PIECES], a0[PIECES];
+#define SG_W(s, at)                                                        \
+  do {                                                                     \
+    const int off = sg_turn(at, first, n) * KC;                            \
+    _Pragma("unroll") for (int h = 0; h < KC / 32; ++h)                    \
+        wr[s][h] = sg_load(wp + off + h * 32);                             \
+  } while (0)
+#define SG_A(regs, at)                                                     \
+  do {                                                                     \
+    const int off = sg_turn(at, first, n) * KC;                            \
+    _Pragma("unroll") for (int p = 0; p < PIECES; ++p)                     \
+        regs[p] = sg_load(ap[p] + off);                                    \
+  } while (0)
+#define SG_PUT(b, regs)                                                    \
+  do {                                                                     \
+    _Pragma("unroll") for (int p = 0; p < PIECES; ++p)                     \
+        *reinterpret_cast<sg_u4*>((b) + put + p * PER * PITCH) = regs[p];  \
+  } while (0)
+#define SG_MATH(s, b)                                                      \
+  do {                                                                     \
+    _Pragma("unroll") for (int h = 0; h < KC / 32; ++h)                    \
+    _Pragma("unroll") for (int i = 0; i < MT; ++i)                         \
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(                  \
+            sg_frag(sg_load((b) + (i * 16 + r) * PITCH + h * 32 + g * 8)), \
+            sg_frag(wr[s][h]), acc[i], 0, 0, 0);                           \
   } while (0)
 
-  // LDS store address for A piece s (rows past A_ROWS never occur: the
-  // last partial piece only exists when A_PIECES*SG_NT > A_ROWS*8, and
-  // then piece s covers i = tid + s*SG_NT < A_ROWS*8 by construction of
-  // A_PIECES for the supported M_TILES set)
-#define SG_AST(st, s) reinterpret_cast<uint4*>(                             \
-    &st[(32 + ((tid + (s) * SG_NT) >> 3)) * SG_LDS_PITCH +                  \
-        ((tid + (s) * SG_NT) & 7) * 8])
-#define SG_WRITE(st, wreg, a0, a1, a2, a3, a4, a5, a6, a7)                  \
-  do {                                                                      \
-    *reinterpret_cast<uint4*>(&st[wrow_st * SG_LDS_PITCH + wchk]) = wreg;   \
-    if (tid < A_ROWS * 8) *SG_AST(st, 0) = a0;                              \
-    if (A_PIECES > 1) *SG_AST(st, 1) = a1;                                  \
-    if (A_PIECES > 2) *SG_AST(st, 2) = a2;                                  \
-    if (A_PIECES > 3) *SG_AST(st, 3) = a3;                                  \
-    if (A_PIECES > 4) *SG_AST(st, 4) = a4;                                  \
-    if (A_PIECES > 5) *SG_AST(st, 5) = a5;                                  \
-    if (A_PIECES > 6) *SG_AST(st, 6) = a6;                                  \
-    if (A_PIECES > 7) *SG_AST(st, 7) = a7;                                  \
-  } while (0)
-
-  f32x4 acc[M_TILES];
+  // everything that the first chunks need is asked for before any wait
+  SG_A(a0, 0);
+  SG_A(ar, min(1, n - 1));
 #pragma unroll
-  for (int mt = 0; mt < M_TILES; ++mt) acc[mt] = {0.f, 0.f, 0.f, 0.f};
-
-  const int kf = k_slice * 32 + gslice * 8;
-  auto compute = [&](const __hip_bfloat16* st) {
-    const gg_bf8 wf = lds_frag(
-        &st[((n_tile << 4) + gl) * SG_LDS_PITCH + kf]);
+  for (int s = 0; s < DEPTH; ++s) SG_W(s, min(s, n - 1));
+  __builtin_amdgcn_sched_barrier(0);
+  SG_PUT(buf[0], a0);
+  int at = 0;
+  for (; at + DEPTH < n; at += DEPTH) {
 #pragma unroll
-    for (int mt = 0; mt < M_TILES; ++mt) {
-      const gg_bf8 af = lds_frag(
-          &st[(32 + mt * 16 + gl) * SG_LDS_PITCH + kf]);
-      acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, wf, acc[mt],
-                                                        0, 0, 0);
+    for (int s = 0; s < DEPTH; ++s) {
+      __syncthreads();
+      SG_PUT(buf[(s + 1) & 1], ar);
+      SG_A(ar, min(at + s + 2, n - 1));
+      __builtin_amdgcn_sched_barrier(0);
+      SG_MATH(s, buf[s & 1]);
+      SG_W(s, min(at + s + DEPTH, n - 1));
+      __builtin_amdgcn_sched_barrier(0);
     }
-  };
-
-  __hip_bfloat16* buf0 = lds.stage[0];
-  __hip_bfloat16* buf1 = lds.stage[1];
-
-  // pipeline prologue: tiles 0,1 in flight; tile 0 lands in buffer 0
-  SG_ISSUE(0, wreg0, a00, a01, a02, a03, a04, a05, a06, a07);
-  SG_ISSUE(1, wreg1, a10, a11, a12, a13, a14, a15, a16, a17);
-  SG_WRITE(buf0, wreg0, a00, a01, a02, a03, a04, a05, a06, a07);
-  SG_ISSUE(2, wreg0, a00, a01, a02, a03, a04, a05, a06, a07);
-
-  // nsteps is even (K % (SPLITS * 2*SG_KSTEP) == 0, enforced host-side);
-  // tile t+1 was issued 2 steps ago so its vmcnt wait is covered, and a
-  // buffer's previous tile was fully read before the barrier, so each
-  // step needs exactly one barrier
-  for (int step = 0; step < nsteps; step += 2) {
-    __syncthreads();
-    compute(buf0);                                 // tile step
-    SG_WRITE(buf1, wreg1, a10, a11, a12, a13, a14, a15, a16, a17);
-    SG_ISSUE(step + 3, wreg1, a10, a11, a12, a13, a14, a15, a16, a17);
-    __syncthreads();
-    compute(buf1);                                 // tile step+1
-    SG_WRITE(buf0, wreg0, a00, a01, a02, a03, a04, a05, a06, a07);
-    SG_ISSUE(step + 4, wreg0, a00, a01, a02, a03, a04, a05, a06, a07);
   }
-#undef SG_ISSUE
-#undef SG_WRITE
-#undef SG_ABASE
-#undef SG_LD
-#undef SG_AST
-
-  // ---- cross-slice reduction through LDS (buffer re-use) ----------------
-  __syncthreads();
 #pragma unroll
-  for (int mt = 0; mt < M_TILES; ++mt) {
-    F32x4U u;
-    u.v = acc[mt];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      lds.red[wave][mt * 256 + r * 64 + lane] = u.e[r];
-  }
-  __syncthreads();
-
-  // fold 2 k-slices; elem e of n-tile nt: lane64 = e & 63,
-  // reg = (e >> 6) & 3, mt = e >> 8 -> m = mt*16 + 4*(lane64>>4) + reg,
-  // n = panel + nt*16 + (lane64 & 15)
-  const int elems = M_TILES * 256 * 2;
-  for (int e = tid; e < elems; e += SG_NT) {
-    const int nt = e >= M_TILES * 256;
-    const int ee = e - nt * M_TILES * 256;
-    const float v = lds.red[nt][ee] + lds.red[2 + nt][ee];
-    const int l64 = ee & 63;
-    const int reg = (ee >> 6) & 3;
-    const int mt = ee >> 8;
-    const int m = mt * 16 + ((l64 >> 4) << 2) + reg;
-    if (m < M) {
-      const int n = (n_group << 5) + (nt << 4) + (l64 & 15);
-      if (SPLITS == 1)
-        c[(size_t)m * N + n] = f2bf(v);
-      else
-        ws[((size_t)split * M + m) * N + n] = v;
+  for (int s = 0; s < DEPTH; ++s) {
+    if (at + s < n) {
+      __syncthreads();
+      SG_PUT(buf[(s + 1) & 1], ar);
+      if (at + s + 2 < n) SG_A(ar, at + s + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      SG_MATH(s, buf[s & 1]);
     }
+  }
+#undef SG_W
+#undef SG_A
+#undef SG_PUT
+#undef SG_MATH
+
+  // lane l, register q: row 4 * g + q of A's tile, column r of the wave's 16
+  if (GLU) {
+    float* meet = (float*)lds;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+      *reinterpret_cast<f32x4*>(&meet[(wave * MT + i) * 256 + lane * 4]) =
+          acc[i];
+    __syncthreads();
+    for (int e = tid; e < SIDE * MT * 256; e += THREADS) {
+      const int i = (e >> 8) % MT, side = (e >> 8) / MT;
+      const int m = i * 16 + ((e >> 6) & 3) * 4 + (e & 3);
+      const int col = (blockIdx.x * SIDE + side) * 16 + ((e >> 2) & 15);
+      if (m < M && col < half)
+        c[(size_t)m * half + col] =
+            f2bf(silu(meet[e]) * meet[e + SIDE * MT * 256]);
+    }
+  } else if (col0 < N) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int m = i * 16 + g * 4 + q;
+        if (m >= M) continue;
+        if (gridDim.y == 1)
+          c[(size_t)m * N + col0 + r] = f2bf(acc[i][q]);
+        else
+          ws[((size_t)blockIdx.y * M + m) * N + col0 + r] = acc[i][q];
+      }
   }
 }
 
 __global__ void reduce_splits_kernel(const float* __restrict__ ws,
                                      __hip_bfloat16* __restrict__ c,
                                      const int splits, const long mn) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= mn) return;
-  float v = 0.f;
-  for (int s = 0; s < splits; ++s) v += ws[(size_t)s * mn + i];
-  c[i] = f2bf(v);
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int s = 0; s < splits; ++s)
+    v += *reinterpret_cast<const f32x4*>(ws + (size_t)s * mn + i);
+  union { __hip_bfloat16 e[4]; uint2 u; } o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) o.e[j] = f2bf(v[j]);
+  *reinterpret_cast<uint2*>(c + i) = o.u;
 }
 
+template <int MT, int NW, bool GLU>
+void launch_tiles(__hip_bfloat16* c, float* ws, const __hip_bfloat16* a,
+                  const __hip_bfloat16* w, int M, int N, int K, int splits,
+                  hipStream_t stream) {
+  const int cols = NW * (GLU ? 8 : 16), out = GLU ? N / 2 : N;
+  skinny_gemm_kernel<MT, NW, GLU>
+      <<<dim3((out + cols - 1) / cols, splits), dim3(64 * NW), 0, stream>>>(
+          a, w, c, ws, M, N, K);
+}
+
+}  // namespace
+
 // ---------------------------------------------------------------------------
-// C launchers (torch glue lives in bindings.cpp)
+// C launchers (torch glue lives in gemm_bindings.h)
 
 extern "C" void launch_skinny_gemm(void* c, void* ws, const void* a,
                                    const void* w, int M, int N, int K,
-                                   int splits, hipStream_t stream) {
-  const dim3 grid((N >> 5) * splits), block(SG_NT);
+                                   int waves, int splits, int glu,
+                                   hipStream_t stream) {
   const __hip_bfloat16* ap = (const __hip_bfloat16*)a;
   const __hip_bfloat16* wp = (const __hip_bfloat16*)w;
   __hip_bfloat16* cp = (__hip_bfloat16*)c;
   float* wsp = (float*)ws;
-  const int m_tiles = (M + 15) >> 4;
-
-#define LAUNCH_MT(MT)                                                        \
-  do {                                                                       \
-    if (splits == 1)                                                         \
-      skinny_gemm_kernel<MT, 1><<<grid, block, 0, stream>>>(                 \
-          ap, wp, cp, nullptr, M, N, K);                                     \
-    else if (splits == 2)                                                    \
-      skinny_gemm_kernel<MT, 2><<<grid, block, 0, stream>>>(                 \
-          ap, wp, cp, wsp, M, N, K);                                         \
-    else if (splits == 4)                                                    \
-      skinny_gemm_kernel<MT, 4><<<grid, block, 0, stream>>>(                 \
-          ap, wp, cp, wsp, M, N, K);                                         \
-    else                                                                     \
-      skinny_gemm_kernel<MT, 8><<<grid, block, 0, stream>>>(                 \
-          ap, wp, cp, wsp, M, N, K);                                         \
+  const int mt = (M + 15) >> 4;
+#define SG_GO(MT, NW)                                                      \
+  do {                                                                     \
+    if (glu)                                                               \
+      launch_tiles<MT, NW, true>(cp, wsp, ap, wp, M, N, K, 1, stream);     \
+    else                                                                   \
+      launch_tiles<MT, NW, false>(cp, wsp, ap, wp, M, N, K, splits,        \
+                                  stream);                                 \
   } while (0)
-
-  if (m_tiles <= 1) LAUNCH_MT(1);
-  else if (m_tiles <= 2) LAUNCH_MT(2);
-  else if (m_tiles <= 4) LAUNCH_MT(4);
-  else if (m_tiles <= 8) LAUNCH_MT(8);
-  else LAUNCH_MT(16);
-#undef LAUNCH_MT
+  if (waves == 0) {             // the kernel of a few rows
+    if (glu)
+      skinny_rows_kernel<true><<<dim3(N / 16), dim3(512), 0, stream>>>(
+          ap, wp, cp, M, N, K);
+    else
+      skinny_rows_kernel<false><<<dim3(N / 16), dim3(512), 0, stream>>>(
+          ap, wp, cp, M, N, K);
+  } else if (mt <= 1 && waves == 4) SG_GO(1, 4);
+  else if (mt <= 2 && waves == 4) SG_GO(2, 4);
+  else if (mt <= 1) SG_GO(1, 8);
+  else if (mt <= 2) SG_GO(2, 8);
+  else if (mt <= 3) SG_GO(3, 8);
+  else if (mt <= 4) SG_GO(4, 8);
+  else if (mt <= 6) SG_GO(6, 8);
+  else if (mt <= 8) SG_GO(8, 8);
+  else if (mt <= 12)
+    launch_tiles<12, 8, false>(cp, wsp, ap, wp, M, N, K, splits, stream);
+  else
+    launch_tiles<16, 8, false>(cp, wsp, ap, wp, M, N, K, splits, stream);
+#undef SG_GO
 }
 
 extern "C" void launch_reduce_splits(void* c, const void* ws, int splits,
                                      long mn, hipStream_t stream) {
   const int threads = 256;
-  reduce_splits_kernel<<<dim3((mn + threads - 1) / threads), dim3(threads),
+  const long vecs = mn / 4;     // N is a multiple of 32
+  reduce_splits_kernel<<<dim3((vecs + threads - 1) / threads), dim3(threads),
                          0, stream>>>((const float*)ws, (__hip_bfloat16*)c,
                                       splits, mn);
 }

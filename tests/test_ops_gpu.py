@@ -391,3 +391,40 @@ def test_prefill_attention_32x32_with_prefix(dev, swz, monkeypatch):
     want = ref.prefill_attention(q, k, v, cu_q, scale, cu_k)
     err = (got.float() - want.float()).abs().max().item()
     assert err < 3e-2, err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 4, 5, 16, 17, 32, 33, 48, 49, 65, 97, 129,
+                               193, 256])
+@pytest.mark.parametrize("n,k", [(32, 256), (160, 768), (8224, 512),
+                                 (2048, 5632), (1312, 2048), (33024, 256)])
+def test_skinny_gemm_edges(m, n, k):
+    """Row tiles of every kernel, columns that leave waves idle, splits of
+    unequal length, fewer chunks of k than are in flight.  f32 sums of bf16
+    products, rounded once: half an ulp of the result (2^-9) and k roundings
+    of 2^-24 of the sums of magnitudes."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(m * 1000003 + n + k)
+    x = torch.randn(m, k, device=dev, generator=gen).bfloat16()
+    w = torch.randn(n, k, device=dev, generator=gen).bfloat16()
+    want = x.double() @ w.double().t().contiguous()
+    bound = want.abs() * 2 ** -8 + \
+        (x.double().abs() @ w.double().abs().t().contiguous()) * k * 2 ** -24
+    got = ops._hip.skinny_gemm(x, w).double()
+    assert ((got - want).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [0, 1, 128, 129])
+@pytest.mark.parametrize("n,k", [(6144, 2048), (12320, 2048), (64, 96)])
+def test_linear_any_shape(rows, n, k):
+    """Both routes of linear, no rows at all among them."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    x = torch.randn(rows, k, device=dev).bfloat16()
+    w = torch.randn(n, k, device=dev).bfloat16()
+    got = ops.linear(x, w)
+    want = x.float() @ w.float().t()
+    assert got.shape == want.shape
+    assert ((got.float() - want).abs() <= want.abs() * 2 ** -7 + 0.05).all()
