@@ -164,6 +164,18 @@ def pick_decode_splits(num_seqs: int, num_kv_heads: int,
     half the dot2 kernel's at equal splits."""
     if variant < 0:
         variant = DECODE_VARIANT
+    if variant == 7:
+        # parts of the table's capacity, whatever the lengths: few (sequence,
+        # head) pairs need short ones to fill the chip, many need long ones,
+        # which start less often (us, 256 / 512 / 1024 / 2048 keys: 8 pairs of
+        # 2048 9.8 / 13 / 16 / 24; 64 pairs of 2048 19.2 / 18.8 / 21 / 30; 128
+        # pairs of up to 2048 32 / 28 / 25 / 32; 1024 pairs of 2080 233 / 211
+        # / 186 / 179)
+        pairs = num_seqs * num_kv_heads
+        span = (max(256, max_context // 32) if pairs <= 32 else
+                max(512, max_context // 16) if pairs <= 96 else
+                max(1024, max_context // 8) if pairs <= 192 else 2048)
+        return max(1, (max_context + span - 1) // span)
     if variant >= 4:
         # v4/v5 pack 2 seqs per WG; v6 runs 1 seq per (2-wave) WG
         per_wg = 2 if variant in (4, 5) else 1
@@ -178,7 +190,7 @@ def pick_decode_splits(num_seqs: int, num_kv_heads: int,
     return int(min(want, by_ctx, 16))
 
 
-DECODE_VARIANT = int(__import__("os").environ.get("RBG_DECODE_VARIANT", "4"))  # MFMA page-pair decode: 5.6 TB/s vs 4.0 dot2 (B128, within-probe)
+DECODE_VARIANT = int(__import__("os").environ.get("RBG_DECODE_VARIANT", "7"))  # decode_pages.hip: 6.1 TB/s against 5.5 of 4 (128 x 2080)
 PREFILL_SWZ = int(__import__("os").environ.get("RBG_PREFILL_SWZ", "6"))  # 8-wave + K/V double-buffer (305 TF/s vs 252 @ swz=4, within-probe)
 
 
@@ -187,9 +199,13 @@ def decode_attention(q, key_cache, value_cache, block_tables, context_lens,
                      variant: int = -1) -> torch.Tensor:
     if _on_gpu(q):
         if num_splits <= 0:
-            max_ctx = int(context_lens.max().item()) if context_lens.numel() else 1
+            if (DECODE_VARIANT if variant < 0 else variant) == 7:
+                max_ctx = block_tables.shape[1] * key_cache.shape[2]
+            else:
+                max_ctx = (int(context_lens.max().item())
+                           if context_lens.numel() else 1)
             num_splits = pick_decode_splits(q.shape[0], key_cache.shape[1],
-                                            max_ctx)
+                                            max_ctx, variant)
         if variant < 0:
             variant = DECODE_VARIANT
         return _require_hip().decode_attention(

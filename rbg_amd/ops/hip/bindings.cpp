@@ -22,6 +22,9 @@ void launch_decode_attention(void*, void*, void*, const void*, const void*,
                              const void*, const void*, const void*, float,
                              int, int, int, int, int, int, int, int,
                              hipStream_t);
+void launch_decode_pages(void*, void*, void*, const void*, const void*,
+                         const void*, const void*, const void*, float, int,
+                         int, int, int, int, int, hipStream_t);
 void launch_prefill_attention(void*, const void*, const void*, const void*,
                               const void*, const void*, float, int, int, int,
                               int, int, int, hipStream_t);
@@ -155,6 +158,15 @@ torch::Tensor decode_attention(torch::Tensor q, torch::Tensor key_cache,
     partial_ml = torch::empty({num_splits, num_seqs, num_q_heads, 2}, opts);
     po = partial_o.data_ptr();
     pml = partial_ml.data_ptr();
+  }
+  if (wide == 7 && page_size == 16) {
+    launch_decode_pages(out.data_ptr(), po, pml, q.data_ptr(),
+                        key_cache.data_ptr(), value_cache.data_ptr(),
+                        block_tables.data_ptr(), context_lens.data_ptr(),
+                        (float)scale, num_seqs, num_q_heads, num_kv_heads,
+                        max_pages, (int)num_splits, (int)q.stride(0),
+                        current_stream());
+    return out;
   }
   launch_decode_attention(out.data_ptr(), po, pml, q.data_ptr(),
                           key_cache.data_ptr(), value_cache.data_ptr(),

@@ -1,0 +1,324 @@
+// Paged flash-decode over pages of 16 keys and head size 128: one query token
+// per sequence, all query heads of a key head in one pass.
+//
+// Bound: the keys and values, read once (a plain read reaches 6.1-6.3 TB/s).
+//  * A page of one key head is 4 KB in one piece.  Keys go from memory
+//    straight into MFMA registers as rows of S^T = K q^T, whose result holds
+//    8 keys of one head per lane: softmax needs two shuffles per 32 keys, and
+//    its weights are the operand of O^T = V^T P^T as they are, with keys
+//    4g..4g+3 of two pages in place of 8g..8g+7.  Only V passes LDS, private
+//    to its wave, to be read transposed: no barrier inside the walk.
+//  * The next 32 keys and values are in flight while these are used: 16 KB
+//    per wave.
+//  * Values, read in whole lines and once, are loaded non-temporally (219 ->
+//    198 us at 128 x 2080); keys, whose lines two loads share, are not.
+//  * Work is cut by keys, not by sequences: every workgroup takes at most
+//    `span` keys of one sequence, whatever the sequence's length, so a batch
+//    of ragged lengths fills the chip as a regular one does.  Workgroups past
+//    the end of their sequence leave at once.
+#include "common.h"
+
+namespace {
+
+constexpr int DIM = 128, PAGE = 16, WAVES = 4, STEP = 32;
+constexpr int VROW = 528;         // of a 16-dim column of 32 values: 512 + pad,
+                                  // so that writes of a row meet no conflicts
+constexpr float LOW = -1e30f;
+
+typedef __attribute__((ext_vector_type(4))) unsigned int dp_u4;
+
+DEV_INLINE dp_u4 dp_load(const __hip_bfloat16* p) {
+  return *reinterpret_cast<const dp_u4*>(p);
+}
+
+DEV_INLINE bf16x8 dp_frag(dp_u4 u) {
+  union { dp_u4 u; bf16x8 v; } c;
+  c.u = u;
+  return c.v;
+}
+
+// TOGETHER: all key heads of a (sequence, part) run on one XCD, workgroup i on
+// XCD i % 8, which then translates an eighth of the pool's addresses (128
+// sequences of 2080 tokens, 8 heads: 198 -> 179 us, 6.1 TB/s).  A small batch
+// of ragged lengths would leave XCDs idle (45 of up to 2500: 63 -> 68 us).
+template <int QPG, bool TOGETHER>
+__global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
+    float* __restrict__ part_o,             // [splits, seqs, QH, DIM]
+    float* __restrict__ part_ml,            // [splits, seqs, QH, 2]
+    __hip_bfloat16* __restrict__ out,       // [seqs, QH, DIM]
+    const __hip_bfloat16* __restrict__ q,   // [seqs, QH, DIM], rows q_stride
+    const __hip_bfloat16* __restrict__ keys,    // [pages, KVH, PAGE, DIM]
+    const __hip_bfloat16* __restrict__ values,
+    const int* __restrict__ tables,         // [seqs, max_pages]
+    const int* __restrict__ lens,           // [seqs]
+    const float scale,                      // to the base of 2
+    const int kv_heads, const int max_pages, const int span,
+    const int q_stride) {
+  int kvh = blockIdx.x, seq = blockIdx.y, split = blockIdx.z;
+  if (TOGETHER) {
+    const int lin = kvh + kv_heads * (seq + gridDim.y * split);
+    const int pairs = gridDim.y * gridDim.z, group = lin / (8 * kv_heads);
+    const int in = lin % (8 * kv_heads);
+    const bool whole = (group + 1) * 8 <= pairs;
+    const int pair = group * 8 + (whole ? in % 8 : in / kv_heads);
+    kvh = whole ? in / 8 : in % kv_heads;
+    seq = pair % gridDim.y;
+    split = pair / gridDim.y;
+  }
+  const int ctx = lens[seq];
+  const int begin = split * span, end = min(ctx, begin + span);
+  if (begin >= ctx && split > 0) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int heads = kv_heads * QPG;
+
+  __shared__ __align__(16) __hip_bfloat16 v_lds[WAVES][8 * VROW];
+  __shared__ float sums[WAVES][QPG][2];
+  static_assert(sizeof(v_lds) >= WAVES * QPG * DIM * 4, "merge fits");
+
+  // the heads' queries as columns (QPG of 16), 4 pieces of 32 dims
+  bf16x8 qf[4];
+  {
+    const __hip_bfloat16* qp = q + (size_t)seq * q_stride +
+                               (size_t)(kvh * QPG + min(c, QPG - 1)) * DIM;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) qf[d] = dp_frag(dp_load(qp + d * 32 + g * 8));
+  }
+  const int* table = tables + (size_t)seq * max_pages;
+  const int last_page = max(end - 1, 0) / PAGE;
+  const size_t head_at = (size_t)kvh * PAGE * DIM;
+  const size_t page_size = (size_t)kv_heads * PAGE * DIM;
+  const int k_at = c * DIM + g * 8;       // this lane's part of a page of keys
+  const int v_at = lane * 8;              // and of values, in 4 pieces of 1 KB
+  __hip_bfloat16* vl = v_lds[wave];
+  // piece j of a page: key 4j + g, dims 8c..; [dim / 16][page][key][dim % 16]
+  const int v_put = (c >> 1) * VROW + g * 16 + (c & 1) * 8;
+
+  f32x4 acc[8];
+  float m = LOW, l = 0.f;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) acc[t] = {0.f, 0.f, 0.f, 0.f};
+
+  dp_u4 kr[2][4], vr[2][4];
+#define DP_PAGE(at, p) table[min((at) / PAGE + (p), last_page)]
+#define DP_KEYS(page)                                                      \
+  _Pragma("unroll") for (int p = 0; p < 2; ++p) {                          \
+    const __hip_bfloat16* src = keys + head_at + k_at +                    \
+                                (size_t)page[p] * page_size;               \
+    _Pragma("unroll") for (int d = 0; d < 4; ++d)                          \
+        kr[p][d] = dp_load(src + d * 32);                                  \
+  }
+#define DP_VALUES(page)                                                    \
+  _Pragma("unroll") for (int p = 0; p < 2; ++p) {                          \
+    const __hip_bfloat16* src = values + head_at + v_at +                  \
+                                (size_t)page[p] * page_size;               \
+    _Pragma("unroll") for (int j = 0; j < 4; ++j)                          \
+        vr[p][j] = __builtin_nontemporal_load(                             \
+            reinterpret_cast<const dp_u4*>(src + j * 512));                \
+  }
+  int at = begin + wave * STEP;
+  int page[2];                    // of the next step, known one step ahead
+  if (at < end) {
+    page[0] = DP_PAGE(at, 0);
+    page[1] = DP_PAGE(at, 1);
+    DP_KEYS(page)
+    DP_VALUES(page)
+    page[0] = DP_PAGE(at + WAVES * STEP, 0);
+    page[1] = DP_PAGE(at + WAVES * STEP, 1);
+  }
+  for (; at < end; at += WAVES * STEP) {
+    const int later[2] = {DP_PAGE(at + 2 * WAVES * STEP, 0),
+                          DP_PAGE(at + 2 * WAVES * STEP, 1)};
+    f32x4 s[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      s[p] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+        s[p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dp_frag(kr[p][d]),
+                                                       qf[d], s[p], 0, 0, 0);
+    }
+    DP_KEYS(page)
+    __builtin_amdgcn_sched_barrier(0);
+
+    // lane: head c, keys at + 16 p + 4 g + r
+    float w[2][4], top = LOW;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        w[p][r] = at + p * PAGE + g * 4 + r < end ? s[p][r] * scale : LOW;
+        top = fmaxf(top, w[p][r]);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16, 64));
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    const float m_new = fmaxf(m, top);
+    const float fade = __builtin_amdgcn_exp2f(m - m_new);
+    m = m_new;
+    l *= fade;
+    union { __hip_bfloat16 e[8]; bf16x8 v; } pf;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = w[p][r] <= LOW
+                            ? 0.f : __builtin_amdgcn_exp2f(w[p][r] - m_new);
+        l += e;
+        pf.e[p * 4 + r] = f2bf(e);
+      }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[t] *= fade;
+
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<dp_u4*>(vl + v_put + p * 256 + j * 64) = vr[p][j];
+    DP_VALUES(page)
+    page[0] = later[0];
+    page[1] = later[1];
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const unsigned va = (unsigned)(unsigned long long)(vl + g * 64 + c * 4);
+    unsigned long long lo[8], hi[8];
+#define DP_READ(t, a, b, off0, off1)                                       \
+    "ds_read_b64_tr_b16 " a ", %16 offset:" off0 "\n\t"                    \
+    "ds_read_b64_tr_b16 " b ", %16 offset:" off1 "\n\t"
+    asm volatile(
+        DP_READ(0, "%0", "%1", "0", "512")
+        DP_READ(1, "%2", "%3", "1056", "1568")
+        DP_READ(2, "%4", "%5", "2112", "2624")
+        DP_READ(3, "%6", "%7", "3168", "3680")
+        DP_READ(4, "%8", "%9", "4224", "4736")
+        DP_READ(5, "%10", "%11", "5280", "5792")
+        DP_READ(6, "%12", "%13", "6336", "6848")
+        DP_READ(7, "%14", "%15", "7392", "7904")
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]),
+          "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]), "=&v"(hi[3]),
+          "=&v"(lo[4]), "=&v"(hi[4]), "=&v"(lo[5]), "=&v"(hi[5]),
+          "=&v"(lo[6]), "=&v"(hi[6]), "=&v"(lo[7]), "=&v"(hi[7])
+        : "v"(va)
+        : "memory");
+#undef DP_READ
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      union { unsigned long long u[2]; bf16x8 v; } vf;
+      vf.u[0] = lo[t];
+      vf.u[1] = hi[t];
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf.v, acc[t], 0,
+                                                       0, 0);
+    }
+  }
+#undef DP_PAGE
+#undef DP_KEYS
+#undef DP_VALUES
+
+  // the waves' sums meet in LDS; lane: head c, dims 16 t + 4 g + r
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  __syncthreads();
+  float* meet = reinterpret_cast<float*>(&v_lds[0][0]);
+  if (c < QPG) {
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      *reinterpret_cast<f32x4*>(
+          &meet[(wave * QPG + c) * DIM + t * 16 + g * 4]) = acc[t];
+    if (g == 0) {
+      sums[wave][c][0] = m;
+      sums[wave][c][1] = l;
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < QPG * DIM; e += 64 * WAVES) {
+    const int h = e / DIM, d = e % DIM;
+    float top = LOW;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) top = fmaxf(top, sums[w][h][0]);
+    float o = 0.f, total = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = __builtin_amdgcn_exp2f(sums[w][h][0] - top);
+      o += meet[(w * QPG + h) * DIM + d] * f;
+      total += sums[w][h][1] * f;
+    }
+    const size_t row = (size_t)seq * heads + kvh * QPG + h;
+    if (ctx <= span) {
+      out[row * DIM + d] = f2bf(total > 0.f ? o / total : 0.f);
+    } else {
+      const size_t at_row = (size_t)split * gridDim.y * heads + row;
+      part_o[at_row * DIM + d] = o;
+      if (d == 0) {
+        part_ml[at_row * 2] = top;
+        part_ml[at_row * 2 + 1] = total;
+      }
+    }
+  }
+}
+
+// Sequences of several workgroups: a workgroup per query head adds their sums.
+// Every load of a thread is independent of the others (one load after another
+// took 9-10 us for 16 splits of one sequence).
+__global__ __launch_bounds__(DIM) void decode_join_kernel(
+    __hip_bfloat16* __restrict__ out, const float* __restrict__ part_o,
+    const float* __restrict__ part_ml, const int* __restrict__ lens,
+    const int span, const int splits) {
+  const int seq = blockIdx.y, d = threadIdx.x;
+  const int ctx = lens[seq];
+  if (ctx <= span) return;
+  const int n = min((ctx + span - 1) / span, splits);
+  const size_t row = (size_t)seq * gridDim.x + blockIdx.x;
+  const size_t step = (size_t)gridDim.y * gridDim.x;
+  float top = LOW;
+#pragma unroll 8
+  for (int s = 0; s < n; ++s)
+    top = fmaxf(top, part_ml[(s * step + row) * 2]);
+  float o = 0.f, total = 0.f;
+#pragma unroll 8
+  for (int s = 0; s < n; ++s) {
+    const float f =
+        __builtin_amdgcn_exp2f(part_ml[(s * step + row) * 2] - top);
+    o += part_o[(s * step + row) * DIM + d] * f;
+    total += part_ml[(s * step + row) * 2 + 1] * f;
+  }
+  out[row * DIM + d] = f2bf(total > 0.f ? o / total : 0.f);
+}
+
+}  // namespace
+
+extern "C" void launch_decode_pages(
+    void* out, void* part_o, void* part_ml, const void* q, const void* keys,
+    const void* values, const void* tables, const void* lens, float scale,
+    int seqs, int heads, int kv_heads, int max_pages, int splits, int q_stride,
+    hipStream_t stream) {
+  // keys per workgroup: the table's capacity over the splits, in whole steps
+  const int steps = (max_pages * PAGE + WAVES * STEP - 1) / (WAVES * STEP);
+  const int span = max(1, (steps + splits - 1) / splits) * WAVES * STEP;
+  const dim3 grid(kv_heads, seqs, splits), block(64 * WAVES);
+#define DP_LAUNCH(QPG, TOGETHER)                                           \
+  decode_pages_kernel<QPG, TOGETHER><<<grid, block, 0, stream>>>(          \
+      (float*)part_o, (float*)part_ml, (__hip_bfloat16*)out,               \
+      (const __hip_bfloat16*)q, (const __hip_bfloat16*)keys,               \
+      (const __hip_bfloat16*)values, (const int*)tables, (const int*)lens, \
+      scale * 1.44269504088896f, kv_heads, max_pages, span, q_stride)
+#define DP_GO(QPG)                                                         \
+  do {                                                                     \
+    if (seqs >= 96) DP_LAUNCH(QPG, true);                                  \
+    else DP_LAUNCH(QPG, false);                                            \
+  } while (0)
+  switch (heads / kv_heads) {
+    case 1: DP_GO(1); break;
+    case 2: DP_GO(2); break;
+    case 4: DP_GO(4); break;
+    case 8: DP_GO(8); break;
+    default: return;        // refused by the caller
+  }
+#undef DP_LAUNCH
+#undef DP_GO
+  if (splits > 1)
+    decode_join_kernel<<<dim3(heads, seqs), dim3(DIM), 0, stream>>>(
+        (__hip_bfloat16*)out, (const float*)part_o, (const float*)part_ml,
+        (const int*)lens, span, splits);
+}

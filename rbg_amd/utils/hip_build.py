@@ -28,6 +28,7 @@ HIP_SOURCES = {
     # bf16 attention/norm/GEMM kernels, KV push, xGMI all-reduce
     "_hip_ops": [
         "attn_decode.hip",
+        "decode_pages.hip",
         "attn_prefill.hip",
         "mfma_probe.hip",
         "rmsnorm.hip",

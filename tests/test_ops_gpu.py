@@ -428,3 +428,57 @@ def test_linear_any_shape(rows, n, k):
     want = x.float() @ w.float().t()
     assert got.shape == want.shape
     assert ((got.float() - want).abs() <= want.abs() * 2 ** -7 + 0.05).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qpg,kvh,lens,splits", [
+    (4, 8, [1, 15, 16, 17, 31, 32, 33, 127, 128, 129, 2080], 1),
+    (1, 3, [1, 128, 129, 255, 257, 640], 5),
+    (8, 2, [700, 1, 500, 384, 385], 4),
+    (2, 1, [2048], 40),                     # more parts than steps
+    (4, 3, [1 + 37 * i % 300 for i in range(97)], 3),   # XCD groups, a rest
+    (4, 8, [2 + 29 * i % 200 for i in range(96)], 1),
+])
+def test_decode_pages(qpg, kvh, lens, splits):
+    """Parts of the table's capacity: ends inside a page, a step and a part,
+    empty parts, sequences of one part beside others of many; spread pages;
+    values far outside the softmax's weights; capture.  Weights are rounded to
+    bf16 (2^-9 of a weighted mean of |v|) and so is the result."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(len(lens) * 100 + splits)
+    pages = [(n + 15) // 16 for n in lens]
+    total = sum(pages) + 1
+    kc = torch.randn(total, kvh, 16, 128, device=dev, generator=gen).bfloat16()
+    vc = torch.randn(total, kvh, 16, 128, device=dev, generator=gen).bfloat16()
+    perm = (torch.randperm(total - 1, device=dev, generator=gen) + 1).int()
+    bt = torch.zeros(len(lens), max(pages) + 3, dtype=torch.int32, device=dev)
+    at = 0
+    for i, n in enumerate(pages):
+        bt[i, :n] = perm[at:at + n]
+        at += n
+    cl = torch.tensor(lens, dtype=torch.int32, device=dev)
+    fused = torch.randn(len(lens), (qpg + 2) * kvh * 128, device=dev,
+                        generator=gen).bfloat16()
+    q = fused[:, :qpg * kvh * 128].view(len(lens), qpg * kvh, 128)
+    def call():
+        return ops._hip.decode_attention(q, kc, vc, bt, cl, 0.4, splits, 7)
+    got = call().double()
+    for i, n in enumerate(lens):
+        rows = [t[bt[i, :pages[i]].long()].transpose(0, 1).reshape(
+            kvh, -1, 128)[:, :n].double() for t in (kc, vc)]
+        for h in range(kvh):
+            w = (q[i, h * qpg:(h + 1) * qpg].double() @
+                 rows[0][h].t().contiguous() * 0.4).softmax(-1)
+            want = w @ rows[1][h]
+            bound = want.abs() * 2 ** -8 + (w @ rows[1][h].abs()) * 2 ** -7
+            err = (got[i, h * qpg:(h + 1) * qpg] - want).abs()
+            assert (err <= bound + 1e-5).all(), (i, n, h)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = call()
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.double(), got)
