@@ -130,11 +130,13 @@ class PPContext:
 
 class LlamaAttention(nn.Module):
     def __init__(self, cfg: ModelConfig, layer_idx: int, tp: TPContext,
-                 device, dtype, gen):
+                 device, dtype, gen, parts: bool = False):
         super().__init__()
         self.cfg = cfg
         self.layer_idx = layer_idx
         self.tp = tp
+        # the next norm adds up what the output GEMM's parts left
+        self.parts = parts
         assert cfg.num_heads % tp.size == 0 and cfg.num_kv_heads % tp.size == 0, \
             "TP degree must divide head counts"
         self.heads = cfg.num_heads // tp.size
@@ -173,27 +175,19 @@ class LlamaAttention(nn.Module):
     def forward(self, x: torch.Tensor, batch: ForwardBatch,
                 kv: PagedKVCache, cos_sin: torch.Tensor) -> torch.Tensor:
         T = x.shape[0]
-        qkv = ops.linear(x, self.wqkv)
-        # q/k/v stay SLICES of the fused projection: the rope and attention
-        # kernels take a token-row stride, so no .contiguous() copies
-        # (~73 ms/bench of pure copy kernels before this)
+        key_cache = kv.key_cache(self.layer_idx)
+        value_cache = kv.value_cache(self.layer_idx)
+        # (Qwen: per-head norms,) RoPE and the paged KV write in one kernel,
+        # which also adds up what a split GEMM left
+        qkv = ops.rope_heads(
+            ops.linear_parts(x, self.wqkv), self.heads, self.q_norm,
+            self.k_norm, self.cfg.rms_eps, key_cache, value_cache, cos_sin,
+            batch.positions, batch.slot_mapping)
+        # q/k/v stay SLICES of the fused projection: the attention kernels
+        # take a token-row stride, so no .contiguous() copies
         q = qkv[:, :self.q_out]
         k = qkv[:, self.q_out:self.q_out + self.kv_out]
         v = qkv[:, self.q_out + self.kv_out:]
-        if self.q_norm is not None:
-            # qwen per-head norm reshapes across rows: materialize
-            q = ops.rmsnorm(q.contiguous().view(-1, self.head_dim),
-                            self.q_norm,
-                            self.cfg.rms_eps).view(T, self.q_out)
-            k = ops.rmsnorm(k.contiguous().view(-1, self.head_dim),
-                            self.k_norm,
-                            self.cfg.rms_eps).view(T, self.kv_out)
-            v = v.contiguous()
-        key_cache = kv.key_cache(self.layer_idx)
-        value_cache = kv.value_cache(self.layer_idx)
-        # fused RoPE + paged KV write (q,k rotated in place)
-        ops.rope_store_kv(q, k, v, key_cache, value_cache, cos_sin,
-                          batch.positions, batch.slot_mapping)
         q3 = q.view(T, self.heads, self.head_dim)
         if batch.mode == "prefill":
             if batch.kv_gather_slots is not None:
@@ -215,14 +209,18 @@ class LlamaAttention(nn.Module):
                                      batch.block_tables, batch.context_lens,
                                      self.scale,
                                      num_splits=batch.decode_num_splits)
-        out = ops.linear(o.view(T, self.q_out).contiguous(), self.wo)
-        return self.tp.all_reduce(out)
+        o = o.view(T, self.q_out).contiguous()
+        if self.parts:
+            return ops.linear_parts(o, self.wo)
+        return self.tp.all_reduce(ops.linear(o, self.wo))
 
 
 class LlamaMLP(nn.Module):
-    def __init__(self, cfg: ModelConfig, tp: TPContext, device, dtype, gen):
+    def __init__(self, cfg: ModelConfig, tp: TPContext, device, dtype, gen,
+                 parts: bool = False):
         super().__init__()
         self.tp = tp
+        self.parts = parts
         assert cfg.intermediate_size % tp.size == 0
         inter = cfg.intermediate_size // tp.size
         wg = _linear_weight(cfg.intermediate_size, cfg.hidden_size, device,
@@ -239,19 +237,21 @@ class LlamaMLP(nn.Module):
         self.inter = inter
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        gu = ops.linear(x, self.w_gate_up)
-        h = ops.silu_mul(gu)
+        h = ops.linear_swiglu(x, self.w_gate_up)
+        if self.parts:
+            return ops.linear_parts(h, self.w_down)
         return self.tp.all_reduce(ops.linear(h, self.w_down))
 
 
 class LlamaLayer(nn.Module):
     def __init__(self, cfg: ModelConfig, layer_idx: int, tp: TPContext,
-                 device, dtype, gen):
+                 device, dtype, gen, parts: bool = False):
         super().__init__()
         # layer_idx here is the KV-cache index LOCAL to this PP stage; the
         # weight generator is already seeded by the GLOBAL layer index
-        self.attn = LlamaAttention(cfg, layer_idx, tp, device, dtype, gen)
-        self.mlp = LlamaMLP(cfg, tp, device, dtype, gen)
+        self.attn = LlamaAttention(cfg, layer_idx, tp, device, dtype, gen,
+                                   parts)
+        self.mlp = LlamaMLP(cfg, tp, device, dtype, gen, parts)
         self.input_norm = nn.Parameter(
             torch.ones(cfg.hidden_size, device=device, dtype=dtype),
             requires_grad=False)
@@ -268,10 +268,9 @@ class LlamaLayer(nn.Module):
             h = ops.rmsnorm(x, self.input_norm, self.eps)
         else:
             # h := rmsnorm(x + residual); residual := x + residual  (fused)
-            ops.fused_add_rmsnorm(x, residual, self.input_norm, self.eps)
-            h = x
+            h = ops.add_rmsnorm(x, residual, self.input_norm, self.eps)
         h = self.attn(h, batch, kv, cos_sin)
-        ops.fused_add_rmsnorm(h, residual, self.post_norm, self.eps)
+        h = ops.add_rmsnorm(h, residual, self.post_norm, self.eps)
         h = self.mlp(h)
         return h, residual
 
@@ -316,8 +315,10 @@ class LlamaForCausalLM(nn.Module):
                             dtype=dtype).normal_(0, 0.02, generator=_gen(0)),
                 requires_grad=False)
         self.layers = nn.ModuleList([
+            # ranks and stages exchange whole rows: no parts between kernels
             LlamaLayer(cfg, i - self.layer_start, self.tp, device, dtype,
-                       _gen(1 + i))
+                       _gen(1 + i),
+                       parts=self.tp.size == 1 and self.pp.size == 1)
             for i in range(self.layer_start, self.layer_end)])
         self.final_norm = None
         self.lm_head = None
@@ -363,11 +364,9 @@ class LlamaForCausalLM(nn.Module):
         residual = None
         for layer in self.layers:
             x, residual = layer(x, residual, batch, kv, self.cos_sin)
-        x = x + residual
         if not self.pp.last:
-            return x
-        x = ops.rmsnorm(x, self.final_norm, self.cfg.rms_eps)
-        return x
+            return x + residual
+        return ops.add_rmsnorm(x, residual, self.final_norm, self.cfg.rms_eps)
 
     @torch.inference_mode()
     def logits(self, hidden: torch.Tensor,

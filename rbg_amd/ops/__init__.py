@@ -115,14 +115,40 @@ def _skinny(rows: int, n: int, k: int) -> bool:
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """Projection GEMM: decode shapes take the hand-written kernel,
     prefill-sized ones the library."""
-    if (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and
-            x.dtype == torch.bfloat16 and
-            _skinny(x.shape[0], w.shape[0], x.shape[1])):
+    if _takes_skinny(x, w):
         # one of these is there whatever the model
         return require("_hip_ops", "_hip_mix", "_hip_gated", "_hip_moe",
                        "_hip_hyper").skinny_gemm(
             x if x.is_contiguous() else x.contiguous(), w)
     return torch.nn.functional.linear(x, w)
+
+
+def _takes_skinny(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and
+            x.dtype == torch.bfloat16 and
+            _skinny(x.shape[0], w.shape[0], x.shape[1]))
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """linear for a reader that adds up: where the GEMM splits k, the f32 sums
+    [parts, T, N] before their reduction, else [T, N] in x's dtype."""
+    if _takes_skinny(x, w):
+        return _require_hip().skinny_parts(
+            x if x.is_contiguous() else x.contiguous(), w)
+    return torch.nn.functional.linear(x, w)
+
+
+def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x Wg^T) * (x Wu^T), w = [Wg; Wu]."""
+    # In the GEMM up to 64 rows of a wide matrix (28672 x 4096: 64 rows 47 us
+    # against 49 of the library and 5 of silu_mul; 128 rows 61 against 58) and
+    # 32 of a narrow one (11264 x 2048: 14 against 15 and 3.5), where the
+    # workgroups of an unsplit k fill the chip
+    if (_takes_skinny(x, w) and w.shape[0] % 64 == 0 and
+            x.shape[0] <= (64 if w.shape[0] > 12288 else 32)):
+        return _require_hip().skinny_swiglu(
+            x if x.is_contiguous() else x.contiguous(), w)
+    return silu_mul(linear(x, w))
 
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
@@ -139,6 +165,21 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor,
     reference.fused_add_rmsnorm(x, residual, weight, eps)
 
 
+def add_rmsnorm(x: torch.Tensor, residual: torch.Tensor,
+                weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """residual += x (in place); returns its RMS norm, perhaps in x.  x may be
+    linear_parts' sums."""
+    if _on_gpu(x):
+        # a workgroup per row with the row in registers: of many rows only few
+        # run at a time (4096 wide: 256 rows 3.4 us against 3.5 of the other, 1024
+        # rows 7.1 against 5.9)
+        if x.dtype == torch.float32 or (
+                x.shape[0] <= 256 and x.shape[-1] <= 16384):
+            return _require_hip().add_rmsnorm(x, residual, weight, eps)
+    fused_add_rmsnorm(x, residual, weight, eps)
+    return x
+
+
 def silu_mul(x: torch.Tensor) -> torch.Tensor:
     if _on_gpu(x):
         return _require_hip().silu_mul(x)
@@ -153,6 +194,28 @@ def rope_store_kv(q, k, v, key_cache, value_cache, cos_sin, positions,
         return
     reference.rope_store_kv(q, k, v, key_cache, value_cache, cos_sin,
                             positions, slot_mapping)
+
+
+def rope_heads(proj, heads: int, q_norm, k_norm, eps: float, key_cache,
+               value_cache, cos_sin, positions, slot_mapping) -> torch.Tensor:
+    """rope_store_kv of a fused projection [T, q | k | v] (in place) or of
+    linear_parts' sums, with RMS norms of the query and key heads before it
+    (None: without); returns the projection in bf16."""
+    dim, kvh = key_cache.shape[3], key_cache.shape[1]
+    if _on_gpu(proj) and dim == 128 and proj.is_contiguous():
+        return _require_hip().rope_heads(
+            proj, heads, q_norm, k_norm, eps, key_cache, value_cache, cos_sin,
+            positions, slot_mapping)
+    if proj.dim() == 3:
+        proj = proj.sum(0).to(key_cache.dtype)
+    q, k, v = proj.split([heads * dim, kvh * dim, kvh * dim], dim=1)
+    if q_norm is not None:
+        for part, w in ((q, q_norm), (k, k_norm)):
+            part.copy_(rmsnorm(part.reshape(-1, dim), w,
+                               eps).view(part.shape))
+    rope_store_kv(q, k, v, key_cache, value_cache, cos_sin, positions,
+                  slot_mapping)
+    return proj
 
 
 def pick_decode_splits(num_seqs: int, num_kv_heads: int,

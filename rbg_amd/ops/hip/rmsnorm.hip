@@ -75,9 +75,92 @@ __global__ void rmsnorm_kernel(__hip_bfloat16* __restrict__ out,      // [T,H]
   }
 }
 
+// residual += src; returns its RMS norm: for decode batches.  src is a row of
+// bf16, or (PARTS) the f32 sums that the parts of a split GEMM left, [parts,
+// rows, hidden], whose own reduction launch this replaces (2 us or more).
+// Bound by latency: a row is one workgroup, so it has as many threads as the
+// row has 8-byte pieces and every load of a thread is independent; the sums
+// stay in registers between the passes (4096 wide, 128 rows: 3.2 us of the
+// kernel above, 3.0 of this one, 4.1 from 8 parts).
+template <bool PARTS>
+__global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(
+    __hip_bfloat16* __restrict__ out, const void* __restrict__ src,
+    __hip_bfloat16* __restrict__ residual,
+    const __hip_bfloat16* __restrict__ w, const float eps, const int parts,
+    const int rows, const int hidden) {
+  constexpr int MOST = 4;         // pieces of 4 per thread: hidden <= 16384
+  const int row = blockIdx.x, tid = threadIdx.x, threads = blockDim.x;
+  const size_t at = (size_t)row * hidden;
+  __shared__ float red[16];
+  union B4 { uint2 u; __hip_bfloat16 e[4]; };
+  B4 sum[MOST];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < MOST; ++i) {
+    const int col = (i * threads + tid) * 4;
+    if (col < hidden) {
+      B4 r;
+      r.u = *reinterpret_cast<const uint2*>(residual + at + col);
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+      if (PARTS) {
+        const float* p = (const float*)src + at + col;
+#pragma unroll 8
+        for (int s = 0; s < parts; ++s)
+          v += *reinterpret_cast<const f32x4*>(p + (size_t)s * rows * hidden);
+      } else {
+        B4 x;
+        x.u = *reinterpret_cast<const uint2*>(
+            (const __hip_bfloat16*)src + at + col);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = bf2f(x.e[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float t = v[j] + bf2f(r.e[j]);
+        sum[i].e[j] = f2bf(t);
+        ss += t * t;
+      }
+      *reinterpret_cast<uint2*>(residual + at + col) = sum[i].u;
+    }
+  }
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  float total = 0.f;
+  for (int k = 0; k < threads >> 6; ++k) total += red[k];
+  const float inv = rsqrtf(total / hidden + eps);
+#pragma unroll
+  for (int i = 0; i < MOST; ++i) {
+    const int col = (i * threads + tid) * 4;
+    if (col < hidden) {
+      B4 g, o;
+      g.u = *reinterpret_cast<const uint2*>(w + col);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        o.e[j] = f2bf(bf2f(sum[i].e[j]) * inv * bf2f(g.e[j]));
+      *reinterpret_cast<uint2*>(out + at + col) = o.u;
+    }
+  }
+}
+
 }  // namespace
 
 extern "C" {
+
+// parts == 0: src is bf16
+void launch_add_rmsnorm_rows(void* out, const void* src, void* residual,
+                             const void* weight, float eps, int parts,
+                             int rows, int hidden, hipStream_t stream) {
+  const int threads = min(1024, (hidden / 4 + 63) / 64 * 64);
+  if (parts)
+    add_rmsnorm_row_kernel<true><<<dim3(rows), dim3(threads), 0, stream>>>(
+        (__hip_bfloat16*)out, src, (__hip_bfloat16*)residual,
+        (const __hip_bfloat16*)weight, eps, parts, rows, hidden);
+  else
+    add_rmsnorm_row_kernel<false><<<dim3(rows), dim3(threads), 0, stream>>>(
+        (__hip_bfloat16*)out, src, (__hip_bfloat16*)residual,
+        (const __hip_bfloat16*)weight, eps, parts, rows, hidden);
+}
 
 void launch_rmsnorm(void* out, void* input, const void* weight, float eps,
                     int tokens, int hidden, hipStream_t stream) {

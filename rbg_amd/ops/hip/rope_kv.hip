@@ -85,9 +85,147 @@ __global__ void rope_store_kv_kernel(
   }
 }
 
+// Heads of 128 from a fused projection [T, q heads | k heads | v heads]: norm
+// of every query and key head (NORM), rotation, paged store.  The projection
+// is bf16, changed in place, or (PARTS) the f32 sums that the parts of a split
+// GEMM left, [parts, T, width], whose result in bf16 goes to `qkv`: neither a
+// reduction nor copies and norms of the slices are launches of their own.
+// Eight lanes hold a head, each 8 neighbouring dims and the 8 they rotate
+// with: 16-byte accesses, and a norm is three shuffles.
+template <bool PARTS, bool NORM>
+__global__ __launch_bounds__(256) void rope_heads_kernel(
+    __hip_bfloat16* __restrict__ q, __hip_bfloat16* __restrict__ k,
+    __hip_bfloat16* __restrict__ v, const float* __restrict__ sums,
+    const int parts, const __hip_bfloat16* __restrict__ q_norm,
+    const __hip_bfloat16* __restrict__ k_norm, const float eps,
+    __hip_bfloat16* __restrict__ key_cache,  // [pages, KVH, page, 128]
+    __hip_bfloat16* __restrict__ val_cache,
+    const float* __restrict__ cos_sin,       // [positions, 128] = cos | sin
+    const int* __restrict__ positions, const int* __restrict__ slot_mapping,
+    const int tokens, const int num_q_heads, const int num_kv_heads,
+    const int page_size, const int q_stride, const int kv_stride) {
+  constexpr int D = 128;
+  const int heads = num_q_heads + 2 * num_kv_heads;
+  const int unit = blockIdx.x * 32 + (threadIdx.x >> 3);
+  const int lane = threadIdx.x & 7;
+  const bool live = unit < tokens * heads;      // shuffles need every lane
+  const int token = live ? unit / heads : tokens - 1;
+  const int head = live ? unit % heads : heads - 1;
+  const bool is_q = head < num_q_heads;
+  const bool is_v = head >= num_q_heads + num_kv_heads;
+  const int kvh = head - num_q_heads - (is_v ? num_kv_heads : 0);
+  __hip_bfloat16* row =
+      is_q ? q + (size_t)token * q_stride + head * D
+           : (is_v ? v : k) + (size_t)token * kv_stride + kvh * D;
+  const int d = lane * 8;
+  float x[2][8];
+  if (PARTS) {
+    const float* p = sums + ((size_t)token * heads + head) * D + d;
+    const size_t step = (size_t)tokens * heads * D;
+    f32x4 t[2][2] = {};
+#pragma unroll 8
+    for (int s = 0; s < parts; ++s)
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+        t[h >> 1][h & 1] += *reinterpret_cast<const f32x4*>(
+            p + s * step + (h >> 1) * 64 + (h & 1) * 4);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[h][j] = t[h][j >> 2][j & 3];
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      Bf16x8U u;
+      u.u = *reinterpret_cast<const uint4*>(row + h * 64 + d);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[h][j] = bf2f(u.e[j]);
+    }
+  }
+  if (NORM) {
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss += x[0][j] * x[0][j] + x[1][j] * x[1][j];
+#pragma unroll
+    for (int off = 4; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    if (!is_v) {
+      const float inv = rsqrtf(ss / D + eps);
+      const __hip_bfloat16* w = is_q ? q_norm : k_norm;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        Bf16x8U u;
+        u.u = *reinterpret_cast<const uint4*>(w + h * 64 + d);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[h][j] *= inv * bf2f(u.e[j]);
+      }
+    }
+  }
+  Bf16x8U o[2];
+  if (!is_v) {
+    const float* cs = cos_sin + (size_t)positions[token] * D + d;
+    float co[8], si[8];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      *reinterpret_cast<f32x4*>(co + j * 4) =
+          *reinterpret_cast<const f32x4*>(cs + j * 4);
+      *reinterpret_cast<f32x4*>(si + j * 4) =
+          *reinterpret_cast<const f32x4*>(cs + 64 + j * 4);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      o[0].e[j] = f2bf(x[0][j] * co[j] - x[1][j] * si[j]);
+      o[1].e[j] = f2bf(x[1][j] * co[j] + x[0][j] * si[j]);
+    }
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[h].e[j] = f2bf(x[h][j]);
+  }
+  if (!live) return;
+  if (PARTS || !is_v) {
+    *reinterpret_cast<uint4*>(row + d) = o[0].u;
+    *reinterpret_cast<uint4*>(row + 64 + d) = o[1].u;
+  }
+  const int slot = slot_mapping[token];
+  if (!is_q && slot >= 0) {
+    __hip_bfloat16* dst =
+        (is_v ? val_cache : key_cache) +
+        (((size_t)(slot / page_size) * num_kv_heads + kvh) * page_size +
+         slot % page_size) * D + d;
+    *reinterpret_cast<uint4*>(dst) = o[0].u;
+    *reinterpret_cast<uint4*>(dst + 64) = o[1].u;
+  }
+}
+
 }  // namespace
 
 extern "C" {
+
+// parts == 0: q, k, v are bf16 and changed in place; q_norm may be null
+void launch_rope_heads(void* q, void* k, void* v, const void* sums, int parts,
+                       const void* q_norm, const void* k_norm, float eps,
+                       void* key_cache, void* val_cache, const void* cos_sin,
+                       const void* positions, const void* slot_mapping,
+                       int tokens, int num_q_heads, int num_kv_heads,
+                       int page_size, int q_stride, int kv_stride,
+                       hipStream_t stream) {
+  const int units = tokens * (num_q_heads + 2 * num_kv_heads);
+  const dim3 grid((units + 31) / 32), block(256);
+#define RH_GO(PARTS, NORM)                                                  \
+  rope_heads_kernel<PARTS, NORM><<<grid, block, 0, stream>>>(               \
+      (__hip_bfloat16*)q, (__hip_bfloat16*)k, (__hip_bfloat16*)v,           \
+      (const float*)sums, parts, (const __hip_bfloat16*)q_norm,             \
+      (const __hip_bfloat16*)k_norm, eps, (__hip_bfloat16*)key_cache,       \
+      (__hip_bfloat16*)val_cache, (const float*)cos_sin,                    \
+      (const int*)positions, (const int*)slot_mapping, tokens, num_q_heads, \
+      num_kv_heads, page_size, q_stride, kv_stride)
+  if (parts && q_norm) RH_GO(true, true);
+  else if (parts) RH_GO(true, false);
+  else if (q_norm) RH_GO(false, true);
+  else RH_GO(false, false);
+#undef RH_GO
+}
 
 void launch_rope_store_kv(void* q, void* k, const void* v, void* key_cache,
                           void* val_cache, const void* cos_sin,

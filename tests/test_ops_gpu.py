@@ -482,3 +482,97 @@ def test_decode_pages(qpg, kvh, lens, splits):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out.double(), got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [0, 1, 5, 16])
+@pytest.mark.parametrize("rows,hidden", [(1, 4096), (7, 256), (3, 20),
+                                         (130, 5120), (2, 16384)])
+def test_add_rmsnorm_rows(parts, rows, hidden):
+    """Both sources, rows that leave threads idle.  The residual is one
+    rounding of the sum, the result another two (2^-8 each, generously)."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(rows * hidden + parts)
+    def rnd(*shape):
+        return torch.randn(*shape, device=dev, generator=gen)
+    x = rnd(parts, rows, hidden) if parts else rnd(rows, hidden).bfloat16()
+    res, w = rnd(rows, hidden).bfloat16(), rnd(hidden).bfloat16()
+    total = (x.double().sum(0) if parts else x.double()) + res.double()
+    want = total * torch.rsqrt(total.square().mean(-1, keepdim=True) + 1e-5) \
+        * w.double()
+    got = ops._hip.add_rmsnorm(x, res, w, 1e-5)
+    assert ((res.double() - total).abs() <= total.abs() * 2 ** -8 +
+            1e-5).all()
+    assert ((got.double() - want).abs() <= want.abs() * 2 ** -7 + 1e-5).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [0, 1, 6])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("tokens,heads,kvh", [(1, 2, 1), (5, 32, 8),
+                                              (37, 6, 3)])
+def test_rope_heads(parts, norm, tokens, heads, kvh):
+    """Head norms, rotation and store from bf16 rows (in place) and from the
+    sums of a split GEMM, with a skipped slot; one rounding of the result."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(tokens * 100 + parts)
+    def rnd(*shape):
+        return torch.randn(*shape, device=dev, generator=gen)
+    width, pages = (heads + 2 * kvh) * 128, 4
+    proj = (rnd(parts, tokens, width) if parts
+            else rnd(tokens, width).bfloat16())
+    x = (proj.double().sum(0) if parts else proj.double()).view(
+        tokens, heads + 2 * kvh, 128)
+    norms = [rnd(128).bfloat16() for _ in range(2)] if norm else [None, None]
+    table = ref.build_cos_sin_table(128, 512, device=dev)
+    pos = torch.randint(0, 512, (tokens,), device=dev, generator=gen).int()
+    slots = torch.randperm(pages * 16, device=dev,
+                           generator=gen)[:tokens].int()
+    if tokens > 1:
+        slots[1] = -1
+    kc = torch.zeros(pages, kvh, 16, 128, dtype=torch.bfloat16, device=dev)
+    vc = torch.zeros_like(kc)
+    want = x.clone()
+    for part, w in zip((want[:, :heads], want[:, heads:heads + kvh]), norms):
+        if norm:
+            part *= torch.rsqrt(part.square().mean(-1, keepdim=True) +
+                                1e-6) * w.double()
+        cs = table[pos.long()].double()[:, None]
+        a, b = part[..., :64].clone(), part[..., 64:].clone()
+        part[..., :64] = a * cs[..., :64] - b * cs[..., 64:]
+        part[..., 64:] = b * cs[..., :64] + a * cs[..., 64:]
+    got = ops.rope_heads(proj, heads, *norms, 1e-6, kc, vc, table, pos, slots)
+    assert got.dtype == torch.bfloat16
+    bound = want.abs() * 2 ** -8 + 2e-5
+    assert ((got.double().view_as(want) - want).abs() <= bound).all()
+    for cache, at in ((kc, heads), (vc, heads + kvh)):
+        held = torch.zeros_like(cache)
+        for t, s in enumerate(slots.tolist()):
+            if s >= 0:
+                held[s // 16, :, s % 16] = got.view(
+                    tokens, -1, 128)[t, at:at + kvh]
+        assert torch.equal(cache, held)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 4, 5, 17, 33, 64, 65])
+@pytest.mark.parametrize("f,k", [(32, 512), (5632, 2048), (8224, 2048)])
+def test_linear_swiglu(m, f, k):
+    """Gate and up tiles of every kernel, columns that leave waves idle; error
+    of the f32 sums through silu and one rounding (the separate kernels round
+    gate and up as well)."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(m * 7 + f)
+    x = torch.randn(m, k, device=dev, generator=gen).bfloat16()
+    w = (torch.randn(2 * f, k, device=dev, generator=gen) / k ** 0.5
+         ).bfloat16()
+    full = x.double() @ w.double().t().contiguous()
+    want = torch.nn.functional.silu(full[:, :f]) * full[:, f:]
+    bound = 2 ** -7 * (full[:, :f].abs() + 1) * (full[:, f:].abs() + 1)
+    for got in (ops._hip.skinny_swiglu(x, w), ops.linear_swiglu(x, w)):
+        assert ((got.double() - want).abs() <= bound).all()
+    got = ops._hip.skinny_swiglu(x, w).double()
+    assert (got - want).norm() <= 2 ** -8 * want.norm()
