@@ -7,7 +7,7 @@ and distinct window, not once per layer.
 """
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 from typing import Dict, List, Optional
 
 import numpy as np
@@ -38,6 +38,23 @@ class ForwardBatch:
     cu_prefill: Optional[torch.Tensor] = None   # cu_seqlens after those rows
     num_decode: int = 0             # leading one-token sequences with a past
     layout: Optional["VarlenLayout"] = None
+    # cu_seqlens and cu_seqlens_k (None: the same) on the host
+    cu_host: Optional[List[int]] = None
+    cu_k_host: Optional[List[int]] = None
+    _plans: Dict = field(default_factory=dict)
+
+    def prefill_plan(self, heads: int, kv_heads: int):
+        """The prompt attention's workgroups, once for all layers; None where
+        cu_seqlens are on the device only."""
+        if self.cu_host is None:
+            return None
+        key = (heads, kv_heads)
+        if key not in self._plans:
+            from ..ops import prefill_plan
+            self._plans[key] = prefill_plan(
+                self.cu_host, self.cu_k_host or self.cu_host, heads, kv_heads,
+                self.positions.device)
+        return self._plans[key]
 
 
 @dataclass

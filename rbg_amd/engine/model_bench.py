@@ -247,11 +247,10 @@ def run_kernels(size: str, batches=(1, 8, 32, 128), ctx: int = 2048,
         q, k, v, g.flatten(1), act, view, 0.05, window))
     out.append(_row(f"window_attention {tag}", us, T * heads * 128 * 10,
                     bf16=pairs * heads * 4 * 128))
-    bi, sl = ops.reference.prefill_block_info(cu.cpu(), qtile=128)
-    bi, sl = bi.to(dev), sl.to(dev)
+    plan = ops.prefill_plan(cu.tolist(), cu.tolist(), heads, kvh, dev)
     kk, vv = k[:, :kvh].contiguous(), v[:, :kvh].contiguous()
-    us = _time(lambda i: ops._require_hip().prefill_attention(
-        q, kk, vv, bi, sl, 0.05, ops.PREFILL_SWZ))
+    us = _time(lambda i: ops.prefill_attention(q, kk, vv, cu, 0.05,
+                                               plan=plan))
     out.append(_row(f"llama prefill_attention {tag}", us, T * heads * 128 * 6,
                     bf16=prompts * ctx * (ctx + 1) // 2 * heads * 4 * 128))
     proj, z, o = rnd(T, hd * 5 + 64), rnd(T, hd), rnd(T, hd)

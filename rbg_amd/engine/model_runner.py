@@ -106,7 +106,7 @@ class ModelRunner:
             mode="prefill",
             positions=self._join(positions),
             slot_mapping=self._join(slots),
-            cu_seqlens=self._i32(cu))
+            cu_seqlens=self._i32(cu), cu_host=cu)
         if self.model.needs_prev:
             batch.prev_tokens = self._join(prev)
         if self.model.varlen:
@@ -123,6 +123,7 @@ class ModelRunner:
                 batch.context_lens = self._i32(ends[:num_decode])
         elif any_past:
             batch.cu_seqlens_k = self._i32(cu_k)
+            batch.cu_k_host = cu_k
             batch.kv_gather_slots = self._join(gather)
         # decode inputs that were left on the device are behind now
         self._dstate = None

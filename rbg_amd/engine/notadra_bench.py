@@ -177,11 +177,9 @@ def notadra_kernels(size: str, batches=(1, 8, 32, 128), ctx: int = 2048,
     out.append(_row(f"paged_prefill {tag}", us, T * (2 * qn + 2 * kn) * 2,
                     bf16=flops))
     cu = i32([i * ctx for i in range(prompts + 1)])
-    bi, sl = ops.reference.prefill_block_info(cu.cpu(), qtile=128)
-    bi, sl = bi.to(dev), sl.to(dev)
+    plan = ops.prefill_plan(cu.tolist(), cu.tolist(), q.shape[1], kvh, dev)
     k, v = rnd(T, kvh, DIM), rnd(T, kvh, DIM)
-    us = _time(lambda i: ops._require_hip().prefill_attention(
-        q, k, v, bi, sl, 0.05, ops.PREFILL_SWZ))
+    us = _time(lambda i: ops.prefill_attention(q, k, v, cu, 0.05, plan=plan))
     out.append(_row(f"llama prefill_attention {tag}", us,
                     T * (2 * qn + 2 * kn) * 2, bf16=flops))
     both(T, tag)

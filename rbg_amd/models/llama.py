@@ -190,20 +190,19 @@ class LlamaAttention(nn.Module):
         v = qkv[:, self.q_out + self.kv_out:]
         q3 = q.view(T, self.heads, self.head_dim)
         if batch.mode == "prefill":
+            plan = None
+            if q3.is_cuda:
+                plan = batch.prefill_plan(self.heads, self.kv_heads)
             if batch.kv_gather_slots is not None:
-                ps = key_cache.shape[2]
-                slots = batch.kv_gather_slots.long()
-                pages, offs = slots // ps, slots % ps
-                k_full = key_cache[pages, :, offs]
-                v_full = value_cache[pages, :, offs]
-                o = ops.prefill_attention(q3, k_full, v_full,
-                                          batch.cu_seqlens, self.scale,
-                                          batch.cu_seqlens_k)
+                # behind a past: all rows, the new ones too, from the pages
+                o = ops.prefill_attention(
+                    q3, key_cache, value_cache, batch.cu_seqlens, self.scale,
+                    batch.cu_seqlens_k, plan, batch.kv_gather_slots)
             else:
                 o = ops.prefill_attention(
                     q3, k.view(T, self.kv_heads, self.head_dim),
                     v.view(T, self.kv_heads, self.head_dim),
-                    batch.cu_seqlens, self.scale)
+                    batch.cu_seqlens, self.scale, plan=plan)
         else:
             o = ops.decode_attention(q3, key_cache, value_cache,
                                      batch.block_tables, batch.context_lens,

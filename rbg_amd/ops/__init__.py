@@ -12,6 +12,7 @@ import importlib
 from dataclasses import dataclass
 from typing import Any, Dict, Optional
 
+import numpy as np
 import torch
 
 from ..utils import hip_build
@@ -254,7 +255,7 @@ def pick_decode_splits(num_seqs: int, num_kv_heads: int,
 
 
 DECODE_VARIANT = int(__import__("os").environ.get("RBG_DECODE_VARIANT", "7"))  # decode_pages.hip: 6.1 TB/s against 5.5 of 4 (128 x 2080)
-PREFILL_SWZ = int(__import__("os").environ.get("RBG_PREFILL_SWZ", "6"))  # 8-wave + K/V double-buffer (305 TF/s vs 252 @ swz=4, within-probe)
+PREFILL_SWZ = int(__import__("os").environ.get("RBG_PREFILL_SWZ", "16"))  # prefill_flash.hip; below 16: the forms of attn_prefill.hip
 
 
 def decode_attention(q, key_cache, value_cache, block_tables, context_lens,
@@ -278,17 +279,72 @@ def decode_attention(q, key_cache, value_cache, block_tables, context_lens,
                                       context_lens, scale)
 
 
-def prefill_attention(q, k, v, cu_seqlens, scale: float,
-                      cu_seqlens_k=None) -> torch.Tensor:
+@dataclass
+class PrefillPlan:
+    """Workgroups of prompt attention (bindings.cpp prefill_flash)."""
+    blocks: torch.Tensor        # [n, 4] int32
+    lens: torch.Tensor          # [n] int32
+
+
+def prefill_plan(cu, cu_k, heads: int, kv_heads: int, device) -> PrefillPlan:
+    """``cu`` and ``cu_k``: where each sequence's query and kv rows begin, on
+    the host."""
+    tokens = 128 // (heads // kv_heads)
+    cu, cu_k = np.asarray(cu), np.asarray(cu_k)
+    rows, lens = np.diff(cu), np.diff(cu_k)
+    count = (rows + tokens - 1) // tokens
+    seq = np.repeat(np.arange(len(rows)), count)
+    nth = np.arange(len(seq)) - np.repeat(np.cumsum(count) - count, count)
+    past = (lens - rows)[seq]
+    need = np.minimum(past + (nth + 1) * tokens, lens[seq])
+    # Most work first.  Where all run at once, two per CU (256 CUs), the second
+    # half is turned round, so that the longest share with the shortest (2048
+    # tokens of 32 heads: 61 -> 56 us).
+    order = np.argsort(-need, kind="stable")
+    if len(order) * kv_heads <= 512:
+        half = 256 // kv_heads
+        order = np.concatenate([order[:half], order[half:][::-1]])
+    info = np.stack([cu[:-1][seq], nth, cu_k[:-1][seq], past], axis=1)
+    both = torch.from_numpy(np.concatenate(
+        [info[order].reshape(-1), lens[seq][order]]).astype(np.int32)
+    ).to(device)
+    n = len(order)
+    return PrefillPlan(both[:4 * n].view(n, 4), both[4 * n:])
+
+
+def prefill_attention(q, k, v, cu_seqlens, scale: float, cu_seqlens_k=None,
+                      plan: Optional[PrefillPlan] = None,
+                      slots=None) -> torch.Tensor:
+    """Varlen causal attention; q [Tq, QH, D], k/v [Tkv, KVH, D], or pages
+    [pages, KVH, page_size, D] of which ``slots`` [Tkv] (page * page_size +
+    place) names the rows.  ``plan``: prefill_plan of the same sequences, made
+    once for all layers of a step."""
+    if _on_gpu(q):
+        kvh = k.shape[1]
+        group = q.shape[1] // kvh
+        if (PREFILL_SWZ >= 16 and q.shape[1] % kvh == 0 and group <= 128 and
+                (slots is None or k.shape[2] & (k.shape[2] - 1) == 0)):
+            if plan is None:
+                cu = cu_seqlens.tolist()
+                plan = prefill_plan(
+                    cu, cu if cu_seqlens_k is None else cu_seqlens_k.tolist(),
+                    q.shape[1], kvh, q.device)
+            return _require_hip().prefill_flash(q, k, v, plan.blocks,
+                                                plan.lens, scale, slots)
+    if slots is not None:
+        at = slots.long()
+        pages, place = at // k.shape[2], at % k.shape[2]
+        k, v = k[pages, :, place], v[pages, :, place]
     if _on_gpu(q):
         # bit 2 = 8-wave 16x16 blocks; bit 3 = 4-wave 32x32 blocks
-        qtile = 128 if (PREFILL_SWZ & 12) else 64
+        swz = PREFILL_SWZ if PREFILL_SWZ < 16 else 6
+        qtile = 128 if (swz & 12) else 64
         block_info, seq_lens = reference.prefill_block_info(
             cu_seqlens.cpu(), qtile=qtile,
             cu_seqlens_k=None if cu_seqlens_k is None else cu_seqlens_k.cpu())
         return _require_hip().prefill_attention(
             q, k, v, block_info.to(q.device), seq_lens.to(q.device), scale,
-            PREFILL_SWZ)
+            swz)
     return reference.prefill_attention(q, k, v, cu_seqlens, scale,
                                        cu_seqlens_k)
 

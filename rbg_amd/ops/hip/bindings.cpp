@@ -34,6 +34,9 @@ void launch_decode_pages(void*, void*, void*, const void*, const void*,
 void launch_prefill_attention(void*, const void*, const void*, const void*,
                               const void*, const void*, float, int, int, int,
                               int, int, int, hipStream_t);
+void launch_prefill_flash(void*, const void*, const void*, const void*,
+                          const void*, const void*, const void*, float, int,
+                          int, int, int, long, long, hipStream_t);
 void launch_mfma_probe(void*, const void*, const void*, int, int, hipStream_t);
 void launch_mfma_probe32(void*, const void*, const void*, int, int, int,
                          hipStream_t);
@@ -343,6 +346,55 @@ torch::Tensor prefill_attention(torch::Tensor q, torch::Tensor k,
   return out;
 }
 
+// Causal attention of prompt rows.  k and v are rows [Tkv, H, 128], or, with
+// slots [Tkv], pages [pages, H, page_size, 128] that the slots name rows of.
+// block_info [n, 4] and seq_lens [n]: a workgroup's first query row of the
+// sequence, its number among the sequence's blocks of 128 / (QH / H) tokens,
+// the sequence's first kv row and the position of its first query row; its kv
+// rows.
+torch::Tensor prefill_flash(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                            torch::Tensor block_info, torch::Tensor seq_lens,
+                            double scale, c10::optional<torch::Tensor> slots) {
+  auto rows3 = [](const torch::Tensor& t, const char* name) {
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
+                t.dim() == 3 && t.stride(2) == 1 &&
+                t.stride(1) == t.size(2) && t.size(2) == 128, name,
+                " must be [T, H, 128] row-sliced");
+  };
+  rows3(q, "q");
+  int shift = 0;
+  if (slots.has_value()) {
+    check_bf16_contig(k, "keys");
+    check_bf16_contig(v, "values");
+    TORCH_CHECK(k.dim() == 4 && k.sizes() == v.sizes() && k.size(3) == 128,
+                "pages must be [pages, H, page_size, 128]");
+    while ((1 << shift) < k.size(2)) ++shift;
+    TORCH_CHECK((1 << shift) == k.size(2), "page size: a power of 2");
+    TORCH_CHECK(slots->is_cuda() && slots->is_contiguous() &&
+                slots->scalar_type() == torch::kInt32, "slots int32");
+  } else {
+    rows3(k, "k");
+    rows3(v, "v");
+    TORCH_CHECK(k.stride(0) == v.stride(0), "k/v stride mismatch");
+  }
+  for (const auto& t : {block_info, seq_lens})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
+                t.scalar_type() == torch::kInt32, "plan int32");
+  const int blocks = seq_lens.numel();
+  TORCH_CHECK(block_info.numel() == 4 * (int64_t)blocks, "plan sizes");
+  const int heads = q.size(1), kv_heads = k.size(1);
+  TORCH_CHECK(kv_heads > 0 && heads % kv_heads == 0 && heads / kv_heads <= 128,
+              "query heads: a multiple of the key heads, at most 128 times");
+  auto out = torch::empty({q.size(0), (int64_t)heads, (int64_t)128},
+                          q.options());
+  launch_prefill_flash(out.data_ptr(), q.data_ptr(), k.data_ptr(),
+                       v.data_ptr(), slots ? slots->data_ptr() : nullptr,
+                       block_info.data_ptr(), seq_lens.data_ptr(),
+                       (float)scale, blocks, heads, kv_heads, shift,
+                       q.stride(0), k.stride(0), current_stream());
+  return out;
+}
+
 torch::Tensor mfma_probe(torch::Tensor a, torch::Tensor b, int64_t a_split,
                          int64_t b_split) {
   auto d = torch::zeros({16, 16}, a.options().dtype(torch::kFloat32));
@@ -512,6 +564,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_store_kv", &rope_store_kv, "RoPE + paged KV write");
   m.def("decode_attention", &decode_attention, "paged flash-decode");
   m.def("prefill_attention", &prefill_attention, "varlen causal flash prefill");
+  m.def("prefill_flash", &prefill_flash, "causal attention of prompts",
+        py::arg("q"), py::arg("k"), py::arg("v"), py::arg("block_info"),
+        py::arg("seq_lens"), py::arg("scale"),
+        py::arg("slots") = c10::nullopt);
   m.def("mfma_probe", &mfma_probe, "MFMA layout probe");
   m.def("mfma_probe32", &mfma_probe32, "32x32x16 MFMA layout probe");
   m.def("skinny_gemm", &skinny_gemm, "decode-shape GEMM (M<=128)",

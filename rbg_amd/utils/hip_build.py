@@ -30,6 +30,7 @@ HIP_SOURCES = {
         "attn_decode.hip",
         "decode_pages.hip",
         "attn_prefill.hip",
+        "prefill_flash.hip",
         "mfma_probe.hip",
         "rmsnorm.hip",
         "rope_kv.hip",
@@ -94,7 +95,7 @@ HIP_SOURCES = {
 }
 
 HIP_HEADERS = {
-    "_hip_ops": ["common.h", "gemm_bindings.h"],
+    "_hip_ops": ["common.h", "gemm_bindings.h", "mfma_util.h"],
     "_hip_mix": ["act.h", "act_kinds.h", "bind_util.h", "common.h",
                  "delta_scan.h", "embed_bindings.h", "gemm_bindings.h",
                  "glu_bindings.h", "mfma_util.h", "mix_args.h", "vec_io.h"],

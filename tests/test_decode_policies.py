@@ -47,3 +47,22 @@ def test_split_policy_is_batch_deterministic():
     a = [pick_decode_splits(b, 8, 4096, variant=4) for b in range(1, 129)]
     b = [pick_decode_splits(b, 8, 4096, variant=4) for b in range(1, 129)]
     assert a == b
+
+
+def test_prefill_plan_covers_every_row():
+    """Every block of rows once, whatever the order."""
+    import torch
+
+    from rbg_amd import ops
+    cu, cu_k = [0, 5, 5, 300, 301], [0, 105, 110, 405, 1406]
+    for heads, kvh in ((32, 8), (6, 2), (8, 8)):
+        tokens = 128 // (heads // kvh)
+        plan = ops.prefill_plan(cu, cu_k, heads, kvh, "cpu")
+        got = sorted(map(tuple, torch.cat(
+            [plan.blocks, plan.lens[:, None]], 1).tolist()))
+        want = sorted(
+            (cu[b], i, cu_k[b], cu_k[b + 1] - cu_k[b] - cu[b + 1] + cu[b],
+             cu_k[b + 1] - cu_k[b])
+            for b in range(4)
+            for i in range(-(-(cu[b + 1] - cu[b]) // tokens)))
+        assert got == want

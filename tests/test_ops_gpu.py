@@ -576,3 +576,64 @@ def test_linear_swiglu(m, f, k):
         assert ((got.double() - want).abs() <= bound).all()
     got = ops._hip.skinny_swiglu(x, w).double()
     assert (got - want).norm() <= 2 ** -8 * want.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kvh", [(4, 1), (8, 8), (6, 2), (16, 2),
+                                       (32, 8), (5, 5)])
+@pytest.mark.parametrize("news,pasts", [
+    ([1], [0]), ([1, 63, 64, 65, 129], [0] * 5),
+    ([31, 33, 1, 200], [1, 64, 500, 63]), ([300], [0])])
+def test_prefill_flash(heads, kvh, news, pasts):
+    """Ends of tiles, waves and blocks, pasts of any length, groups that do
+    not divide 128, key heads in and out of step with the XCDs; rows beside
+    pages, scale of either sign, scores large enough to move the maximum, and
+    sums that a capture replays.  Weights are rounded to bf16 (2^-9 of a
+    weighted mean of |v|) and so is the result."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(heads * 1000 + sum(news))
+    cu = [0] + torch.tensor(news).cumsum(0).tolist()
+    cu_k = [0] + (torch.tensor(news) + torch.tensor(pasts)).cumsum(0).tolist()
+    q = torch.randn(cu[-1], heads, 128, device=dev, generator=gen).bfloat16()
+    rows = torch.randn(cu_k[-1], 2 * kvh, 128, device=dev,
+                       generator=gen).bfloat16()
+    rows[::50] *= 4
+    rows = rows.view(cu_k[-1], -1)
+    k = rows[:, :kvh * 128].view(-1, kvh, 128)
+    v = rows[:, kvh * 128:].view(-1, kvh, 128)
+    n = cu_k[-1] // 32 + 1
+    slots = torch.randperm(n * 32, device=dev, generator=gen)[:cu_k[-1]]
+    pages = torch.zeros(2, n, kvh, 32, 128, dtype=torch.bfloat16, device=dev)
+    pages[0, slots // 32, :, slots % 32] = k
+    pages[1, slots // 32, :, slots % 32] = v
+    cut = torch.tensor(cu, dtype=torch.int32, device=dev)
+    cut_k = torch.tensor(cu_k, dtype=torch.int32, device=dev)
+    for scale in (0.3, -0.09, 0.0):
+        got = ops.prefill_attention(q, k, v, cut, scale, cut_k)
+        for b, past in enumerate(pasts):
+            kb, vb = (t[cu_k[b]:cu_k[b + 1]].double() for t in (k, v))
+            at = past + torch.arange(news[b], device=dev)
+            hide = torch.arange(len(kb), device=dev)[None] > at[:, None]
+            for h in range(heads):
+                g = h // (heads // kvh)
+                qb = q[cu[b]:cu[b + 1], h].double()
+                s = (qb @ kb[:, g].t().contiguous() * scale).masked_fill(
+                    hide, -math.inf)
+                w = s.softmax(-1)
+                want = w @ vb[:, g]
+                bound = want.abs() * 2 ** -8 + (w @ vb[:, g].abs()) * 2 ** -7
+                err = (got[cu[b]:cu[b + 1], h].double() - want).abs()
+                assert (err <= bound + 1e-5).all(), (scale, b, h)
+        paged = ops.prefill_attention(q, pages[0], pages[1], cut, scale,
+                                      cut_k, slots=slots.int())
+        assert torch.equal(paged, got)
+    plan = ops.prefill_plan(cu, cu_k, heads, kvh, dev)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = ops.prefill_attention(q, k, v, cut, 0.0, cut_k, plan)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, got)
