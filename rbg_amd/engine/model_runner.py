@@ -18,6 +18,7 @@ import torch
 
 from ..models.llama import PPContext, TPContext
 from ..models.registry import build_model
+from ..utils.upload import upload
 from .batch import ForwardBatch, VarlenLayout, table_array
 from .config import EngineConfig
 from .sequence import Sequence
@@ -52,11 +53,8 @@ class ModelRunner:
 
     # ------------------------------------------------------------------
 
-    def _i32(self, data) -> torch.Tensor:
-        return torch.tensor(data, dtype=torch.int32, device=self.device)
-
-    def _join(self, parts: List[np.ndarray]) -> torch.Tensor:
-        return torch.from_numpy(np.concatenate(parts)).to(self.device)
+    def _index(self, rows: List[int]) -> torch.Tensor:
+        return upload([np.array(rows, dtype=np.int64)], self.device)[0]
 
     # one sequence's part of a varlen step: tokens at [start, start + len)
     Chunk = Tuple[Sequence, int, List[int]]
@@ -102,29 +100,39 @@ class ModelRunner:
             starts.append(start)
             ends.append(end)
             tables.append(seq.block_table)
-        batch = ForwardBatch(
-            mode="prefill",
-            positions=self._join(positions),
-            slot_mapping=self._join(slots),
-            cu_seqlens=self._i32(cu), cu_host=cu)
+        # everything the step needs from the host is one transfer
+        i32 = lambda a: np.asarray(a, dtype=np.int32)   # noqa: E731
+        parts = {"tokens": np.concatenate(tokens),
+                 "positions": np.concatenate(positions),
+                 "slots": np.concatenate(slots), "cu": i32(cu)}
         if self.model.needs_prev:
-            batch.prev_tokens = self._join(prev)
+            parts["prev"] = np.concatenate(prev)
         if self.model.varlen:
-            batch.starts = self._i32(starts)
-            batch.state_slots = self._i32([t.state_slot for t in tables])
+            parts["starts"] = i32(starts)
+            parts["state_slots"] = i32([t.state_slot for t in tables])
+            parts["cu_prefill"] = i32([c - num_decode
+                                       for c in cu[num_decode:]])
+            if num_decode:
+                parts["tables"] = table_array(tables[:num_decode])
+                parts["ends"] = i32(ends[:num_decode])
+        elif any_past:
+            parts["cu_k"] = i32(cu_k)
+            parts["gather"] = np.concatenate(gather)
+        dev = dict(zip(parts, upload(list(parts.values()), self.device)))
+        batch = ForwardBatch(
+            mode="prefill", positions=dev["positions"],
+            slot_mapping=dev["slots"], cu_seqlens=dev["cu"], cu_host=cu,
+            prev_tokens=dev.get("prev"), starts=dev.get("starts"),
+            state_slots=dev.get("state_slots"),
+            cu_prefill=dev.get("cu_prefill"),
+            block_tables=dev.get("tables"), context_lens=dev.get("ends"),
+            cu_seqlens_k=dev.get("cu_k"),
+            cu_k_host=cu_k if "cu_k" in dev else None,
+            kv_gather_slots=dev.get("gather"))
+        if self.model.varlen:
             batch.num_decode = num_decode
             batch.layout = VarlenLayout(starts, ends, tables, num_decode,
                                         self.cfg.page_size, self.device)
-            batch.cu_prefill = self._i32([c - num_decode
-                                          for c in cu[num_decode:]])
-            if num_decode:
-                batch.block_tables = torch.from_numpy(table_array(
-                    tables[:num_decode])).to(self.device)
-                batch.context_lens = self._i32(ends[:num_decode])
-        elif any_past:
-            batch.cu_seqlens_k = self._i32(cu_k)
-            batch.cu_k_host = cu_k
-            batch.kv_gather_slots = self._join(gather)
         # decode inputs that were left on the device are behind now
         self._dstate = None
         hidden_in = None
@@ -132,7 +140,7 @@ class ModelRunner:
             hidden_in = self.pp.recv_prev(
                 (cu[-1], self.model.stream_width),
                 self.model.stream_dtype, self.device)
-        hidden = self.model.forward(self._join(tokens), batch, self.cache,
+        hidden = self.model.forward(dev["tokens"], batch, self.cache,
                                     hidden=hidden_in)
         if not self.pp.last:
             self.pp.send_next(hidden)
@@ -169,7 +177,7 @@ class ModelRunner:
             return []
         if self.pp.last:
             last = [first_row[i] + len(chunks[i][2]) - 1 for i in at]
-            logits = self.model.logits(hidden, self._i32(last))
+            logits = self.model.logits(hidden, self._index(last))
             next_dev = self.sample_device(logits, sampled)[0]
         else:
             next_dev = torch.empty(len(sampled), dtype=torch.int64,
@@ -191,39 +199,71 @@ class ModelRunner:
             self._dstate = None
             logits = self._decode_logits([seq for seq, _, _ in chunks])
             rows = [i for i, w in enumerate(want) for _ in w]
-            return logits[torch.tensor(rows, dtype=torch.int64,
-                                       device=self.device)]
+            if rows == list(range(len(chunks))):
+                return logits.clone()   # the next step writes these again
+            return logits[self._index(rows)]
         hidden, first_row = self.run_chunks(chunks)
         rows = [first_row[i] + p for i, w in enumerate(want) for p in w]
-        return self.model.logits(hidden, self._i32(rows))
+        return self.model.logits(hidden, self._index(rows))
 
     # ------------------------------------------------------------------
 
-    def _build_decode_state(self, seqs: List[Sequence]) -> dict:
+    def _build_decode_state(self, seqs: List[Sequence],
+                            bucket: int = 0) -> dict:
         """Device-resident decode inputs.  Valid across steps for the same
         batch composition: positions/ctx advance on-device, the block tables
         never change mid-decode (pages are reserved for prompt+max_new at
         admission — engine/scheduler.py), so the only host->device traffic
         per step is nothing at all; sampled tokens stay on-device as the
-        next step's input."""
-        dev = self.device
-        positions = self._i32([seq.num_tokens - 1 for seq in seqs])
-        ctx = self._i32([seq.num_tokens for seq in seqs])
-        tokens = torch.tensor([seq.last_token for seq in seqs],
-                              dtype=torch.int64, device=dev)
-        bt_np = table_array([seq.block_table for seq in seqs])
-        state = {"ids": tuple(s.seq_id for s in seqs),
-                 "positions": positions, "ctx": ctx, "tokens": tokens,
-                 "bt": torch.from_numpy(bt_np).to(dev), "fresh": True,
-                 "state_slots": None, "prev": None}
+        next step's input.  With a ``bucket`` they live in the inputs of its
+        captured step."""
+        n, rows = len(seqs), bucket or len(seqs)
+        ps = self.cfg.page_size
+        # one transfer: per sequence 2 int64 and 4 int32, then the tables.
+        # Padding rows decode position 0 against page 0 with ctx=1: harmless
+        # work; their slot writes land in reserved scratch page 0
+        fields = np.zeros(4 * rows, dtype=np.int64)
+        words = fields[2 * rows:].view(np.int32).reshape(4, rows)
+        positions = np.array([seq.num_tokens - 1 for seq in seqs])
+        fields[:n] = [seq.last_token for seq in seqs]
         if self.model.needs_prev:
-            state["prev"] = torch.tensor(
-                [seq.token_at(seq.num_tokens - 2) for seq in seqs],
-                dtype=torch.int64, device=dev)
+            fields[rows:rows + n] = [seq.token_at(seq.num_tokens - 2)
+                                     for seq in seqs]
+        bt = table_array([seq.block_table for seq in seqs])
+        words[0, :n] = positions
+        words[1, :n] = (bt[np.arange(n), positions // ps] * ps +
+                        positions % ps)
+        words[2] = 1
+        words[2, :n] = positions + 1
         if self.model.stateful:
-            state["state_slots"] = self._i32(
-                [seq.block_table.state_slot for seq in seqs])
+            words[3, :n] = [seq.block_table.state_slot for seq in seqs]
+        fields_dev, bt_dev = upload([fields, bt], self.device)
+        if bucket:
+            static = self._graphs[bucket][1]
+            static["fields"].copy_(fields_dev)
+            static["bt"].zero_()
+            static["bt"][:n, :bt.shape[1]].copy_(bt_dev)
+        else:
+            static = dict(self._fields(fields_dev), bt=bt_dev)
+        state = {k: static[k][:n] for k in ("tokens", "prev", "positions",
+                                            "slots", "ctx", "state_slots")}
+        state["bt"] = static["bt"][:n]
+        if not self.model.needs_prev:
+            state["prev"] = None
+        if not self.model.stateful:
+            state["state_slots"] = None
+        state.update(ids=tuple(s.seq_id for s in seqs), fresh=True,
+                     bucket=bucket)
         return state
+
+    @staticmethod
+    def _fields(fields: torch.Tensor) -> Dict[str, torch.Tensor]:
+        """The parts of a step's per-sequence inputs, 4 * rows int64."""
+        rows = fields.numel() // 4
+        words = fields[2 * rows:].view(torch.int32).view(4, rows)
+        return {"tokens": fields[:rows], "prev": fields[rows:2 * rows],
+                "positions": words[0], "slots": words[1], "ctx": words[2],
+                "state_slots": words[3]}
 
     def _decode_slots(self, state: dict) -> torch.Tensor:
         ps = self.cfg.page_size
@@ -236,22 +276,38 @@ class ModelRunner:
         """Forward of one decode step; logits [n, vocab] on the last stage."""
         n = len(seqs)
         ids = tuple(s.seq_id for s in seqs)
+        bucket = 0
+        if (not self.cfg.enforce_eager and
+                self.device.type == "cuda" and
+                self.pp.size == 1 and           # p2p hops: eager path
+                self.model.tp.graph_safe and    # xGMI AR or no TP
+                n <= GRAPH_BATCH_SIZES[-1]):
+            bucket = self._graph_bucket(n)
+            if bucket not in self._graphs:
+                self._build_graph(bucket)
         state = self._dstate
-        if state is None or state["ids"] != ids:
-            state = self._build_decode_state(seqs)
+        if state is None or state["ids"] != ids or state["bucket"] != bucket:
+            state = self._build_decode_state(seqs, bucket)
             self._dstate = state
         elif not state["fresh"]:
             state["positions"] += 1
             state["ctx"] += 1
+            slots = self._decode_slots(state)
+            if bucket:
+                state["slots"].copy_(slots)
+                static = self._graphs[bucket][1]
+                # the first step's tokens, its prev now, are static's own
+                for key in ("prev", "tokens"):
+                    if state[key] is not None:
+                        static[key][:n].copy_(state[key])
+            else:
+                state["slots"] = slots
         state["fresh"] = False
-        slots = self._decode_slots(state)
-        use_graph = (not self.cfg.enforce_eager and
-                     self.device.type == "cuda" and
-                     self.pp.size == 1 and           # p2p hops: eager path
-                     self.model.tp.graph_safe and    # xGMI AR or no TP
-                     n <= GRAPH_BATCH_SIZES[-1])
-        if use_graph:
-            return self._decode_graph(state, slots, n)[:n]
+        if bucket:
+            graph, _, logits = self._graphs[bucket]
+            graph.replay()
+            return logits[:n]
+        slots = state["slots"]
         batch = self._decode_batch(state, slots, n)
         hidden_in = None
         if not self.pp.first:
@@ -304,18 +360,11 @@ class ModelRunner:
 
     def _build_graph(self, bs: int):
         """Capture one decode step at batch size ``bs`` into a hipGraph."""
-        static = {
-            "tokens": torch.zeros(bs, dtype=torch.int64, device=self.device),
-            "prev": torch.zeros(bs, dtype=torch.int64, device=self.device),
-            "positions": torch.zeros(bs, dtype=torch.int32, device=self.device),
-            "slots": torch.zeros(bs, dtype=torch.int32, device=self.device),
-            "ctx": torch.ones(bs, dtype=torch.int32, device=self.device),
-            "bt": torch.zeros(bs, self.max_pages_per_seq, dtype=torch.int32,
-                              device=self.device),
-            # padding rows use the scratch slot 0
-            "state_slots": torch.zeros(bs, dtype=torch.int32,
-                                       device=self.device),
-        }
+        fields = torch.zeros(4 * bs, dtype=torch.int64, device=self.device)
+        static = dict(self._fields(fields), fields=fields)
+        static["ctx"].fill_(1)
+        static["bt"] = torch.zeros(bs, self.max_pages_per_seq,
+                                   dtype=torch.int32, device=self.device)
         batch = self._decode_batch(static, static["slots"], bs)
         # warm up allocations outside capture
         torch.cuda.synchronize()
@@ -331,36 +380,6 @@ class ModelRunner:
         self._graphs[bs] = (graph, static, logits)
         log.info("captured decode hipGraph for batch %d", bs)
         return self._graphs[bs]
-
-    def _decode_graph(self, state: dict, slots: torch.Tensor,
-                      n: int) -> torch.Tensor:
-        bs = self._graph_bucket(n)
-        if bs not in self._graphs:
-            self._build_graph(bs)
-        graph, static, logits = self._graphs[bs]
-        static["tokens"][:n].copy_(state["tokens"][:n])
-        static["positions"][:n].copy_(state["positions"])
-        static["slots"][:n].copy_(slots)
-        static["ctx"][:n].copy_(state["ctx"])
-        if state["state_slots"] is not None:
-            static["state_slots"][:n].copy_(state["state_slots"])
-        if state["prev"] is not None:
-            static["prev"][:n].copy_(state["prev"])
-        bt = state["bt"]
-        if state.get("graph_bt_loaded") != (state["ids"], bs):
-            # block tables are stable for this batch: upload once per batch
-            static["bt"].zero_()
-            static["bt"][:n, :bt.shape[1]].copy_(bt)
-            if n < bs:
-                # padding rows decode against page 0 with ctx=1: harmless
-                # work; their slot writes land in reserved scratch page 0
-                static["slots"][n:] = 0
-                static["positions"][n:] = 0
-                static["ctx"][n:] = 1
-                static["state_slots"][n:] = 0
-            state["graph_bt_loaded"] = (state["ids"], bs)
-        graph.replay()
-        return logits
 
     # ------------------------------------------------------------------
 

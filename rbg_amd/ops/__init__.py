@@ -16,6 +16,7 @@ import numpy as np
 import torch
 
 from ..utils import hip_build
+from ..utils.upload import upload
 from . import reference
 
 # Extension modules by name, loaded as far as they are built; a process needs
@@ -305,11 +306,8 @@ def prefill_plan(cu, cu_k, heads: int, kv_heads: int, device) -> PrefillPlan:
         half = 256 // kv_heads
         order = np.concatenate([order[:half], order[half:][::-1]])
     info = np.stack([cu[:-1][seq], nth, cu_k[:-1][seq], past], axis=1)
-    both = torch.from_numpy(np.concatenate(
-        [info[order].reshape(-1), lens[seq][order]]).astype(np.int32)
-    ).to(device)
-    n = len(order)
-    return PrefillPlan(both[:4 * n].view(n, 4), both[4 * n:])
+    return PrefillPlan(*upload([info[order].astype(np.int32),
+                                lens[seq][order].astype(np.int32)], device))
 
 
 def prefill_attention(q, k, v, cu_seqlens, scale: float, cu_seqlens_k=None,
