@@ -2,8 +2,8 @@
 // as rows or, behind a past, straight from the pages.
 //
 // Bound: the matrix cores (4 * 128 operations per pair of tokens) and beside
-// them the exponentials: 936 TFLOP/s at 8192 tokens of 32 heads, where the
-// 16-row form this replaces reached 346, and 570 at 2048, where few workgroups
+// them the exponentials: 925 TFLOP/s at 8192 tokens of 32 heads, where the
+// 16-row form this replaces reached 346, and 590 at 2048, where few workgroups
 // have most of the work.  A workgroup is 4 waves of 32 query rows each; tiles
 // of 64 keys pass LDS in two buffers, one barrier a tile, the next tile's rows
 // in flight meanwhile.  (Forming the next tile's scores beside this tile's
@@ -17,9 +17,9 @@
 //    operand of O^T = V^T P^T as they are, with keys 4h..4h+3, 8+4h.. of 16 in
 //    place of 8h..8h+7: probabilities never pass LDS, the softmax exchanges one
 //    value per 32 keys.  V is read transposed.
-//  * The running maximum moves only when a score exceeds it by 2^8 (weights
-//    stay below 256 times their true scale, sums are f32), so sums are hardly
-//    ever rescaled; scale and maximum are one fma per score.
+//  * Scale and maximum are one fma per score, and sums are rescaled only when
+//    some row's maximum grows.  (Letting scores exceed it by 2^8 would be 1 to
+//    2% faster, but the largest weight, 1 here, would then be rounded too.)
 #include "mfma_util.h"
 
 namespace {
@@ -28,7 +28,6 @@ constexpr int DIM = 128, TILE = 64, WAVES = 4, ROWS = WAVES * 32;
 constexpr int THREADS = WAVES * 64;
 constexpr int KP = DIM + 8;       // row pitch of K in LDS: no bank conflicts
 constexpr float LOW = -1e30f;
-constexpr float SLACK = 8.f;      // to the base of 2
 
 typedef __attribute__((ext_vector_type(4))) unsigned int pf_u4;
 
@@ -40,6 +39,11 @@ DEV_INLINE bf16x8 pf_frag(pf_u4 u) {
   union { pf_u4 u; bf16x8 v; } c;
   c.u = u;
   return c.v;
+}
+
+DEV_INLINE float pf_add2(__bf16 a, __bf16 b, float sum) {
+  const bf16x2 ab = {a, b}, ones = {(__bf16)1.f, (__bf16)1.f};
+  return __builtin_amdgcn_fdot2_f32_bf16(ab, ones, sum, false);
 }
 
 // PAGED: kv rows are named by `slots` ((page << page_shift) + place) and lie in
@@ -195,7 +199,7 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) top = fmaxf(top, s[p][i]);
       top = fmaxf(top, __shfl_xor(top, 32, 64)) * scale;
-      if (__any(top > m + SLACK)) {
+      if (__any(top > m)) {
         const float m_new = fmaxf(m, top);
         const float fade = __builtin_amdgcn_exp2f(m - m_new);
         m = m_new;
@@ -210,11 +214,16 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
       for (int p = 0; p < 2; ++p)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const float e =
-              __builtin_amdgcn_exp2f(__builtin_fmaf(s[p][i], scale, -m));
-          l += e;
-          pf[p * 2 + i / 8][i % 8] = (__bf16)e;
+          pf[p * 2 + i / 8][i % 8] = (__bf16)__builtin_amdgcn_exp2f(
+              __builtin_fmaf(s[p][i], scale, -m));
         }
+      // the sum of the weights as they are used, rounded: an error that the
+      // largest share with it cancels
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 8; i += 2)
+          l = pf_add2(pf[e][i], pf[e][i + 1], l);
       // 16 keys x 32 dims: lanes of a half read blocks of 4 keys x 16 dims
       const __hip_bfloat16* vp =
           v_lds[b] + h * 512 + ((lane >> 4) & 1) * 64 + (lane & 15) * 4;
