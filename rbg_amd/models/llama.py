@@ -172,16 +172,18 @@ class LlamaAttention(nn.Module):
                                                   dtype=dtype),
                                        requires_grad=False)
 
-    def forward(self, x: torch.Tensor, batch: ForwardBatch,
-                kv: PagedKVCache, cos_sin: torch.Tensor) -> torch.Tensor:
-        T = x.shape[0]
+    def forward(self, x: Optional[torch.Tensor], residual: torch.Tensor,
+                norm: torch.Tensor, batch: ForwardBatch, kv: PagedKVCache,
+                cos_sin: torch.Tensor):
+        """Attention of the norm of residual + x; and that sum."""
+        T = residual.shape[0]
         key_cache = kv.key_cache(self.layer_idx)
         value_cache = kv.value_cache(self.layer_idx)
         # (Qwen: per-head norms,) RoPE and the paged KV write in one kernel,
         # which also adds up what a split GEMM left
-        qkv = ops.rope_heads(
-            ops.linear_parts(x, self.wqkv), self.heads, self.q_norm,
-            self.k_norm, self.cfg.rms_eps, key_cache, value_cache, cos_sin,
+        qkv, residual = ops.norm_heads(
+            x, residual, norm, self.cfg.rms_eps, self.wqkv, self.heads,
+            self.q_norm, self.k_norm, key_cache, value_cache, cos_sin,
             batch.positions, batch.slot_mapping)
         # q/k/v stay SLICES of the fused projection: the attention kernels
         # take a token-row stride, so no .contiguous() copies
@@ -210,8 +212,8 @@ class LlamaAttention(nn.Module):
                                      num_splits=batch.decode_num_splits)
         o = o.view(T, self.q_out).contiguous()
         if self.parts:
-            return ops.linear_parts(o, self.wo)
-        return self.tp.all_reduce(ops.linear(o, self.wo))
+            return ops.linear_parts(o, self.wo), residual
+        return self.tp.all_reduce(ops.linear(o, self.wo)), residual
 
 
 class LlamaMLP(nn.Module):
@@ -235,11 +237,13 @@ class LlamaMLP(nn.Module):
                                      tp_size=tp.size, tp_rank=tp.rank)
         self.inter = inter
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        h = ops.linear_swiglu(x, self.w_gate_up)
+    def forward(self, x: torch.Tensor, residual: torch.Tensor,
+                norm: torch.Tensor, eps: float):
+        """Of the norm of residual + x; and that sum."""
+        h, residual = ops.norm_swiglu(x, residual, norm, eps, self.w_gate_up)
         if self.parts:
-            return ops.linear_parts(h, self.w_down)
-        return self.tp.all_reduce(ops.linear(h, self.w_down))
+            return ops.linear_parts(h, self.w_down), residual
+        return self.tp.all_reduce(ops.linear(h, self.w_down)), residual
 
 
 class LlamaLayer(nn.Module):
@@ -263,14 +267,10 @@ class LlamaLayer(nn.Module):
                 batch: ForwardBatch, kv: PagedKVCache,
                 cos_sin: torch.Tensor):
         if residual is None:
-            residual = x.clone()
-            h = ops.rmsnorm(x, self.input_norm, self.eps)
-        else:
-            # h := rmsnorm(x + residual); residual := x + residual  (fused)
-            h = ops.add_rmsnorm(x, residual, self.input_norm, self.eps)
-        h = self.attn(h, batch, kv, cos_sin)
-        h = ops.add_rmsnorm(h, residual, self.post_norm, self.eps)
-        h = self.mlp(h)
+            x, residual = None, x       # nothing to add yet
+        h, residual = self.attn(x, residual, self.input_norm, batch, kv,
+                                cos_sin)
+        h, residual = self.mlp(h, residual, self.post_norm, self.eps)
         return h, residual
 
 

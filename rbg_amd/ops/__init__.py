@@ -220,6 +220,54 @@ def rope_heads(proj, heads: int, q_norm, k_norm, eps: float, key_cache,
     return proj
 
 
+def _takes_rows(src, residual: torch.Tensor, w: torch.Tensor) -> bool:
+    """Can norm and GEMM be one launch (hip/skinny_rows.h)?  The shapes that its
+    kernel without a norm takes, in bf16 without parts."""
+    return (_takes_skinny(residual, w) and residual.shape[0] <= 4 and
+            residual.shape[1] % 2048 == 0 and residual.is_contiguous() and
+            (src is None or (src.dtype == torch.bfloat16 and
+                             src.is_contiguous())))
+
+
+def _normed(src, residual, weight, eps: float) -> torch.Tensor:
+    if src is None:
+        return rmsnorm(residual, weight, eps)
+    return add_rmsnorm(src, residual, weight, eps)
+
+
+def norm_heads(src, residual, weight, eps: float, w, heads: int, q_norm,
+               k_norm, key_cache, value_cache, cos_sin, positions,
+               slot_mapping):
+    """rope_heads of the projection by ``w`` of the RMS norm of residual + src
+    (src: linear_parts' result, or None).  Returns the projection in bf16 and
+    the new residual, perhaps in the old one's memory."""
+    store = (key_cache, value_cache, cos_sin, positions, slot_mapping)
+    # every workgroup norms the rows: 384 of them repay that for up to 16384
+    # values (us, norm + GEMM + rotation against one launch: 6144 x 4096, 1 row
+    # 19.3 / 13.7, 4 rows 20.2 / 15.2; 10240 x 8192, 2 rows 41.0 / 38.3, 4 rows
+    # 42.3 / 44.6)
+    if (_takes_rows(src, residual, w) and residual.numel() <= 16384 and
+            key_cache.shape[3] == 128):
+        mod = _require_hip()
+        if q_norm is None:
+            return mod.norm_rows(src, residual, weight, eps, w, 2, heads,
+                                 *store)
+        proj, residual = mod.norm_rows(src, residual, weight, eps, w, 0)
+    else:
+        proj = linear_parts(_normed(src, residual, weight, eps), w)
+    return rope_heads(proj, heads, q_norm, k_norm, eps, *store), residual
+
+
+def norm_swiglu(src, residual, weight, eps: float, w):
+    """linear_swiglu of the RMS norm of residual + src, and the new residual."""
+    # 1792 workgroups repay it for one row only (28672 x 4096: 1 row 45.2 / 43.3,
+    # 2 rows 44.0 / 47.2)
+    if (_takes_rows(src, residual, w) and residual.shape[0] == 1 and
+            w.shape[0] % 64 == 0):
+        return _require_hip().norm_rows(src, residual, weight, eps, w, 1)
+    return linear_swiglu(_normed(src, residual, weight, eps), w), residual
+
+
 def pick_decode_splits(num_seqs: int, num_kv_heads: int,
                        max_context: int, variant: int = -1) -> int:
     """Fill the chip: MI355X has 256 CUs / 8 XCDs; measured optimum is

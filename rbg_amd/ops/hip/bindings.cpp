@@ -20,6 +20,10 @@ void launch_rope_heads(void*, void*, void*, const void*, int, const void*,
                        const void*, float, void*, void*, const void*,
                        const void*, const void*, int, int, int, int, int, int,
                        hipStream_t);
+void launch_norm_rows(void*, const void*, const void*, void*, const void*,
+                      float, const void*, int, int, int, int, const void*,
+                      const void*, const void*, void*, void*, int, int, int,
+                      hipStream_t);
 void launch_silu_mul(void*, const void*, int, int, hipStream_t);
 void launch_rope_store_kv(void*, void*, const void*, void*, void*,
                           const void*, const void*, const void*, int, int,
@@ -263,6 +267,61 @@ torch::Tensor rope_heads(torch::Tensor proj, int64_t num_q_heads,
                     (int)kv_heads, (int)key_cache.size(2), (int)width,
                     (int)width, current_stream());
   return out;
+}
+
+// Up to 4 rows: the RMS norm of residual + src (src may be missing), a GEMM and
+// its end in one launch: nothing (0), silu(gate) * up (1), or rotation and
+// paged store of fused heads (2, as rope_heads).  Returns the product and the
+// new residual, which is another tensor unless src is missing.
+std::vector<torch::Tensor> norm_rows(
+    c10::optional<torch::Tensor> src, torch::Tensor residual,
+    torch::Tensor norm_weight, double eps, torch::Tensor w, int64_t end,
+    int64_t heads, c10::optional<torch::Tensor> key_cache,
+    c10::optional<torch::Tensor> value_cache,
+    c10::optional<torch::Tensor> cos_sin,
+    c10::optional<torch::Tensor> positions,
+    c10::optional<torch::Tensor> slots) {
+  check_skinny(residual, w);
+  check_bf16_contig(norm_weight, "norm weight");
+  const int64_t M = residual.size(0), K = residual.size(1), N = w.size(0);
+  TORCH_CHECK(M <= 4 && M * K <= 32768, "at most 4 rows, 64 KB of them");
+  TORCH_CHECK(norm_weight.numel() == K, "norm weight of K");
+  TORCH_CHECK(end >= 0 && end <= 2, "unknown end");
+  if (src.has_value()) {
+    check_bf16_contig(*src, "src");
+    TORCH_CHECK(src->sizes() == residual.sizes(), "src like residual");
+  }
+  int64_t kv_heads = 0, page_size = 1;
+  if (end == 2) {
+    TORCH_CHECK(key_cache && value_cache && cos_sin && positions && slots,
+                "the rotation's inputs");
+    check_bf16_contig(*key_cache, "key_cache");
+    check_bf16_contig(*value_cache, "value_cache");
+    kv_heads = key_cache->size(1);
+    page_size = key_cache->size(2);
+    TORCH_CHECK(key_cache->size(3) == 128 &&
+                value_cache->sizes() == key_cache->sizes() &&
+                N == (heads + 2 * kv_heads) * 128, "heads of 128, q | k | v");
+    TORCH_CHECK(cos_sin->scalar_type() == torch::kFloat32 &&
+                cos_sin->is_contiguous() && cos_sin->size(1) == 128,
+                "cos_sin must be fp32 [positions, 128]");
+    for (const auto& t : {*positions, *slots})
+      TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kInt32 &&
+                  t.is_contiguous() && t.numel() == M,
+                  "an int32 position and slot per row");
+  }
+  auto out = torch::empty({M, end == 1 ? N / 2 : N}, residual.options());
+  auto next = src ? torch::empty_like(residual) : residual;
+  const auto ptr = [](const c10::optional<torch::Tensor>& t) -> void* {
+    return t ? t->data_ptr() : nullptr;
+  };
+  launch_norm_rows(out.data_ptr(), ptr(src), residual.data_ptr(),
+                   next.data_ptr(), norm_weight.data_ptr(), (float)eps,
+                   w.data_ptr(), (int)M, (int)N, (int)K, (int)end,
+                   ptr(cos_sin), ptr(positions), ptr(slots), ptr(key_cache),
+                   ptr(value_cache), (int)heads, (int)kv_heads,
+                   (int)page_size, current_stream());
+  return {out, next};
 }
 
 torch::Tensor decode_attention(torch::Tensor q, torch::Tensor key_cache,
@@ -574,6 +633,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("a"), py::arg("w"), py::arg("force_splits") = 0);
   m.def("skinny_parts", &skinny_parts, "decode GEMM as its parts' sums");
   m.def("skinny_swiglu", &skinny_swiglu, "decode gate/up GEMM with silu");
+  m.def("norm_rows", &norm_rows, "norm, GEMM of a few rows and its end",
+        py::arg("src"), py::arg("residual"), py::arg("norm_weight"),
+        py::arg("eps"), py::arg("w"), py::arg("end"), py::arg("heads") = 0,
+        py::arg("key_cache") = c10::nullopt,
+        py::arg("value_cache") = c10::nullopt,
+        py::arg("cos_sin") = c10::nullopt, py::arg("positions") = c10::nullopt,
+        py::arg("slots") = c10::nullopt);
   m.def("add_rmsnorm", &add_rmsnorm, "residual += x; its RMS norm");
   m.def("rope_heads", &rope_heads, "head norms, RoPE, paged store");
   // gil_scoped_release on the IPC/copy entry points: mapping or launching

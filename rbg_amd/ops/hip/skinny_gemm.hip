@@ -20,113 +20,12 @@
 //  * workgroups begin at different places of K.  All rows of A and W are K
 //    apart, so workgroups in step ask the same few L2 channels (128 rows: 78
 //    -> 75 us).
-#include "common.h"
+#include "skinny_rows.h"
 
 namespace {
 
 constexpr int KC = 128;           // k per chunk
 constexpr int DEPTH = 2;          // chunks of weights in flight per wave
-constexpr int ROWS_KC = 64, ROWS_DEPTH = 4;     // of skinny_rows_kernel
-
-typedef __attribute__((ext_vector_type(4))) unsigned int sg_u4;
-
-DEV_INLINE sg_u4 sg_load(const __hip_bfloat16* p) {
-  return *reinterpret_cast<const sg_u4*>(p);
-}
-
-DEV_INLINE bf16x8 sg_frag(sg_u4 u) {
-  union { sg_u4 u; bf16x8 v; } c;
-  c.u = u;
-  return c.v;
-}
-
-DEV_INLINE float silu(float g) { return g / (1.f + __expf(-g)); }
-
-// The chunk that a workgroup takes as its c-th.
-DEV_INLINE int sg_turn(int c, int first, int n) {
-  c += first;
-  return c >= n ? c - n : c;
-}
-
-// A few rows: 8 waves share one 16-row tile of W and take its K in turns,
-// without a barrier until their sums meet in LDS, and without splits whose
-// sums a second launch would add.  4096 x 4096, one row: 8.5 us against 10.5 of
-// the kernel below with its reduction.  Its time grows with the rows, since
-// every workgroup reads all of A (28672 x 4096: 4 rows 40 us, 16 rows 56).
-// GLU: the tile is 8 rows of the gate and the same 8 of the up matrix.
-template <bool GLU>
-__global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
-    const __hip_bfloat16* __restrict__ a,   // [M, K]
-    const __hip_bfloat16* __restrict__ w,   // [N, K]
-    __hip_bfloat16* __restrict__ c,         // [M, N], GLU: [M, N / 2]
-    const int M, const int N, const int K) {
-  constexpr int WAVES = 8;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const int row = GLU ? blockIdx.x * 8 + (r & 7) + (r >> 3) * (N / 2)
-                      : blockIdx.x * 16 + r;
-  const __hip_bfloat16* wp = w + (size_t)row * K + wave * ROWS_KC + g * 8;
-  const __hip_bfloat16* ap = a + (size_t)min(r, M - 1) * K + wave * ROWS_KC + g * 8;
-  const int n = (K / ROWS_KC - wave + WAVES - 1) / WAVES;
-  const int first = n ? ((blockIdx.x >> 3) + (blockIdx.x & 7) * (n >> 3)) % n
-                      : 0;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  sg_u4 wr[ROWS_DEPTH][2], ar[ROWS_DEPTH][2];
-#define SR_LOAD(s, at)                                                     \
-  do {                                                                     \
-    const int off = sg_turn(at, first, n) * (ROWS_KC * WAVES);                  \
-    wr[s][0] = sg_load(wp + off);                                          \
-    wr[s][1] = sg_load(wp + off + 32);                                     \
-    ar[s][0] = sg_load(ap + off);                                          \
-    ar[s][1] = sg_load(ap + off + 32);                                     \
-  } while (0)
-#define SR_MATH(s)                                                         \
-  do {                                                                     \
-    _Pragma("unroll") for (int h = 0; h < 2; ++h)                          \
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(                     \
-            sg_frag(ar[s][h]), sg_frag(wr[s][h]), acc, 0, 0, 0);           \
-  } while (0)
-  if (n > 0) {
-#pragma unroll
-    for (int s = 0; s < ROWS_DEPTH; ++s) SR_LOAD(s, min(s, n - 1));
-    int at = 0;
-    for (; at + ROWS_DEPTH < n; at += ROWS_DEPTH) {
-#pragma unroll
-      for (int s = 0; s < ROWS_DEPTH; ++s) {
-        SR_MATH(s);
-        SR_LOAD(s, min(at + ROWS_DEPTH + s, n - 1));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < ROWS_DEPTH; ++s)
-      if (at + s < n) SR_MATH(s);
-  }
-#undef SR_LOAD
-#undef SR_MATH
-
-  // lane l, register q: row 4 * (l >> 4) + q of A, row l & 15 of the tile
-  __shared__ float red[WAVES][256];
-  *reinterpret_cast<f32x4*>(&red[wave][lane * 4]) = acc;
-  __syncthreads();
-  const int e = threadIdx.x;
-  if (e < 256) {
-    const int col = (e >> 2) & 15, m = (e >> 6) * 4 + (e & 3);
-    float v = 0.f;
-#pragma unroll
-    for (int k = 0; k < WAVES; ++k) v += red[k][e];
-    if (GLU) {
-      if (m < M && col < 8) {
-        float up = 0.f;
-#pragma unroll
-        for (int k = 0; k < WAVES; ++k) up += red[k][e + 8 * 4];
-        c[(size_t)m * (N / 2) + blockIdx.x * 8 + col] = f2bf(silu(v) * up);
-      }
-    } else if (m < M) {
-      c[(size_t)m * N + blockIdx.x * 16 + col] = f2bf(v);
-    }
-  }
-}
 
 // NW waves of 16 rows of W each share MT * 16 rows of A through LDS, a chunk
 // at a time, two buffers, one barrier a chunk.  blockIdx.y: a part of K, whose
@@ -312,11 +211,10 @@ extern "C" void launch_skinny_gemm(void* c, void* ws, const void* a,
   } while (0)
   if (waves == 0) {             // the kernel of a few rows
     if (glu)
-      skinny_rows_kernel<true><<<dim3(N / 16), dim3(512), 0, stream>>>(
-          ap, wp, cp, M, N, K);
+      launch_skinny_rows<ROWS_GLU, false>(cp, ap, wp, M, N, K, {}, {}, stream);
     else
-      skinny_rows_kernel<false><<<dim3(N / 16), dim3(512), 0, stream>>>(
-          ap, wp, cp, M, N, K);
+      launch_skinny_rows<ROWS_PLAIN, false>(cp, ap, wp, M, N, K, {}, {},
+                                            stream);
   } else if (mt <= 1 && waves == 4) SG_GO(1, 4);
   else if (mt <= 2 && waves == 4) SG_GO(2, 4);
   else if (mt <= 1) SG_GO(1, 8);

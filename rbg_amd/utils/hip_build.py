@@ -29,6 +29,7 @@ HIP_SOURCES = {
     "_hip_ops": [
         "attn_decode.hip",
         "decode_pages.hip",
+        "decode_rows.hip",
         "attn_prefill.hip",
         "prefill_flash.hip",
         "mfma_probe.hip",
@@ -95,24 +96,28 @@ HIP_SOURCES = {
 }
 
 HIP_HEADERS = {
-    "_hip_ops": ["common.h", "gemm_bindings.h", "mfma_util.h"],
+    "_hip_ops": ["common.h", "gemm_bindings.h", "mfma_util.h",
+                 "skinny_rows.h"],
     "_hip_mix": ["act.h", "act_kinds.h", "bind_util.h", "common.h",
                  "delta_scan.h", "embed_bindings.h", "gemm_bindings.h",
-                 "glu_bindings.h", "mfma_util.h", "mix_args.h", "vec_io.h"],
+                 "glu_bindings.h", "mfma_util.h", "mix_args.h",
+                 "skinny_rows.h", "vec_io.h"],
     "_hip_latent": ["bind_util.h", "common.h", "latent_args.h", "lds_stream.h",
                     "mfma_util.h", "rotary.h", "vec_io.h"],
     "_hip_experts": ["act.h", "act_kinds.h", "bind_util.h", "common.h",
                      "expert_args.h", "expert_rows.h", "lds_stream.h",
                      "mfma_util.h", "vec_io.h"],
     "_hip_moe": ["bind_util.h", "common.h", "expert_rows.h", "gemm_bindings.h",
-                 "mfma_util.h", "moe_args.h", "vec_io.h"],
+                 "mfma_util.h", "moe_args.h", "skinny_rows.h", "vec_io.h"],
     "_hip_hyper": ["act.h", "act_kinds.h", "bind_util.h", "common.h",
                    "embed_bindings.h", "expert_rows.h", "gemm_bindings.h",
-                   "glu_bindings.h", "hyper_args.h", "vec_io.h"],
+                   "glu_bindings.h", "hyper_args.h",
+                   "skinny_rows.h", "vec_io.h"],
     "_hip_gated": ["act.h", "act_kinds.h", "bind_util.h", "common.h",
                    "delta_scan.h", "embed_bindings.h", "expert_rows.h",
                    "gated_args.h", "gated_delta.h", "gemm_bindings.h",
-                   "glu_bindings.h", "mfma_util.h", "vec_io.h"],
+                   "glu_bindings.h", "mfma_util.h", "skinny_rows.h",
+                   "vec_io.h"],
 }
 
 # model architecture -> the extensions with its kernels (default: _hip_ops)

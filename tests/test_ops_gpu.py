@@ -637,3 +637,55 @@ def test_prefill_flash(heads, kvh, news, pasts):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 3, 4])
+@pytest.mark.parametrize("k", [2048, 8192])
+@pytest.mark.parametrize("first", [False, True])
+def test_norm_rows(rows, k, first):
+    """Norm, GEMM and each of its ends in one launch against float64.  The
+    operand is rounded once, as the separate norm rounds it: 2^-8 of the sums'
+    size, which for rows of a norm is the root of k times the weights'."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(rows * 10 + k)
+    def rnd(*shape):
+        return torch.randn(*shape, device=dev, generator=gen).bfloat16()
+    heads, kvh = 4, 2
+    src = None if first else rnd(rows, k)
+    res, nw = rnd(rows, k) * 3, rnd(k)
+    w = (torch.randn(1024, k, device=dev, generator=gen) / k ** 0.5).bfloat16()
+    total = res.double() + (0 if first else src.double())
+    h = total * torch.rsqrt(total.square().mean(-1, keepdim=True) + 1e-5) * \
+        nw.double()
+    full = h @ w.double().t().contiguous()
+    for end, want in ((0, full), (1, torch.nn.functional.silu(full[:, :512]) *
+                                  full[:, 512:])):
+        old = res.clone()
+        out, new = ops._hip.norm_rows(src, res, nw, 1e-5, w, end)
+        assert torch.equal(res, old)
+        assert ((new.double() - total).abs() <= total.abs() * 2 ** -8).all()
+        assert (out.double() - want).norm() <= 2 ** -7 * want.norm(), end
+    table = ref.build_cos_sin_table(128, 512, device=dev)
+    pos = torch.randint(0, 512, (rows,), device=dev, generator=gen).int()
+    slots = torch.randperm(32, device=dev, generator=gen)[:rows].int()
+    slots[-1] = -1
+    caches = [torch.zeros(2, kvh, 16, 128, dtype=torch.bfloat16, device=dev)
+              for _ in range(4)]
+    for norms in ((None, None), (rnd(128), rnd(128))):
+        got, _ = ops.norm_heads(src, res.clone(), nw, 1e-5, w, heads, *norms,
+                                *caches[:2], table, pos, slots)
+        want = ops.rope_heads(full.float()[None], heads, *norms, 1e-5,
+                              *caches[2:], table, pos, slots)
+        assert (got.double() - want.double()).norm() <= \
+            2 ** -6.5 * want.double().norm()
+        for a, b in zip(caches[:2], caches[2:]):
+            assert ((a != 0) == (b != 0)).all()
+            held = got.view(rows, -1, 128)
+        for t, s in enumerate(slots.tolist()):
+            if s >= 0:
+                assert torch.equal(caches[0][s // 16, :, s % 16],
+                                   held[t, heads:heads + kvh])
+                assert torch.equal(caches[1][s // 16, :, s % 16],
+                                   held[t, heads + kvh:])
