@@ -113,8 +113,9 @@ torch::Tensor skinny_swiglu(torch::Tensor a, torch::Tensor w) {
   TORCH_CHECK(M <= 128, "at most 128 rows");
   auto c = torch::empty({M, N / 2}, a.options());
   // as pick_skinny, unsplit; the smaller workgroups where they fill the chip
-  const int waves = M <= 4 && K % 2048 == 0 ? 0 : M <= 32 && N <= 12288 ? 4
-                                                                        : 8;
+  const int waves = pick_skinny((int)M, (int)N, (int)K).waves == 0 ? 0
+                    : M <= 32 && N <= 12288                        ? 4
+                                                                   : 8;
   launch_skinny_gemm(c.data_ptr(), nullptr, a.data_ptr(), w.data_ptr(),
                      (int)M, (int)N, (int)K, waves, 1, 1, current_stream());
   return c;
