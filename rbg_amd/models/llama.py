@@ -356,7 +356,7 @@ class LlamaForCausalLM(nn.Module):
         Non-last stages return the combined stream to send onward; the last
         stage returns final-normed hidden states ready for logits()."""
         if self.pp.first:
-            x = self.embed[tokens.long()]
+            x = torch.nn.functional.embedding(tokens.long(), self.embed)
         else:
             assert hidden is not None, "non-first PP stage needs hidden"
             x = hidden

@@ -282,12 +282,13 @@ def pick_decode_splits(num_seqs: int, num_kv_heads: int,
         # head) pairs need short ones to fill the chip, many need long ones,
         # which start less often (us, 256 / 512 / 1024 / 2048 keys: 8 pairs of
         # 2048 10 / 13 / 18 / 26; 56 pairs of up to 3000 18.9 / 21.7 / 19.7 /
-        # 29.8; 128 pairs of up to 2048 31 / 26 / 24 / 29; 1024 pairs of 2080
-        # 224 / 191 / 177 / 174)
+        # 29.8; 128 pairs of up to 2048 31 / 26 / 24 / 29; 360 pairs of up to
+        # 2500 63 / 59 / 58 / 68; 512 pairs of up to 2048, 8 query heads each,
+        # 98 / 89 / 84 / 76; 1024 pairs of 2080 224 / 191 / 177 / 174)
         pairs = num_seqs * num_kv_heads
         span = (max(256, max_context // 32) if pairs <= 64 else
                 max(512, max_context // 16) if pairs <= 96 else
-                max(1024, max_context // 8) if pairs <= 192 else 2048)
+                max(1024, max_context // 8) if pairs <= 384 else 2048)
         return max(1, (max_context + span - 1) // span)
     if variant >= 4:
         # v4/v5 pack 2 seqs per WG; v6 runs 1 seq per (2-wave) WG
