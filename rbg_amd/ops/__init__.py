@@ -99,19 +99,33 @@ SKINNY_GEMM = int(__import__("os").environ.get("RBG_SKINNY_GEMM", "1"))
 def _skinny(rows: int, n: int, k: int) -> bool:
     """Does the hand-written decode GEMM (hip/skinny_gemm.hip) take a [rows, k]
     x [n, k] product, rather than hipBLASLt?  Measured with cold weights (us,
-    own against library): narrow matrices at any decode batch (4096 x 14336:
-    1 row 22 against 24, 64 rows 28 against 38, 128 rows 38 against 73; 10240 x
-    8192: 39 against 41 and 50 against 55), but the short ones only up to 64
-    (3072 x 2048: 16 rows 7.6 against 8.6, 64 rows 9.5 against 9.2, 128 rows
-    12.5 against 12.0).  Wide
-    ones up to 64 rows (28672 x 4096: 1 row 40 against 57, 64 rows 46 against
-    49, 128 rows 58 against 53), where rows are a multiple of 4 KB apart
-    (51200 x 5120: 1 row 94 against 89, 64 rows 122 against 98)."""
+    own with its reduction against library).  Narrow matrices at any decode
+    batch (4096 x 14336: 1 row 22 against 24, 64 rows 28 / 38, 128 rows 38 / 73;
+    10240 x 8192: 64 rows 39 / 41, 128 rows 50 / 55), the short ones up to 64
+    rows (3072 x 2048: 16 rows 7.6 / 8.6, 64 rows 9.5 / 9.2, 128 rows 12.5 /
+    12.0), the long ones further, as the library does not split k (4096 x 14336:
+    192 rows 47 / 99, 256 rows 62 / 59; 5120 x 25600: 256 rows 119 / 260).  Wide
+    matrices up to 64 rows (28672 x 4096: 1 row 40 / 57, 64 rows 46 / 49, 128
+    rows 58 / 53), where their rows are a multiple of 4 KB apart (51200 x 5120:
+    1 row 94 / 89, 64 rows 122 / 98)."""
     if rows < 1 or n % 32 or k % 512:
         return False
     if n <= 12288:
-        return rows <= (128 if k > 2048 else 64)
+        return rows <= (256 if k > 16384 else 192 if k >= 12288 else
+                        128 if k > 2048 else 64)
     return rows <= 64 and k % 2048 == 0
+
+
+def _takes_skinny(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
+            x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and
+            _skinny(x.shape[0], w.shape[0], x.shape[1]) and
+            # what only the library takes: strides, rows that begin between
+            # multiples of 16 bytes, gradients
+            w.is_contiguous() and
+            (x.data_ptr() | w.data_ptr()) % 16 == 0 and
+            not (torch.is_grad_enabled() and
+                 (x.requires_grad or w.requires_grad)))
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -123,12 +137,6 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
                        "_hip_hyper").skinny_gemm(
             x if x.is_contiguous() else x.contiguous(), w)
     return torch.nn.functional.linear(x, w)
-
-
-def _takes_skinny(x: torch.Tensor, w: torch.Tensor) -> bool:
-    return (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and
-            x.dtype == torch.bfloat16 and
-            _skinny(x.shape[0], w.shape[0], x.shape[1]))
 
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -475,10 +475,11 @@ def test_decode_pages(qpg, kvh, lens, splits):
             err = (got[i, h * qpg:(h + 1) * qpg] - want).abs()
             assert (err <= bound + 1e-5).all(), (i, n, h)
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    with torch.inference_mode(), torch.cuda.graph(g):
         out = call()
     for _ in range(3):
-        out.zero_()
+        with torch.inference_mode():
+            out.zero_()
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out.double(), got)
@@ -630,10 +631,11 @@ def test_prefill_flash(heads, kvh, news, pasts):
         assert torch.equal(paged, got)
     plan = ops.prefill_plan(cu, cu_k, heads, kvh, dev)
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    with torch.inference_mode(), torch.cuda.graph(g):
         out = ops.prefill_attention(q, k, v, cut, 0.0, cut_k, plan)
     for _ in range(3):
-        out.zero_()
+        with torch.inference_mode():
+            out.zero_()
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, got)
@@ -689,3 +691,26 @@ def test_norm_rows(rows, k, first):
                                    held[t, heads:heads + kvh])
                 assert torch.equal(caches[1][s // 16, :, s % 16],
                                    held[t, heads + kvh:])
+
+
+@pytest.mark.gpu
+def test_linear_takes_what_the_library_takes():
+    """Transposed and misaligned operands and gradients, at a shape that the
+    decode GEMM would take otherwise."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    x = torch.randn(8, 1024, device=dev).bfloat16()
+    w = torch.randn(1024, 256, device=dev).bfloat16()
+    want = x.float() @ w.float()
+    def near(got):
+        return ((got.float() - want).abs() <=
+                want.abs() * 2 ** -7 + 0.05).all()
+    assert near(ops.linear(x, w.t()))
+    odd = torch.empty(8 * 1024 + 1, device=dev, dtype=torch.bfloat16)[1:]
+    odd.copy_(x.flatten())
+    wt = w.t().contiguous()
+    assert near(ops.linear(odd.view(8, 1024), wt))
+    x.requires_grad_(True)
+    got = ops.linear(x, wt)
+    got.float().sum().backward()
+    assert near(got) and x.grad is not None
