@@ -158,7 +158,7 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             x.shape[0] <= (64 if w.shape[0] > 12288 else 32)):
         return _require_hip().skinny_swiglu(
             x if x.is_contiguous() else x.contiguous(), w)
-    return silu_mul(linear(x, w))
+    return silu_mul(linear_parts(x, w))
 
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:

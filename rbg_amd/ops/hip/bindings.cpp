@@ -24,6 +24,7 @@ void launch_norm_rows(void*, const void*, const void*, void*, const void*,
                       float, const void*, int, int, int, int, const void*,
                       const void*, const void*, void*, void*, int, int, int,
                       hipStream_t);
+void launch_silu_parts(void*, const void*, int, int, int, hipStream_t);
 void launch_silu_mul(void*, const void*, int, int, hipStream_t);
 void launch_rope_store_kv(void*, void*, const void*, void*, void*,
                           const void*, const void*, const void*, int, int,
@@ -148,6 +149,17 @@ torch::Tensor add_rmsnorm(torch::Tensor x, torch::Tensor residual,
 }
 
 torch::Tensor silu_mul(torch::Tensor x) {
+  if (x.scalar_type() == torch::kFloat32) {     // sums of skinny_parts
+    TORCH_CHECK(x.is_cuda() && x.is_contiguous() && x.dim() == 3 &&
+                x.size(2) % 8 == 0, "f32 parts [parts, T, 2 I], I % 4 == 0");
+    const int64_t tokens = x.size(1), inter = x.size(2) / 2;
+    auto out = torch::empty({tokens, inter},
+                            x.options().dtype(torch::kBFloat16));
+    if (tokens)
+      launch_silu_parts(out.data_ptr(), x.data_ptr(), (int)x.size(0),
+                        (int)tokens, (int)inter, current_stream());
+    return out;
+  }
   check_bf16_contig(x, "x");
   const int inter2 = x.size(-1);
   TORCH_CHECK(inter2 % 16 == 0, "2*inter must be a multiple of 16");

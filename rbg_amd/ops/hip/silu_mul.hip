@@ -27,9 +27,43 @@ __global__ void silu_mul_kernel(__hip_bfloat16* __restrict__ out,   // [T, I]
   }
 }
 
+// The same of the f32 sums [parts, T, 2I] that a split GEMM left, for decode
+// batches: the reduction's launch (2 us) and its result's way through memory
+// are saved.
+__global__ void silu_parts_kernel(__hip_bfloat16* __restrict__ out,  // [T, I]
+                                  const float* __restrict__ x,
+                                  const int parts, const int inter,
+                                  const long total_vec) {
+  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+  if (i >= total_vec) return;
+  const int nvec_row = inter / 4;
+  const long row = i / nvec_row;
+  const int col = (int)(i % nvec_row) * 4;
+  const float* p = x + row * 2 * inter + col;
+  const size_t step = (size_t)total_vec * 8;
+  f32x4 g = {0.f, 0.f, 0.f, 0.f}, u = g;
+#pragma unroll 4
+  for (int s = 0; s < parts; ++s) {
+    g += *reinterpret_cast<const f32x4*>(p + s * step);
+    u += *reinterpret_cast<const f32x4*>(p + s * step + inter);
+  }
+  union { __hip_bfloat16 e[4]; uint2 u; } o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    o.e[j] = f2bf(g[j] / (1.f + __expf(-g[j])) * u[j]);
+  *reinterpret_cast<uint2*>(out + row * inter + col) = o.u;
+}
+
 }  // namespace
 
 extern "C" {
+
+void launch_silu_parts(void* out, const void* x, int parts, int tokens,
+                       int inter, hipStream_t stream) {
+  const long vecs = (long)tokens * (inter / 4);
+  silu_parts_kernel<<<dim3((vecs + 255) / 256), dim3(256), 0, stream>>>(
+      (__hip_bfloat16*)out, (const float*)x, parts, inter, vecs);
+}
 
 void launch_silu_mul(void* out, const void* x, int tokens, int inter,
                      hipStream_t stream) {

@@ -559,7 +559,8 @@ def test_rope_heads(parts, norm, tokens, heads, kvh):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("m", [1, 4, 5, 17, 33, 64, 65])
-@pytest.mark.parametrize("f,k", [(32, 512), (5632, 2048), (8224, 2048)])
+@pytest.mark.parametrize("f,k", [(32, 512), (36, 4096), (5632, 2048),
+                                 (8224, 2048)])
 def test_linear_swiglu(m, f, k):
     """Gate and up tiles of every kernel, columns that leave waves idle; error
     of the f32 sums through silu and one rounding (the separate kernels round
@@ -573,7 +574,14 @@ def test_linear_swiglu(m, f, k):
     full = x.double() @ w.double().t().contiguous()
     want = torch.nn.functional.silu(full[:, :f]) * full[:, f:]
     bound = 2 ** -7 * (full[:, :f].abs() + 1) * (full[:, f:].abs() + 1)
-    for got in (ops._hip.skinny_swiglu(x, w), ops.linear_swiglu(x, w)):
+    if f % 32:
+        with pytest.raises(RuntimeError):
+            ops._hip.skinny_swiglu(x, w)
+        w = torch.cat([w[:32], w[f:f + 32]])    # 1 to 16 parts
+        full, f = torch.cat([full[:, :32], full[:, f:f + 32]], 1), 32
+        want, bound = want[:, :32], bound[:, :32]
+    for got in (ops._hip.skinny_swiglu(x, w), ops.linear_swiglu(x, w),
+                ops.silu_mul(ops.linear_parts(x, w))):
         assert ((got.double() - want).abs() <= bound).all()
     got = ops._hip.skinny_swiglu(x, w).double()
     assert (got - want).norm() <= 2 ** -8 * want.norm()
