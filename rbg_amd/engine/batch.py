@@ -24,8 +24,8 @@ class ForwardBatch:
     cu_seqlens: Optional[torch.Tensor] = None   # [B+1] int32 (q rows)
     cu_seqlens_k: Optional[torch.Tensor] = None  # [B+1] int32 (total KV)
     kv_gather_slots: Optional[torch.Tensor] = None  # [Tkv] int32 — prefix
-    #   caching / chunked prefill: gather the FULL [past; new] K/V from the
-    #   paged pool (the new tokens' rows were just written by rope_store_kv)
+    #   caching / chunked prefill: where the FULL [past; new] K/V lies in the
+    #   paged pool (the new tokens' rows were just written there)
     # decode (and the leading decode rows of a mixed step)
     block_tables: Optional[torch.Tensor] = None  # [S, max_pages] int32
     context_lens: Optional[torch.Tensor] = None  # [S] int32

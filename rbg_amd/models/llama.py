@@ -1,10 +1,10 @@
 """Llama-family decoder built directly on the rbg_amd CDNA4 ops.
 
-MI355X-first structure: the four hot non-GEMM ops (RMSNorm with fused
-residual add, RoPE fused with the paged-KV write, prefill/decode paged
-attention, SiLU*up) are the hand-written HIP kernels of rbg_amd.ops; plain
-projections go through hipBLASLt via torch.nn.functional.linear with QKV and
-gate/up fused into single GEMMs so each layer runs 4 GEMMs total.
+MI355X-first structure: norms with the residual add, RoPE with the paged-KV
+write, prefill and decode attention, SiLU*up and the GEMMs of decode batches are
+the hand-written HIP kernels of rbg_amd.ops, fused with one another where a
+batch is small; the GEMMs of prompts go through hipBLASLt (ops.linear), with QKV
+and gate/up fused so that each layer runs 4 of them.
 
 Tensor parallelism is Megatron-style over RCCL/xGMI: QKV and gate_up are
 column-parallel (head-aligned shards), o_proj and down_proj row-parallel
