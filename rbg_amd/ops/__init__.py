@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import importlib
 from dataclasses import dataclass
-from typing import Any, Dict, Optional
+from typing import Any, Dict, Optional, Tuple
 
 import numpy as np
 import torch
@@ -276,6 +276,23 @@ def norm_swiglu(src, residual, weight, eps: float, w):
     return linear_swiglu(_normed(src, residual, weight, eps), w), residual
 
 
+def _decode_span(pairs: int) -> Tuple[int, int]:
+    """Keys of a part, and the most parts of a sequence, for that many
+    (sequence, key head) pairs.  Few pairs need short parts to fill the chip,
+    many need long ones, which start less often (us, 256 / 512 / 1024 / 2048
+    keys: 8 pairs of 2048 10 / 13 / 18 / 26; 56 pairs of up to 3000 18.9 / 21.7 /
+    19.7 / 29.8; 128 pairs of up to 2048 31 / 26 / 24 / 29; 360 pairs of up to
+    2500 63 / 59 / 58 / 68; 512 pairs of up to 2048, 8 query heads each, 98 / 89 /
+    84 / 76; 1024 pairs of 2080 224 / 191 / 177 / 174)."""
+    if pairs <= 64:
+        return 256, 32
+    if pairs <= 96:
+        return 512, 16
+    if pairs <= 384:
+        return 1024, 8
+    return 2048, 1 << 16
+
+
 def pick_decode_splits(num_seqs: int, num_kv_heads: int,
                        max_context: int, variant: int = -1) -> int:
     """Fill the chip: MI355X has 256 CUs / 8 XCDs; measured optimum is
@@ -286,18 +303,10 @@ def pick_decode_splits(num_seqs: int, num_kv_heads: int,
     if variant < 0:
         variant = DECODE_VARIANT
     if variant == 7:
-        # parts of the table's capacity, whatever the lengths: few (sequence,
-        # head) pairs need short ones to fill the chip, many need long ones,
-        # which start less often (us, 256 / 512 / 1024 / 2048 keys: 8 pairs of
-        # 2048 10 / 13 / 18 / 26; 56 pairs of up to 3000 18.9 / 21.7 / 19.7 /
-        # 29.8; 128 pairs of up to 2048 31 / 26 / 24 / 29; 360 pairs of up to
-        # 2500 63 / 59 / 58 / 68; 512 pairs of up to 2048, 8 query heads each,
-        # 98 / 89 / 84 / 76; 1024 pairs of 2080 224 / 191 / 177 / 174)
-        pairs = num_seqs * num_kv_heads
-        span = (max(256, max_context // 32) if pairs <= 64 else
-                max(512, max_context // 16) if pairs <= 96 else
-                max(1024, max_context // 8) if pairs <= 384 else 2048)
-        return max(1, (max_context + span - 1) // span)
+        # as many as the table's capacity may need of _decode_span, or up to a
+        # limit, above which parts grow with the sequence (hip/decode_pages.hip)
+        span, most = _decode_span(num_seqs * num_kv_heads)
+        return max(1, min((max_context + span - 1) // span, most))
     if variant >= 4:
         # v4/v5 pack 2 seqs per WG; v6 runs 1 seq per (2-wave) WG
         per_wg = 2 if variant in (4, 5) else 1
@@ -332,7 +341,8 @@ def decode_attention(q, key_cache, value_cache, block_tables, context_lens,
             variant = DECODE_VARIANT
         return _require_hip().decode_attention(
             q, key_cache, value_cache, block_tables, context_lens, scale,
-            num_splits, variant)
+            num_splits, variant,
+            _decode_span(q.shape[0] * key_cache.shape[1])[0])
     return reference.decode_attention(q, key_cache, value_cache, block_tables,
                                       context_lens, scale)
 

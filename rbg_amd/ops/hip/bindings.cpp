@@ -35,7 +35,7 @@ void launch_decode_attention(void*, void*, void*, const void*, const void*,
                              hipStream_t);
 void launch_decode_pages(void*, void*, void*, const void*, const void*,
                          const void*, const void*, const void*, float, int,
-                         int, int, int, int, int, hipStream_t);
+                         int, int, int, int, int, int, hipStream_t);
 void launch_prefill_attention(void*, const void*, const void*, const void*,
                               const void*, const void*, float, int, int, int,
                               int, int, int, hipStream_t);
@@ -337,11 +337,13 @@ std::vector<torch::Tensor> norm_rows(
   return {out, next};
 }
 
+// span: of form 7, the fewest keys that a part has, where the sequence is longer
 torch::Tensor decode_attention(torch::Tensor q, torch::Tensor key_cache,
                                torch::Tensor value_cache,
                                torch::Tensor block_tables,
                                torch::Tensor context_lens, double scale,
-                               int64_t num_splits, int64_t wide) {
+                               int64_t num_splits, int64_t wide,
+                               int64_t span) {
   // q may be a slice of the fused QKV projection: 3-D bf16 with
   // contiguous (head, dim) rows and an arbitrary token stride
   TORCH_CHECK(q.is_cuda() && q.scalar_type() == torch::kBFloat16 &&
@@ -374,8 +376,8 @@ torch::Tensor decode_attention(torch::Tensor q, torch::Tensor key_cache,
                         key_cache.data_ptr(), value_cache.data_ptr(),
                         block_tables.data_ptr(), context_lens.data_ptr(),
                         (float)scale, num_seqs, num_q_heads, num_kv_heads,
-                        max_pages, (int)num_splits, (int)q.stride(0),
-                        current_stream());
+                        max_pages, (int)num_splits, (int)span,
+                        (int)q.stride(0), current_stream());
     return out;
   }
   launch_decode_attention(out.data_ptr(), po, pml, q.data_ptr(),
@@ -634,7 +636,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm, "x,residual += ; rmsnorm");
   m.def("silu_mul", &silu_mul, "silu(gate)*up");
   m.def("rope_store_kv", &rope_store_kv, "RoPE + paged KV write");
-  m.def("decode_attention", &decode_attention, "paged flash-decode");
+  m.def("decode_attention", &decode_attention, "paged flash-decode",
+        py::arg("q"), py::arg("key_cache"), py::arg("value_cache"),
+        py::arg("block_tables"), py::arg("context_lens"), py::arg("scale"),
+        py::arg("num_splits"), py::arg("wide"), py::arg("span") = 128);
   m.def("prefill_attention", &prefill_attention, "varlen causal flash prefill");
   m.def("prefill_flash", &prefill_flash, "causal attention of prompts",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("block_info"),

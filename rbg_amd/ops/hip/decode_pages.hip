@@ -12,10 +12,11 @@
 //    per wave.
 //  * Values, read in whole lines and once, are loaded non-temporally (219 ->
 //    198 us at 128 x 2080); keys, whose lines two loads share, are not.
-//  * Work is cut by keys, not by sequences: every workgroup takes at most
-//    `span` keys of one sequence, whatever the sequence's length, so a batch
-//    of ragged lengths fills the chip as a regular one does.  Workgroups past
-//    the end of their sequence leave at once.
+//  * Work is cut by keys, not by sequences: every workgroup takes `span` keys
+//    of one sequence, whatever the sequence's length, so a batch of ragged
+//    lengths fills the chip as a regular one does; longer ones only where the
+//    grid has too few for the sequence.  The grid is fixed when a step is
+//    captured; workgroups past the end of their sequence leave at once.
 #include "common.h"
 
 namespace {
@@ -37,6 +38,15 @@ DEV_INLINE bf16x8 dp_frag(dp_u4 u) {
   return c.v;
 }
 
+// Keys of a workgroup: not a share of the table's capacity, which may be many
+// times a sequence's length (one of 2048 keys, 8 heads, tables of 8192 / 40960 /
+// 131072 keys: 11.0 / 20.7 / 27.4 us with shares of the capacity, 11.1 of any).
+DEV_INLINE int part_keys(int ctx, int span, int splits) {
+  constexpr int ROUND = WAVES * STEP;
+  const int all = splits * ROUND;
+  return max(span, (ctx + all - 1) / all * ROUND);
+}
+
 // TOGETHER: all key heads of a (sequence, part) run on one XCD, workgroup i on
 // XCD i % 8, which then translates an eighth of the pool's addresses (128
 // sequences of 2080 tokens, 8 heads: 198 -> 179 us, 6.1 TB/s).  A small batch
@@ -52,7 +62,7 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     const int* __restrict__ tables,         // [seqs, max_pages]
     const int* __restrict__ lens,           // [seqs]
     const float scale,                      // to the base of 2
-    const int kv_heads, const int max_pages, const int span,
+    const int kv_heads, const int max_pages, const int least,
     const int q_stride) {
   int kvh = blockIdx.x, seq = blockIdx.y, split = blockIdx.z;
   if (TOGETHER) {
@@ -66,6 +76,7 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     split = pair / gridDim.y;
   }
   const int ctx = lens[seq];
+  const int span = part_keys(ctx, least, gridDim.z);
   const int begin = split * span, end = min(ctx, begin + span);
   if (begin >= ctx && split > 0) return;
   const int lane = threadIdx.x & 63;
@@ -268,10 +279,11 @@ template <int SHARES>
 __global__ __launch_bounds__(DIM * SHARES) void decode_join_kernel(
     __hip_bfloat16* __restrict__ out, const float* __restrict__ part_o,
     const float* __restrict__ part_ml, const int* __restrict__ lens,
-    const int span, const int splits) {
+    const int least, const int splits) {
   const int seq = blockIdx.y, d = threadIdx.x % DIM;
   const int share = threadIdx.x / DIM;
   const int ctx = lens[seq];
+  const int span = part_keys(ctx, least, splits);
   if (ctx <= span) return;
   const int n = min((ctx + span - 1) / span, splits);
   const size_t row = (size_t)seq * gridDim.x + blockIdx.x;
@@ -327,11 +339,10 @@ __global__ __launch_bounds__(DIM * SHARES) void decode_join_kernel(
 extern "C" void launch_decode_pages(
     void* out, void* part_o, void* part_ml, const void* q, const void* keys,
     const void* values, const void* tables, const void* lens, float scale,
-    int seqs, int heads, int kv_heads, int max_pages, int splits, int q_stride,
-    hipStream_t stream) {
-  // keys per workgroup: the table's capacity over the splits, in whole steps
-  const int steps = (max_pages * PAGE + WAVES * STEP - 1) / (WAVES * STEP);
-  const int span = max(1, (steps + splits - 1) / splits) * WAVES * STEP;
+    int seqs, int heads, int kv_heads, int max_pages, int splits, int span,
+    int q_stride, hipStream_t stream) {
+  // in whole rounds of the waves
+  span = max(1, (span + WAVES * STEP - 1) / (WAVES * STEP)) * WAVES * STEP;
   const dim3 grid(kv_heads, seqs, splits), block(64 * WAVES);
 #define DP_LAUNCH(QPG, TOGETHER)                                           \
   decode_pages_kernel<QPG, TOGETHER><<<grid, block, 0, stream>>>(          \

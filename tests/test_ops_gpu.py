@@ -722,3 +722,72 @@ def test_linear_takes_what_the_library_takes():
     got = ops.linear(x, wt)
     got.float().sum().backward()
     assert near(got) and x.grad is not None
+
+
+def _paged(dev, lens, kvh, capacity, page=16, seed=0):
+    """Keys, values, tables of that many keys, lengths; pages in no order."""
+    gen = torch.Generator(device=dev).manual_seed(seed + len(lens))
+    pages = [(n + page - 1) // page for n in lens]
+    total = sum(pages) + 1
+    kv = torch.randn(2, total, kvh, page, 128, device=dev,
+                     generator=gen).bfloat16()
+    perm = (torch.randperm(total - 1, device=dev, generator=gen) + 1).int()
+    tables = torch.zeros(len(lens), capacity // page, dtype=torch.int32,
+                         device=dev)
+    at = 0
+    for i, n in enumerate(pages):
+        tables[i, :n] = perm[at:at + n]
+        at += n
+    return kv[0], kv[1], tables, torch.tensor(lens, dtype=torch.int32,
+                                              device=dev)
+
+
+def _near_decode(got, q, kc, vc, tables, lens, scale):
+    """Weights are rounded to bf16 (2^-9 of a weighted mean of |v|) and so is
+    the result."""
+    qpg, kvh, page = q.shape[1] // kc.shape[1], kc.shape[1], kc.shape[2]
+    for i, n in enumerate(lens.tolist()):
+        at = tables[i, :(n + page - 1) // page].long()
+        k, v = (t[at].transpose(0, 1).reshape(kvh, -1, 128)[:, :n].double()
+                for t in (kc, vc))
+        qi = q[i].view(kvh, qpg, 128).double()
+        w = torch.stack([qi[h] @ k[h].t().contiguous() * scale
+                         for h in range(kvh)]).softmax(-1)
+        want = torch.stack([w[h] @ v[h] for h in range(kvh)]).view(-1, 128)
+        most = torch.stack([w[h] @ v[h].abs()
+                            for h in range(kvh)]).view(-1, 128)
+        err = (got[i].double() - want).abs()
+        assert (err <= want.abs() * 2 ** -8 + most * 2 ** -7 + 1e-5).all(), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens", [
+    [2048], [2900 - 390 * i for i in range(7)],
+    [2500 - 40 * i for i in range(45)]])
+def test_decode_parts_follow_the_lengths(lens):
+    """The same parts, and so the same bits, whatever a table could hold."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    q = torch.randn(len(lens), 32, 128, device=dev).bfloat16()
+    outs = []
+    for capacity in (8192, 40960, 131072):
+        kv = _paged(dev, lens, 8, capacity)
+        outs.append(ops.decode_attention(
+            q, *kv, 0.1, ops.pick_decode_splits(len(lens), 8, capacity)))
+    _near_decode(outs[0], q, *kv, 0.1)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits,span", [(1, 256), (4, 256), (4, 100),
+                                         (12, 128)])
+def test_decode_part_lengths(splits, span):
+    """Lengths about the end of a part, and beyond what the grid holds of the
+    least parts, whose parts grow."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    lens = [1, 255, 256, 257, 512, 1023, 1024, 1025, 1536, 1537, 2100]
+    q = torch.randn(len(lens), 8, 128, device=dev).bfloat16()
+    kv = _paged(dev, lens, 2, 4096)
+    got = ops._hip.decode_attention(q, *kv, 0.3, splits, 7, span)
+    _near_decode(got, q, *kv, 0.3)
