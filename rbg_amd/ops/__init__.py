@@ -290,7 +290,12 @@ def _decode_span(pairs: int) -> Tuple[int, int]:
         return 512, 16
     if pairs <= 384:
         return 1024, 8
-    return 2048, 1 << 16
+    # Pairs alone fill the chip here: parts only even out ragged lengths, and
+    # every workgroup without keys costs its start (128 sequences of 2080, 4 /
+    # 8 / 20 / 64 parts: 184 / 179 / 191 / 218 us; one of 60000 beside 48 of 500,
+    # 8 / 16 / 64 parts: 187 / 113 / 77 us).  8192 workgroups at most, as the sums
+    # of each are 512 bytes a query head.
+    return 2048, max(1, min(16, 8192 // pairs))
 
 
 def pick_decode_splits(num_seqs: int, num_kv_heads: int,

@@ -66,3 +66,21 @@ def test_prefill_plan_covers_every_row():
             for b in range(4)
             for i in range(-(-(cu[b + 1] - cu[b]) // tokens)))
         assert got == want
+
+
+def test_default_parts_are_bounded():
+    """Of the default form: no more for a longer table than fill the chip, and
+    so a bounded workspace; about as many for one sequence more."""
+    for kvh in (1, 2, 4, 8, 16):
+        for bs in GRAPH_BATCH_SIZES + (49,):
+            counts = [pick_decode_splits(bs, kvh, c, variant=7)
+                      for c in (64, 2048, 8192, 40960, 131072, 1 << 20)]
+            assert counts == sorted(counts) and counts[0] == 1
+            assert counts[-1] <= 32
+            # a head's sums are 128 floats; groups of 8
+            assert counts[-1] * bs * kvh * 8 * 512 <= 32 << 20
+    for cap in (8192, 40960, 131072):
+        counts = [pick_decode_splits(b, 8, cap, variant=7)
+                  for b in range(1, 257)]
+        assert all(b >= a / 2 and a >= b / 2
+                   for a, b in zip(counts, counts[1:]))
