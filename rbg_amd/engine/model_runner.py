@@ -329,7 +329,7 @@ class ModelRunner:
             starts=inputs["positions"], state_slots=inputs["state_slots"],
             prev_tokens=inputs["prev"],
             decode_num_splits=self.model.decode_splits(
-                n, self.cfg.max_seq_len))
+                n, self.cfg.max_seq_len, self.cfg.page_size))
 
     @torch.inference_mode()
     def decode(self, seqs: List[Sequence]) -> List[int]:

@@ -338,12 +338,13 @@ class LlamaForCausalLM(nn.Module):
     def make_cache(self, cfg: EngineConfig) -> PagedKVCache:
         return PagedKVCache(cfg, self.device, num_layers=self.num_local_layers)
 
-    def decode_splits(self, batch_size: int, max_seq_len: int) -> int:
+    def decode_splits(self, batch_size: int, max_seq_len: int,
+                      page_size: int = 16) -> int:
         """Sync-free split-KV policy (graph-safe: depends only on the padded
-        batch size and the config's max context)."""
+        batch size and the config's max context and page size)."""
         tp = max(1, self.tp.size)
         return ops.pick_decode_splits(batch_size, self.cfg.num_kv_heads // tp,
-                                      max_seq_len)
+                                      max_seq_len, page_size=page_size)
 
     @torch.inference_mode()
     def forward(self, tokens: torch.Tensor, batch: ForwardBatch,

@@ -105,7 +105,8 @@ class StreamForCausalLM(nn.Module):
         """Columns of what one pipeline stage hands to the next."""
         return self.cfg.hidden_size
 
-    def decode_splits(self, batch_size: int, max_seq_len: int) -> int:
+    def decode_splits(self, batch_size: int, max_seq_len: int,
+                      page_size: int = 16) -> int:
         return 0                        # per layer, from its sizes
 
     @torch.inference_mode()

@@ -299,7 +299,8 @@ def _decode_span(pairs: int) -> Tuple[int, int]:
 
 
 def pick_decode_splits(num_seqs: int, num_kv_heads: int,
-                       max_context: int, variant: int = -1) -> int:
+                       max_context: int, variant: int = -1,
+                       page_size: int = 16) -> int:
     """Fill the chip: MI355X has 256 CUs / 8 XCDs; measured optimum is
     ~1024 workgroups for BOTH kernels (profiles/decode_breakdown r59
     sweep: V4 B128 peaks at splits=2 = 1024 WGs, B64 at splits=4 = 1024).
@@ -307,6 +308,12 @@ def pick_decode_splits(num_seqs: int, num_kv_heads: int,
     half the dot2 kernel's at equal splits."""
     if variant < 0:
         variant = DECODE_VARIANT
+    # Pages of other sizes take the dot2 form, whatever the variant.  Few pairs
+    # gain by short parts there too (pages of 32, 8 heads, 32 / 16 parts: 1 x
+    # 2048 12.4 / 16.0 us, 1 x 30000 85 / 159; 8 / 5: 45 of up to 2500 100 / 108),
+    # many do not (8 / 2: 128 x 2080 311 / 307).
+    if variant == 7 and page_size != 16 and num_seqs * num_kv_heads > 384:
+        variant = 4
     if variant == 7:
         # as many as the table's capacity may need of _decode_span, or up to a
         # limit, above which parts grow with the sequence (hip/decode_pages.hip)
@@ -341,7 +348,8 @@ def decode_attention(q, key_cache, value_cache, block_tables, context_lens,
                 max_ctx = (int(context_lens.max().item())
                            if context_lens.numel() else 1)
             num_splits = pick_decode_splits(q.shape[0], key_cache.shape[1],
-                                            max_ctx, variant)
+                                            max_ctx, variant,
+                                            key_cache.shape[2])
         if variant < 0:
             variant = DECODE_VARIANT
         return _require_hip().decode_attention(

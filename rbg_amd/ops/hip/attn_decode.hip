@@ -11,7 +11,7 @@
 //
 // Capability analog: the decode-side paged attention of the engines the
 // reference orchestrates (SURVEY §2.3 decode engine row).
-#include "common.h"
+#include "decode_join.h"
 
 namespace {
 
@@ -922,31 +922,6 @@ __global__ __launch_bounds__(128, 4) void decode_attn_pc_kernel(
   }
 }
 
-// Merge split partials: one block per (seq, q_head).
-__global__ void decode_combine_kernel(
-    __hip_bfloat16* __restrict__ out,       // [seqs, QH, D]
-    const float* __restrict__ partial_o,    // [splits, seqs, QH, D]
-    const float* __restrict__ partial_ml,   // [splits, seqs, QH, 2]
-    const int num_splits, const int num_q_heads) {
-  const int seq = blockIdx.x, qh = blockIdx.y, d = threadIdx.x;
-  const int seqs = gridDim.x;
-  float m_star = NEG_INF;
-  for (int s = 0; s < num_splits; ++s)
-    m_star = fmaxf(m_star,
-                   partial_ml[(((size_t)s * seqs + seq) * num_q_heads + qh) * 2]);
-  float o = 0.f, lsum = 0.f;
-  for (int s = 0; s < num_splits; ++s) {
-    const float* ml =
-        partial_ml + (((size_t)s * seqs + seq) * num_q_heads + qh) * 2;
-    const float f = __expf(ml[0] - m_star);
-    o += partial_o[(((size_t)s * seqs + seq) * num_q_heads + qh) * HEAD_DIM +
-                   d] * f;
-    lsum += ml[1] * f;
-  }
-  out[((size_t)seq * num_q_heads + qh) * HEAD_DIM + d] =
-      f2bf(lsum > 0.f ? o / lsum : 0.f);
-}
-
 }  // namespace
 
 extern "C" {
@@ -969,6 +944,11 @@ void launch_decode_attention(void* out, void* partial_o, void* partial_ml,
                      (const int*)block_tables, (const int*)context_lens,      \
                      scale, num_kv_heads, page_size, max_pages, num_splits,  \
                      q_stride)
+  // every part leaves sums, to the base of e
+#define DECODE_JOIN()                                                         \
+  launch_decode_join((__hip_bfloat16*)out, (const float*)partial_o,           \
+                     (const float*)partial_ml, nullptr, 0, num_splits,        \
+                     num_q_heads, num_seqs, 1.44269504088896f, stream)
   if (variant == 6 && page_size == 16) {
     dim3 pgrid(num_kv_heads, num_seqs, num_splits), pblock(128);
 #define LAUNCH_PC(QPG)                                                       \
@@ -986,12 +966,7 @@ void launch_decode_attention(void* out, void* partial_o, void* partial_ml,
     else if (qpg == 8) LAUNCH_PC(8);
     else return;
 #undef LAUNCH_PC
-    if (num_splits > 1) {
-      dim3 cgrid(num_seqs, num_q_heads), cblock(HEAD_DIM);
-      hipLaunchKernelGGL(decode_combine_kernel, cgrid, cblock, 0, stream,
-                         (__hip_bfloat16*)out, (const float*)partial_o,
-                         (const float*)partial_ml, num_splits, num_q_heads);
-    }
+    DECODE_JOIN();
     return;
   }
   if ((variant == 4 || variant == 5) && page_size == 16) {
@@ -1020,12 +995,7 @@ void launch_decode_attention(void* out, void* partial_o, void* partial_ml,
       else return;
     }
 #undef LAUNCH_MFMA
-    if (num_splits > 1) {
-      dim3 cgrid(num_seqs, num_q_heads), cblock(HEAD_DIM);
-      hipLaunchKernelGGL(decode_combine_kernel, cgrid, cblock, 0, stream,
-                         (__hip_bfloat16*)out, (const float*)partial_o,
-                         (const float*)partial_ml, num_splits, num_q_heads);
-    }
+    DECODE_JOIN();
     return;
   }
   // variant 4 with a non-16 page size falls back to the dot2 kernel
@@ -1050,12 +1020,8 @@ void launch_decode_attention(void* out, void* partial_o, void* partial_ml,
     default: return;   // validated host-side
   }
 #undef LAUNCH_QPG
-  if (num_splits > 1) {
-    dim3 cgrid(num_seqs, num_q_heads), cblock(HEAD_DIM);
-    hipLaunchKernelGGL(decode_combine_kernel, cgrid, cblock, 0, stream,
-                       (__hip_bfloat16*)out, (const float*)partial_o,
-                       (const float*)partial_ml, num_splits, num_q_heads);
-  }
+  DECODE_JOIN();
+#undef DECODE_JOIN
 }
 
 }  // extern "C"

@@ -1,0 +1,104 @@
+// Parts of a sequence in decode attention, and the sum of what they left.
+#pragma once
+#include "common.h"
+
+namespace {
+
+constexpr int DIM = 128, PART_ROUND = 128;
+constexpr float LOW = -1e30f;
+
+// Keys of a part: not a share of the table's capacity, which may be many times
+// a sequence's length (one of 2048 keys, 8 heads, tables of 8192 / 40960 /
+// 131072 keys: 11.0 / 20.7 / 27.4 us with shares of the capacity, 11.1 of any).
+DEV_INLINE int part_keys(int ctx, int least, int splits) {
+  const int all = splits * PART_ROUND;
+  return max(least, (ctx + all - 1) / all * PART_ROUND);
+}
+
+// A workgroup per query head adds the parts' sums, in shares that meet in LDS.
+// Bound by latency: the loads of a round of 8 parts are independent (one load
+// after another took 9-10 us for 16 parts of one sequence).  Of more than 8
+// parts there are four shares (3 sequences of up to 15000 tokens, 30 parts: 40.7
+// -> 36.7 us with the attention); else one, whose workgroups are a quarter of
+// the threads (128 x 2080: 174 us against 180).
+// lens: parts are of part_keys(length, least, splits), a sequence of one part
+// has no sums.  null: every sequence has `splits` of them, perhaps empty ones.
+// to_base2: of the maxima, 1 or log2(e).
+template <int SHARES>
+__global__ __launch_bounds__(DIM * SHARES) void decode_join_kernel(
+    __hip_bfloat16* __restrict__ out,       // [seqs, QH, DIM]
+    const float* __restrict__ part_o,       // [splits, seqs, QH, DIM]
+    const float* __restrict__ part_ml,      // [splits, seqs, QH, 2]
+    const int* __restrict__ lens, const int least, const int splits,
+    const float to_base2) {
+  const int seq = blockIdx.y, d = threadIdx.x % DIM;
+  const int share = threadIdx.x / DIM;
+  int n = splits;
+  if (lens) {
+    const int ctx = lens[seq], span = part_keys(ctx, least, splits);
+    if (ctx <= span) return;
+    n = min((ctx + span - 1) / span, splits);
+  }
+  const size_t row = (size_t)seq * gridDim.x + blockIdx.x;
+  const size_t step = (size_t)gridDim.y * gridDim.x;
+  __shared__ float meet[SHARES][DIM + 2];
+  float top = LOW, o = 0.f, total = 0.f;
+  for (int first = share; first < n; first += 8 * SHARES) {
+    float ms[8], ls[8], os[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      // past the end: the last part again, without weight
+      const size_t at = min(first + i * SHARES, n - 1) * step + row;
+      ms[i] = part_ml[at * 2] * to_base2;
+      ls[i] = part_ml[at * 2 + 1];
+      os[i] = part_o[at * DIM + d];
+    }
+    float most = top;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) most = fmaxf(most, ms[i]);
+    const float fade = __builtin_amdgcn_exp2f(top - most);
+    top = most;
+    o *= fade;
+    total *= fade;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (first + i * SHARES < n) {
+        const float f = __builtin_amdgcn_exp2f(ms[i] - top);
+        o += os[i] * f;
+        total += ls[i] * f;
+      }
+  }
+  meet[share][d] = o;
+  if (d == 0) {
+    meet[share][DIM] = top;
+    meet[share][DIM + 1] = total;
+  }
+  __syncthreads();
+  if (share) return;
+#pragma unroll
+  for (int k = 0; k < SHARES; ++k) top = fmaxf(top, meet[k][DIM]);
+  o = total = 0.f;
+#pragma unroll
+  for (int k = 0; k < SHARES; ++k) {
+    const float f = __builtin_amdgcn_exp2f(meet[k][DIM] - top);
+    o += meet[k][d] * f;
+    total += meet[k][DIM + 1] * f;
+  }
+  out[row * DIM + d] = f2bf(total > 0.f ? o / total : 0.f);
+}
+
+inline void launch_decode_join(__hip_bfloat16* out, const float* part_o,
+                               const float* part_ml, const int* lens,
+                               int least, int splits, int heads, int seqs,
+                               float to_base2, hipStream_t stream) {
+  if (splits <= 1) return;
+  const dim3 grid(heads, seqs);
+  if (splits <= 8)
+    decode_join_kernel<1><<<grid, dim3(DIM), 0, stream>>>(
+        out, part_o, part_ml, lens, least, splits, to_base2);
+  else
+    decode_join_kernel<4><<<grid, dim3(DIM * 4), 0, stream>>>(
+        out, part_o, part_ml, lens, least, splits, to_base2);
+}
+
+}  // namespace

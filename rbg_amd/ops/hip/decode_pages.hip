@@ -17,14 +17,14 @@
 //    lengths fills the chip as a regular one does; longer ones only where the
 //    grid has too few for the sequence.  The grid is fixed when a step is
 //    captured; workgroups past the end of their sequence leave at once.
-#include "common.h"
+#include "decode_join.h"
 
 namespace {
 
-constexpr int DIM = 128, PAGE = 16, WAVES = 4, STEP = 32;
+constexpr int PAGE = 16, WAVES = 4, STEP = 32;
 constexpr int VROW = 528;         // of a 16-dim column of 32 values: 512 + pad,
                                   // so that writes of a row meet no conflicts
-constexpr float LOW = -1e30f;
+static_assert(WAVES * STEP == PART_ROUND, "parts are whole rounds");
 
 typedef __attribute__((ext_vector_type(4))) unsigned int dp_u4;
 
@@ -36,15 +36,6 @@ DEV_INLINE bf16x8 dp_frag(dp_u4 u) {
   union { dp_u4 u; bf16x8 v; } c;
   c.u = u;
   return c.v;
-}
-
-// Keys of a workgroup: not a share of the table's capacity, which may be many
-// times a sequence's length (one of 2048 keys, 8 heads, tables of 8192 / 40960 /
-// 131072 keys: 11.0 / 20.7 / 27.4 us with shares of the capacity, 11.1 of any).
-DEV_INLINE int part_keys(int ctx, int span, int splits) {
-  constexpr int ROUND = WAVES * STEP;
-  const int all = splits * ROUND;
-  return max(span, (ctx + all - 1) / all * ROUND);
 }
 
 // TOGETHER: all key heads of a (sequence, part) run on one XCD, workgroup i on
@@ -269,71 +260,6 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
   }
 }
 
-// Sequences of several workgroups: a workgroup per query head adds their sums,
-// in shares that meet in LDS.  Bound by latency: the loads of a round of 8 parts
-// are independent (one load after another took 9-10 us for 16 parts of one
-// sequence).  Of more than 8 parts there are four shares (3 sequences of up to
-// 15000 tokens, 30 parts: 40.7 -> 36.7 us with the attention); else one, whose
-// workgroups are a quarter of the threads (128 x 2080: 174 us against 180).
-template <int SHARES>
-__global__ __launch_bounds__(DIM * SHARES) void decode_join_kernel(
-    __hip_bfloat16* __restrict__ out, const float* __restrict__ part_o,
-    const float* __restrict__ part_ml, const int* __restrict__ lens,
-    const int least, const int splits) {
-  const int seq = blockIdx.y, d = threadIdx.x % DIM;
-  const int share = threadIdx.x / DIM;
-  const int ctx = lens[seq];
-  const int span = part_keys(ctx, least, splits);
-  if (ctx <= span) return;
-  const int n = min((ctx + span - 1) / span, splits);
-  const size_t row = (size_t)seq * gridDim.x + blockIdx.x;
-  const size_t step = (size_t)gridDim.y * gridDim.x;
-  __shared__ float meet[SHARES][DIM + 2];
-  float top = LOW, o = 0.f, total = 0.f;
-  for (int first = share; first < n; first += 8 * SHARES) {
-    float ms[8], ls[8], os[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      // past the end: the last part again, without weight
-      const size_t at = min(first + i * SHARES, n - 1) * step + row;
-      ms[i] = part_ml[at * 2];
-      ls[i] = part_ml[at * 2 + 1];
-      os[i] = part_o[at * DIM + d];
-    }
-    float most = top;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) most = fmaxf(most, ms[i]);
-    const float fade = __builtin_amdgcn_exp2f(top - most);
-    top = most;
-    o *= fade;
-    total *= fade;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (first + i * SHARES < n) {
-        const float f = __builtin_amdgcn_exp2f(ms[i] - top);
-        o += os[i] * f;
-        total += ls[i] * f;
-      }
-  }
-  meet[share][d] = o;
-  if (d == 0) {
-    meet[share][DIM] = top;
-    meet[share][DIM + 1] = total;
-  }
-  __syncthreads();
-  if (share) return;
-#pragma unroll
-  for (int k = 0; k < SHARES; ++k) top = fmaxf(top, meet[k][DIM]);
-  o = total = 0.f;
-#pragma unroll
-  for (int k = 0; k < SHARES; ++k) {
-    const float f = __builtin_amdgcn_exp2f(meet[k][DIM] - top);
-    o += meet[k][d] * f;
-    total += meet[k][DIM + 1] * f;
-  }
-  out[row * DIM + d] = f2bf(total > 0.f ? o / total : 0.f);
-}
-
 }  // namespace
 
 extern "C" void launch_decode_pages(
@@ -342,7 +268,7 @@ extern "C" void launch_decode_pages(
     int seqs, int heads, int kv_heads, int max_pages, int splits, int span,
     int q_stride, hipStream_t stream) {
   // in whole rounds of the waves
-  span = max(1, (span + WAVES * STEP - 1) / (WAVES * STEP)) * WAVES * STEP;
+  span = max(1, (span + PART_ROUND - 1) / PART_ROUND) * PART_ROUND;
   const dim3 grid(kv_heads, seqs, splits), block(64 * WAVES);
 #define DP_LAUNCH(QPG, TOGETHER)                                           \
   decode_pages_kernel<QPG, TOGETHER><<<grid, block, 0, stream>>>(          \
@@ -364,12 +290,8 @@ extern "C" void launch_decode_pages(
   }
 #undef DP_LAUNCH
 #undef DP_GO
-#define DP_JOIN(SHARES)                                                    \
-  decode_join_kernel<SHARES>                                               \
-      <<<dim3(heads, seqs), dim3(DIM * SHARES), 0, stream>>>(              \
-          (__hip_bfloat16*)out, (const float*)part_o,                      \
-          (const float*)part_ml, (const int*)lens, span, splits)
-  if (splits > 1 && splits <= 8) DP_JOIN(1);
-  if (splits > 8) DP_JOIN(4);
-#undef DP_JOIN
+  // sums to the base of 2
+  launch_decode_join((__hip_bfloat16*)out, (const float*)part_o,
+                     (const float*)part_ml, (const int*)lens, span, splits,
+                     heads, seqs, 1.f, stream);
 }

@@ -84,3 +84,14 @@ def test_default_parts_are_bounded():
                   for b in range(1, 257)]
         assert all(b >= a / 2 and a >= b / 2
                    for a, b in zip(counts, counts[1:]))
+
+
+def test_parts_of_other_pages():
+    """Only pages of 16 have the form whose parts many pairs gain by."""
+    for cap in (8192, 131072):
+        for bs in (64, 128, 256):
+            assert pick_decode_splits(bs, 8, cap, variant=7, page_size=32) == \
+                pick_decode_splits(bs, 8, cap, variant=4)
+        for bs in (1, 8, 48):
+            assert pick_decode_splits(bs, 8, cap, variant=7, page_size=32) == \
+                pick_decode_splits(bs, 8, cap, variant=7)

@@ -791,3 +791,20 @@ def test_decode_part_lengths(splits, span):
     kv = _paged(dev, lens, 2, 4096)
     got = ops._hip.decode_attention(q, *kv, 0.3, splits, 7, span)
     _near_decode(got, q, *kv, 0.3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("variant", [4, 7])
+@pytest.mark.parametrize("page", [8, 16, 32, 64])
+@pytest.mark.parametrize("splits", [1, 2, 8, 9, 31])
+def test_decode_parts_of_any_page(variant, page, splits):
+    """Forms whose every part leaves sums, empty ones too: one share and four,
+    more than a round of eight each."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    lens = [1, 17, 300, 497, 1000]
+    q = torch.randn(len(lens), 8, 128, device=dev).bfloat16()
+    kv = _paged(dev, lens, 2, 2048, page)
+    got = ops.decode_attention(q, *kv, 0.2, splits, variant)
+    _near_decode(got, q, *kv, 0.2)
+    _near_decode(ops.decode_attention(q, *kv, 0.2), q, *kv, 0.2)
