@@ -84,7 +84,8 @@ __global__ __launch_bounds__(DIM * SHARES) void decode_join_kernel(
     o += meet[k][d] * f;
     total += meet[k][DIM + 1] * f;
   }
-  out[row * DIM + d] = f2bf(total > 0.f ? o / total : 0.f);
+  // no keys: 0; weights that are no numbers: no number
+  out[row * DIM + d] = f2bf(total == 0.f ? 0.f : o / total);
 }
 
 inline void launch_decode_join(__hip_bfloat16* out, const float* part_o,

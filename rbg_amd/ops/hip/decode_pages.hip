@@ -247,8 +247,8 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
       total += sums[w][h][1] * f;
     }
     const size_t row = (size_t)seq * heads + kvh * QPG + h;
-    if (ctx <= span) {
-      out[row * DIM + d] = f2bf(total > 0.f ? o / total : 0.f);
+    if (ctx <= span) {        // no keys: 0; NaN stays
+      out[row * DIM + d] = f2bf(total == 0.f ? 0.f : o / total);
     } else {
       const size_t at_row = (size_t)split * gridDim.y * heads + row;
       part_o[at_row * DIM + d] = o;

@@ -808,3 +808,24 @@ def test_decode_parts_of_any_page(variant, page, splits):
     got = ops.decode_attention(q, *kv, 0.2, splits, variant)
     _near_decode(got, q, *kv, 0.2)
     _near_decode(ops.decode_attention(q, *kv, 0.2), q, *kv, 0.2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [1, 4, 12])
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+def test_decode_shows_broken_rows(splits, bad):
+    """A query or key that is no number leaves no plausible zeros, and stays
+    in its row; a sequence without keys is zeros."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    q = torch.randn(4, 8, 128, device=dev).bfloat16()
+    kc, vc, tables, lens = _paged(dev, [900, 900, 900, 1], 2, 1024)
+    q[1, 5, 7] = bad
+    kc[tables[2, 3], 0, 5, 0] = math.nan
+    lens[3] = 0
+    got = ops._hip.decode_attention(q, kc, vc, tables, lens, 0.1, splits, 7)
+    assert got[1, 5].isnan().all() and got[2, :4].isnan().all()
+    assert (got[3] == 0).all()
+    rest = got.clone()
+    rest[1, 5] = rest[2, :4] = 0
+    assert rest.isfinite().all()
