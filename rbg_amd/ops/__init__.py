@@ -230,8 +230,10 @@ def rope_heads(proj, heads: int, q_norm, k_norm, eps: float, key_cache,
 
 def _takes_rows(src, residual: torch.Tensor, w: torch.Tensor) -> bool:
     """Can norm and GEMM be one launch (hip/skinny_rows.h)?  The shapes that its
-    kernel without a norm takes, in bf16 without parts."""
+    kernel without a norm takes, in bf16 without parts, whose normed rows are at
+    most 64 KB, as every workgroup keeps them in LDS."""
     return (_takes_skinny(residual, w) and residual.shape[0] <= 4 and
+            residual.numel() <= 32768 and
             residual.shape[1] % 2048 == 0 and residual.is_contiguous() and
             (src is None or (src.dtype == torch.bfloat16 and
                              src.is_contiguous())))

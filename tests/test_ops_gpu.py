@@ -829,3 +829,27 @@ def test_decode_shows_broken_rows(splits, bad):
     rest = got.clone()
     rest[1, 5] = rest[2, :4] = 0
     assert rest.isfinite().all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [32768, 34816])
+def test_norm_swiglu_widest_row(k):
+    """The widest row that the one launch holds, and one that it does not."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(k)
+    def rnd(*shape):
+        return torch.randn(*shape, device=dev, generator=gen)
+    x, res, nw = rnd(1, k).bfloat16(), rnd(1, k).bfloat16(), rnd(k).bfloat16()
+    w = (rnd(64, k) / k ** 0.5).bfloat16()
+    total = x.double() + res.double()
+    h = total * torch.rsqrt(total.square().mean() + 1e-5) * nw.double()
+    full = h @ w.double().t().contiguous()
+    want = torch.nn.functional.silu(full[:, :32]) * full[:, 32:]
+    for src in (x, None):
+        got, new = ops.norm_swiglu(src, res.clone(), nw, 1e-5, w)
+        if src is not None:
+            assert (got.double() - want).norm() <= 2 ** -7 * want.norm()
+            assert (new.double() - total).norm() <= 2 ** -8 * total.norm()
+        else:
+            assert torch.equal(new, res) and got.isfinite().all()
