@@ -113,7 +113,9 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
   }
 
   const int last = min(offset + q_first + tokens, len) - 1;   // key needed
-  const int tiles = last / TILE + 1;
+  // a sequence of fewer keys than queries has queries before its first key,
+  // whose result is 0: a block of only those reads no rows
+  const int tiles = last < 0 ? 0 : last / TILE + 1;
   const int wave_first = offset + q_first + wave * 32 / group;
   const int wave_end = offset + q_first + (wave * 32 + 31) / group;
   const int wave_tiles = min(tiles, min(wave_end, len - 1) / TILE + 1);
@@ -156,10 +158,12 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[d][i] = 0.f;
 
-  PF_SLOTS(0)
-  PF_ROWS(0)
-  PF_SLOTS(min(1, tiles - 1))
-  PF_PUT(0)
+  if (tiles > 0) {
+    PF_SLOTS(0)
+    PF_ROWS(0)
+    PF_SLOTS(min(1, tiles - 1))
+    PF_PUT(0)
+  }
   // A wave stages rows for the others beyond its own last tile, in a loop of
   // its own: a condition around the sums would have them copied every tile.
 #define PF_STAGE(t)                                                        \
@@ -253,6 +257,7 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
   l += __shfl_xor(l, 32, 64);
   if (my_row < q_rows && in < tokens * group) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
+    const bool seen = my_pos >= 0;      // else the sums are of masked scores
     __hip_bfloat16* op =
         out + ((size_t)(q_start + my_row) * num_q_heads + qh) * DIM + 4 * h;
 #pragma unroll
@@ -261,7 +266,8 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
       for (int i = 0; i < 4; ++i) {
         union { __hip_bfloat16 e[4]; uint2 u; } o;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) o.e[j] = f2bf(acc[d][i * 4 + j] * inv);
+        for (int j = 0; j < 4; ++j)
+          o.e[j] = f2bf(seen ? acc[d][i * 4 + j] * inv : 0.f);
         *reinterpret_cast<uint2*>(op + d * 32 + i * 8) = o.u;
       }
   }

@@ -853,3 +853,39 @@ def test_norm_swiglu_widest_row(k):
             assert (new.double() - total).norm() <= 2 ** -8 * total.norm()
         else:
             assert torch.equal(new, res) and got.isfinite().all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kvh", [(4, 1), (32, 8), (6, 2)])
+def test_prefill_fewer_keys_than_queries(heads, kvh):
+    """Queries before the first key are zeros; no keys at all, first, between
+    and last; rows beside pages."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    news, lens = [70, 200, 33, 130, 40], [0, 100, 40, 1, 0]
+    cu = [0] + torch.tensor(news).cumsum(0).tolist()
+    cu_k = [0] + torch.tensor(lens).cumsum(0).tolist()
+    q = torch.randn(cu[-1], heads, 128, device=dev).bfloat16()
+    k, v = torch.randn(2, cu_k[-1], kvh, 128, device=dev).bfloat16()
+    slots = torch.randperm(160, device=dev)[:cu_k[-1]]
+    pages = torch.zeros(2, 10, kvh, 16, 128, dtype=torch.bfloat16, device=dev)
+    pages[0, slots // 16, :, slots % 16] = k
+    pages[1, slots // 16, :, slots % 16] = v
+    cut = torch.tensor(cu, dtype=torch.int32, device=dev)
+    cut_k = torch.tensor(cu_k, dtype=torch.int32, device=dev)
+    got = ops.prefill_attention(q, k, v, cut, 0.2, cut_k)
+    assert torch.equal(got, ops.prefill_attention(
+        q, pages[0], pages[1], cut, 0.2, cut_k, slots=slots.int()))
+    for b, (new, n) in enumerate(zip(news, lens)):
+        rows = got[cu[b]:cu[b + 1]]
+        behind = max(0, new - n)
+        assert (rows[:behind] == 0).all()
+        if behind == new:
+            continue
+        at = torch.tensor([0, new - behind], dtype=torch.int32, device=dev)
+        at_k = torch.tensor([0, n], dtype=torch.int32, device=dev)
+        kb, vb = (t[cu_k[b]:cu_k[b + 1]] for t in (k, v))
+        want = ref.prefill_attention(q[cu[b] + behind:cu[b + 1]].float(),
+                                     kb.float(), vb.float(), at, 0.2, at_k)
+        # bf16 weights and result, values of unit variance
+        assert (rows[behind:].float() - want).abs().max() < 3e-2
