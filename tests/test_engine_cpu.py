@@ -132,3 +132,14 @@ def test_qwen3_family_qk_norm():
     # qwen3-32b preset has the reference benchmark shapes
     q32 = ModelConfig.preset("qwen3-32b")
     assert q32.qk_norm and q32.num_layers == 64 and q32.hidden_size == 5120
+
+
+def test_ids_count_from_the_end():
+    """An id of -1 is the vocabulary's last, as a tensor's index is."""
+    outs = []
+    for last in (511, -1):
+        eng = tiny_engine()
+        (s,) = eng.generate([[3, last, 7, last]],
+                            SamplingParams(max_new_tokens=3))
+        outs.append(s.output_tokens)
+    assert outs[0] == outs[1]
