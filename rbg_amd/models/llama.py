@@ -362,7 +362,7 @@ class LlamaForCausalLM(nn.Module):
             x = self.embed[tokens.long()]
         else:
             assert hidden is not None, "non-first PP stage needs hidden"
-            x = hidden
+            x = hidden.clone()      # the layers add to it in place
         residual = None
         for layer in self.layers:
             x, residual = layer(x, residual, batch, kv, self.cos_sin)

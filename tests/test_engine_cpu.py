@@ -143,3 +143,26 @@ def test_ids_count_from_the_end():
                             SamplingParams(max_new_tokens=3))
         outs.append(s.output_tokens)
     assert outs[0] == outs[1]
+
+
+def test_stage_leaves_its_input():
+    """A later stage does not write into the stream that it was given."""
+    from rbg_amd.engine.batch import ForwardBatch
+    from rbg_amd.models.llama import LlamaForCausalLM, PPContext
+    cfg = EngineConfig(model=ModelConfig.preset("tiny"), device="cpu",
+                       kv_pool_tokens=256)
+    model = LlamaForCausalLM(cfg.model, torch.device("cpu"),
+                             pp=PPContext(size=2, stage=1))
+    cache = PagedKVCache(cfg, torch.device("cpu"),
+                         num_layers=model.num_local_layers)
+    at = torch.arange(5, dtype=torch.int32)
+    hidden = torch.randn(5, cfg.model.hidden_size).bfloat16()
+    given = hidden.clone()
+    outs = []
+    for _ in range(2):
+        batch = ForwardBatch(mode="prefill", positions=at,
+                             slot_mapping=at + 16,
+                             cu_seqlens=torch.tensor([0, 5]).int())
+        outs.append(model.forward(None, batch, cache, hidden=hidden))
+    assert torch.equal(hidden, given)
+    assert torch.equal(outs[0], outs[1])
