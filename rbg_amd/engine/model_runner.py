@@ -10,6 +10,7 @@ delegates to SGLang (SURVEY §2.3 prefill/decode engine rows).
 """
 from __future__ import annotations
 
+import gc
 import logging
 from typing import Dict, List, Optional, Tuple
 
@@ -366,6 +367,9 @@ class ModelRunner:
         static["bt"] = torch.zeros(bs, self.max_pages_per_seq,
                                    dtype=torch.int32, device=self.device)
         batch = self._decode_batch(static, static["slots"], bs)
+        # an engine that was dropped in a cycle frees its pool when Python
+        # collects it, and a free ends a capture: now, not in the middle of one
+        gc.collect()
         # warm up allocations outside capture
         torch.cuda.synchronize()
         hidden = self.model.forward(static["tokens"], batch, self.cache)

@@ -1,6 +1,7 @@
 """Whole Llama-family steps against a plain float64 implementation: what one
 fused kernel hands the next, the paged cache, and decode inputs that stay on the
 device between steps."""
+import gc
 import math
 
 import pytest
@@ -200,3 +201,35 @@ def test_generated_steps(device, eager, norms, first, later):
         for at, tok in enumerate(s.output_tokens):
             row = wants[s.seq_id][s.num_prompt_tokens + at - 1]
             assert row.max() - row[tok] < NEAR * row.norm()
+
+
+@pytest.mark.gpu
+def test_capture_beside_garbage():
+    """An engine in a cycle of references, dropped before another captures its
+    step: its pool is not freed in the middle of that."""
+    def runner():
+        r = ModelRunner(engine_config(False, "cuda"))
+        seq = Sequence([1, 2, 3])
+        seq.block_table = BlockTable(r.cache)
+        seq.block_table.ensure(4)
+        r.feed([(seq, 0, [1, 2])], [[1]])
+        return r, seq
+    live, seq = runner()
+    inner, calls = live.model.logits, []
+
+    def logits(hidden):
+        calls.append(hidden)
+        if torch.cuda.is_current_stream_capturing():
+            gc.collect()
+        return inner(hidden)
+    live.model.logits = logits
+    gc.disable()
+    try:
+        dropped, _ = runner()
+        dropped.itself = dropped
+        del dropped, _
+        out = live.feed([(seq, 2, [3])], [[0]])
+    finally:
+        gc.enable()
+        del live.model.logits
+    assert len(calls) == 2 and out.isfinite().all()
