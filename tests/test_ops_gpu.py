@@ -889,3 +889,46 @@ def test_prefill_fewer_keys_than_queries(heads, kvh):
                                      kb.float(), vb.float(), at, 0.2, at_k)
         # bf16 weights and result, values of unit variance
         assert (rows[behind:].float() - want).abs().max() < 3e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,shift", [(64, 0), (128, 1), (128, 4), (256, 0)])
+@pytest.mark.parametrize("tokens", [1, 37])
+def test_rope_store_kv_any_rows(dim, shift, tokens):
+    """Head sizes and rows that the kernel of heads of 128 does not take: others
+    than 128, and queries and keys that begin between multiples of 16 bytes."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    heads, kvh = 6, 2
+    gen = torch.Generator(device=dev).manual_seed(dim + tokens)
+    q, k = (torch.randn(tokens, h * dim + 8, device=dev, generator=gen)
+            .bfloat16()[:, shift:shift + h * dim] for h in (heads, kvh))
+    v = torch.randn(tokens, kvh * dim + 8, device=dev,
+                    generator=gen).bfloat16()[:, :kvh * dim]
+    table = ref.build_cos_sin_table(dim, 512, device=dev)
+    pos = torch.randint(0, 512, (tokens,), device=dev, generator=gen).int()
+    slots = torch.randperm(48, device=dev, generator=gen)[:tokens].int()
+    if tokens > 1:
+        slots[1] = -1
+    kc, vc = torch.zeros(2, 3, kvh, 16, dim, device=dev).bfloat16()
+    cs = table[pos.long()].double()[:, None]
+    half = dim // 2
+
+    def rotated(t):
+        t = t.double().view(tokens, -1, dim)
+        a, b = t[..., :half], t[..., half:]
+        return torch.cat([a * cs[..., :half] - b * cs[..., half:],
+                          b * cs[..., :half] + a * cs[..., half:]], -1)
+    wants = [rotated(q), rotated(k)]
+    old = v.clone()
+    ops.rope_store_kv(q, k, v, kc, vc, table, pos, slots)
+    for got, want in zip((q, k), wants):
+        err = (got.double().view_as(want) - want).abs()
+        assert (err <= want.abs() * 2 ** -8 + 2e-5).all()
+    assert torch.equal(v, old)
+    for cache, rows in ((kc, k), (vc, v)):
+        want = torch.zeros_like(cache)
+        for t, s in enumerate(slots.tolist()):
+            if s >= 0:
+                want[s // 16, :, s % 16] = rows[t].view(kvh, dim)
+        assert torch.equal(cache, want)
