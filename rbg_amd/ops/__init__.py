@@ -120,9 +120,13 @@ def _takes_skinny(x: torch.Tensor, w: torch.Tensor) -> bool:
     return (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
             x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and
             _skinny(x.shape[0], w.shape[0], x.shape[1]) and
-            # what only the library takes: strides, rows that begin between
-            # multiples of 16 bytes, gradients
-            w.is_contiguous() and
+            _plain(x, w))
+
+
+def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Not what only the library takes: strides, rows that begin between
+    multiples of 16 bytes, gradients."""
+    return (w.is_contiguous() and
             (x.data_ptr() | w.data_ptr()) % 16 == 0 and
             not (torch.is_grad_enabled() and
                  (x.requires_grad or w.requires_grad)))
@@ -148,14 +152,37 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, w)
 
 
+def _glu(rows: int, n: int, k: int) -> bool:
+    """Does a gate/up product apply silu in the decode GEMM, which then
+    cannot split k?  Where its workgroups fill the chip all the same (us,
+    against the product, by linear_parts or the library, and silu_mul): up to
+    64 rows of a wide matrix (28672 x 4096: 64 rows 47 / 55; 18432 x 2560: 16
+    rows 26 / 57; not 38912 x 4096, a round and a small rest: 16 rows 76 / 72),
+    32 rows to 16384 columns (14336 x 4096: 32 rows 27 / 29, 64 rows 42 / 30;
+    not x 8192: 16 rows 60 / 48), and narrow ones of short k (7168 x 2048: 16
+    rows 13.1 / 15.4, x 4096 23.9 / 18.4; 11264 x 2048: 32 rows 14.1 / 17.5;
+    12288 x 4096: 16 rows 25.6 / 29.5, x 5120: 32 rows 33.6 / 29.7).  The form
+    of a few rows splits k within a workgroup (7168 x 8192: 4 rows 25 / 27)."""
+    if rows < 1 or n % 64 or k % 512:
+        return False
+    if rows <= 4 and k % 2048 == 0:
+        return True
+    if n <= 12288:
+        return (rows <= 2 and k <= 8192 or rows <= 32 and
+                (k <= (1536 if n <= 4096 else 2048) or
+                 n >= 10240 and k <= 4096))
+    if rows <= 16 and n <= 24576 and k <= 4096:
+        return True
+    return (k % 2048 == 0 and rows <= (32 if n <= 16384 else 64) and
+            not (32768 < n < 49152 and k > 2048) and
+            not (n <= 16384 and 6144 < k < 12288))
+
+
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T), w = [Wg; Wu]."""
-    # In the GEMM up to 64 rows of a wide matrix (28672 x 4096: 64 rows 47 us
-    # against 49 of the library and 5 of silu_mul; 128 rows 61 against 58) and
-    # 32 of a narrow one (11264 x 2048: 14 against 15 and 3.5), where the
-    # workgroups of an unsplit k fill the chip
-    if (_takes_skinny(x, w) and w.shape[0] % 64 == 0 and
-            x.shape[0] <= (64 if w.shape[0] > 12288 else 32)):
+    if (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
+            x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and
+            _glu(x.shape[0], w.shape[0], x.shape[1]) and _plain(x, w)):
         return _require_hip().skinny_swiglu(
             x if x.is_contiguous() else x.contiguous(), w)
     return silu_mul(linear_parts(x, w))

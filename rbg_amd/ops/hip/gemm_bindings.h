@@ -29,7 +29,8 @@ inline SkinnyPlan pick_skinny(int M, int N, int K) {
   // behind (5120 x 25600: 66 us against 50, 4096 x 14336: 22.4 against 24.3),
   // on short rows by less than a reduction costs (2048 x 5632, 1 row: 9.0
   // against 9.7, 4 rows 10.1 against 10.0)
-  if ((M <= 4 && K % 2048 == 0) || (M <= 2 && K <= 8192)) return {0, 1};
+  if ((M <= 4 && K % 2048 == 0) || (M <= 2 && K <= 8192 && N <= 12288))
+    return {0, 1};
   // up to 32 rows of a narrow matrix: workgroups of half the size, half again
   // as many as fit at once (6144 x 4096, one row: 13.2 us against 14.2; above
   // 32 rows A's copies cost more, 14336 x 4096, 64 rows: 30.1 against 26.7)

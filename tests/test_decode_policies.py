@@ -95,3 +95,17 @@ def test_parts_of_other_pages():
         for bs in (1, 8, 48):
             assert pick_decode_splits(bs, 8, cap, variant=7, page_size=32) == \
                 pick_decode_splits(bs, 8, cap, variant=7)
+
+
+def test_silu_in_the_product_fits_its_kernel():
+    """What the rule hands to the decode GEMM with silu is what it takes."""
+    from rbg_amd.ops import _glu
+    taken = 0
+    for n in (32, 64, 96, 1024, 4096, 10240, 12288, 12320, 14336, 18432, 51200):
+        for k in (256, 512, 1000, 2048, 2560, 4096, 8192):
+            for rows in (0, 1, 2, 4, 5, 16, 17, 32, 33, 64, 65):
+                glu = _glu(rows, n, k)
+                assert not glu or 1 <= rows <= 64
+                assert not glu or n % 64 == 0 and k % 512 == 0
+                taken += glu
+    assert taken > 100

@@ -932,3 +932,23 @@ def test_rope_store_kv_any_rows(dim, shift, tokens):
             if s >= 0:
                 want[s // 16, :, s % 16] = rows[t].view(kvh, dim)
         assert torch.equal(cache, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 2, 4, 5, 17, 32, 33, 64])
+@pytest.mark.parametrize("f,k", [(3584, 4096), (7168, 2048), (6176, 2560),
+                                 (8160, 2048), (9216, 2560), (19456, 2048)])
+def test_swiglu_routes(m, f, k):
+    """Both sides of the rule for silu within the GEMM, workgroups of 4 waves
+    up to 16384 columns and of 8 beyond; the bound of test_linear_swiglu."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(m * 7 + f)
+    x = torch.randn(m, k, device=dev, generator=gen).bfloat16()
+    w = (torch.randn(2 * f, k, device=dev, generator=gen) / k ** 0.5
+         ).bfloat16()
+    full = x.double() @ w.double().t().contiguous()
+    want = torch.nn.functional.silu(full[:, :f]) * full[:, f:]
+    bound = 2 ** -7 * (full[:, :f].abs() + 1) * (full[:, f:].abs() + 1)
+    for got in (ops._hip.skinny_swiglu(x, w), ops.linear_swiglu(x, w)):
+        assert ((got.double() - want).abs() <= bound).all()
