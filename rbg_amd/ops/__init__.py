@@ -96,30 +96,54 @@ def _on_gpu(t: torch.Tensor) -> bool:
 SKINNY_GEMM = int(__import__("os").environ.get("RBG_SKINNY_GEMM", "1"))
 
 
-def _skinny(rows: int, n: int, k: int) -> bool:
-    """Does the hand-written decode GEMM (hip/skinny_gemm.hip) take a [rows, k]
-    x [n, k] product, rather than hipBLASLt?  Measured with cold weights (us,
-    own with its reduction against library).  Narrow matrices at any decode
-    batch (4096 x 14336: 1 row 22 against 24, 64 rows 28 / 38, 128 rows 38 / 73;
-    10240 x 8192: 64 rows 39 / 41, 128 rows 50 / 55), the short ones up to 64
-    rows (3072 x 2048: 16 rows 7.6 / 8.6, 64 rows 9.5 / 9.2, 128 rows 12.5 /
-    12.0), the long ones further, as the library does not split k (4096 x 14336:
-    192 rows 47 / 99, 256 rows 62 / 59; 5120 x 25600: 256 rows 119 / 260).  Wide
-    matrices up to 64 rows (28672 x 4096: 1 row 40 / 57, 64 rows 46 / 49, 128
-    rows 58 / 53), where their rows are a multiple of 4 KB apart (51200 x 5120:
-    1 row 94 / 89, 64 rows 122 / 98)."""
+def _skinny(rows: int, n: int, k: int, parts: bool = False) -> bool:
+    """Does the hand-written decode GEMM (hip/skinny_gemm.hip) take a
+    [rows, k] x [n, k] product, rather than hipBLASLt?  ``parts``: its reader
+    adds up the parts of a split k, which saves a launch.  Measured over the
+    whole range with cold weights (us, own / library): the library is uneven.
+
+    Up to 10240 columns, as it splits k and the library does not: long ones at
+    any decode batch (4096 x 4096: 128 rows 19.5 / 24.4, 129 rows 22.1 / 22.1;
+    4096 x 14336: 192 rows 48 / 103, 256 rows 63 / 62; 5120 x 25600: 256 rows
+    121 / 261), short ones for few rows (4096 x 2048: 32 rows 9.8 / 11.9, 64
+    rows 13.1 / 12.4; 1024 x 4096: 64 rows 10.3 / 12.1, 128 rows 14.6 / 9.4).
+
+    Beyond, a few rows by the form for them (12288 x 8192: 4 rows 37 / 40,
+    28672 x 4096: 42 / 60), and short k up to 16 rows (18432 x 2560: 16 rows
+    26 / 55, 17 rows 25 / 23).  To 12288 columns its workgroups fill only two
+    thirds of the chip (12288 x 8192: 16 rows 43 / 40).
+
+    Wide ones up to 64 rows where rows of W are a multiple of 4 KB apart: the
+    library reads those at 4.6 TB/s and others at 5.8, and this kernel, whose
+    workgroups begin at different k, both at 5.3 to 6 (28672 x 4096: 64 rows
+    47 / 52, 128 rows 60 / 54; 1 row of 51200 x 4096 72 / 91, x 5120 98 / 91).
+    Not where there is a round of workgroups and a small rest (40960 x 4096: 64
+    rows 82 / 78), nor near 16384 x 8192, where the library is good (14336 x
+    8192: 16 rows 50 / 45, 64 rows 57 / 48)."""
     if rows < 1 or n % 32 or k % 512:
         return False
+    if n <= 10240:
+        if k <= 2048:
+            return rows <= (64 if parts else 32)
+        if n <= 2048 and not parts:
+            return rows <= min(256, k // 64)
+        return rows <= (256 if k > 16384 else 192 if k >= 12288 else 128)
+    if rows <= 4 and k % 2048 == 0 or rows <= 16 and n <= 24576 and k <= 4096:
+        return True
     if n <= 12288:
-        return rows <= (256 if k > 16384 else 192 if k >= 12288 else
-                        128 if k > 2048 else 64)
-    return rows <= 64 and k % 2048 == 0
+        return (16 < rows <= 256 if k > 16384 else
+                rows <= 64 and k <= 4096 if parts else
+                rows <= 32 and k <= 2048)
+    return (rows <= 64 and k % 2048 == 0 and
+            not (32768 < n < 49152 and k > 2048) and
+            not (n <= 16384 and 6144 < k < 12288))
 
 
-def _takes_skinny(x: torch.Tensor, w: torch.Tensor) -> bool:
+def _takes_skinny(x: torch.Tensor, w: torch.Tensor,
+                  parts: bool = False) -> bool:
     return (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
             x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and
-            _skinny(x.shape[0], w.shape[0], x.shape[1]) and
+            _skinny(x.shape[0], w.shape[0], x.shape[1], parts) and
             _plain(x, w))
 
 
@@ -146,7 +170,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear for a reader that adds up: where the GEMM splits k, the f32 sums
     [parts, T, N] before their reduction, else [T, N] in x's dtype."""
-    if _takes_skinny(x, w):
+    if _takes_skinny(x, w, parts=True):
         return _require_hip().skinny_parts(
             x if x.is_contiguous() else x.contiguous(), w)
     return torch.nn.functional.linear(x, w)

@@ -45,6 +45,45 @@ inline SkinnyPlan pick_skinny(int M, int N, int K) {
   return {8, std::max(1, std::min({256 / tiles, K / 256, 16}))};
 }
 
+// The same for a product whose parts a launch of its own adds up, which a few
+// long parts repay and many short ones do not: the form with the least time by
+// a model of it in us, fitted to all forms at 5083 shapes of 1 to 256 rows, 1024
+// to 128256 columns and 512 to 28672 k with cold weights.  Its choices take 0.7%
+// longer than the fastest form on average; pick_skinny's take 5.4% (8 rows, 1024
+// x 512: two parts 5.6, one 4.2 us; 128 rows, 10240 x 1024: 19.9 and 17.9).
+inline SkinnyPlan pick_summed(int M, int N, int K) {
+  // a few rows: where one round of workgroups covers N, or rows of W are a
+  // multiple of 4 KB apart (1 row, 4096 x 1536: 5.2 us against 7.3 of the other
+  // forms; 5120 x 2048 7.8 against 9.0, 5120 x 2560 13.1 against 11.0)
+  if (M <= 4 && K >= 1024 &&
+      (N <= 4096 ? K <= 3 * N
+                 : (N <= 8192 && K < 2048) || (K % 2048 == 0 && K <= 8192)))
+    return {0, 1};
+  const int tiles = (M + 15) / 16;
+  SkinnyPlan best{8, 1};
+  float least = 1e30f;
+  for (int waves = M <= 32 ? 4 : 8; waves <= 8; waves += 4)
+    for (int splits : {1, 2, 3, 4, 5, 6, 8, 12, 16}) {
+      if (splits > std::max(1, K / 256)) break;
+      const int groups = (N + 16 * waves - 1) / (16 * waves) * splits;
+      const int chunks = (K / 128 + splits - 1) / splits;
+      float t;
+      if (waves == 4)   // two on a CU share its bandwidth
+        t = (groups + 511) / 512 * chunks *
+            std::max(0.67f, std::min(2, (groups + 255) / 256) *
+                                (0.46f + 0.088f * tiles));
+      else
+        t = (groups + 255) / 256 * (0.69f + chunks * (0.63f + 0.16f * tiles));
+      if (splits > 1) t += 3.57f + 1.83e-6f * splits * M * N;
+      t *= 1.f + 0.0084f * (splits - 1);
+      if (t < least) {
+        least = t;
+        best = {waves, splits};
+      }
+    }
+  return best;
+}
+
 inline bool skinny_gemm_supported(int64_t M, int64_t N, int64_t K) {
   return M >= 1 && M <= 256 && (N % 32) == 0 && (K % 256) == 0;
 }
@@ -64,7 +103,7 @@ inline torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor w,
   check_skinny(a, w);
   const int64_t M = a.size(0), K = a.size(1), N = w.size(0);
   auto c = torch::empty({M, N}, a.options());
-  SkinnyPlan plan = pick_skinny((int)M, (int)N, (int)K);
+  SkinnyPlan plan = pick_summed((int)M, (int)N, (int)K);
   if (force_splits > 0 && K % (force_splits * 256) == 0)
     plan = {plan.waves ? plan.waves : 8, (int)force_splits};
   torch::Tensor ws;

@@ -109,3 +109,23 @@ def test_silu_in_the_product_fits_its_kernel():
                 assert not glu or n % 64 == 0 and k % 512 == 0
                 taken += glu
     assert taken > 100
+
+
+def test_decode_products_fit_their_kernels():
+    """What the rules hand to the decode GEMM is what it takes, and a reader of
+    parts gets them wherever a sum is worth its launch."""
+    from rbg_amd.ops import _skinny
+    sizes = (32, 64, 96, 1000, 1024, 2048, 4096, 5120, 10240, 10272, 12288,
+             12320, 14336, 16384, 24576, 32768, 40960, 51200, 128256)
+    taken = 0
+    for n in sizes:
+        for k in (256, 512, 1000, 2048, 2560, 4096, 8192, 12288, 25600):
+            for rows in (0, 1, 2, 4, 5, 16, 17, 32, 33, 64, 65, 128, 129, 192,
+                         256, 257):
+                own = _skinny(rows, n, k)
+                assert not own or 1 <= rows <= 256
+                assert not own or n % 32 == 0 and k % 512 == 0
+                if own and n <= 10240 and k > 2048 and rows <= 128:
+                    assert _skinny(rows, n, k, parts=True)
+                taken += own
+    assert taken > 500

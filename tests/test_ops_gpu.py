@@ -935,6 +935,26 @@ def test_rope_store_kv_any_rows(dim, shift, tokens):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 4, 5, 16, 32, 33, 65, 200])
+@pytest.mark.parametrize("n,k", [(64, 512), (96, 8192), (1024, 14336),
+                                 (4128, 1536), (9216, 2560), (14336, 1024)])
+def test_skinny_gemm_forms(m, n, k):
+    """The forms of summed products: a few rows, one part, up to 16 parts of
+    unequal length, workgroups of 4 and 8 waves.  Bounds as above: half an ulp
+    of the result and k roundings of 2^-24 of the sums of magnitudes."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(m * 1000003 + n + k)
+    x = torch.randn(m, k, device=dev, generator=gen).bfloat16()
+    w = torch.randn(n, k, device=dev, generator=gen).bfloat16()
+    want = x.double() @ w.double().t().contiguous()
+    bound = want.abs() * 2 ** -8 + \
+        (x.double().abs() @ w.double().abs().t().contiguous()) * k * 2 ** -24
+    for got in (ops._hip.skinny_gemm(x, w), ops.linear(x, w)):
+        assert ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [1, 2, 4, 5, 17, 32, 33, 64])
 @pytest.mark.parametrize("f,k", [(3584, 4096), (7168, 2048), (6176, 2560),
                                  (8160, 2048), (9216, 2560), (19456, 2048)])
