@@ -367,18 +367,25 @@ class ModelRunner:
         static["bt"] = torch.zeros(bs, self.max_pages_per_seq,
                                    dtype=torch.int32, device=self.device)
         batch = self._decode_batch(static, static["slots"], bs)
-        # an engine that was dropped in a cycle frees its pool when Python
-        # collects it, and a free ends a capture: now, not in the middle of one
-        gc.collect()
         # warm up allocations outside capture
         torch.cuda.synchronize()
         hidden = self.model.forward(static["tokens"], batch, self.cache)
         logits = self.model.logits(hidden)
         torch.cuda.synchronize()
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, pool=self._graph_pool):
-            hidden = self.model.forward(static["tokens"], batch, self.cache)
-            logits = self.model.logits(hidden)
+        # Python must not collect another engine, dropped in a cycle of
+        # references, just now: freeing its pool ends a capture, and its
+        # captured steps end the process
+        collects = gc.isenabled()
+        gc.disable()
+        try:
+            with torch.cuda.graph(graph, pool=self._graph_pool):
+                hidden = self.model.forward(static["tokens"], batch,
+                                            self.cache)
+                logits = self.model.logits(hidden)
+        finally:
+            if collects:
+                gc.enable()
         if self._graph_pool is None:
             self._graph_pool = graph.pool()
         self._graphs[bs] = (graph, static, logits)

@@ -204,32 +204,27 @@ def test_generated_steps(device, eager, norms, first, later):
 
 
 @pytest.mark.gpu
-def test_capture_beside_garbage():
-    """An engine in a cycle of references, dropped before another captures its
-    step: its pool is not freed in the middle of that."""
-    def runner():
-        r = ModelRunner(engine_config(False, "cuda"))
-        seq = Sequence([1, 2, 3])
-        seq.block_table = BlockTable(r.cache)
-        seq.block_table.ensure(4)
-        r.feed([(seq, 0, [1, 2])], [[1]])
-        return r, seq
-    live, seq = runner()
-    inner, calls = live.model.logits, []
+@pytest.mark.parametrize("collects", [True, False])
+def test_nothing_is_collected_in_a_capture(collects):
+    """Python's own collection, which may free a dropped engine's pool and
+    captured steps, rests while a step is captured."""
+    runner = ModelRunner(engine_config(False, "cuda"))
+    seq = Sequence([1, 2, 3])
+    seq.block_table = BlockTable(runner.cache)
+    seq.block_table.ensure(4)
+    runner.feed([(seq, 0, [1, 2])], [[1]])
+    inner, seen = runner.model.logits, []
 
     def logits(hidden):
-        calls.append(hidden)
         if torch.cuda.is_current_stream_capturing():
-            gc.collect()
+            seen.append(gc.isenabled())
         return inner(hidden)
-    live.model.logits = logits
-    gc.disable()
+    runner.model.logits = logits
     try:
-        dropped, _ = runner()
-        dropped.itself = dropped
-        del dropped, _
-        out = live.feed([(seq, 2, [3])], [[0]])
+        gc.enable() if collects else gc.disable()
+        out = runner.feed([(seq, 2, [3])], [[0]])
+        assert gc.isenabled() == collects
     finally:
         gc.enable()
-        del live.model.logits
-    assert len(calls) == 2 and out.isfinite().all()
+        del runner.model.logits
+    assert seen == [False] and out.isfinite().all()
