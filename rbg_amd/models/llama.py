@@ -357,9 +357,7 @@ class LlamaForCausalLM(nn.Module):
         Non-last stages return the combined stream to send onward; the last
         stage returns final-normed hidden states ready for logits()."""
         if self.pp.first:
-            # not embedding(), which takes no ids that count from the end (and
-            # ends the process on a GPU), though a row's gather is 3 us less
-            x = self.embed[tokens.long()]
+            x = ops.embed_rows(tokens, self.embed)
         else:
             assert hidden is not None, "non-first PP stage needs hidden"
             x = hidden.clone()      # the layers add to it in place

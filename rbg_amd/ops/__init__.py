@@ -212,6 +212,17 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return silu_mul(linear_parts(x, w))
 
 
+def embed_rows(ids: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
+    """table[ids]; NaN for an id outside where the kernel takes the call (1.8 us
+    for a row of 4096, the indexing kernel 3.0; 128 rows 2.0 both)."""
+    if (_on_gpu(table) and table.dtype == torch.bfloat16 and
+            table.dim() == 2 and ids.dim() == 1 and
+            table.is_contiguous() and table.shape[1] % 8 == 0 and
+            table.data_ptr() % 16 == 0):
+        return _require_hip().embed_rows(ids.long().contiguous(), table)
+    return table[ids.long()]
+
+
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     if _on_gpu(x):
         return _require_hip().rmsnorm(x, weight, eps)

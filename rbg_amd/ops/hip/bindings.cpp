@@ -24,6 +24,8 @@ void launch_norm_rows(void*, const void*, const void*, void*, const void*,
                       float, const void*, int, int, int, int, const void*,
                       const void*, const void*, void*, void*, int, int, int,
                       hipStream_t);
+void launch_embed_rows(void*, const void*, const void*, long, int, int,
+                       hipStream_t);
 void launch_silu_parts(void*, const void*, int, int, int, hipStream_t);
 void launch_silu_mul(void*, const void*, int, int, hipStream_t);
 void launch_rope_store_kv(void*, void*, const void*, void*, void*,
@@ -145,6 +147,23 @@ torch::Tensor add_rmsnorm(torch::Tensor x, torch::Tensor residual,
                             weight.data_ptr(), (float)eps,
                             split ? (int)x.size(0) : 0, rows, hidden,
                             current_stream());
+  return out;
+}
+
+// table's rows of the ids, bf16; below 0 from its end, NaN where there is none
+torch::Tensor embed_rows(torch::Tensor ids, torch::Tensor table) {
+  check_bf16_contig(table, "table");
+  TORCH_CHECK(ids.is_cuda() && ids.is_contiguous() && ids.dim() == 1 &&
+              ids.scalar_type() == torch::kInt64, "ids must be int64 on GPU");
+  TORCH_CHECK(table.dim() == 2 && table.size(1) % 8 == 0 &&
+              (reinterpret_cast<uintptr_t>(table.data_ptr()) & 15) == 0,
+              "rows of whole, aligned 16 bytes");
+  TORCH_CHECK(table.size(1) > 0 && ids.numel() < (1ll << 31), "sizes");
+  auto out = torch::empty({ids.numel(), table.size(1)}, table.options());
+  if (ids.numel())
+    launch_embed_rows(out.data_ptr(), table.data_ptr(), ids.data_ptr(),
+                      table.size(0), (int)table.size(1), (int)ids.numel(),
+                      current_stream());
   return out;
 }
 
@@ -634,6 +653,7 @@ torch::Tensor xgmi_allreduce(torch::Tensor inp,
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm", &rmsnorm, "RMSNorm (bf16)");
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm, "x,residual += ; rmsnorm");
+  m.def("embed_rows", &embed_rows, "rows of an embedding table");
   m.def("silu_mul", &silu_mul, "silu(gate)*up");
   m.def("rope_store_kv", &rope_store_kv, "RoPE + paged KV write");
   m.def("decode_attention", &decode_attention, "paged flash-decode",

@@ -30,6 +30,7 @@ HIP_SOURCES = {
         "attn_decode.hip",
         "decode_pages.hip",
         "decode_rows.hip",
+        "embed_rows.hip",
         "attn_prefill.hip",
         "prefill_flash.hip",
         "mfma_probe.hip",

@@ -972,3 +972,26 @@ def test_swiglu_routes(m, f, k):
     bound = 2 ** -7 * (full[:, :f].abs() + 1) * (full[:, f:].abs() + 1)
     for got in (ops._hip.skinny_swiglu(x, w), ops.linear_swiglu(x, w)):
         assert ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,width", [(7, 8), (300, 256), (512, 4096),
+                                        (64, 8200), (50, 20)])
+@pytest.mark.parametrize("count", [0, 1, 131])
+def test_embed_rows(rows, width, count):
+    """The indexed rows, from the end below 0; ids without a row touch no
+    memory and give NaN; a width that only indexing takes."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    table = torch.randn(rows, width, device=dev).bfloat16()
+    ids = torch.randint(-rows, rows, (count,), device=dev)
+    if count > 1:
+        ids[0], ids[1] = -rows, rows - 1
+    want = table.cpu()[ids.cpu()]
+    assert torch.equal(ops.embed_rows(ids, table).cpu(), want)
+    assert torch.equal(ops.embed_rows(ids.int(), table).cpu(), want)
+    if count > 1 and width % 8 == 0:
+        ids[2], ids[3], ids[4] = rows, -rows - 1, 1 << 40
+        got = ops.embed_rows(ids, table)
+        assert got[2:5].isnan().all()
+        assert torch.equal(got[5:].cpu(), want[5:])
