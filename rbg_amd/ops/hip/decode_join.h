@@ -11,8 +11,9 @@ constexpr float LOW = -1e30f;
 // a sequence's length (one of 2048 keys, 8 heads, tables of 8192 / 40960 /
 // 131072 keys: 11.0 / 20.7 / 27.4 us with shares of the capacity, 11.1 of any).
 DEV_INLINE int part_keys(int ctx, int least, int splits) {
+  if (ctx <= least * splits) return least;
   const int all = splits * PART_ROUND;
-  return max(least, (ctx + all - 1) / all * PART_ROUND);
+  return (ctx + all - 1) / all * PART_ROUND;
 }
 
 // A workgroup per query head adds the parts' sums, in shares that meet in LDS.
