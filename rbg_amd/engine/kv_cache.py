@@ -40,7 +40,7 @@ class PagedKVCache:
         self.ipc_exportable = False
         self._alloc_storage(device)
         # page 0 is reserved scratch: hipGraph decode padding rows write
-        # their (dead) KV slot there (model_runner._decode_graph)
+        # their (dead) KV slot there (ModelRunner._build_decode_state)
         self._free: List[int] = list(range(num_pages - 1, 0, -1))
         import threading
         self._lock = threading.Lock()   # alloc/free may race import threads

@@ -115,7 +115,8 @@ def _skinny(rows: int, n: int, k: int, parts: bool = False) -> bool:
 
     Wide ones up to 64 rows where rows of W are a multiple of 4 KB apart: the
     library reads those at 4.6 TB/s and others at 5.8, and this kernel, whose
-    workgroups begin at different k, both at 5.3 to 6 (28672 x 4096: 64 rows
+    workgroups begin at different k, both at 5.3 to 6; the form of a few rows
+    loads more than once where k is no multiple of 2048 (28672 x 4096: 64 rows
     47 / 52, 128 rows 60 / 54; 1 row of 51200 x 4096 72 / 91, x 5120 98 / 91).
     Not where there is a round of workgroups and a small rest (40960 x 4096: 64
     rows 82 / 78), nor near 16384 x 8192, where the library is good (14336 x

@@ -256,6 +256,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gated_chunk", &gated_chunk, "gated delta rule, by chunks");
   m.attr("CHUNK") = gated_chunk_tokens();
   m.attr("CHUNK_MAX_DIM") = gated_chunk_max_dim();
-  m.def("skinny_gemm", &skinny_gemm, "decode-shape GEMM (M<=128)",
+  m.def("skinny_gemm", &skinny_gemm, "decode-shape GEMM (M<=256)",
         py::arg("a"), py::arg("w"), py::arg("force_splits") = 0);
 }

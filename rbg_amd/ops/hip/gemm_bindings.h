@@ -25,10 +25,11 @@ struct SkinnyPlan {
 };
 
 inline SkinnyPlan pick_skinny(int M, int N, int K) {
-  // a few rows; where rows of W are no multiple of 4 KB apart the kernel falls
-  // behind (5120 x 25600: 66 us against 50, 4096 x 14336: 22.4 against 24.3),
-  // on short rows by less than a reduction costs (2048 x 5632, 1 row: 9.0
-  // against 9.7, 4 rows 10.1 against 10.0)
+  // a few rows, where K is whole turns of that kernel (8 waves x 4 chunks of 64
+  // in flight; in a part of one it loads the last chunk again, with K = 2560 8
+  // times for 5 chunks), or short, where that costs less than a reduction (2048 x
+  // 5632, 1 row: 9.0 us against 9.7, 4 rows 10.1 against 10.0).  5120 x 25600
+  // takes 66 us against 50, most of it for 320 workgroups on 256 CUs.
   if ((M <= 4 && K % 2048 == 0) || (M <= 2 && K <= 8192 && N <= 12288))
     return {0, 1};
   // up to 32 rows of a narrow matrix: workgroups of half the size, half again
@@ -52,9 +53,9 @@ inline SkinnyPlan pick_skinny(int M, int N, int K) {
 // longer than the fastest form on average; pick_skinny's take 5.4% (8 rows, 1024
 // x 512: two parts 5.6, one 4.2 us; 128 rows, 10240 x 1024: 19.9 and 17.9).
 inline SkinnyPlan pick_summed(int M, int N, int K) {
-  // a few rows: where one round of workgroups covers N, or rows of W are a
-  // multiple of 4 KB apart (1 row, 4096 x 1536: 5.2 us against 7.3 of the other
-  // forms; 5120 x 2048 7.8 against 9.0, 5120 x 2560 13.1 against 11.0)
+  // a few rows: where one round of workgroups covers N, or K is whole turns of
+  // that kernel (1 row, 4096 x 1536: 5.2 us against 7.3 of the other forms; 5120
+  // x 2048 7.8 against 9.0, 5120 x 2560 13.1 against 11.0)
   if (M <= 4 && K >= 1024 &&
       (N <= 4096 ? K <= 3 * N
                  : (N <= 8192 && K < 2048) || (K % 2048 == 0 && K <= 8192)))

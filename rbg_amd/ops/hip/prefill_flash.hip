@@ -2,9 +2,9 @@
 // as rows or, behind a past, straight from the pages.
 //
 // Bound: the matrix cores (4 * 128 operations per pair of tokens) and beside
-// them the exponentials: 920 TFLOP/s at 8192 tokens of 32 heads, where the
-// 16-row form this replaces reached 346, and 590 at 2048, where few workgroups
-// have most of the work.  A workgroup is 4 waves of 32 query rows each; tiles
+// them the exponentials: 870 to 910 TFLOP/s at 8192 tokens of 32 heads, where
+// the 16-row form this replaces reached 346, and 580 to 630 at 2048, where few
+// workgroups have most of the work.  A workgroup is 4 waves of 32 query rows each; tiles
 // of 64 keys pass LDS in two buffers, one barrier a tile, the next tile's rows
 // in flight meanwhile.  (Forming the next tile's scores beside this tile's
 // exponentials, for 28 more registers, measured the same.)

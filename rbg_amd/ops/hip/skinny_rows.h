@@ -56,7 +56,7 @@ struct RowsRope {
 // barrier until their sums meet in LDS, and without splits whose sums another
 // launch would add.  4096 x 4096, one row: 8.5 us against 10.5 of
 // skinny_gemm_kernel with its reduction.  Its time grows with the rows, since
-// every workgroup reads all of A (28672 x 4096: 4 rows 40 us, 16 rows 56).
+// every workgroup reads all of A (28672 x 4096: 1 row 41.8 us, 4 rows 44.3).
 // GLU and ROPE: the tile is 8 rows of W and the 8 that they meet, N / 2 or 64
 // further on.
 // NORM: every workgroup forms A for itself, in LDS, while its first weights are
