@@ -168,9 +168,42 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, w)
 
 
+def _tile(rows: int, n: int, k: int) -> bool:
+    """Does the GEMM of prompts (hip/tile_gemm.hip) take a [rows, k] x [n, k]
+    product whose reader adds up parts, rather than the decode GEMM or
+    hipBLASLt?  It splits k where its tiles are few, which the library does not,
+    and picks a tile by the shape.  Against what is taken without it, with the
+    norm that reads the sums (us): from 129 rows (4096 x 4096: 160 rows 25 / 17;
+    4096 x 14336: 256 rows 62 / 44, 2048 rows 214 / 182; 5120 x 25600: 512 rows
+    270 / 128; 6144 x 4096: 1500 rows 76 / 60), before that only of long rows
+    (4096 x 14336: 128 rows 34 / 32; 5120 x 25600: 97 rows 71 / 61).  Not short k
+    (2048 x 2048: 256 rows 10 / 11), and from 257 rows to 999 only k from 5120 on
+    (6144 x 4096: 512 rows 36 / 38), then not matrices with little to split
+    (4096 x 4096: 1280 rows 56 / 60; 2048 x 5632: 1400 rows 42 / 45).  Above 4096
+    rows the library's tiles are as full (8192 rows: 6144 x 4096 276 / 293, 4096 x
+    14336 615 / 644), and wide matrices give it enough of them (16384 x 4096: 2048
+    rows 243 / 256)."""
+    if k < 3584 or k % 64 or n % 64 or not 2048 <= n <= 14336:
+        return False
+    if rows <= 128:
+        return rows > 64 and k >= 12288
+    if rows < 1000:
+        return rows <= 256 or k >= 5120
+    return rows <= 4096 and (k >= 8192 or n >= 4096 and n * k > 2 ** 24)
+
+
+def _takes_tile(x: torch.Tensor, w: torch.Tensor, rule) -> bool:
+    return (_on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
+            x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and
+            x.shape[1] == w.shape[1] and
+            rule(x.shape[0], w.shape[0], x.shape[1]) and _plain(x, w))
+
+
 def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear for a reader that adds up: where the GEMM splits k, the f32 sums
     [parts, T, N] before their reduction, else [T, N] in x's dtype."""
+    if x.shape[0] > 64 and _takes_tile(x, w, _tile):
+        return _require_hip().tile_parts(x.contiguous(), w)
     if _takes_skinny(x, w, parts=True):
         return _require_hip().skinny_parts(
             x if x.is_contiguous() else x.contiguous(), w)
@@ -203,8 +236,30 @@ def _glu(rows: int, n: int, k: int) -> bool:
             not (n <= 16384 and 6144 < k < 12288))
 
 
+def _tile_glu(rows: int, n: int, k: int) -> bool:
+    """Does it take a gate/up product, with silu?  Against the product and
+    silu_mul, or the decode GEMM (us): from 129 rows (28672 x 4096: 256 rows 74 /
+    64, 512 rows 113 / 105, 2048 rows 387 / 350, 8192 rows 1417 / 1341; 11264 x
+    2048: 256 rows 30 / 22, 2048 rows 95 / 82).  Not where parts of k, which silu
+    cannot have, fill the chip better (16384 x 4096: 176 rows 46 / 51; 12288 x
+    6144: 640 rows 100 / 122; 8192 x 28672: 1200 rows 472 / 495), and around 320
+    rows, a round and a quarter of its tiles, only of narrower matrices (51200 x
+    5120: 199 / 217; 14336 x 4096: 53 / 53).  From 65 rows where tiles of 128 x 128
+    nearly fill the chip once (28672 x 4096: 65 rows 56 / 45, 128 rows 58 / 51;
+    not 51200 x 5120, 128 rows 120 / 128, nor 14336 x 4096, 65 rows 34 / 37)."""
+    if k < 1024 or k % 64 or n % 64 or n < 8192 or k > n:
+        return False
+    if rows <= 128:
+        return rows > 64 and 24576 <= n <= 32768
+    if k >= 3584 and n <= (16384 if rows <= 256 else 12288) and rows < 1000:
+        return False
+    return rows <= 256 or rows > 384 or n <= 16384
+
+
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T), w = [Wg; Wu]."""
+    if x.shape[0] > 64 and _takes_tile(x, w, _tile_glu):
+        return _require_hip().tile_swiglu(x.contiguous(), w)
     if (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
             x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and
             _glu(x.shape[0], w.shape[0], x.shape[1]) and _plain(x, w)):

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "gemm_bindings.h"
+#include "tile_bindings.h"
 
 extern "C" {
 void launch_rmsnorm(void*, void*, const void*, float, int, int, hipStream_t);
@@ -671,6 +672,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("a"), py::arg("w"), py::arg("force_splits") = 0);
   m.def("skinny_parts", &skinny_parts, "decode GEMM as its parts' sums");
   m.def("skinny_swiglu", &skinny_swiglu, "decode gate/up GEMM with silu");
+  m.def("tile_swiglu", &tile_swiglu, "gate/up GEMM of a prompt with silu");
+  m.def("tile_parts", &tile_parts, "GEMM of a prompt, perhaps as parts' sums");
+  m.def("tile_form", &tile_form, "one form of these");
   m.def("norm_rows", &norm_rows, "norm, GEMM of a few rows and its end",
         py::arg("src"), py::arg("residual"), py::arg("norm_weight"),
         py::arg("eps"), py::arg("w"), py::arg("end"), py::arg("heads") = 0,

@@ -1,0 +1,184 @@
+// Forms of the GEMM of prompts (tile_gemm.hip): which tiles, how many parts.
+#pragma once
+#include <torch/extension.h>
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "gemm_bindings.h"
+
+extern "C" int launch_tile_gemm(void*, const void*, const void*, int, int, int,
+                                int, int, int, int, int, int, int, hipStream_t);
+
+enum TileEnd { TILE_PLAIN, TILE_PARTS, TILE_GLU };
+
+// A tile of 32 wm rows and 32 wn rows of W and the time of a launch in us: fixed
+// + rounds * (round + stages * (step + busy * share of workgroups with work)) +
+// write * MB / 2 of the result.  Fitted to 300 to 1300 launches of each form, 65
+// to 8192 rows, 1536 to 57344 columns, 2048 to 28672 k with cold weights (half of
+// them within 4 to 10%).  A stage takes longer where more CUs are busy, as the
+// chip lowers its clock.
+struct TileForm {
+  int wm, wn, fill;             // fill: fewest stages of an item
+  bool glu;
+  float fixed, round, step, busy, write;
+};
+
+constexpr TileForm TILE_FORMS[] = {
+    {8, 8, 2, true, 4.21f, 5.85f, 0.961f, 0.404f, 0.100f},
+    {6, 8, 2, true, 8.79f, -1.90f, 0.903f, 0.216f, 0.208f},
+    {8, 6, 2, false, 6.00f, 0.60f, 0.843f, 0.211f, 0.199f},
+    {6, 6, 3, false, 7.05f, -1.24f, 0.650f, 0.168f, 0.280f},
+    {8, 4, 3, true, 5.98f, -0.38f, 0.556f, 0.255f, 0.206f},
+    {4, 4, 4, true, 7.58f, -3.47f, 0.378f, 0.187f, 0.298f},
+};
+
+struct TilePlan {
+  float time;                   // us
+  const TileForm* form;
+  int parts;
+  const TileForm* rest;         // of the columns from `to` on; null: none
+  int to;
+};
+
+// `cols` of the result, which for GLU are half of W's rows
+inline float tile_time(const TileForm& f, int M, int cols, int K, int end,
+                       int parts) {
+  const int wide = end == TILE_GLU ? 16 * f.wn : 32 * f.wn;
+  const long items = (long)((M + 32 * f.wm - 1) / (32 * f.wm)) *
+                     ((cols + wide - 1) / wide) * parts;
+  const long rounds = ((items + 7) / 8 + 31) / 32;
+  const float stages = K / 64.f / parts;
+  const float share = items / (256.f * rounds);
+  const float mb = 1e-6f * M * cols *
+                   (end == TILE_PARTS ? 4.f * parts : end == TILE_GLU ? 2 : 2);
+  return f.fixed +
+         rounds * (f.round + stages * (f.step + f.busy * share)) + f.write * mb;
+}
+
+inline TilePlan pick_tile(int M, int N, int K, int end) {
+  const int cols = end == TILE_GLU ? N / 2 : N;
+  TilePlan best{1e30f, nullptr, 1, nullptr, cols};
+  auto consider = [&](const TilePlan& p) {
+    if (p.time < best.time) best = p;
+  };
+  for (const TileForm& f : TILE_FORMS) {
+    if ((end == TILE_GLU && !f.glu) || K / 64 < f.fill) continue;
+    consider({tile_time(f, M, cols, K, end, 1), &f, 1, nullptr, cols});
+    // whole rounds of these tiles, and others for the columns that are left:
+    // 2048 x 28672 x 4096 is 3.5 rounds, whose half takes as long as a whole
+    const int wide = end == TILE_GLU ? 16 * f.wn : 32 * f.wn;
+    const int down = (M + 32 * f.wm - 1) / (32 * f.wm);
+    const long items = (long)down * ((cols + wide - 1) / wide);
+    const int to = (int)(items / 256 * 256 / down * wide);
+    if (to > 0 && to < cols && f.wm == 8 && f.wn == 8)
+      for (const TileForm& r : TILE_FORMS) {
+        if ((end == TILE_GLU && !r.glu) || K / 64 < r.fill) continue;
+        consider({tile_time(f, M, to, K, end, 1) +
+                      tile_time(r, M, cols - to, K, end, 1),
+                  &f, 1, &r, to});
+      }
+  }
+  return best;
+}
+
+// Parts of K whose f32 sums a reader adds up, where that is faster by 7% with
+// what it reads more than bf16, at 5 TB/s.
+inline TilePlan pick_tile_parts(int M, int N, int K) {
+  TilePlan best = pick_tile(M, N, K, TILE_PLAIN);
+  float least = best.time * 0.93f;
+  for (const TileForm& f : TILE_FORMS)
+    for (int parts : {2, 3, 4, 6, 8}) {
+      const int tiles =
+          ((M + 32 * f.wm - 1) / (32 * f.wm)) * ((N + 32 * f.wn - 1) / (32 * f.wn));
+      // one round, which also bounds the sums (80 MB)
+      if (tiles * parts > 320 || K / 64 / parts < f.fill) break;
+      const float time = tile_time(f, M, N, K, TILE_PARTS, parts) +
+                         (4 * parts - 2) * 2e-7f * M * N;
+      if (time < least) {
+        least = time;
+        best = {time, &f, parts, nullptr, N};
+      }
+    }
+  return best;
+}
+
+inline void check_tile(const torch::Tensor& a, const torch::Tensor& w) {
+  for (const auto& t : {a, w})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
+                t.is_contiguous() && t.dim() == 2 &&
+                (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0,
+                "operands must be contiguous, aligned bf16 matrices on GPU");
+  const int64_t M = a.size(0), K = a.size(1), N = w.size(0);
+  TORCH_CHECK(w.size(1) == K, "K mismatch");
+  // offsets within a tile's rows and W's halves are 32 bits, tiles' numbers too
+  TORCH_CHECK(M >= 1 && N >= 64 && N % 64 == 0 && K >= 256 && K % 64 == 0 &&
+              M < (1 << 24) && (N / 2 + 256) * K < (1ll << 31) &&
+              ((M + 127) / 128) * ((N + 127) / 128) < (1 << 24),
+              "unsupported shape");
+}
+
+inline void launch_tile_plan(const TilePlan& p, void* out, const torch::Tensor& a,
+                             const torch::Tensor& w, int end) {
+  const int M = a.size(0), K = a.size(1), N = w.size(0);
+  const int cols = end == TILE_GLU ? N / 2 : N;
+  // Workgroups begin at different k where the weights are the bound and rows of
+  // A fit an L2: all rows are K apart, and in step they ask the same channels
+  // (128 rows, 28672 x 4096: 57 -> 53 us).  In step they share rows of A and W,
+  // which many rows need.
+  const int turn = M <= 256;
+  auto go = [&](const TileForm* f, int from, int to) {
+    TORCH_CHECK(launch_tile_gemm(out, a.data_ptr(), w.data_ptr(), M, N, K, end,
+                                 f->wm, f->wn, from, to, p.parts, turn,
+                                 gemm_stream()), "no such tile");
+  };
+  go(p.form, 0, p.to);
+  if (p.rest) go(p.rest, p.to, cols);
+}
+
+// silu(a Wg^T) * (a Wu^T), w = [Wg; Wu].
+inline torch::Tensor tile_swiglu(torch::Tensor a, torch::Tensor w) {
+  check_tile(a, w);
+  auto c = torch::empty({a.size(0), w.size(0) / 2}, a.options());
+  launch_tile_plan(pick_tile(a.size(0), w.size(0), a.size(1), TILE_GLU),
+                   c.data_ptr(), a, w, TILE_GLU);
+  return c;
+}
+
+// a W^T in bf16, or where K is split its parts' sums, f32 [parts, M, N].
+inline torch::Tensor tile_parts(torch::Tensor a, torch::Tensor w) {
+  check_tile(a, w);
+  const int64_t M = a.size(0), N = w.size(0);
+  const TilePlan p = pick_tile_parts(M, N, a.size(1));
+  const bool split = p.parts > 1;
+  auto c = split ? torch::empty({p.parts, M, N},
+                                a.options().dtype(torch::kFloat32))
+                 : torch::empty({M, N}, a.options());
+  launch_tile_plan(p, c.data_ptr(), a, w, split ? TILE_PARTS : TILE_PLAIN);
+  return c;
+}
+
+// One form of the above, for tests: its number, the parts, and for a second form
+// the column that it begins at.
+inline torch::Tensor tile_form(torch::Tensor a, torch::Tensor w, int64_t end,
+                               int64_t form, int64_t parts, int64_t rest,
+                               int64_t to) {
+  check_tile(a, w);
+  const int64_t M = a.size(0), N = w.size(0), K = a.size(1);
+  const int64_t cols = end == TILE_GLU ? N / 2 : N;
+  const int64_t forms = sizeof(TILE_FORMS) / sizeof(TILE_FORMS[0]);
+  TORCH_CHECK(end >= 0 && end <= TILE_GLU && form >= 0 && form < forms &&
+              rest < forms && parts >= 1 && (parts == 1 || end == TILE_PARTS) &&
+              K / 64 / parts >= TILE_FORMS[form].fill &&
+              (rest < 0 || (to > 0 && to < cols && to % 32 == 0 &&
+                            K / 64 / parts >= TILE_FORMS[rest].fill)), "form");
+  auto c = end == TILE_PARTS
+               ? torch::empty({parts, M, N}, a.options().dtype(torch::kFloat32))
+               : torch::empty({M, cols}, a.options());
+  launch_tile_plan({0.f, TILE_FORMS + form, (int)parts,
+                    rest < 0 ? nullptr : TILE_FORMS + rest,
+                    (int)(rest < 0 ? cols : to)},
+                   c.data_ptr(), a, w, (int)end);
+  return c;
+}

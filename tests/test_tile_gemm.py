@@ -1,0 +1,136 @@
+"""The GEMM of prompts (ops/hip/tile_gemm.hip) and the rules that choose it."""
+import pytest
+import torch
+
+FORMS = [(8, 8), (6, 8), (8, 6), (6, 6), (8, 4), (4, 4)]
+PLAIN, PARTS, GLU = 0, 1, 2
+
+
+def _operands(m, n, k):
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(m * 1000003 + n + k)
+    x = torch.randn(m, k, device=dev, generator=gen).bfloat16()
+    w = (torch.randn(n, k, device=dev, generator=gen) / k ** 0.5).bfloat16()
+    full = x.double() @ w.double().t().contiguous()
+    # f32 sums of bf16 products: k roundings of 2^-24 of the magnitudes' sums
+    sums = (x.double().abs() @ w.double().abs().t().contiguous()) * k * 2 ** -24
+    return x, w, full, sums
+
+
+def _near(got, end, full, sums):
+    if end == PARTS:
+        return ((got.double().sum(0) - full).abs() <= sums).all()
+    if end == PLAIN:        # and half an ulp of the result
+        return ((got.double() - full).abs() <= full.abs() * 2 ** -8 + sums).all()
+    f = full.shape[1] // 2
+    g, u = full[:, :f], full[:, f:]
+    want = torch.nn.functional.silu(g) * u
+    # |silu'| < 1.1; the exponential and the division to a few 2^-23
+    bound = want.abs() * (2 ** -8 + 2 ** -20) + \
+        1.1 * sums[:, :f] * u.abs() + (g.abs() + 1) * sums[:, f:]
+    return ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", range(len(FORMS)))
+@pytest.mark.parametrize("m,n,k", [
+    (1, 64, 256), (127, 320, 320), (129, 1088, 1024), (255, 192, 640),
+    (257, 2176, 832), (300, 576, 1088), (769, 1600, 256)])
+def test_forms(form, m, n, k):
+    """Every tile: rows and columns short of a tile and past one, few and odd
+    numbers of stages, parts of unequal length, several tiles a workgroup."""
+    from rbg_amd import ops
+    x, w, full, sums = _operands(m, n, k)
+    wm, wn = FORMS[form]
+    for end in (PLAIN, PARTS, GLU):
+        if end == GLU and wn % 4:
+            continue
+        for parts in (1, 2, 3) if end == PARTS else (1,):
+            if k // 64 // parts < 4:
+                continue
+            got = ops._hip.tile_form(x, w, end, form, parts, -1, 0)
+            assert _near(got, end, full, sums), (end, parts)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("end", [PLAIN, GLU])
+def test_second_form_for_the_rest(end):
+    from rbg_amd import ops
+    x, w, full, sums = _operands(500, 2048, 512)
+    for form, rest, to in ((0, 4, 512), (0, 5, 768), (4, 0, 256)):
+        got = ops._hip.tile_form(x, w, end, form, 1, rest, to)
+        assert _near(got, end, full, sums)
+
+
+@pytest.mark.gpu
+def test_many_tiles_a_workgroup():
+    """More tiles than workgroups, of a few stages each: loads run several
+    tiles ahead."""
+    from rbg_amd import ops
+    x, w, full, sums = _operands(2100, 9280, 256)
+    for form in range(len(FORMS)):
+        for end in (PLAIN, GLU):
+            if end == GLU and FORMS[form][1] % 4:
+                continue
+            got = ops._hip.tile_form(x, w, end, form, 1, -1, 0)
+            assert _near(got, end, full, sums), (form, end)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [
+    (65, 2048, 12288), (128, 4096, 12288), (129, 2048, 3584),
+    (256, 6144, 4096), (257, 2048, 5120), (999, 3136, 5120),
+    (1000, 6144, 4096), (1500, 14336, 3584), (2048, 4096, 8192)])
+def test_parts_route(m, n, k):
+    from rbg_amd import ops
+    assert ops._tile(m, n, k)
+    x, w, full, sums = _operands(m, n, k)
+    got = ops.linear_parts(x, w)
+    assert _near(got, PARTS if got.dim() == 3 else PLAIN, full, sums)
+    # rows further apart than they are long
+    wide = torch.cat([x, x], dim=1)
+    assert torch.equal(ops.linear_parts(wide[:, :k], w), got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [
+    (65, 24576, 1024), (128, 28672, 1088), (129, 8192, 2048),
+    (256, 18432, 2048), (385, 28672, 1024), (1000, 11264, 2048),
+    (2048, 28672, 1024)])
+def test_swiglu_route(m, n, k):
+    from rbg_amd import ops
+    assert ops._tile_glu(m, n, k)
+    x, w, full, sums = _operands(m, n, k)
+    assert _near(ops.linear_swiglu(x, w), GLU, full, sums)
+
+
+@pytest.mark.gpu
+def test_refuses_what_it_cannot_take():
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    x = torch.randn(300, 512, device=dev).bfloat16()
+    w = torch.randn(256, 512, device=dev).bfloat16()
+    for bad in ((x[:, :500].contiguous(), w[:, :500].contiguous()),
+                (x, w[:250].contiguous()), (x[:, ::2], w[:, :256]),
+                (x.float(), w.float())):
+        for f in (ops._hip.tile_swiglu, ops._hip.tile_parts):
+            with pytest.raises(RuntimeError):
+                f(*bad)
+    with pytest.raises(RuntimeError):       # parts of too few stages
+        ops._hip.tile_form(x, w, PARTS, 5, 4, -1, 0)
+
+
+def test_rules_hand_over_what_it_takes():
+    from rbg_amd.ops import _tile, _tile_glu
+    taken = [0, 0]
+    for n in (64, 1024, 2048, 4096, 6144, 8192, 8200, 10240, 14336, 16384,
+              28672, 57344):
+        for k in (256, 1000, 2048, 3584, 4096, 5120, 12288, 25600):
+            for rows in (0, 1, 64, 65, 128, 129, 256, 257, 999, 1000, 4096,
+                         4097, 8192):
+                for i, rule in enumerate((_tile, _tile_glu)):
+                    if rule(rows, n, k):
+                        assert rows > 64 and n % 64 == 0 and k % 64 == 0
+                        assert k >= 256
+                        taken[i] += 1
+    assert min(taken) > 50
