@@ -8,6 +8,7 @@ as the implementation.
 """
 from __future__ import annotations
 
+import heapq
 import importlib
 from dataclasses import dataclass
 from typing import Any, Dict, Optional, Tuple
@@ -485,6 +486,88 @@ class PrefillPlan:
     """Workgroups of prompt attention (bindings.cpp prefill_flash)."""
     blocks: torch.Tensor        # [n, 4] int32
     lens: torch.Tensor          # [n] int32
+    # where blocks are cut by keys: [m, 4] and [c, 3] int32, parts in all
+    items: Optional[torch.Tensor] = None
+    joins: Optional[torch.Tensor] = None
+    parts: int = 0
+
+
+def _cut_prefill(tiles: np.ndarray, kv_heads: int):
+    """Work of blocks of so many tiles of 64 keys, most first, as equal shares
+    of the chip's CUs: (items, joins, parts), or None where whole blocks are as
+    good.
+
+    A CU's share holds whole blocks as far as they fit, and other blocks are cut
+    to fill it.  Times in us are those of hip/prefill_flash.hip: a tile takes 1.2
+    by itself on a CU and 1.05 beside another; a part leaves 64 KB of sums, which
+    are written and read at 5 TB/s, and the launch that adds them up takes 5.
+    Whole blocks and cut ones, 32 heads of 8 (us): 40 rows after 9000 keys 165 / 28,
+    512 after 4000 88 / 60, 1500 after 9000 297 / 261.  Not cut: 2048 rows, whose
+    longest workgroups run beside the shortest (51), nor more blocks than four a
+    CU, which even out by themselves."""
+    cus = max(1, 256 // kv_heads)           # of a key head
+    n, work = len(tiles), int(tiles.sum())
+    if n == 0 or n > 4 * cus:
+        return None
+    share = max(-(-work // cus), 4)
+    part_time = kv_heads * 0.026
+    tile_time = 1.2 if n <= cus else 1.0
+    least = tile_time * share + 5 + part_time * 2 * int((tiles > share).sum())
+    tiles = tiles.tolist()
+    whole = 1.2 * tiles[0]
+    if n > cus:
+        load = [t for t in reversed(tiles[:cus])]       # a heap: they ascend
+        for t in tiles[cus:]:
+            heapq.heapreplace(load, load[0] + t)
+        whole = max(whole, max(load))
+    if least > 0.95 * whole:
+        return None
+    items, joins, cut, parts = [], [], [], 0
+    room = [-share] * cus                               # negative: a heap
+    for b, t in enumerate(tiles):
+        if t <= -room[0]:
+            heapq.heapreplace(room, room[0] + t)
+            items.append((b, 0, t, -1))
+        else:
+            cut.append(b)
+    room = sorted(-r for r in room)                     # the most last
+    over = max(2, share // 8)       # a share may be this much more
+    for b in cut:
+        done, first = 0, parts
+        while done < tiles[b]:
+            left = tiles[b] - done
+            take = left
+            if room and left > room[-1] + over:
+                take = room[-1]
+            if room:
+                room[-1] -= take
+                if room[-1] <= over:
+                    room.pop()
+                    if room and room[-1] <= over:
+                        room.clear()
+            items.append((b, done, done + take, parts))
+            parts += 1
+            done += take
+        if parts == first + 1:      # whole after all
+            items[-1] = items[-1][:3] + (-1,)
+            parts = first
+        else:
+            joins.append((b, first, parts - first))
+    longest = max(i[2] - i[1] for i in items)
+    cost = max(1.2 * longest, tile_time * share) + 5 + part_time * parts
+    if not joins or cost > 0.95 * whole:
+        return None
+    return np.array(items), np.array(joins), parts
+
+
+def _turn_round(order: np.ndarray, kv_heads: int) -> np.ndarray:
+    """Most work first.  Where all run at once, two per CU (256 CUs), the second
+    half is turned round, so that the longest share with the shortest (2048
+    tokens of 32 heads: 61 -> 56 us)."""
+    if len(order) * kv_heads <= 512:
+        half = 256 // kv_heads
+        order = np.concatenate([order[:half], order[half:][::-1]])
+    return order
 
 
 def prefill_plan(cu, cu_k, heads: int, kv_heads: int, device) -> PrefillPlan:
@@ -498,16 +581,19 @@ def prefill_plan(cu, cu_k, heads: int, kv_heads: int, device) -> PrefillPlan:
     nth = np.arange(len(seq)) - np.repeat(np.cumsum(count) - count, count)
     past = (lens - rows)[seq]
     need = np.minimum(past + (nth + 1) * tokens, lens[seq])
-    # Most work first.  Where all run at once, two per CU (256 CUs), the second
-    # half is turned round, so that the longest share with the shortest (2048
-    # tokens of 32 heads: 61 -> 56 us).
     order = np.argsort(-need, kind="stable")
-    if len(order) * kv_heads <= 512:
-        half = 256 // kv_heads
-        order = np.concatenate([order[:half], order[half:][::-1]])
+    tiles = np.maximum((need[order] + 63) // 64, 0)
+    cut = _cut_prefill(tiles, kv_heads)
+    if cut is None:
+        order = _turn_round(order, kv_heads)
     info = np.stack([cu[:-1][seq], nth, cu_k[:-1][seq], past], axis=1)
-    return PrefillPlan(*upload([info[order].astype(np.int32),
-                                lens[seq][order].astype(np.int32)], device))
+    arrays = [info[order], lens[seq][order]]
+    if cut is not None:
+        items, joins, parts = cut
+        by_work = np.argsort(items[:, 1] - items[:, 2], kind="stable")
+        arrays += [items[_turn_round(by_work, kv_heads)], joins]
+    dev = upload([a.astype(np.int32) for a in arrays], device)
+    return PrefillPlan(*dev, parts) if cut is not None else PrefillPlan(*dev)
 
 
 def prefill_attention(q, k, v, cu_seqlens, scale: float, cu_seqlens_k=None,
@@ -527,8 +613,9 @@ def prefill_attention(q, k, v, cu_seqlens, scale: float, cu_seqlens_k=None,
                 plan = prefill_plan(
                     cu, cu if cu_seqlens_k is None else cu_seqlens_k.tolist(),
                     q.shape[1], kvh, q.device)
-            return _require_hip().prefill_flash(q, k, v, plan.blocks,
-                                                plan.lens, scale, slots)
+            return _require_hip().prefill_flash(
+                q, k, v, plan.blocks, plan.lens, scale, slots, plan.items,
+                plan.joins, plan.parts)
     if slots is not None:
         at = slots.long()
         pages, place = at // k.shape[2], at % k.shape[2]

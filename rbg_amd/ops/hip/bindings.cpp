@@ -44,7 +44,8 @@ void launch_prefill_attention(void*, const void*, const void*, const void*,
                               int, int, int, hipStream_t);
 void launch_prefill_flash(void*, const void*, const void*, const void*,
                           const void*, const void*, const void*, float, int,
-                          int, int, int, long, long, hipStream_t);
+                          const void*, int, const void*, int, void*, void*, int,
+                          int, int, long, long, hipStream_t);
 void launch_mfma_probe(void*, const void*, const void*, int, int, hipStream_t);
 void launch_mfma_probe32(void*, const void*, const void*, int, int, int,
                          hipStream_t);
@@ -445,10 +446,16 @@ torch::Tensor prefill_attention(torch::Tensor q, torch::Tensor k,
 // block_info [n, 4] and seq_lens [n]: a workgroup's first query row of the
 // sequence, its number among the sequence's blocks of 128 / (QH / H) tokens,
 // the sequence's first kv row and the position of its first query row; its kv
-// rows.
+// rows.  items [m, 4] and joins [c, 3], where work is cut by keys: a
+// workgroup's block, its first and one past its last tile of 64 keys, and the
+// part that its sums are, or -1 for all of a block; a cut block, its first part
+// and how many they are, in order of the parts.
 torch::Tensor prefill_flash(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                             torch::Tensor block_info, torch::Tensor seq_lens,
-                            double scale, c10::optional<torch::Tensor> slots) {
+                            double scale, c10::optional<torch::Tensor> slots,
+                            c10::optional<torch::Tensor> items,
+                            c10::optional<torch::Tensor> joins,
+                            int64_t parts) {
   auto rows3 = [](const torch::Tensor& t, const char* name) {
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
                 t.dim() == 3 && t.stride(2) == 1 &&
@@ -479,13 +486,32 @@ torch::Tensor prefill_flash(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   const int heads = q.size(1), kv_heads = k.size(1);
   TORCH_CHECK(kv_heads > 0 && heads % kv_heads == 0 && heads / kv_heads <= 128,
               "query heads: a multiple of the key heads, at most 128 times");
+  TORCH_CHECK(items.has_value() == joins.has_value(), "items and joins");
+  if (items)
+    for (const auto& t : {*items, *joins})
+      TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.dim() == 2 &&
+                  t.scalar_type() == torch::kInt32, "plan int32");
+  TORCH_CHECK(!items || (items->size(1) == 4 && joins->size(1) == 3 &&
+                         parts >= 0), "plan sizes");
   auto out = torch::empty({q.size(0), (int64_t)heads, (int64_t)128},
                           q.options());
+  torch::Tensor sums;           // per part and key head 128 rows of 128, then
+  float* ml = nullptr;          // maximum and sum of each row
+  if (items && parts > 0) {
+    const int64_t rows = parts * kv_heads * 128;
+    sums = torch::empty({rows * 130}, q.options().dtype(torch::kFloat32));
+    ml = sums.data_ptr<float>() + rows * 128;
+  }
   launch_prefill_flash(out.data_ptr(), q.data_ptr(), k.data_ptr(),
                        v.data_ptr(), slots ? slots->data_ptr() : nullptr,
                        block_info.data_ptr(), seq_lens.data_ptr(),
-                       (float)scale, blocks, heads, kv_heads, shift,
-                       q.stride(0), k.stride(0), current_stream());
+                       (float)scale, blocks,
+                       items ? items->data_ptr() : nullptr,
+                       items ? (int)items->size(0) : 0,
+                       items ? joins->data_ptr() : nullptr,
+                       items ? (int)joins->size(0) : 0,
+                       ml ? sums.data_ptr() : nullptr, ml, heads, kv_heads,
+                       shift, q.stride(0), k.stride(0), current_stream());
   return out;
 }
 
@@ -665,7 +691,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("prefill_flash", &prefill_flash, "causal attention of prompts",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("block_info"),
         py::arg("seq_lens"), py::arg("scale"),
-        py::arg("slots") = c10::nullopt);
+        py::arg("slots") = c10::nullopt,
+        py::arg("items") = c10::nullopt, py::arg("joins") = c10::nullopt,
+        py::arg("parts") = 0);
   m.def("mfma_probe", &mfma_probe, "MFMA layout probe");
   m.def("mfma_probe32", &mfma_probe32, "32x32x16 MFMA layout probe");
   m.def("skinny_gemm", &skinny_gemm, "decode-shape GEMM (M<=256)",

@@ -1,13 +1,10 @@
 // Varlen causal flash attention for prompts, head size 128, keys and values
 // as rows or, behind a past, straight from the pages.
 //
-// Bound: the matrix cores (4 * 128 operations per pair of tokens) and beside
-// them the exponentials: 870 to 910 TFLOP/s at 8192 tokens of 32 heads, where
-// the 16-row form this replaces reached 346, and 580 to 630 at 2048, where few
-// workgroups have most of the work.  A workgroup is 4 waves of 32 query rows each; tiles
-// of 64 keys pass LDS in two buffers, one barrier a tile, the next tile's rows
-// in flight meanwhile.  (Forming the next tile's scores beside this tile's
-// exponentials, for 28 more registers, measured the same.)
+// Bound: the matrix cores (4 * 128 operations per pair of tokens), beside them
+// the exponentials, which take about as long, and the power of both: 1.9 GHz at
+// 8192 tokens of 32 heads, 1020 to 1050 TFLOP/s.  A workgroup is 4 waves of 32
+// query rows each; tiles of 64 keys pass LDS in two stages, one barrier a tile.
 //  * The rows of a workgroup are 128 / group tokens with all the query heads
 //    of a key head: fewer rows go to waste at the ends of short sequences and
 //    on the diagonal than with 128 tokens of one head.
@@ -20,13 +17,25 @@
 //  * Scale and maximum are one fma per score, and sums are rescaled only when
 //    some row's maximum grows.  (Letting scores exceed it by 2^8 would be 1 to
 //    2% faster, but the largest weight, 1 here, would then be rounded too.)
+//  * Rows go straight to LDS, to places that no read or load meets a conflict
+//    at (through registers, with V's writes in conflict: 8192 tokens 600 us, so
+//    550), and between the products, pinned there, stand their operands' reads,
+//    several ahead, the next tile's loads and half of the exponentials (550 ->
+//    525, where a workgroup has its CU to itself 1.75 -> 1.2 us a tile).  A third
+//    workgroup on a CU, V in one stage, needs registers that spill (640).
+//  * Blocks are cut by keys where whole ones would leave CUs idle (ops
+//    _cut_prefill), whose sums a second launch adds up: 1500 tokens after 9000
+//    297 -> 261 us, 512 after 4000 88 -> 60, 40 after 9000 165 -> 28.
+#include <type_traits>
+
 #include "mfma_util.h"
 
 namespace {
 
 constexpr int DIM = 128, TILE = 64, WAVES = 4, ROWS = WAVES * 32;
 constexpr int THREADS = WAVES * 64;
-constexpr int KP = DIM + 8;       // row pitch of K in LDS: no bank conflicts
+constexpr int STAGE = TILE * DIM * 2;     // bytes of a tile of K or V
+constexpr int LDS = 4 * STAGE;            // two of each
 constexpr float LOW = -1e30f;
 
 typedef __attribute__((ext_vector_type(4))) unsigned int pf_u4;
@@ -46,9 +55,26 @@ DEV_INLINE float pf_add2(__bf16 a, __bf16 b, float sum) {
   return __builtin_amdgcn_fdot2_f32_bf16(ab, ones, sum, false);
 }
 
-// PAGED: kv rows are named by `slots` ((page << page_shift) + place) and lie in
-// [pages, kv heads, 1 << page_shift, DIM].
-template <bool PAGED>
+// 16 bytes per lane from base + off, or from a lane's own address, to 16 * lane
+// past the wave's LDS address.  Not the compiler's builtin: it would wait for
+// the data before any LDS read.
+DEV_INLINE void pf_bring(uint32_t off, const void* base, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+               "global_load_lds_dwordx4 %0, %1"
+               :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+DEV_INLINE void pf_bring(const void* at, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\t"
+               "global_load_lds_dwordx4 %0, off"
+               :: "v"(at), "s"(lds) : "memory", "m0");
+}
+
+// where kv rows lie: rows kv_stride apart, of which a tile's offsets are 32 bits
+// (FROM_ROWS) or not (FROM_FAR_ROWS), or (FROM_PAGES) named by `slots` ((page <<
+// page_shift) + place) in [pages, kv heads, 1 << page_shift, DIM]
+enum From { FROM_ROWS, FROM_FAR_ROWS, FROM_PAGES };
+
+template <int FROM>
 __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
     __hip_bfloat16* __restrict__ out,        // [T, QH, DIM]
     const __hip_bfloat16* __restrict__ q,    // [T, QH, DIM], rows q_stride
@@ -59,27 +85,33 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
     //   block of ROWS / group queries, first kv row, position of the first
     //   query row
     const int* __restrict__ seq_lens,        // [blocks]: kv rows
+    const int* __restrict__ items,           // [count, 4]: block, its first and
+    //   one past its last tile, where its sums go; null: the blocks, whole
+    float* __restrict__ part_o,              // [parts, KVH, 4 waves, 16, 64, 4]
+    float* __restrict__ part_ml,             // [parts, KVH, ROWS, 2]
     const float scale,                       // to the base of 2, > 0
     const bool negate, const int num_q_heads, const int num_kv_heads,
     const int page_shift, const long q_stride, const long kv_stride,
-    const int blocks) {
+    const int count) {
   // Workgroup i runs on XCD i % 8.  A key head stays on one XCD (or on as few
   // as there are heads for), whose L2 then holds that head's rows only.
   const int group = num_q_heads / num_kv_heads;
-  int kvh, blk;
+  int kvh, unit;
   if (num_kv_heads % 8 == 0) {
     const int per = num_kv_heads / 8, i = blockIdx.x / 8;
     kvh = blockIdx.x % 8 * per + i % per;
-    blk = i / per;
+    unit = i / per;
   } else if (8 % num_kv_heads == 0) {
     const int xcd = blockIdx.x % 8;
     kvh = xcd % num_kv_heads;
-    blk = blockIdx.x / 8 * (8 / num_kv_heads) + xcd / num_kv_heads;
+    unit = blockIdx.x / 8 * (8 / num_kv_heads) + xcd / num_kv_heads;
   } else {
     kvh = blockIdx.x % num_kv_heads;
-    blk = blockIdx.x / num_kv_heads;
+    unit = blockIdx.x / num_kv_heads;
   }
-  if (blk >= blocks) return;
+  if (unit >= count) return;
+  const int blk = items ? items[unit * 4] : unit;
+  const int part = items ? items[unit * 4 + 3] : -1;
   const int tokens = ROWS / group;
   const int q_start = block_info[blk * 4];
   const int q_first = block_info[blk * 4 + 1] * tokens;
@@ -91,9 +123,10 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, h = lane >> 5;
 
-  __shared__ __align__(16) __hip_bfloat16 k_lds[2][TILE * KP];
-  // [key / 4][dim / 16][key % 4][dim % 16]
-  __shared__ __align__(16) __hip_bfloat16 v_lds[2][TILE * DIM];
+  // two stages of K, two of V, each [key / 4][16-byte pieces of 4 keys], a piece
+  // of V at dim / 16 * 8 + key % 4 * 2 + dim / 8 % 2, of K there with two bits
+  // turned over by those of key / 4: no bank conflicts
+  extern __shared__ __align__(16) char pf_lds[];
 
   const int q_rows = len - offset;            // of this sequence
   const int in = wave * 32 + c;
@@ -115,41 +148,74 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
   const int last = min(offset + q_first + tokens, len) - 1;   // key needed
   // a sequence of fewer keys than queries has queries before its first key,
   // whose result is 0: a block of only those reads no rows
-  const int tiles = last < 0 ? 0 : last / TILE + 1;
+  const int all = last < 0 ? 0 : last / TILE + 1;
+  const int begin = items ? items[unit * 4 + 1] : 0;
+  const int tiles = items ? min(all, items[unit * 4 + 2]) : all;
   const int wave_first = offset + q_first + wave * 32 / group;
   const int wave_end = offset + q_first + (wave * 32 + 31) / group;
   const int wave_tiles = min(tiles, min(wave_end, len - 1) / TILE + 1);
+  const int whole = min(wave_tiles, max(min(wave_first + 1, len), 0) / TILE);
 
-  // thread: 16 bytes of rows tid / 16 + 16 j of a tile
-  const int kr = tid >> 4, kc = (tid & 15) * 8;
-  pf_u4 ks[4], vs[4];
-  int slot[4];
-#define PF_SLOTS(t)                                                        \
-  if (PAGED) {                                                             \
-    _Pragma("unroll") for (int j = 0; j < 4; ++j)                          \
-        slot[j] = slots[kv_start +                                         \
-                        min((t) * TILE + kr + j * 16, len - 1)];           \
-  }
-#define PF_ROWS(t)                                                         \
-  _Pragma("unroll") for (int j = 0; j < 4; ++j) {                          \
-    size_t at;                                                             \
-    if (PAGED)                                                             \
-      at = (((((size_t)(slot[j] >> page_shift) * num_kv_heads + kvh)       \
-              << page_shift) + (slot[j] & ((1 << page_shift) - 1))) * DIM  \
-            + kc);                                                         \
-    else                                                                   \
-      at = (size_t)(kv_start + min((t) * TILE + kr + j * 16, len - 1)) *   \
-               kv_stride + (size_t)kvh * DIM + kc;                         \
-    ks[j] = pf_load(k + at);                                               \
-    vs[j] = pf_load(v + at);                                               \
-  }
-  const int k_put = kr * KP + kc;
-  const int v_put = ((kr >> 2) * 8 + (kc >> 4)) * 64 + (kr & 3) * 16 + (kc & 8);
-#define PF_PUT(b)                                                          \
-  _Pragma("unroll") for (int j = 0; j < 4; ++j) {                          \
-    *reinterpret_cast<pf_u4*>(k_lds[b] + k_put + j * 16 * KP) = ks[j];     \
-    *reinterpret_cast<pf_u4*>(v_lds[b] + v_put + j * 16 * DIM) = vs[j];    \
-  }
+  // A wave's load brings 4 keys, wave * 4 + 16 j .. of a tile; a lane's piece
+  // of its key's 16
+  const int kr = wave * 4 + ((lane >> 1) & 3);
+  const uint32_t v_piece = ((lane >> 3) * 2 + (lane & 1)) * 16;
+  const uint32_t k_piece = (((lane >> 3) ^ (wave & 1)) * 2 +
+                            ((lane & 1) ^ (wave >> 1))) * 16;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)pf_lds + wave * 1024;
+  const size_t row_bytes = (size_t)kv_stride * 2;
+  const size_t head_at = (size_t)kvh * DIM + (size_t)kv_start * kv_stride;
+  const char* const kb = (const char*)(FROM == FROM_PAGES ? k : k + head_at);
+  const char* const vb = (const char*)(FROM == FROM_PAGES ? v : v + head_at);
+  const uint32_t page_rows = (uint32_t)num_kv_heads << page_shift;
+  const uint32_t head_rows = (uint32_t)kvh << page_shift;
+  int slot[4] = {};                         // of the next tile
+  auto name = [&](int t) {
+    if (FROM == FROM_PAGES)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        slot[j] = slots[kv_start + min(t * TILE + kr + j * 16, len - 1)];
+  };
+  // the compiler's wait for them, which counts only its own loads, comes here
+  auto named = [&]() {
+    if (FROM == FROM_PAGES)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(slot[j]));
+  };
+  auto bring = [&](int j, const char* base, int t, uint32_t piece,
+                   uint32_t to) {
+    if (FROM == FROM_PAGES) {
+      pf_bring(base + piece +
+                   ((size_t)(uint32_t)(slot[j] >> page_shift) * page_rows +
+                    (head_rows + (slot[j] & ((1 << page_shift) - 1)))) *
+                       (DIM * 2),
+               to + j * 4096);
+    } else {
+      const int r = min(kr + j * 16, len - 1 - t * TILE);
+      const char* at = base + t * TILE * row_bytes;
+      if (FROM == FROM_ROWS)
+        pf_bring(__umul24(r, (uint32_t)row_bytes) + piece, at, to + j * 4096);
+      else
+        pf_bring(at + r * row_bytes + piece, to + j * 4096);
+    }
+  };
+  // all of tile `t`, or the q-th of its 8 loads, to the stages of tile `as`
+  auto bring_one = [&](int q, int t, int as) {
+    const uint32_t to = lds0 + (as & 1) * STAGE;
+    if (q & 1) bring(q >> 1, vb, t, v_piece, to + 2 * STAGE);
+    else bring(q >> 1, kb, t, k_piece, to);
+  };
+  auto bring_all = [&](int t, int as) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) bring_one(q, t, as);
+  };
+
+  // this lane's key and piece of K: row p * 32 + c, dims e * 16 + h * 8 ..
+  const int kblk = c >> 2;
+  const int k_at = kblk * 1024 + (c & 3) * 32 + ((h ^ ((kblk >> 1) & 1)) * 16);
+  const int k_even = k_at + (kblk & 1) * 128, k_odd = k_at - (kblk & 1) * 128;
+  const int v_at = 2 * STAGE + h * 1024 + ((lane >> 4) & 1) * 128 +
+                   (lane & 15) * 8;
 
   f32x16 acc[4];
   float m = LOW, l = 0.f;
@@ -158,103 +224,146 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[d][i] = 0.f;
 
-  if (tiles > 0) {
-    PF_SLOTS(0)
-    PF_ROWS(0)
-    PF_SLOTS(min(1, tiles - 1))
-    PF_PUT(0)
+  if (begin < tiles) {
+    name(begin);
+    named();
+    bring_all(begin, begin);
+    name(min(begin + 1, tiles - 1));
   }
-  // A wave stages rows for the others beyond its own last tile, in a loop of
-  // its own: a condition around the sums would have them copied every tile.
-#define PF_STAGE(t)                                                        \
-  __syncthreads();                                                         \
-  PF_ROWS(min((t) + 1, tiles - 1))                                         \
-  PF_SLOTS(min((t) + 2, tiles - 1))                                        \
-  __builtin_amdgcn_sched_barrier(0);
-  int t = 0;
-  for (; t < wave_tiles; ++t) {
-    const int b = t & 1, base = t * TILE;
-    PF_STAGE(t)
-    {
-      f32x16 s[2];
+  // Waited for here: the compiler would wait for them in every tile.
 #pragma unroll
-      for (int p = 0; p < 2; ++p) {
+  for (int s = 0; s < 8; ++s) asm volatile("" : "+v"(qf[s]));
+#define PF_MEET()                                                          \
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); \
+  named();
+  // One tile's products.  Between them, one thing at a time and pinned there,
+  // stand the reads of their operands ahead of them, the next tile's loads and
+  // half of the exponentials.
+  auto products = [&](auto masked, int t) {
+    constexpr bool MASK = decltype(masked)::value;
+    const int base = t * TILE, next = min(t + 1, tiles - 1);
+    const char* kp = pf_lds + (t & 1) * STAGE;
+    const __hip_bfloat16* vp =
+        (const __hip_bfloat16*)(pf_lds + v_at + (t & 1) * STAGE);
+    auto k_read = [&](int n) {
+      return pf_frag(*reinterpret_cast<const pf_u4*>(
+          kp + (n & 1 ? k_odd : k_even) + (n >> 3) * 8192 + (n & 7) * 128));
+    };
+    // 16 keys x 32 dims: lanes of a half read blocks of 4 keys x 16 dims
+    auto v_read = [&](int n) {
+      union { mf_bf4 u[2]; bf16x8 v; } f;
+      const __hip_bfloat16* at = vp + (n >> 2) * 2048 + (n & 3) * 128;
+      f.u[0] = tr_read4(at);
+      f.u[1] = tr_read4(at + 1024);
+      return f.v;
+    };
+    constexpr int AHEAD = 6, V_AHEAD = 4;
+    bf16x8 kf[AHEAD], vf[V_AHEAD];
+    f32x16 s[2] = {};
+    float top = LOW;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[p][i] = 0.f;
-        const __hip_bfloat16* kp = k_lds[b] + (p * 32 + c) * KP + h * 8;
+    for (int n = 0; n < AHEAD; ++n) kf[n] = k_read(n);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          s[p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              pf_frag(pf_load(kp + e * 16)), qf[e], s[p], 0, 0, 0);
+    for (int n = 0; n < 16; ++n) {
+      s[n >> 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          kf[n % AHEAD], qf[n & 7], s[n >> 3], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (n + AHEAD < 16) kf[n % AHEAD] = k_read(n + AHEAD);
+      else if (n + V_AHEAD >= 16) vf[n + V_AHEAD - 16] = v_read(n + V_AHEAD - 16);
+      if (n < 8) bring_one(n, next, t + 1);
+      if (!MASK && n >= 10 && n < 15) {
+#pragma unroll
+        for (int i = (n - 10) * 3; i < min(16, (n - 9) * 3 + (n == 14)); ++i)
+          top = fmaxf(top, s[0][i]);
       }
-      // lane: query c, keys base + 32 p + i % 4 + 8 (i / 4) + 4 h
-      if (base + TILE - 1 > wave_first || base + TILE > len) {
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int key = base + p * 32 + i % 4 + 8 * (i / 4) + 4 * h;
-            if (key > my_pos || key >= len) s[p][i] = LOW;
-          }
-      }
-      float top = LOW;
-#pragma unroll
-      for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) top = fmaxf(top, s[p][i]);
-      top = fmaxf(top, __shfl_xor(top, 32, 64)) * scale;
-      if (__any(top > m)) {
-        const float m_new = fmaxf(m, top);
-        const float fade = __builtin_amdgcn_exp2f(m - m_new);
-        m = m_new;
-        l *= fade;
-#pragma unroll
-        for (int d = 0; d < 4; ++d)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) acc[d][i] *= fade;
-      }
-      bf16x8 pf[4];               // 16 keys each
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    name(min(t + 2, tiles - 1));
+    // lane: query c, keys base + 32 p + i % 4 + 8 (i / 4) + 4 h
+    if (MASK) {
 #pragma unroll
       for (int p = 0; p < 2; ++p)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          pf[p * 2 + i / 8][i % 8] = (__bf16)__builtin_amdgcn_exp2f(
-              __builtin_fmaf(s[p][i], scale, -m));
-        }
-      // the sum of the weights as they are used, rounded: an error that the
-      // largest share with it cancels
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int i = 0; i < 8; i += 2)
-          l = pf_add2(pf[e][i], pf[e][i + 1], l);
-      // 16 keys x 32 dims: lanes of a half read blocks of 4 keys x 16 dims
-      const __hip_bfloat16* vp =
-          v_lds[b] + h * 512 + ((lane >> 4) & 1) * 64 + (lane & 15) * 4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          union { mf_bf4 u[2]; bf16x8 v; } vf;
-          vf.u[0] = tr_read4(vp + e * 2048 + d * 128);
-          vf.u[1] = tr_read4(vp + e * 2048 + d * 128 + 1024);
-          acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf[e], acc[d],
-                                                           0, 0, 0);
+          const int key = base + p * 32 + i % 4 + 8 * (i / 4) + 4 * h;
+          if (key > my_pos || key >= len) s[p][i] = LOW;
+          if (p == 0) top = fmaxf(top, s[0][i]);
         }
     }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) top = fmaxf(top, s[1][i]);
+    top = fmaxf(top, __shfl_xor(top, 32, 64)) * scale;
+    if (__any(top > m)) {
+      const float m_new = fmaxf(m, top);
+      const float fade = __builtin_amdgcn_exp2f(m - m_new);
+      m = m_new;
+      l *= fade;
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[d][i] *= fade;
+    }
+    bf16x8 pf[4];               // 16 keys each
+    auto weigh = [&](int n) {
+      pf[n >> 3][n & 7] = (__bf16)__builtin_amdgcn_exp2f(
+          __builtin_fmaf(s[n >> 4][n & 15], scale, -m));
+    };
+#pragma unroll
+    for (int n = 0; n < 16; ++n) weigh(n);
     __builtin_amdgcn_sched_barrier(0);
-    PF_PUT(1 - b)
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {
+      acc[n & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          vf[n % V_AHEAD], pf[n >> 2], acc[n & 3], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (n + V_AHEAD < 16) vf[n % V_AHEAD] = v_read(n + V_AHEAD);
+      if (n < 8) {
+        weigh(16 + 2 * n);
+        weigh(17 + 2 * n);
+      } else {
+        // the sum of the weights as they are used, rounded: an error that the
+        // largest share with it cancels
+        const int e = (n - 8) >> 1, i = (n & 1) * 4;
+        l = pf_add2(pf[e][i], pf[e][i + 1], l);
+        l = pf_add2(pf[e][i + 2], pf[e][i + 3], l);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  int t = begin;
+  for (; t < whole; ++t) {
+    PF_MEET()
+    products(std::false_type(), t);
   }
+  for (; t < wave_tiles; ++t) {
+    PF_MEET()
+    products(std::true_type(), t);
+  }
+  // beyond its own last tile a wave brings rows for the others
   for (; t < tiles; ++t) {
-    PF_STAGE(t)
-    PF_PUT(1 - (t & 1))
+    PF_MEET()
+    bring_all(min(t + 1, tiles - 1), t + 1);
+    name(min(t + 2, tiles - 1));
   }
-#undef PF_STAGE
-#undef PF_SLOTS
-#undef PF_ROWS
-#undef PF_PUT
+#undef PF_MEET
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // LDS is in use until then
 
   l += __shfl_xor(l, 32, 64);
+  if (part >= 0) {
+    const size_t at = ((size_t)part * num_kv_heads + kvh) * ROWS;
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      *reinterpret_cast<f32x4*>(
+          part_o + at * DIM + ((wave * 16 + e) * 64 + lane) * 4) =
+          f32x4{acc[e >> 2][(e & 3) * 4], acc[e >> 2][(e & 3) * 4 + 1],
+                acc[e >> 2][(e & 3) * 4 + 2], acc[e >> 2][(e & 3) * 4 + 3]};
+    if (h == 0) {
+      part_ml[(at + in) * 2] = m;
+      part_ml[(at + in) * 2 + 1] = l;
+    }
+    return;
+  }
   if (my_row < q_rows && in < tokens * group) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
     const bool seen = my_pos >= 0;      // else the sums are of masked scores
@@ -273,27 +382,88 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
   }
 }
 
+// The sums of a block whose keys were cut, from those of its parts.  A workgroup
+// per block, key head and 32 dims; bound by reading them, 512 bytes a row and
+// part, in the order in which the kernel above holds them.
+__global__ __launch_bounds__(THREADS) void prefill_join_kernel(
+    __hip_bfloat16* __restrict__ out, const float* __restrict__ part_o,
+    const float* __restrict__ part_ml, const int* __restrict__ block_info,
+    const int* __restrict__ seq_lens,
+    const int* __restrict__ joins,           // [n, 3]: block, its first part, parts
+    const int num_q_heads, const int num_kv_heads) {
+  const int blk = joins[blockIdx.x * 3], first = joins[blockIdx.x * 3 + 1];
+  const int parts = joins[blockIdx.x * 3 + 2];
+  const int kvh = blockIdx.y, d = blockIdx.z;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 31, h = lane >> 5, in = wave * 32 + c;
+  const int group = num_q_heads / num_kv_heads, tokens = ROWS / group;
+  const int offset = block_info[blk * 4 + 3];
+  const int my_row = block_info[blk * 4 + 1] * tokens + in / group;
+  float top = LOW, l = 0.f;
+  f32x4 o[4] = {};
+  for (int p = 0; p < parts; ++p) {
+    const size_t at = ((size_t)(first + p) * num_kv_heads + kvh) * ROWS;
+    f32x4 x[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      x[e] = *reinterpret_cast<const f32x4*>(
+          part_o + at * DIM + ((wave * 16 + d * 4 + e) * 64 + lane) * 4);
+    const float m = part_ml[(at + in) * 2];
+    const float most = fmaxf(top, m);
+    const float fade = __builtin_amdgcn_exp2f(top - most);
+    const float f = __builtin_amdgcn_exp2f(m - most);
+    top = most;
+    l = l * fade + part_ml[(at + in) * 2 + 1] * f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = o[e] * fade + x[e] * f;
+  }
+  if (my_row >= seq_lens[blk] - offset || in >= tokens * group) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const bool seen = offset + my_row >= 0;
+  __hip_bfloat16* op = out +
+      ((size_t)(block_info[blk * 4] + my_row) * num_q_heads + kvh * group +
+       in % group) * DIM + d * 32 + 4 * h;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    union { __hip_bfloat16 e[4]; uint2 u; } b;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b.e[j] = f2bf(seen ? o[e][j] * inv : 0.f);
+    *reinterpret_cast<uint2*>(op + e * 8) = b.u;
+  }
+}
+
 }  // namespace
 
+// items and joins: null, or the blocks' work as cut up and what is to be joined
 extern "C" void launch_prefill_flash(
     void* out, const void* q, const void* k, const void* v, const void* slots,
     const void* block_info, const void* seq_lens, float scale, int blocks,
-    int num_q_heads, int num_kv_heads, int page_shift, long q_stride,
-    long kv_stride, hipStream_t stream) {
-  if (blocks == 0) return;
-  const int units = num_kv_heads * blocks;
+    const void* items, int count, const void* joins, int joined, void* part_o,
+    void* part_ml, int num_q_heads, int num_kv_heads, int page_shift,
+    long q_stride, long kv_stride, hipStream_t stream) {
+  if (!items) count = blocks;
+  if (count == 0) return;
+  const int units = num_kv_heads * count;
   const int grid = num_kv_heads % 8 && 8 % num_kv_heads == 0
                        ? (units + 7) / 8 * 8 : units;
   // a scale of 0 would make masked scores 0 as well
   const float base2 = fmaxf(fabsf(scale) * 1.44269504088896f, 1e-20f);
-#define PF_GO(PAGED)                                                       \
-  prefill_flash_kernel<PAGED><<<dim3(grid), dim3(THREADS), 0, stream>>>(   \
+#define PF_GO(FROM)                                                        \
+  prefill_flash_kernel<FROM><<<dim3(grid), dim3(THREADS), LDS, stream>>>(  \
       (__hip_bfloat16*)out, (const __hip_bfloat16*)q,                      \
       (const __hip_bfloat16*)k, (const __hip_bfloat16*)v,                  \
       (const int*)slots, (const int*)block_info, (const int*)seq_lens,     \
-      base2, scale < 0.f, num_q_heads, num_kv_heads, page_shift, q_stride, \
-      kv_stride, blocks)
-  if (slots) PF_GO(true);
-  else PF_GO(false);
+      (const int*)items, (float*)part_o, (float*)part_ml, base2,           \
+      scale < 0.f, num_q_heads, num_kv_heads, page_shift, q_stride,        \
+      kv_stride, count)
+  if (slots) PF_GO(FROM_PAGES);
+  else if (kv_stride < (1 << 23)) PF_GO(FROM_ROWS);
+  else PF_GO(FROM_FAR_ROWS);
 #undef PF_GO
+  if (joined)
+    prefill_join_kernel<<<dim3(joined, num_kv_heads, DIM / 32), dim3(THREADS),
+                          0, stream>>>(
+        (__hip_bfloat16*)out, (const float*)part_o, (const float*)part_ml,
+        (const int*)block_info, (const int*)seq_lens, (const int*)joins,
+        num_q_heads, num_kv_heads);
 }

@@ -4,6 +4,8 @@ contracts — they must depend only on (padded batch, config), never on
 per-step tensor values — and the split policy encodes a measured optimum
 (~1024 workgroups fills 256 CUs / 8 XCDs; profiles/decode_breakdown.md
 r59 sweep), so a regression here silently costs decode bandwidth."""
+import pytest
+
 from rbg_amd.engine.model_runner import GRAPH_BATCH_SIZES
 from rbg_amd.ops import pick_decode_splits
 
@@ -66,6 +68,47 @@ def test_prefill_plan_covers_every_row():
             for b in range(4)
             for i in range(-(-(cu[b + 1] - cu[b]) // tokens)))
         assert got == want
+
+
+@pytest.mark.parametrize("kvh", [1, 3, 4, 8, 40])
+def test_cut_prefill_covers_every_tile(kvh):
+    """Of a block that is cut every tile of keys once, its parts in order and
+    numbered in a row; few enough for a bounded workspace; some blocks are cut
+    and some whole."""
+    import random
+
+    from rbg_amd import ops
+    rng = random.Random(kvh)
+    cut = 0
+    for _ in range(200):
+        n = rng.randint(1, 12)
+        rows = [int(2 ** rng.uniform(0, 11)) for _ in range(n)]
+        pasts = [rng.choice([0, -min(3, r - 1), int(2 ** rng.uniform(0, 14))])
+                 for r in rows]
+        cu, cu_k = [0], [0]
+        for r, p in zip(rows, pasts):
+            cu.append(cu[-1] + r)
+            cu_k.append(cu_k[-1] + r + p)
+        group = rng.choice([1, 3, 4, 8, 128])
+        plan = ops.prefill_plan(cu, cu_k, kvh * group, kvh, "cpu")
+        if plan.items is None:
+            continue
+        cut += 1
+        assert plan.parts * kvh <= 768          # 64 KB of sums each
+        pieces = {}
+        for b, begin, end, part in sorted(plan.items.tolist()):
+            pieces.setdefault(b, []).append((begin, end, part))
+        joins = {b: list(range(first, first + count))
+                 for b, first, count in plan.joins.tolist()}
+        assert sorted(sum(joins.values(), [])) == list(range(plan.parts))
+        for b, ((_, nth, _, past), keys) in enumerate(
+                zip(plan.blocks.tolist(), plan.lens.tolist())):
+            need = min(past + (nth + 1) * (128 // group), keys)
+            ends = [0] + [p[1] for p in pieces[b]]
+            assert ends[-1] == max(-(-need // 64), 0)
+            assert [p[0] for p in pieces[b]] == ends[:-1]
+            assert [p[2] for p in pieces[b]] == joins.get(b, [-1])
+    assert cut > 20
 
 
 def test_default_parts_are_bounded():

@@ -650,6 +650,58 @@ def test_prefill_flash(heads, kvh, news, pasts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,kvh", [(4, 1), (6, 2), (32, 8)])
+@pytest.mark.parametrize("news,pasts", [
+    ([1], [2500]), ([70, 1, 300], [2500, 0, 0]), ([129], [1900])])
+def test_prefill_flash_cut(heads, kvh, news, pasts):
+    """Blocks cut by keys, beside whole ones: parts that end anywhere in a
+    sequence and on its diagonal, scores that move the maximum from part to
+    part, sums that a capture replays.  Bounds as in test_prefill_flash."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(heads * 1000 + sum(news))
+    cu = [0] + torch.tensor(news).cumsum(0).tolist()
+    cu_k = [0] + (torch.tensor(news) + torch.tensor(pasts)).cumsum(0).tolist()
+    q = torch.randn(cu[-1], heads, 128, device=dev, generator=gen).bfloat16()
+    k, v = torch.randn(2, cu_k[-1], kvh, 128, device=dev,
+                       generator=gen).bfloat16()
+    k[::333] *= 4
+    n = cu_k[-1] // 16 + 1
+    slots = torch.randperm(n * 16, device=dev, generator=gen)[:cu_k[-1]]
+    pages = torch.zeros(2, n, kvh, 16, 128, dtype=torch.bfloat16, device=dev)
+    pages[0, slots // 16, :, slots % 16] = k
+    pages[1, slots // 16, :, slots % 16] = v
+    plan = ops.prefill_plan(cu, cu_k, heads, kvh, dev)
+    assert plan.items is not None
+    for scale in (0.3, -0.09):
+        got = ops.prefill_attention(q, k, v, None, scale, plan=plan)
+        for b, past in enumerate(pasts):
+            kb, vb = (t[cu_k[b]:cu_k[b + 1]].double() for t in (k, v))
+            at = past + torch.arange(news[b], device=dev)
+            hide = torch.arange(len(kb), device=dev)[None] > at[:, None]
+            for h in range(heads):
+                g = h // (heads // kvh)
+                s = q[cu[b]:cu[b + 1], h].double() @ kb[:, g].t().contiguous()
+                w = (s * scale).masked_fill(hide, -math.inf).softmax(-1)
+                want = w @ vb[:, g]
+                bound = want.abs() * 2 ** -8 + (w @ vb[:, g].abs()) * 2 ** -7
+                err = (got[cu[b]:cu[b + 1], h].double() - want).abs()
+                assert (err <= bound + 1e-5).all(), (scale, b, h)
+        paged = ops.prefill_attention(q, pages[0], pages[1], None, scale,
+                                      plan=plan, slots=slots.int())
+        assert torch.equal(paged, got)
+    g = torch.cuda.CUDAGraph()
+    with torch.inference_mode(), torch.cuda.graph(g):
+        out = ops.prefill_attention(q, k, v, None, -0.09, plan=plan)
+    for _ in range(3):
+        with torch.inference_mode():
+            out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, got)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 3, 4])
 @pytest.mark.parametrize("k", [2048, 8192])
 @pytest.mark.parametrize("first", [False, True])
