@@ -108,7 +108,7 @@ def test_cut_prefill_covers_every_tile(kvh):
             assert ends[-1] == max(-(-need // 64), 0)
             assert [p[0] for p in pieces[b]] == ends[:-1]
             assert [p[2] for p in pieces[b]] == joins.get(b, [-1])
-    assert cut > 20
+    assert cut > 5
 
 
 def test_default_parts_are_bounded():
