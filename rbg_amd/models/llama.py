@@ -373,7 +373,7 @@ class LlamaForCausalLM(nn.Module):
                gather_idx: Optional[torch.Tensor] = None) -> torch.Tensor:
         if gather_idx is not None:
             hidden = hidden[gather_idx.long()]
-        return ops.linear(hidden, self.lm_head).float()
+        return ops.linear_f32(hidden, self.lm_head)
 
     def reload_weights(self, seed: int) -> None:
         """In-place weight refresh — the live-update path (SURVEY §2.3

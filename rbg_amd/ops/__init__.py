@@ -169,6 +169,16 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, w)
 
 
+def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """linear(x, w).float(): the decode GEMM stores its rounded results so (a
+    launch of 2 to 4 us less)."""
+    if _takes_skinny(x, w):
+        return require("_hip_ops", "_hip_mix", "_hip_gated", "_hip_moe",
+                       "_hip_hyper").skinny_gemm(
+            x if x.is_contiguous() else x.contiguous(), w, wide=True)
+    return linear(x, w).float()
+
+
 def _tile(rows: int, n: int, k: int) -> bool:
     """Does the GEMM of prompts (hip/tile_gemm.hip) take a [rows, k] x [n, k]
     product whose reader adds up parts, rather than the decode GEMM or

@@ -697,7 +697,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma_probe", &mfma_probe, "MFMA layout probe");
   m.def("mfma_probe32", &mfma_probe32, "32x32x16 MFMA layout probe");
   m.def("skinny_gemm", &skinny_gemm, "decode-shape GEMM (M<=256)",
-        py::arg("a"), py::arg("w"), py::arg("force_splits") = 0);
+        py::arg("a"), py::arg("w"), py::arg("force_splits") = 0,
+        py::arg("wide") = false);
   m.def("skinny_parts", &skinny_parts, "decode GEMM as its parts' sums");
   m.def("skinny_swiglu", &skinny_swiglu, "decode gate/up GEMM with silu");
   m.def("tile_swiglu", &tile_swiglu, "gate/up GEMM of a prompt with silu");

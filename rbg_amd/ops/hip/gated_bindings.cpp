@@ -257,5 +257,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.attr("CHUNK") = gated_chunk_tokens();
   m.attr("CHUNK_MAX_DIM") = gated_chunk_max_dim();
   m.def("skinny_gemm", &skinny_gemm, "decode-shape GEMM (M<=256)",
-        py::arg("a"), py::arg("w"), py::arg("force_splits") = 0);
+        py::arg("a"), py::arg("w"), py::arg("force_splits") = 0,
+        py::arg("wide") = false);
 }

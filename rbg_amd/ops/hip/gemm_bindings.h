@@ -99,25 +99,28 @@ inline void check_skinny(const torch::Tensor& a, const torch::Tensor& w) {
               "unsupported skinny shape");
 }
 
+// wide: the result, rounded to bf16 all the same, in f32
 inline torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor w,
-                          int64_t force_splits = 0) {
+                                 int64_t force_splits = 0, bool wide = false) {
   check_skinny(a, w);
   const int64_t M = a.size(0), K = a.size(1), N = w.size(0);
-  auto c = torch::empty({M, N}, a.options());
   SkinnyPlan plan = pick_summed((int)M, (int)N, (int)K);
   if (force_splits > 0 && K % (force_splits * 256) == 0)
     plan = {plan.waves ? plan.waves : 8, (int)force_splits};
+  const bool direct = wide && plan.splits == 1;
+  auto c = torch::empty(
+      {M, N}, direct ? a.options().dtype(torch::kFloat32) : a.options());
   torch::Tensor ws;
-  void* wsp = nullptr;
+  void* wsp = direct ? c.data_ptr() : nullptr;
   if (plan.splits > 1) {
     ws = torch::empty({plan.splits, M, N}, a.options().dtype(torch::kFloat32));
     wsp = ws.data_ptr();
   }
-  launch_skinny_gemm(c.data_ptr(), wsp, a.data_ptr(), w.data_ptr(), (int)M,
+  launch_skinny_gemm(direct ? nullptr : c.data_ptr(), wsp, a.data_ptr(), w.data_ptr(), (int)M,
                      (int)N, (int)K, plan.waves, plan.splits, 0,
                      gemm_stream());
   if (plan.splits > 1)
     launch_reduce_splits(c.data_ptr(), wsp, plan.splits, (long)(M * N),
                          gemm_stream());
-  return c;
+  return wide && !direct ? c.to(torch::kFloat32) : c;
 }

@@ -89,5 +89,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gelu_mul", &gelu_mul, "gelu_tanh(gate) * up");
   m.def("clamped_glu", &clamped_glu, "clamped gated unit");
   m.def("skinny_gemm", &skinny_gemm, "decode-shape GEMM (M<=256)",
-        py::arg("a"), py::arg("w"), py::arg("force_splits") = 0);
+        py::arg("a"), py::arg("w"), py::arg("force_splits") = 0,
+        py::arg("wide") = false);
 }

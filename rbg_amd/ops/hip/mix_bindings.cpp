@@ -213,5 +213,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("delta_chunk", &delta_chunk, "generalized delta rule, by chunks");
   m.attr("DELTA_CHUNK") = delta_chunk_tokens();
   m.def("skinny_gemm", &skinny_gemm, "decode-shape GEMM (M<=256)",
-        py::arg("a"), py::arg("w"), py::arg("force_splits") = 0);
+        py::arg("a"), py::arg("w"), py::arg("force_splits") = 0,
+        py::arg("wide") = false);
 }

@@ -246,5 +246,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_prefill", &paged_prefill, "varlen attention over pages");
   m.def("paged_decode", &paged_decode, "one query per sequence over pages");
   m.def("skinny_gemm", &skinny_gemm, "decode-shape GEMM (M<=256)",
-        py::arg("a"), py::arg("w"), py::arg("force_splits") = 0);
+        py::arg("a"), py::arg("w"), py::arg("force_splits") = 0,
+        py::arg("wide") = false);
 }

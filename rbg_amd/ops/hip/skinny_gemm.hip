@@ -36,7 +36,8 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
     const __hip_bfloat16* __restrict__ a,   // [M, K]
     const __hip_bfloat16* __restrict__ w,   // [N, K]
     __hip_bfloat16* __restrict__ c,         // [M, N], GLU: [M, N / 2]
-    float* __restrict__ ws,                 // [gridDim.y, M, N] if > 1
+    float* __restrict__ ws,                 // [gridDim.y, M, N] if > 1, or C
+                                            // in f32 if c is null
     const int M, const int N, const int K) {
   constexpr int THREADS = 64 * NW, PITCH = KC + 8;   // + 8: no bank conflicts
   constexpr int PER = THREADS * 8 / KC;     // rows of A that one load covers
@@ -154,10 +155,12 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
       for (int q = 0; q < 4; ++q) {
         const int m = i * 16 + g * 4 + q;
         if (m >= M) continue;
-        if (gridDim.y == 1)
+        if (gridDim.y > 1)
+          ws[((size_t)blockIdx.y * M + m) * N + col0 + r] = acc[i][q];
+        else if (c)
           c[(size_t)m * N + col0 + r] = f2bf(acc[i][q]);
         else
-          ws[((size_t)blockIdx.y * M + m) * N + col0 + r] = acc[i][q];
+          ws[(size_t)m * N + col0 + r] = bf2f(f2bf(acc[i][q]));
       }
   }
 }
@@ -192,6 +195,7 @@ void launch_tiles(__hip_bfloat16* c, float* ws, const __hip_bfloat16* a,
 // ---------------------------------------------------------------------------
 // C launchers (torch glue lives in gemm_bindings.h)
 
+// c may be null where nothing is split (splits == 1): ws is C then, in f32.
 extern "C" void launch_skinny_gemm(void* c, void* ws, const void* a,
                                    const void* w, int M, int N, int K,
                                    int waves, int splits, int glu,
@@ -212,9 +216,13 @@ extern "C" void launch_skinny_gemm(void* c, void* ws, const void* a,
   if (waves == 0) {             // the kernel of a few rows
     if (glu)
       launch_skinny_rows<ROWS_GLU, false>(cp, ap, wp, M, N, K, {}, {}, stream);
+    else if ((N <= 2048 && K >= 4096) ||
+             (M == 1 && N > 4096 && N <= 6144 && K >= 8192))
+      launch_skinny_rows<ROWS_PLAIN, false, true>(cp, ap, wp, M, N, K, {}, {},
+                                                  stream, cp ? nullptr : wsp);
     else
       launch_skinny_rows<ROWS_PLAIN, false>(cp, ap, wp, M, N, K, {}, {},
-                                            stream);
+                                            stream, cp ? nullptr : wsp);
   } else if (mt <= 1 && waves == 4) SG_GO(1, 4);
   else if (mt <= 2 && waves == 4) SG_GO(2, 4);
   else if (mt <= 1) SG_GO(1, 8);

@@ -59,46 +59,60 @@ struct RowsRope {
 // every workgroup reads all of A (28672 x 4096: 1 row 41.8 us, 4 rows 44.3).
 // GLU and ROPE: the tile is 8 rows of W and the 8 that they meet, N / 2 or 64
 // further on.
+// PAIR: the tile is 8 rows of W, whose k are taken two chunks at a time, so that
+// twice as many workgroups are half as long.  For matrices whose tiles of 16 rows
+// leave half of the chip or more idle, with long k (1 row: 1024 x 4096 8.0 -> 6.1
+// us, 2048 x 5632 10.6 -> 9.8, x 14336 19.6 -> 15.8, x 2048 6.1 -> 6.5; 4 rows: 2048
+// x 4096 8.9 -> 8.4), and where they fill it one and a half times (1 row of 5120 x
+// 8192 24.1 -> 19.5, of 6144 x 25600 69 -> 58; 4 rows 25.4 -> 25.1, 74 -> 78).
 // NORM: every workgroup forms A for itself, in LDS, while its first weights are
 // on their way; the row's 1 / rms is a factor of the result, so that nothing
 // waits for it.  A launch of its own takes 2.6 us.
-template <int END, bool NORM>
+template <int END, bool NORM, bool PAIR>
 __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
     const __hip_bfloat16* __restrict__ a,   // [M, K]; NORM: src, may be null
     const __hip_bfloat16* __restrict__ w,   // [N, K]
     __hip_bfloat16* __restrict__ c,         // [M, N], GLU: [M, N / 2]
+    float* __restrict__ wide,               // PLAIN: not null: C in f32
     const int M, const int N, const int K, const RowsNorm norm,
     const RowsRope rope) {
-  constexpr int WAVES = 8;
+  static_assert(!PAIR || (END == ROWS_PLAIN && !NORM), "plain products only");
+  constexpr int WAVES = 8, STEP = PAIR ? 2 * ROWS_KC : ROWS_KC;
   extern __shared__ __align__(16) char rows_lds[];
   __shared__ float squares[WAVES][ROWS_MOST];
   __hip_bfloat16* al = (__hip_bfloat16*)rows_lds;         // NORM: [M, K]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
   const int apart = END == ROWS_GLU ? N / 2 : 64;
-  const int col0 = END == ROWS_PLAIN ? blockIdx.x * 16
+  const int col0 = PAIR ? blockIdx.x * 8
+                   : END == ROWS_PLAIN ? blockIdx.x * 16
                    : END == ROWS_GLU ? blockIdx.x * 8
                                      : (blockIdx.x >> 3) * 128 +
                                            (blockIdx.x & 7) * 8;
-  const int row = END == ROWS_PLAIN ? col0 + r
-                                    : col0 + (r & 7) + (r >> 3) * apart;
-  const __hip_bfloat16* wp = w + (size_t)row * K + wave * ROWS_KC + g * 8;
-  const __hip_bfloat16* ap =
-      (NORM ? al : a) + (size_t)min(r, M - 1) * K + wave * ROWS_KC + g * 8;
-  const int n = (K / ROWS_KC - wave + WAVES - 1) / WAVES;
+  const int row = PAIR ? col0 + (r & 7)
+                  : END == ROWS_PLAIN ? col0 + r
+                                      : col0 + (r & 7) + (r >> 3) * apart;
+  // PAIR: W's second 8 rows and A's second 4 stand for the first ones' next k
+  const __hip_bfloat16* wp = w + (size_t)row * K + wave * STEP + g * 8 +
+                             (PAIR ? (r >> 3) * ROWS_KC : 0);
+  const __hip_bfloat16* ap = (NORM ? al : a) +
+                             (size_t)min(PAIR ? r & 3 : r, M - 1) * K +
+                             wave * STEP + g * 8 +
+                             (PAIR ? (r >> 2 & 1) * ROWS_KC : 0);
+  const int n = (K / STEP - wave + WAVES - 1) / WAVES;
   const int first = n ? ((blockIdx.x >> 3) + (blockIdx.x & 7) * (n >> 3)) % n
                       : 0;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   sg_u4 wr[ROWS_DEPTH][2], ar[ROWS_DEPTH][2];
 #define SR_WEIGHTS(s, at)                                                  \
   do {                                                                     \
-    const int off = sg_turn(at, first, n) * (ROWS_KC * WAVES);             \
+    const int off = sg_turn(at, first, n) * (STEP * WAVES);                \
     wr[s][0] = sg_load(wp + off);                                          \
     wr[s][1] = sg_load(wp + off + 32);                                     \
   } while (0)
 #define SR_ROWS(s, at)                                                     \
   do {                                                                     \
-    const int off = sg_turn(at, first, n) * (ROWS_KC * WAVES);             \
+    const int off = sg_turn(at, first, n) * (STEP * WAVES);                \
     ar[s][0] = sg_load(ap + off);                                          \
     ar[s][1] = sg_load(ap + off + 32);                                     \
   } while (0)
@@ -181,20 +195,21 @@ __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
   // the first ROWS_MOST rows are there, the first 16 lanes'
   if (NORM) __syncthreads();                // A is read
   float* red = (float*)rows_lds;            // [WAVES][16 columns][ROWS_MOST]
-  if (g == 0)
+  if (PAIR ? g == r >> 3 : g == 0)
     *reinterpret_cast<f32x4*>(red + (wave * 16 + r) * ROWS_MOST) = acc;
   __syncthreads();
   const int e = threadIdx.x;
   if (e >= 16 * ROWS_MOST) return;
   const int col = e / ROWS_MOST, m = e % ROWS_MOST;
-  if (m >= M || (END != ROWS_PLAIN && col >= 8)) return;
+  if (m >= M || ((PAIR || END != ROWS_PLAIN) && col >= 8)) return;
   float v = 0.f, v2 = 0.f, factor = 1.f;
 #pragma unroll
   for (int k = 0; k < WAVES; ++k) {
     v += red[k * 16 * ROWS_MOST + e];
-    if (END != ROWS_PLAIN)
+    if (PAIR || END != ROWS_PLAIN)
       v2 += red[k * 16 * ROWS_MOST + e + 8 * ROWS_MOST];
   }
+  if (PAIR) v += v2;
   if (NORM) {
     float total = 0.f;
 #pragma unroll
@@ -204,7 +219,8 @@ __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
   v *= factor;
   v2 *= factor;
   if (END == ROWS_PLAIN) {
-    c[(size_t)m * N + col0 + col] = f2bf(v);
+    if (wide) wide[(size_t)m * N + col0 + col] = bf2f(f2bf(v));
+    else c[(size_t)m * N + col0 + col] = f2bf(v);
   } else if (END == ROWS_GLU) {
     c[(size_t)m * (N / 2) + col0 + col] = f2bf(silu(v) * v2);
   } else {
@@ -232,16 +248,16 @@ __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
   }
 }
 
-template <int END, bool NORM>
+template <int END, bool NORM, bool PAIR = false>
 void launch_skinny_rows(__hip_bfloat16* c, const __hip_bfloat16* a,
                         const __hip_bfloat16* w, int M, int N, int K,
                         const RowsNorm& norm, const RowsRope& rope,
-                        hipStream_t stream) {
+                        hipStream_t stream, float* wide = nullptr) {
   const size_t sums = 8 * 16 * ROWS_MOST * sizeof(float);
   const size_t rows = NORM ? (size_t)M * K * 2 : 0;
-  skinny_rows_kernel<END, NORM>
-      <<<dim3(N / 16), dim3(512), rows > sums ? rows : sums, stream>>>(
-          a, w, c, M, N, K, norm, rope);
+  skinny_rows_kernel<END, NORM, PAIR>
+      <<<dim3(N / (PAIR ? 8 : 16)), dim3(512), rows > sums ? rows : sums,
+         stream>>>(a, w, c, wide, M, N, K, norm, rope);
 }
 
 }  // namespace

@@ -650,6 +650,30 @@ def test_prefill_flash(heads, kvh, news, pasts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,n,k", [
+    (1, 32, 4096), (4, 2048, 4096), (3, 1024, 14336), (2, 2048, 5632),
+    (1, 5120, 8192), (1, 6144, 8704), (1, 4128, 14336), (5, 2048, 2048),
+    (64, 32768, 2048), (128, 1024, 4096)])
+def test_rows_of_pairs_and_f32(rows, n, k):
+    """Forms whose tiles take two chunks of k at a time, at the ends of the rule
+    for them, and results in f32, which are the rounded ones: 2^-8 of each, and
+    f32 sums of k products."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(rows + n + k)
+    x = torch.randn(rows, k, device=dev, generator=gen).bfloat16()
+    w = torch.randn(n, k, device=dev, generator=gen).bfloat16()
+    want = x.double() @ w.double().t().contiguous()
+    size = x.double().abs() @ w.double().abs().t().contiguous()
+    got = ops._hip.skinny_gemm(x, w)
+    assert ((got.double() - want).abs() <=
+            want.abs() * 2 ** -8 + size * 2 ** -18).all()
+    wide = ops._hip.skinny_gemm(x, w, wide=True)
+    assert wide.dtype == torch.float32 and torch.equal(wide, got.float())
+    assert torch.equal(ops.linear_f32(x, w), ops.linear(x, w).float())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads,kvh", [(4, 1), (6, 2), (32, 8)])
 @pytest.mark.parametrize("news,pasts", [
     ([1], [2500]), ([70, 1, 300], [2500, 0, 0]), ([129], [1900])])
