@@ -30,6 +30,8 @@ class ForwardBatch:
     block_tables: Optional[torch.Tensor] = None  # [S, max_pages] int32
     context_lens: Optional[torch.Tensor] = None  # [S] int32
     decode_num_splits: int = 0      # 0 = pick host-side (sync-free in graphs)
+    tickets: Optional[torch.Tensor] = None  # [S * kv heads] int32 zeros of this
+    #   batch's stream, for ops.decode_attention
     # models that look at pairs of tokens: [T] int64, -1 before the first
     prev_tokens: Optional[torch.Tensor] = None
     # models with per-sequence state

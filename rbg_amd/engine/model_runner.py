@@ -19,6 +19,7 @@ import torch
 
 from ..models.llama import PPContext, TPContext
 from ..models.registry import build_model
+from ..ops import place_inputs
 from ..utils.upload import upload
 from .batch import ForwardBatch, VarlenLayout, table_array
 from .config import EngineConfig
@@ -241,14 +242,14 @@ class ModelRunner:
         fields_dev, bt_dev = upload([fields, bt], self.device)
         if bucket:
             static = self._graphs[bucket][1]
-            static["fields"].copy_(fields_dev)
-            static["bt"].zero_()
-            static["bt"][:n, :bt.shape[1]].copy_(bt_dev)
+            place_inputs(static["fields"], static["bt"], fields_dev, bt_dev)
         else:
-            static = dict(self._fields(fields_dev), bt=bt_dev)
+            static = dict(self._fields(fields_dev), bt=bt_dev,
+                          tickets=self.model.decode_tickets(rows))
         state = {k: static[k][:n] for k in ("tokens", "prev", "positions",
                                             "slots", "ctx", "state_slots")}
         state["bt"] = static["bt"][:n]
+        state["tickets"] = static["tickets"]
         if not self.model.needs_prev:
             state["prev"] = None
         if not self.model.stateful:
@@ -328,7 +329,7 @@ class ModelRunner:
             mode="decode", positions=inputs["positions"], slot_mapping=slots,
             block_tables=inputs["bt"], context_lens=inputs["ctx"],
             starts=inputs["positions"], state_slots=inputs["state_slots"],
-            prev_tokens=inputs["prev"],
+            prev_tokens=inputs["prev"], tickets=inputs["tickets"],
             decode_num_splits=self.model.decode_splits(
                 n, self.cfg.max_seq_len, self.cfg.page_size))
 
@@ -364,6 +365,7 @@ class ModelRunner:
         fields = torch.zeros(4 * bs, dtype=torch.int64, device=self.device)
         static = dict(self._fields(fields), fields=fields)
         static["ctx"].fill_(1)
+        static["tickets"] = self.model.decode_tickets(bs)
         static["bt"] = torch.zeros(bs, self.max_pages_per_seq,
                                    dtype=torch.int32, device=self.device)
         batch = self._decode_batch(static, static["slots"], bs)

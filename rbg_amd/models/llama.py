@@ -209,7 +209,8 @@ class LlamaAttention(nn.Module):
             o = ops.decode_attention(q3, key_cache, value_cache,
                                      batch.block_tables, batch.context_lens,
                                      self.scale,
-                                     num_splits=batch.decode_num_splits)
+                                     num_splits=batch.decode_num_splits,
+                                     tickets=batch.tickets)
         o = o.view(T, self.q_out).contiguous()
         if self.parts:
             return ops.linear_parts(o, self.wo), residual
@@ -337,6 +338,11 @@ class LlamaForCausalLM(nn.Module):
 
     def make_cache(self, cfg: EngineConfig) -> PagedKVCache:
         return PagedKVCache(cfg, self.device, num_layers=self.num_local_layers)
+
+    def decode_tickets(self, rows: int) -> torch.Tensor:
+        """For the decode attention of that many sequences."""
+        return torch.zeros(rows * self.cfg.num_kv_heads // self.tp.size,
+                           dtype=torch.int32, device=self.device)
 
     def decode_splits(self, batch_size: int, max_seq_len: int,
                       page_size: int = 16) -> int:

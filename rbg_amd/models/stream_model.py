@@ -105,6 +105,9 @@ class StreamForCausalLM(nn.Module):
         """Columns of what one pipeline stage hands to the next."""
         return self.cfg.hidden_size
 
+    def decode_tickets(self, rows: int) -> None:
+        return None         # ops.decode_attention is not used
+
     def decode_splits(self, batch_size: int, max_seq_len: int,
                       page_size: int = 16) -> int:
         return 0                        # per layer, from its sizes

@@ -279,6 +279,18 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return silu_mul(linear_parts(x, w))
 
 
+def place_inputs(fields, tables, new_fields, new_tables) -> None:
+    """A captured decode step's inputs from new ones: ``fields``, and ``tables``
+    [rows, width] with page 0 beyond ``new_tables`` [seqs, used]."""
+    if _on_gpu(fields) and _hip is not None:
+        _hip.place_inputs(fields, tables, new_fields, new_tables)
+        return
+    n, used = new_tables.shape
+    fields.copy_(new_fields)
+    tables.zero_()
+    tables[:n, :used].copy_(new_tables)
+
+
 def embed_rows(ids: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
     """table[ids]; NaN for an id outside where the kernel takes the call (1.8 us
     for a row of 4096, the indexing kernel 3.0; 128 rows 2.0 both)."""
@@ -470,7 +482,10 @@ PREFILL_SWZ = int(__import__("os").environ.get("RBG_PREFILL_SWZ", "16"))  # pref
 
 def decode_attention(q, key_cache, value_cache, block_tables, context_lens,
                      scale: float, num_splits: int = 0,
-                     variant: int = -1) -> torch.Tensor:
+                     variant: int = -1, tickets=None) -> torch.Tensor:
+    """``tickets``: int32 zeros, one for every sequence and key head, which only
+    this stream uses and which are zeros again afterwards: the parts of a sequence
+    are then added up without a launch of their own."""
     if _on_gpu(q):
         if num_splits <= 0:
             if (DECODE_VARIANT if variant < 0 else variant) == 7:
@@ -486,7 +501,7 @@ def decode_attention(q, key_cache, value_cache, block_tables, context_lens,
         return _require_hip().decode_attention(
             q, key_cache, value_cache, block_tables, context_lens, scale,
             num_splits, variant,
-            _decode_span(q.shape[0] * key_cache.shape[1])[0])
+            _decode_span(q.shape[0] * key_cache.shape[1])[0], tickets)
     return reference.decode_attention(q, key_cache, value_cache, block_tables,
                                       context_lens, scale)
 

@@ -947,7 +947,7 @@ void launch_decode_attention(void* out, void* partial_o, void* partial_ml,
   // every part leaves sums, to the base of e
 #define DECODE_JOIN()                                                         \
   launch_decode_join((__hip_bfloat16*)out, (const float*)partial_o,           \
-                     (const float*)partial_ml, nullptr, 0, num_splits,        \
+                     (const float*)partial_ml, nullptr, 0, 0, num_splits,     \
                      num_q_heads, num_seqs, 1.44269504088896f, stream)
   if (variant == 6 && page_size == 16) {
     dim3 pgrid(num_kv_heads, num_seqs, num_splits), pblock(128);

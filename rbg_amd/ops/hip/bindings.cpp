@@ -38,7 +38,9 @@ void launch_decode_attention(void*, void*, void*, const void*, const void*,
                              hipStream_t);
 void launch_decode_pages(void*, void*, void*, const void*, const void*,
                          const void*, const void*, const void*, float, int,
-                         int, int, int, int, int, int, hipStream_t);
+                         int, int, int, int, int, int, void*, hipStream_t);
+void launch_place_inputs(void*, const void*, int, void*, const void*, int, int,
+                         int, int, hipStream_t);
 void launch_prefill_attention(void*, const void*, const void*, const void*,
                               const void*, const void*, float, int, int, int,
                               int, int, int, hipStream_t);
@@ -358,13 +360,38 @@ std::vector<torch::Tensor> norm_rows(
   return {out, next};
 }
 
-// span: of form 7, the fewest keys that a part has, where the sequence is longer
+// fields and tables [rows, width]: a captured step's inputs, from new ones, whose
+// tables are [seqs, used]
+void place_inputs(torch::Tensor fields, torch::Tensor tables,
+                  torch::Tensor new_fields, torch::Tensor new_tables) {
+  for (const auto& t : {fields, new_fields})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
+                t.scalar_type() == torch::kInt64, "fields: int64 on GPU");
+  for (const auto& t : {tables, new_tables})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.dim() == 2 &&
+                t.scalar_type() == torch::kInt32, "tables: int32 on GPU");
+  TORCH_CHECK(fields.numel() == new_fields.numel() &&
+              new_tables.size(0) <= tables.size(0) &&
+              new_tables.size(1) <= tables.size(1), "sizes disagree");
+  TORCH_CHECK(fields.numel() < (1 << 30) && tables.numel() < (1 << 30),
+              "too many");
+  launch_place_inputs(fields.data_ptr(), new_fields.data_ptr(),
+                      (int)fields.numel(), tables.data_ptr(),
+                      new_tables.data_ptr(), (int)tables.size(0),
+                      (int)tables.size(1), (int)new_tables.size(0),
+                      (int)new_tables.size(1), current_stream());
+}
+
+// span: of form 7, the fewest keys that a part has, where the sequence is longer.
+// tickets: of form 7 on pages of 16, zeros for every sequence and key head, which
+// they are again afterwards: the sequences' last workgroups add up the parts.
 torch::Tensor decode_attention(torch::Tensor q, torch::Tensor key_cache,
                                torch::Tensor value_cache,
                                torch::Tensor block_tables,
                                torch::Tensor context_lens, double scale,
                                int64_t num_splits, int64_t wide,
-                               int64_t span) {
+                               int64_t span,
+                               c10::optional<torch::Tensor> tickets) {
   // q may be a slice of the fused QKV projection: 3-D bf16 with
   // contiguous (head, dim) rows and an arbitrary token stride
   TORCH_CHECK(q.is_cuda() && q.scalar_type() == torch::kBFloat16 &&
@@ -392,13 +419,20 @@ torch::Tensor decode_attention(torch::Tensor q, torch::Tensor key_cache,
     po = partial_o.data_ptr();
     pml = partial_ml.data_ptr();
   }
+  if (tickets)
+    TORCH_CHECK(tickets->is_cuda() && tickets->is_contiguous() &&
+                tickets->scalar_type() == torch::kInt32 &&
+                tickets->numel() >= (int64_t)num_seqs * num_kv_heads,
+                "an int32 ticket per sequence and key head");
   if (wide == 7 && page_size == 16) {
     launch_decode_pages(out.data_ptr(), po, pml, q.data_ptr(),
                         key_cache.data_ptr(), value_cache.data_ptr(),
                         block_tables.data_ptr(), context_lens.data_ptr(),
                         (float)scale, num_seqs, num_q_heads, num_kv_heads,
                         max_pages, (int)num_splits, (int)span,
-                        (int)q.stride(0), current_stream());
+                        (int)q.stride(0),
+                        tickets ? tickets->data_ptr() : nullptr,
+                        current_stream());
     return out;
   }
   launch_decode_attention(out.data_ptr(), po, pml, q.data_ptr(),
@@ -686,7 +720,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_attention", &decode_attention, "paged flash-decode",
         py::arg("q"), py::arg("key_cache"), py::arg("value_cache"),
         py::arg("block_tables"), py::arg("context_lens"), py::arg("scale"),
-        py::arg("num_splits"), py::arg("wide"), py::arg("span") = 128);
+        py::arg("num_splits"), py::arg("wide"), py::arg("span") = 128,
+        py::arg("tickets") = c10::nullopt);
+  m.def("place_inputs", &place_inputs, "a decode step's inputs to their place");
   m.def("prefill_attention", &prefill_attention, "varlen causal flash prefill");
   m.def("prefill_flash", &prefill_flash, "causal attention of prompts",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("block_info"),

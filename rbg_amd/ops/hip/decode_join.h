@@ -10,7 +10,10 @@ constexpr float LOW = -1e30f;
 // Keys of a part: not a share of the table's capacity, which may be many times
 // a sequence's length (one of 2048 keys, 8 heads, tables of 8192 / 40960 /
 // 131072 keys: 11.0 / 20.7 / 27.4 us with shares of the capacity, 11.1 of any).
-DEV_INLINE int part_keys(int ctx, int least, int splits) {
+// Up to `whole` keys are one part all the same.
+DEV_INLINE int part_keys(int ctx, int least, int whole, int splits) {
+  if (ctx > least && ctx <= whole)
+    return (ctx + PART_ROUND - 1) / PART_ROUND * PART_ROUND;
   if (ctx <= least * splits) return least;
   const int all = splits * PART_ROUND;
   return (ctx + all - 1) / all * PART_ROUND;
@@ -22,7 +25,7 @@ DEV_INLINE int part_keys(int ctx, int least, int splits) {
 // parts there are four shares (3 sequences of up to 15000 tokens, 30 parts: 40.7
 // -> 36.7 us with the attention); else one, whose workgroups are a quarter of
 // the threads (128 x 2080: 174 us against 180).
-// lens: parts are of part_keys(length, least, splits), a sequence of one part
+// lens: parts are of part_keys(length, least, whole, splits), a sequence of one part
 // has no sums.  null: every sequence has `splits` of them, perhaps empty ones.
 // to_base2: of the maxima, 1 or log2(e).
 template <int SHARES>
@@ -30,13 +33,13 @@ __global__ __launch_bounds__(DIM * SHARES) void decode_join_kernel(
     __hip_bfloat16* __restrict__ out,       // [seqs, QH, DIM]
     const float* __restrict__ part_o,       // [splits, seqs, QH, DIM]
     const float* __restrict__ part_ml,      // [splits, seqs, QH, 2]
-    const int* __restrict__ lens, const int least, const int splits,
-    const float to_base2) {
+    const int* __restrict__ lens, const int least, const int whole,
+    const int splits, const float to_base2) {
   const int seq = blockIdx.y, d = threadIdx.x % DIM;
   const int share = threadIdx.x / DIM;
   int n = splits;
   if (lens) {
-    const int ctx = lens[seq], span = part_keys(ctx, least, splits);
+    const int ctx = lens[seq], span = part_keys(ctx, least, whole, splits);
     if (ctx <= span) return;
     n = min((ctx + span - 1) / span, splits);
   }
@@ -91,16 +94,16 @@ __global__ __launch_bounds__(DIM * SHARES) void decode_join_kernel(
 
 inline void launch_decode_join(__hip_bfloat16* out, const float* part_o,
                                const float* part_ml, const int* lens,
-                               int least, int splits, int heads, int seqs,
-                               float to_base2, hipStream_t stream) {
+                               int least, int whole, int splits, int heads,
+                               int seqs, float to_base2, hipStream_t stream) {
   if (splits <= 1) return;
   const dim3 grid(heads, seqs);
   if (splits <= 8)
     decode_join_kernel<1><<<grid, dim3(DIM), 0, stream>>>(
-        out, part_o, part_ml, lens, least, splits, to_base2);
+        out, part_o, part_ml, lens, least, whole, splits, to_base2);
   else
     decode_join_kernel<4><<<grid, dim3(DIM * 4), 0, stream>>>(
-        out, part_o, part_ml, lens, least, splits, to_base2);
+        out, part_o, part_ml, lens, least, whole, splits, to_base2);
 }
 
 }  // namespace

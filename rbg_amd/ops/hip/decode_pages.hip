@@ -17,6 +17,11 @@
 //    lengths fills the chip as a regular one does; longer ones only where the
 //    grid has too few for the sequence.  The grid is fixed when a step is
 //    captured; workgroups past the end of their sequence leave at once.
+//  * With a ticket per (sequence, key head), which the caller keeps and which is
+//    0 between launches, the last workgroup of a sequence adds up what its parts
+//    left: no launch of its own, which costs 1 to 3 us (1 sequence of 100 keys
+//    6.3 -> 4.8 us, 64 of up to 2048 68 -> 65).  (Read after a fence, which
+//    invalidates caches that others use, 128 of 2080 took 9 us more instead.)
 #include "decode_join.h"
 
 namespace {
@@ -38,6 +43,17 @@ DEV_INLINE bf16x8 dp_frag(dp_u4 u) {
   return c.v;
 }
 
+DEV_INLINE void dp_share(float* to, float x) {
+  __hip_atomic_store(to, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+DEV_INLINE f32x2 dp_shared(const float* from) {
+  union { unsigned long long u; f32x2 v; } x;
+  x.u = __hip_atomic_load((const unsigned long long*)from, __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_AGENT);
+  return x.v;
+}
+
 // TOGETHER: all key heads of a (sequence, part) run on one XCD, workgroup i on
 // XCD i % 8, which then translates an eighth of the pool's addresses (128
 // sequences of 2080 tokens, 8 heads: 198 -> 179 us, 6.1 TB/s).  A small batch
@@ -54,7 +70,8 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     const int* __restrict__ lens,           // [seqs]
     const float scale,                      // to the base of 2
     const int kv_heads, const int max_pages, const int least,
-    const int q_stride) {
+    const int whole, const int q_stride,
+    int* __restrict__ tickets) {            // [seqs, KVH], or null
   int kvh = blockIdx.x, seq = blockIdx.y, split = blockIdx.z;
   if (TOGETHER) {
     const int lin = kvh + kv_heads * (seq + gridDim.y * split);
@@ -67,7 +84,7 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     split = pair / gridDim.y;
   }
   const int ctx = lens[seq];
-  const int span = part_keys(ctx, least, gridDim.z);
+  const int span = part_keys(ctx, least, whole, gridDim.z);
   const int begin = split * span, end = min(ctx, begin + span);
   if (begin >= ctx && split > 0) return;
   const int lane = threadIdx.x & 63;
@@ -77,7 +94,8 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
 
   __shared__ __align__(16) __hip_bfloat16 v_lds[WAVES][8 * VROW];
   __shared__ float sums[WAVES][QPG][2];
-  static_assert(sizeof(v_lds) >= WAVES * QPG * DIM * 4, "merge fits");
+  static_assert(sizeof(v_lds) >= WAVES * QPG * DIM * 4 &&
+                    sizeof(v_lds) >= 64 * WAVES * 6 * 4, "merges fit");
 
   // the heads' queries as columns (QPG of 16), 4 pieces of 32 dims
   bf16x8 qf[4];
@@ -251,13 +269,97 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
       out[row * DIM + d] = f2bf(total == 0.f ? 0.f : o / total);
     } else {
       const size_t at_row = (size_t)split * gridDim.y * heads + row;
-      part_o[at_row * DIM + d] = o;
+      // past the L2, which other XCDs' workgroups do not see
+      dp_share(&part_o[at_row * DIM + d], o);
       if (d == 0) {
-        part_ml[at_row * 2] = top;
-        part_ml[at_row * 2 + 1] = total;
+        dp_share(&part_ml[at_row * 2], top);
+        dp_share(&part_ml[at_row * 2 + 1], total);
       }
     }
   }
+  if (!tickets || ctx <= span) return;
+
+  // every thread's sums are there before the ticket is
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __shared__ int taken;
+  __syncthreads();
+  const int parts = min((ctx + span - 1) / span, (int)gridDim.z);
+  if (threadIdx.x == 0) {
+    int* ticket = tickets + (size_t)seq * kv_heads + kvh;
+    taken = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+    if (taken == parts - 1)
+      __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (taken != parts - 1) return;
+  // four dims a thread, the parts in shares that meet in LDS; rounds of 8
+  // independent loads
+  constexpr int PIECES = QPG * DIM / 4, SHARES = 64 * WAVES / PIECES;
+  const int piece = threadIdx.x % PIECES, share = threadIdx.x / PIECES;
+  const int h = piece / (DIM / 4), d = piece % (DIM / 4) * 4;
+  const size_t row = (size_t)seq * heads + kvh * QPG + h;
+  const size_t step = (size_t)gridDim.y * heads;
+  float top = LOW, total = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int first = share; first < parts; first += 8 * SHARES) {
+    float ms[8], ls[8];
+    f32x4 os[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      // past the end: the last part again, without weight
+      const size_t from = min(first + i * SHARES, parts - 1) * step + row;
+      const f32x2 ml = dp_shared(part_ml + from * 2);
+      const f32x2 lo = dp_shared(part_o + from * DIM + d);
+      const f32x2 hi = dp_shared(part_o + from * DIM + d + 2);
+      ms[i] = ml[0];
+      ls[i] = ml[1];
+      os[i] = f32x4{lo[0], lo[1], hi[0], hi[1]};
+    }
+    float most = top;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) most = fmaxf(most, ms[i]);
+    const float fade = __builtin_amdgcn_exp2f(top - most);
+    top = most;
+    o *= fade;
+    total *= fade;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (first + i * SHARES < parts) {
+        const float f = __builtin_amdgcn_exp2f(ms[i] - top);
+        o += os[i] * f;
+        total += ls[i] * f;
+      }
+  }
+  if (SHARES > 1) {
+    // `meet` was read before the barriers above; [share][piece][o, top, total]
+    float* mine = meet + (share * PIECES + piece) * 6;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mine[j] = o[j];
+    mine[4] = top;
+    mine[5] = total;
+    __syncthreads();
+    if (share) return;
+    float most = LOW;
+#pragma unroll
+    for (int k = 0; k < SHARES; ++k)
+      most = fmaxf(most, meet[(k * PIECES + piece) * 6 + 4]);
+    o = f32x4{0.f, 0.f, 0.f, 0.f};
+    total = 0.f;
+#pragma unroll
+    for (int k = 0; k < SHARES; ++k) {
+      const float* theirs = meet + (k * PIECES + piece) * 6;
+      const float f = __builtin_amdgcn_exp2f(theirs[4] - most);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] += theirs[j] * f;
+      total += theirs[5] * f;
+    }
+  }
+  union { __hip_bfloat16 e[4]; uint2 u; } b;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) b.e[j] = f2bf(total == 0.f ? 0.f : o[j] / total);
+  *reinterpret_cast<uint2*>(out + row * DIM + d) = b.u;
 }
 
 }  // namespace
@@ -266,16 +368,22 @@ extern "C" void launch_decode_pages(
     void* out, void* part_o, void* part_ml, const void* q, const void* keys,
     const void* values, const void* tables, const void* lens, float scale,
     int seqs, int heads, int kv_heads, int max_pages, int splits, int span,
-    int q_stride, hipStream_t stream) {
+    int q_stride, void* tickets, hipStream_t stream) {
   // in whole rounds of the waves
   span = max(1, (span + PART_ROUND - 1) / PART_ROUND) * PART_ROUND;
+  // Where pairs of sequence and key head fill the chip three times, no part of a
+  // few keys beside one of many (128 sequences of 2080 and 8 heads 181 -> 171 us,
+  // 96 of up to 2500 106 -> 101; 64 of up to 4000 143 -> 146, so not for fewer).
+  const int whole = seqs * kv_heads >= 768 ? span + span / 4 : span;
   const dim3 grid(kv_heads, seqs, splits), block(64 * WAVES);
 #define DP_LAUNCH(QPG, TOGETHER)                                           \
   decode_pages_kernel<QPG, TOGETHER><<<grid, block, 0, stream>>>(          \
       (float*)part_o, (float*)part_ml, (__hip_bfloat16*)out,               \
       (const __hip_bfloat16*)q, (const __hip_bfloat16*)keys,               \
       (const __hip_bfloat16*)values, (const int*)tables, (const int*)lens, \
-      scale * 1.44269504088896f, kv_heads, max_pages, span, q_stride)
+      scale * 1.44269504088896f, kv_heads, max_pages, span, whole,        \
+      q_stride,                                                            \
+      (int*)tickets)
 #define DP_GO(QPG)                                                         \
   do {                                                                     \
     if (seqs >= 96) DP_LAUNCH(QPG, true);                                  \
@@ -290,8 +398,9 @@ extern "C" void launch_decode_pages(
   }
 #undef DP_LAUNCH
 #undef DP_GO
+  if (tickets) return;
   // sums to the base of 2
   launch_decode_join((__hip_bfloat16*)out, (const float*)part_o,
-                     (const float*)part_ml, (const int*)lens, span, splits,
-                     heads, seqs, 1.f, stream);
+                     (const float*)part_ml, (const int*)lens, span, whole,
+                     splits, heads, seqs, 1.f, stream);
 }

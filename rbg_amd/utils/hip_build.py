@@ -34,6 +34,7 @@ HIP_SOURCES = {
         "attn_prefill.hip",
         "prefill_flash.hip",
         "mfma_probe.hip",
+        "place_inputs.hip",
         "rmsnorm.hip",
         "rope_kv.hip",
         "silu_mul.hip",

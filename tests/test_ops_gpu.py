@@ -650,6 +650,69 @@ def test_prefill_flash(heads, kvh, news, pasts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("group", [1, 2, 4, 8])
+@pytest.mark.parametrize("lens,splits", [
+    ([1, 256, 257, 0, 513, 5000], 32), ([16000], 32), ([300], 2),
+    ([2080] * 100, 4), ([2049, 2560, 2561, 2048] * 100, 4)])
+def test_decode_attention_tickets(group, lens, splits):
+    """Parts added up by a sequence's last workgroup as by a launch of its own:
+    one part, two, more than a round of loads, longer ones than the least, and a
+    longer single one where there are many; again and again with the same tickets,
+    and replayed.  The same f32 sums in another order: a rounding of the result
+    apart, 2^-8 of it, or of the values' size where they cancel."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(group + len(lens))
+    kvh, width = 2, (max(lens) + 15) // 16
+    n = len(lens)
+    q = torch.randn(n, kvh * group, 128, device=dev,
+                    generator=gen).bfloat16()
+    k, v = torch.randn(2, 1200, kvh, 16, 128, device=dev,
+                       generator=gen).bfloat16()
+    tables = torch.randint(0, 1200, (n, width), device=dev, generator=gen,
+                           dtype=torch.int32)
+    lens = torch.tensor(lens, dtype=torch.int32, device=dev)
+    tickets = torch.zeros(n * kvh, dtype=torch.int32, device=dev)
+
+    def run(t):
+        return ops.decode_attention(q, k, v, tables, lens, 0.2,
+                                    num_splits=splits, variant=7, tickets=t)
+    want = run(None).float()
+    bound = want.abs() * 2 ** -7 + 2 ** -9
+    for _ in range(3):
+        got = run(tickets)
+        assert ((got.float() - want).abs() <= bound).all()
+        assert not tickets.any()
+    g = torch.cuda.CUDAGraph()
+    with torch.inference_mode(), torch.cuda.graph(g):
+        out = run(tickets)
+    for _ in range(3):
+        with torch.inference_mode():
+            out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, got) and not tickets.any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,width,seqs,used", [
+    (1, 512, 1, 1), (4, 7, 3, 7), (128, 1024, 97, 131), (2, 512, 1, 512)])
+def test_place_inputs(rows, width, seqs, used):
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    fields = torch.randint(0, 1 << 40, (4 * rows,), device=dev)
+    tables = torch.randint(1, 1 << 30, (seqs, used), device=dev,
+                           dtype=torch.int32)
+    to_fields = torch.full_like(fields, -1)
+    to_tables = torch.full((rows, width), -1, device=dev, dtype=torch.int32)
+    ops.place_inputs(to_fields, to_tables, fields, tables)
+    assert torch.equal(to_fields, fields)
+    assert torch.equal(to_tables[:seqs, :used], tables)
+    to_tables[:seqs, :used] = 0
+    assert not to_tables.any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,n,k", [
     (1, 32, 4096), (4, 2048, 4096), (3, 1024, 14336), (2, 2048, 5632),
     (1, 5120, 8192), (1, 6144, 8704), (1, 4128, 14336), (5, 2048, 2048),
