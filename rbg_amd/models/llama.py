@@ -21,6 +21,7 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from .. import ops
 from ..engine.batch import ForwardBatch
@@ -269,10 +270,33 @@ class LlamaLayer(nn.Module):
                 cos_sin: torch.Tensor):
         if residual is None:
             x, residual = None, x       # nothing to add yet
+        if batch.routes is not None:
+            out = self.issue(x, residual, batch, kv, cos_sin)
+            if out:
+                return out
         h, residual = self.attn(x, residual, self.input_norm, batch, kv,
                                 cos_sin)
         h, residual = self.mlp(h, residual, self.post_norm, self.eps)
         return h, residual
+
+
+    def issue(self, x: Optional[torch.Tensor], residual: torch.Tensor,
+              batch: ForwardBatch, kv: PagedKVCache, cos_sin: torch.Tensor):
+        """forward of a prompt's rows in one native call; None where parts of
+        the layer are hooked, whose calls would be missed."""
+        attn, mlp = self.attn, self.mlp
+        if (attn._forward_hooks or attn._forward_pre_hooks or
+                mlp._forward_hooks or mlp._forward_pre_hooks or
+                _has_any_global_hook()):
+            return None
+        plan = batch.prefill_plan(attn.heads, attn.kv_heads)
+        return ops.prompt_layer(
+            x, residual, self.input_norm, self.post_norm, self.eps, attn.wqkv,
+            attn.wo, mlp.w_gate_up, mlp.w_down, batch.routes, attn.heads,
+            attn.q_norm, attn.k_norm, kv.key_cache(attn.layer_idx),
+            kv.value_cache(attn.layer_idx), cos_sin, batch.positions,
+            batch.slot_mapping, attn.scale, plan.blocks, plan.lens, plan.items,
+            plan.joins, plan.parts, batch.kv_gather_slots)
 
 
 class LlamaForCausalLM(nn.Module):
@@ -368,11 +392,30 @@ class LlamaForCausalLM(nn.Module):
             assert hidden is not None, "non-first PP stage needs hidden"
             x = hidden.clone()      # the layers add to it in place
         residual = None
+        batch.routes = self.routes(x, batch, kv)
         for layer in self.layers:
             x, residual = layer(x, residual, batch, kv, self.cos_sin)
         if not self.pp.last:
             return x + residual
         return ops.add_rmsnorm(x, residual, self.final_norm, self.cfg.rms_eps)
+
+    def routes(self, x: torch.Tensor, batch: ForwardBatch, kv: PagedKVCache):
+        """Of a prompt whose layers one call each can issue.  Up to four rows
+        take norm and product in one launch, ranks exchange rows between
+        launches."""
+        page = kv.page_size
+        if (batch.mode != "prefill" or not x.is_cuda or x.shape[0] <= 4 or
+                self.tp.size > 1 or self.pp.size > 1 or
+                batch.cu_host is None or self.cfg.head_dim != 128 or
+                ops.PREFILL_SWZ < 16 or x.shape[1] % 8 or
+                (batch.kv_gather_slots is not None and page & (page - 1))):
+            return None
+        attn, mlp = self.layers[0].attn, self.layers[0].mlp
+        if attn.heads // attn.kv_heads > 128:
+            return None
+        return ops.prompt_routes(x.shape[0], tuple(
+            tuple(w.shape)
+            for w in (attn.wqkv, attn.wo, mlp.w_gate_up, mlp.w_down)))
 
     @torch.inference_mode()
     def logits(self, hidden: torch.Tensor,

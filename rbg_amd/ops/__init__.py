@@ -8,6 +8,7 @@ as the implementation.
 """
 from __future__ import annotations
 
+import functools
 import heapq
 import importlib
 from dataclasses import dataclass
@@ -289,6 +290,29 @@ def place_inputs(fields, tables, new_fields, new_tables) -> None:
     fields.copy_(new_fields)
     tables.zero_()
     tables[:n, :used].copy_(new_tables)
+
+
+@functools.lru_cache(maxsize=1024)
+def prompt_routes(rows: int, shapes: Tuple[Tuple[int, int], ...]
+                  ) -> Tuple[int, ...]:
+    """What linear_parts and linear_swiglu (the third) take for products of that
+    many rows and weights of ``shapes``, as numbers of bindings.cpp's Route."""
+    def parts(n, k):
+        if rows > 64 and _tile(rows, n, k):
+            return 2
+        return 1 if SKINNY_GEMM and _skinny(rows, n, k, True) else 0
+
+    def glu(n, k):
+        if rows > 64 and _tile_glu(rows, n, k):
+            return 4
+        return 3 if SKINNY_GEMM and _glu(rows, n, k) else parts(n, k)
+    return tuple((glu if i == 2 else parts)(n, k)
+                 for i, (n, k) in enumerate(shapes))
+
+
+def prompt_layer(*args):
+    """bindings.cpp prompt_layer; an empty list where it does not take the call."""
+    return _require_hip().prompt_layer(*args)
 
 
 def embed_rows(ids: torch.Tensor, table: torch.Tensor) -> torch.Tensor:

@@ -549,6 +549,76 @@ torch::Tensor prefill_flash(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   return out;
 }
 
+// Who takes a product of a prompt's rows (ops.prompt_routes).
+enum Route { BY_LIBRARY, BY_SKINNY, BY_TILE, GLU_BY_SKINNY, GLU_BY_TILE };
+
+static torch::Tensor routed(const torch::Tensor& x, const torch::Tensor& w,
+                            int64_t route) {
+  switch (route) {
+    case BY_SKINNY: return skinny_parts(x, w);
+    case BY_TILE: return tile_parts(x, w);
+    case GLU_BY_SKINNY: return skinny_swiglu(x, w);
+    case GLU_BY_TILE: return tile_swiglu(x, w);
+    default: return at::linear(x, w);
+  }
+}
+
+// ops.add_rmsnorm, or the norm of the residual alone
+static torch::Tensor prompt_norm(const c10::optional<torch::Tensor>& src,
+                                 const torch::Tensor& residual,
+                                 const torch::Tensor& weight, double eps) {
+  if (!src) return rmsnorm(residual, weight, eps);
+  if (src->scalar_type() == torch::kFloat32 ||
+      (src->size(0) <= 256 && src->size(-1) <= 16384))
+    return add_rmsnorm(*src, residual, weight, eps);
+  fused_add_rmsnorm(*src, residual, weight, eps);
+  return *src;
+}
+
+// A Llama layer on the rows of prompts: the launches of its parts' operations
+// (models/llama.py), issued by one call.  Short prompts waited for the host: 37
+// tokens of 2048 wide are 62 launches, whose kernels take 400 us and which took 576
+// to issue, 412 so.  routes: of wqkv, wo, w_gate_up and w_down.  Returns the layer's result for the next norm to add, and the
+// residual, which is changed in place; nothing, and does nothing, for weights
+// that only the library takes.
+std::vector<torch::Tensor> prompt_layer(
+    c10::optional<torch::Tensor> src, torch::Tensor residual,
+    torch::Tensor input_norm, torch::Tensor post_norm, double eps,
+    torch::Tensor wqkv, torch::Tensor wo, torch::Tensor w_gate_up,
+    torch::Tensor w_down, std::vector<int64_t> routes, int64_t heads,
+    c10::optional<torch::Tensor> q_norm, c10::optional<torch::Tensor> k_norm,
+    torch::Tensor key_cache, torch::Tensor value_cache, torch::Tensor cos_sin,
+    torch::Tensor positions, torch::Tensor slot_mapping, double scale,
+    torch::Tensor block_info, torch::Tensor seq_lens,
+    c10::optional<torch::Tensor> items, c10::optional<torch::Tensor> joins,
+    int64_t parts, c10::optional<torch::Tensor> gather_slots) {
+  TORCH_CHECK(routes.size() == 4, "a route per product");
+  for (const auto& w : {wqkv, wo, w_gate_up, w_down})
+    if (!w.is_cuda() || !w.is_contiguous() || w.dim() != 2 ||
+        w.scalar_type() != torch::kBFloat16 ||
+        (reinterpret_cast<uintptr_t>(w.data_ptr()) & 15))
+      return {};
+  const int64_t rows = residual.size(0), kvh = key_cache.size(1);
+  auto x = prompt_norm(src, residual, input_norm, eps);
+  auto qkv = rope_heads(routed(x, wqkv, routes[0]), heads, q_norm, k_norm, eps,
+                        key_cache, value_cache, cos_sin, positions,
+                        slot_mapping);
+  const auto part = [&](int64_t from, int64_t n) {
+    return qkv.narrow(1, from * 128, n * 128).view({rows, n, 128});
+  };
+  // behind a past: all rows, the new ones too, from the pages
+  auto o = prefill_flash(part(0, heads),
+                         gather_slots ? key_cache : part(heads, kvh),
+                         gather_slots ? value_cache : part(heads + kvh, kvh),
+                         block_info, seq_lens, scale, gather_slots, items,
+                         joins, parts);
+  x = routed(o.view({rows, heads * 128}), wo, routes[1]);
+  x = prompt_norm(x, residual, post_norm, eps);
+  x = routed(x, w_gate_up, routes[2]);
+  if (routes[2] != GLU_BY_SKINNY && routes[2] != GLU_BY_TILE) x = silu_mul(x);
+  return {routed(x, w_down, routes[3]), residual};
+}
+
 torch::Tensor mfma_probe(torch::Tensor a, torch::Tensor b, int64_t a_split,
                          int64_t b_split) {
   auto d = torch::zeros({16, 16}, a.options().dtype(torch::kFloat32));
@@ -722,6 +792,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("block_tables"), py::arg("context_lens"), py::arg("scale"),
         py::arg("num_splits"), py::arg("wide"), py::arg("span") = 128,
         py::arg("tickets") = c10::nullopt);
+  m.def("prompt_layer", &prompt_layer, "a Llama layer on rows of prompts");
   m.def("place_inputs", &place_inputs, "a decode step's inputs to their place");
   m.def("prefill_attention", &prefill_attention, "varlen causal flash prefill");
   m.def("prefill_flash", &prefill_flash, "causal attention of prompts",

@@ -228,3 +228,40 @@ def test_nothing_is_collected_in_a_capture(collects):
         gc.enable()
         del runner.model.logits
     assert seen == [False] and out.isfinite().all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("norms", [False, True])
+@pytest.mark.parametrize("rows", [5, 37, 65, 300, 1100])
+def test_layers_issued_by_one_call(norms, rows, monkeypatch):
+    """The same launches as of a layer's parts, so the same bits: prompts, and
+    portions behind a past; a hooked part is called."""
+    runner = ModelRunner(engine_config(norms, "cuda"))
+    spread_norms(runner.model)
+    gen = torch.Generator().manual_seed(rows)
+    seqs = []
+    for count in (rows - 2, 2):
+        seqs.append(Sequence(torch.randint(0, 512, (2 * count,),
+                                           generator=gen).tolist()))
+        seqs[-1].block_table = BlockTable(runner.cache)
+        seqs[-1].block_table.ensure(2 * count)
+    seen = []
+
+    def step(half):
+        chunks = []
+        for s in seqs:
+            n = len(s.prompt_tokens) // 2
+            chunks.append((s, half * n, s.prompt_tokens[half * n:][:n]))
+        return runner.feed(chunks, [[0, len(c[2]) - 1] for c in chunks])
+    got = [step(0), step(1), runner.cache.kv.clone()]
+    assert seen == []
+    hook = runner.model.layers[1].mlp.register_forward_hook(
+        lambda *a: seen.append(1))
+    again = step(0)
+    hook.remove()
+    assert seen and torch.equal(again, got[0])
+    monkeypatch.setattr(type(runner.model), "routes", lambda *a: None)
+    runner.cache.kv.zero_()
+    want = [step(0), step(1), runner.cache.kv]
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
