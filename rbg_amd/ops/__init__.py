@@ -230,13 +230,17 @@ def _glu(rows: int, n: int, k: int) -> bool:
     rows 26 / 57; not 38912 x 4096, a round and a small rest: 16 rows 76 / 72),
     32 rows to 16384 columns (14336 x 4096: 32 rows 27 / 29, 64 rows 42 / 30;
     not x 8192: 16 rows 60 / 48), and narrow ones of short k (7168 x 2048: 16
-    rows 13.1 / 15.4, x 4096 23.9 / 18.4; 11264 x 2048: 32 rows 14.1 / 17.5;
+    rows 13.1 / 15.4, x 4096 23.9 / 18.4; 11264 x 2048: 32 rows 14.1 / 17.5, 37
+    rows 16.8 / 18.5; 16384 x 2048, 64 rows 19.4 / 21.3; 4096 x 1024, 48 rows 8.6 /
+    9.8, but 8192 x 2048 15.6 / 14.5, 12288 x 3072 25.1 / 25.1;
     12288 x 4096: 16 rows 25.6 / 29.5, x 5120: 32 rows 33.6 / 29.7).  The form
     of a few rows splits k within a workgroup (7168 x 8192: 4 rows 25 / 27)."""
     if rows < 1 or n % 64 or k % 512:
         return False
     if rows <= 4 and k % 2048 == 0:
         return True
+    if 32 < rows <= 64 and n <= 16384:
+        return k <= 1024 or n >= 10240 and k <= 2048
     if n <= 12288:
         return (rows <= 2 and k <= 8192 or rows <= 32 and
                 (k <= (1536 if n <= 4096 else 2048) or

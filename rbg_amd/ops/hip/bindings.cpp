@@ -121,7 +121,7 @@ torch::Tensor skinny_swiglu(torch::Tensor a, torch::Tensor w) {
   auto c = torch::empty({M, N / 2}, a.options());
   // as pick_skinny, unsplit; the smaller workgroups where they fill the chip
   const int waves = pick_skinny((int)M, (int)N, (int)K).waves == 0 ? 0
-                    : M <= 32 && N <= 16384                        ? 4
+                    : M <= 64 && N <= 16384                        ? 4
                                                                    : 8;
   launch_skinny_gemm(c.data_ptr(), nullptr, a.data_ptr(), w.data_ptr(),
                      (int)M, (int)N, (int)K, waves, 1, 1, current_stream());

@@ -213,6 +213,8 @@ extern "C" void launch_skinny_gemm(void* c, void* ws, const void* a,
       launch_tiles<MT, NW, false>(cp, wsp, ap, wp, M, N, K, splits,        \
                                   stream);                                 \
   } while (0)
+#define SG_GLU(MT)                                                         \
+  launch_tiles<MT, 4, true>(cp, wsp, ap, wp, M, N, K, 1, stream)
   if (waves == 0) {             // the kernel of a few rows
     if (glu)
       launch_skinny_rows<ROWS_GLU, false>(cp, ap, wp, M, N, K, {}, {}, stream);
@@ -227,6 +229,8 @@ extern "C" void launch_skinny_gemm(void* c, void* ws, const void* a,
   else if (mt <= 2 && waves == 4) SG_GO(2, 4);
   else if (mt <= 1) SG_GO(1, 8);
   else if (mt <= 2) SG_GO(2, 8);
+  else if (mt <= 3 && waves == 4 && glu) SG_GLU(3);
+  else if (mt <= 4 && waves == 4 && glu) SG_GLU(4);
   else if (mt <= 3) SG_GO(3, 8);
   else if (mt <= 4) SG_GO(4, 8);
   else if (mt <= 6) SG_GO(6, 8);
@@ -236,6 +240,7 @@ extern "C" void launch_skinny_gemm(void* c, void* ws, const void* a,
   else
     launch_tiles<16, 8, false>(cp, wsp, ap, wp, M, N, K, splits, stream);
 #undef SG_GO
+#undef SG_GLU
 }
 
 extern "C" void launch_reduce_splits(void* c, const void* ws, int splits,

@@ -650,6 +650,32 @@ def test_prefill_flash(heads, kvh, news, pasts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [33, 48, 49, 64])
+@pytest.mark.parametrize("n,k", [(64, 512), (4160, 1024), (10240, 2048),
+                                 (16384, 1536)])
+def test_swiglu_of_small_workgroups(rows, n, k):
+    """silu within the decode GEMM of 33 to 64 rows, and gates as large as make
+    its exponential infinite or 0; an f32 sum of k products, silu and one
+    rounding."""
+    from rbg_amd import ops
+    assert ops._glu(rows, n, k)
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(rows + n)
+    x = torch.randn(rows, k, device=dev, generator=gen).bfloat16()
+    w = (torch.randn(n, k, device=dev, generator=gen) / k ** 0.5).bfloat16()
+    w[:8] *= 64
+    full = x.double() @ w.double().t().contiguous()
+    size = (x.double().abs() @ w.double().abs().t().contiguous()) * 2 ** -18
+    gate, up = full.chunk(2, 1)
+    want = torch.nn.functional.silu(gate) * up
+    # silu grows by at most 1.1 of what its argument does
+    bound = want.abs() * 2 ** -8 + 1.1 * size[:, :n // 2] * up.abs() + \
+        size[:, n // 2:] * gate.abs() + 1e-6
+    got = ops.linear_swiglu(x, w)
+    assert ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("group", [1, 2, 4, 8])
 @pytest.mark.parametrize("lens,splits", [
     ([1, 256, 257, 0, 513, 5000], 32), ([16000], 32), ([300], 2),
