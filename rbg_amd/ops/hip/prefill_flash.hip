@@ -13,19 +13,20 @@
 //  * S^T = K Q^T leaves a lane 16 keys of one query, and those weights are the
 //    operand of O^T = V^T P^T as they are, with keys 4h..4h+3, 8+4h.. of 16 in
 //    place of 8h..8h+7: probabilities never pass LDS, the softmax exchanges one
-//    value per 32 keys.  V is read transposed.
+//    value per 64 keys.  V is read transposed.
 //  * Scale and maximum are one fma per score, and sums are rescaled only when
 //    some row's maximum grows.  (Letting scores exceed it by 2^8 would be 1 to
 //    2% faster, but the largest weight, 1 here, would then be rounded too.)
 //  * Rows go straight to LDS, to places that no read or load meets a conflict
 //    at (through registers, with V's writes in conflict: 8192 tokens 600 us, so
 //    550), and between the products, pinned there, stand their operands' reads,
-//    several ahead, the next tile's loads and half of the exponentials (550 ->
-//    525, where a workgroup has its CU to itself 1.75 -> 1.2 us a tile).  A third
-//    workgroup on a CU, V in one stage, needs registers that spill (640).
+//    several ahead, the next tile's loads and three quarters of the exponentials
+//    (550 -> 520, where a workgroup has its CU to itself 1.75 -> 1.2 us a tile; half
+//    of the exponentials there 1 to 3% more).  A third workgroup on a CU, V in one
+//    stage, needs registers that spill (640).
 //  * Blocks are cut by keys where whole ones would leave CUs idle (ops
 //    _cut_prefill), whose sums a second launch adds up: 1500 tokens after 9000
-//    297 -> 261 us, 512 after 4000 88 -> 60, 40 after 9000 165 -> 28.
+//    297 -> 255 us, 512 after 4000 88 -> 60, 40 after 9000 165 -> 28.
 #include <type_traits>
 
 #include "mfma_util.h"
@@ -53,6 +54,16 @@ DEV_INLINE bf16x8 pf_frag(pf_u4 u) {
 DEV_INLINE float pf_add2(__bf16 a, __bf16 b, float sum) {
   const bf16x2 ab = {a, b}, ones = {(__bf16)1.f, (__bf16)1.f};
   return __builtin_amdgcn_fdot2_f32_bf16(ab, ones, sum, false);
+}
+
+// of a lane and the one 32 away
+DEV_INLINE float pf_other_half_max(float x) {
+  union { float f; unsigned u; } a, b;
+  a.f = x;
+  const auto both = __builtin_amdgcn_permlane32_swap(a.u, a.u, false, false);
+  a.u = both[0];
+  b.u = both[1];
+  return fmaxf(a.f, b.f);
 }
 
 // 16 bytes per lane from base + off, or from a lane's own address, to 16 * lane
@@ -238,7 +249,7 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
   named();
   // One tile's products.  Between them, one thing at a time and pinned there,
   // stand the reads of their operands ahead of them, the next tile's loads and
-  // half of the exponentials.
+  // three quarters of the exponentials.
   auto products = [&](auto masked, int t) {
     constexpr bool MASK = decltype(masked)::value;
     const int base = t * TILE, next = min(t + 1, tiles - 1);
@@ -293,7 +304,7 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) top = fmaxf(top, s[1][i]);
-    top = fmaxf(top, __shfl_xor(top, 32, 64)) * scale;
+    top = pf_other_half_max(top) * scale;
     if (__any(top > m)) {
       const float m_new = fmaxf(m, top);
       const float fade = __builtin_amdgcn_exp2f(m - m_new);
@@ -310,7 +321,7 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
           __builtin_fmaf(s[n >> 4][n & 15], scale, -m));
     };
 #pragma unroll
-    for (int n = 0; n < 16; ++n) weigh(n);
+    for (int n = 0; n < 8; ++n) weigh(n);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int n = 0; n < 16; ++n) {
@@ -318,15 +329,15 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
           vf[n % V_AHEAD], pf[n >> 2], acc[n & 3], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if (n + V_AHEAD < 16) vf[n % V_AHEAD] = v_read(n + V_AHEAD);
-      if (n < 8) {
-        weigh(16 + 2 * n);
-        weigh(17 + 2 * n);
+      if (n < 12) {
+        weigh(8 + 2 * n);
+        weigh(9 + 2 * n);
       } else {
         // the sum of the weights as they are used, rounded: an error that the
         // largest share with it cancels
-        const int e = (n - 8) >> 1, i = (n & 1) * 4;
-        l = pf_add2(pf[e][i], pf[e][i + 1], l);
-        l = pf_add2(pf[e][i + 2], pf[e][i + 3], l);
+#pragma unroll
+        for (int i = 0; i < 8; i += 2)
+          l = pf_add2(pf[n - 12][i], pf[n - 12][i + 1], l);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
