@@ -3,8 +3,9 @@
 MI355X-first structure: norms with the residual add, RoPE with the paged-KV
 write, prefill and decode attention, SiLU*up and the GEMMs of decode batches are
 the hand-written HIP kernels of rbg_amd.ops, fused with one another where a
-batch is small; the GEMMs of prompts go through hipBLASLt (ops.linear), with QKV
-and gate/up fused so that each layer runs 4 of them.
+batch is small; the GEMMs of prompts go through hand-written tiles or hipBLASLt,
+by the shape (ops.linear_parts, ops.linear_swiglu), with QKV and gate/up fused so
+that each layer runs 4 of them.
 
 Tensor parallelism is Megatron-style over RCCL/xGMI: QKV and gate_up are
 column-parallel (head-aligned shards), o_proj and down_proj row-parallel
