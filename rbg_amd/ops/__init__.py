@@ -187,8 +187,13 @@ def _tile(rows: int, n: int, k: int) -> bool:
     and picks a tile by the shape.  Against what is taken without it, with the
     norm that reads the sums (us): from 129 rows (4096 x 4096: 160 rows 25 / 17;
     4096 x 14336: 256 rows 62 / 44, 2048 rows 214 / 182; 5120 x 25600: 512 rows
-    270 / 128; 6144 x 4096: 1500 rows 76 / 60), before that only of long rows
-    (4096 x 14336: 128 rows 34 / 32; 5120 x 25600: 97 rows 71 / 61).  Not short k
+    270 / 128; 6144 x 4096: 1500 rows 76 / 60), from 97 rows
+    of matrices that give parts enough to do (6144 x 4096: 128 rows 26.3 / 24.0; 8192 x
+    8192: 45.2 / 42.1; 4096 x 8192: 29.0 / 27.1, x 4096 21.3 / 22.0; 3072 x 8192 26.3 /
+    23.7), from 65 rows of long rows (4096 x 14336: 128 rows 34 / 32; 5120 x 25600: 97
+    rows 71 / 61), of wide matrices (12288 x 8192: 80 rows 59.7 / 50.7; not of rows that
+    are no multiple of 4 KB apart: x 5120, 112 rows 41.8 / 46.3) and of 2048 columns (x
+    4096: 65 rows 15.2 / 13.7, x 6144 15.7 / 17.1).  Not short k
     (2048 x 2048: 256 rows 10 / 11), and from 257 rows to 999 only k from 5120 on
     (6144 x 4096: 512 rows 36 / 38), then not matrices with little to split
     (4096 x 4096: 1280 rows 56 / 60; 2048 x 5632: 1400 rows 42 / 45).  Above 4096
@@ -198,7 +203,14 @@ def _tile(rows: int, n: int, k: int) -> bool:
     if k < 3584 or k % 64 or n % 64 or not 2048 <= n <= 14336:
         return False
     if rows <= 128:
-        return rows > 64 and k >= 12288
+        if n >= 12288:
+            wide = k <= 4096 or k >= 6144
+        elif n < 3072:
+            wide = k <= 4096
+        else:
+            wide = rows > 96 and k >= (3584 if n >= 5120 else
+                                       5120 if n >= 4096 else 8192)
+        return rows > 64 and (k >= 12288 or wide)
     if rows < 1000:
         return rows <= 256 or k >= 5120
     return rows <= 4096 and (k >= 8192 or n >= 4096 and n * k > 2 ** 24)
@@ -252,6 +264,29 @@ def _glu(rows: int, n: int, k: int) -> bool:
             not (n <= 16384 and 6144 < k < 12288))
 
 
+def _tile_few(rows: int, n: int, k: int) -> bool:
+    """Does the GEMM of prompts take gate/up of 5 to 64 rows, in tiles of 64?  Its
+    ring of weights in LDS is deeper than the decode GEMM's registers, but a CU has
+    one tile at a time, so that it gains where there is about one for each.  Against
+    what is taken without it, over 16384 to 65536 columns, 2048, 4096, 5120 and 8192 k,
+    5 to 64 rows (us): to 20480 columns (18432 x 4096: 8 rows 39.6 / 31.3, 64 rows 43.1 /
+    36.6; 20480 x 8192: 16 rows 74.5 / 64.1), from there to 28672 for more rows (24576 x
+    4096: 48 rows 44.0 / 38.7, 16 rows 37.0 / 37.0; 28672 x 4096: 48 rows 45.4 / 43.1, 33
+    rows 43.0 / 43.0), and beyond 32768 with tiles of 256 (36864 x 2048: 5 rows 38.9 /
+    30.3; 45056 x 4096: 64 rows 93.7 / 70.3; 57344 x 8192: 16 rows 180 / 169, 64 rows 192 /
+    167; not 57344 x 4096, 8 rows 83.6 / 88.6).  Rows that are no multiple of 4 KB apart
+    the library reads better (40960 x 5120: 64 rows 95 / 101), but not where they are few
+    and it has few tiles (18432 x 5120: 16 rows 85 / 46, 32 rows 45 / 50)."""
+    if not 4 < rows <= 64 or k < 2048 or k > 8192 or n <= 16384:
+        return False
+    if k % 2048:
+        return rows <= 16 and k >= 4096 and n <= 32768
+    if n <= 32768:
+        return n <= 20480 or (n <= 28672 and
+                              rows > (32 if n <= 26624 else 40))
+    return n <= 53248 or (n <= 65536 and k == 8192)
+
+
 def _tile_glu(rows: int, n: int, k: int) -> bool:
     """Does it take a gate/up product, with silu?  Against the product and
     silu_mul, or the decode GEMM (us): from 129 rows (28672 x 4096: 256 rows 74 /
@@ -265,8 +300,10 @@ def _tile_glu(rows: int, n: int, k: int) -> bool:
     not 51200 x 5120, 128 rows 120 / 128, nor 14336 x 4096, 65 rows 34 / 37)."""
     if k < 1024 or k % 64 or n % 64 or n < 8192 or k > n:
         return False
+    if rows <= 64:
+        return _tile_few(rows, n, k)
     if rows <= 128:
-        return rows > 64 and 24576 <= n <= 32768
+        return 24576 <= n <= 32768
     if k >= 3584 and n <= (16384 if rows <= 256 else 12288) and rows < 1000:
         return False
     return rows <= 256 or rows > 384 or n <= 16384
@@ -274,7 +311,7 @@ def _tile_glu(rows: int, n: int, k: int) -> bool:
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T), w = [Wg; Wu]."""
-    if x.shape[0] > 64 and _takes_tile(x, w, _tile_glu):
+    if x.shape[0] > 4 and _takes_tile(x, w, _tile_glu):
         return _require_hip().tile_swiglu(x.contiguous(), w)
     if (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
             x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and
@@ -307,7 +344,7 @@ def prompt_routes(rows: int, shapes: Tuple[Tuple[int, int], ...]
         return 1 if SKINNY_GEMM and _skinny(rows, n, k, True) else 0
 
     def glu(n, k):
-        if rows > 64 and _tile_glu(rows, n, k):
+        if _tile_glu(rows, n, k):
             return 4
         return 3 if SKINNY_GEMM and _glu(rows, n, k) else parts(n, k)
     return tuple((glu if i == 2 else parts)(n, k)

@@ -34,6 +34,14 @@ constexpr TileForm TILE_FORMS[] = {
     {4, 4, 4, true, 7.58f, -3.47f, 0.378f, 0.187f, 0.298f},
 };
 
+// Of gate/up of up to 64 rows, which ops._tile_few names: rings of W 6 and 4 stages
+// deep.  Tiles of 128 rows of W while the chip has a CU for each, then of 256 (us,
+// 64 rows, 128 / 256: 28672 x 4096 43.6 / 57.7, 40960 x 4096 78 / 68).
+constexpr TileForm TILE_FEW[] = {
+    {2, 4, 6, true, 0.f, 0.f, 0.f, 0.f, 0.f},
+    {2, 8, 4, true, 0.f, 0.f, 0.f, 0.f, 0.f},
+};
+
 struct TilePlan {
   float time;                   // us
   const TileForm* form;
@@ -141,8 +149,12 @@ inline void launch_tile_plan(const TilePlan& p, void* out, const torch::Tensor& 
 inline torch::Tensor tile_swiglu(torch::Tensor a, torch::Tensor w) {
   check_tile(a, w);
   auto c = torch::empty({a.size(0), w.size(0) / 2}, a.options());
-  launch_tile_plan(pick_tile(a.size(0), w.size(0), a.size(1), TILE_GLU),
-                   c.data_ptr(), a, w, TILE_GLU);
+  const TileForm* few = TILE_FEW + (w.size(0) > 32768);
+  const bool takes = a.size(0) <= 64 && a.size(1) / 64 >= few->fill;
+  launch_tile_plan(
+      takes ? TilePlan{0.f, few, 1, nullptr, (int)(w.size(0) / 2)}
+            : pick_tile(a.size(0), w.size(0), a.size(1), TILE_GLU),
+      c.data_ptr(), a, w, TILE_GLU);
   return c;
 }
 
@@ -159,8 +171,8 @@ inline torch::Tensor tile_parts(torch::Tensor a, torch::Tensor w) {
   return c;
 }
 
-// One form of the above, for tests: its number, the parts, and for a second form
-// the column that it begins at.
+// One form of the above, for tests: its number (TILE_FEW's after the others), the
+// parts, and for a second form the column that it begins at.
 inline torch::Tensor tile_form(torch::Tensor a, torch::Tensor w, int64_t end,
                                int64_t form, int64_t parts, int64_t rest,
                                int64_t to) {
@@ -168,15 +180,18 @@ inline torch::Tensor tile_form(torch::Tensor a, torch::Tensor w, int64_t end,
   const int64_t M = a.size(0), N = w.size(0), K = a.size(1);
   const int64_t cols = end == TILE_GLU ? N / 2 : N;
   const int64_t forms = sizeof(TILE_FORMS) / sizeof(TILE_FORMS[0]);
-  TORCH_CHECK(end >= 0 && end <= TILE_GLU && form >= 0 && form < forms &&
+  const int64_t few = sizeof(TILE_FEW) / sizeof(TILE_FEW[0]);
+  TORCH_CHECK(form >= 0 && form < forms + few, "form");
+  const TileForm* f = form < forms ? TILE_FORMS + form : TILE_FEW + form - forms;
+  TORCH_CHECK(end >= 0 && end <= TILE_GLU &&
               rest < forms && parts >= 1 && (parts == 1 || end == TILE_PARTS) &&
-              K / 64 / parts >= TILE_FORMS[form].fill &&
+              K / 64 / parts >= f->fill &&
               (rest < 0 || (to > 0 && to < cols && to % 32 == 0 &&
                             K / 64 / parts >= TILE_FORMS[rest].fill)), "form");
   auto c = end == TILE_PARTS
                ? torch::empty({parts, M, N}, a.options().dtype(torch::kFloat32))
                : torch::empty({M, cols}, a.options());
-  launch_tile_plan({0.f, TILE_FORMS + form, (int)parts,
+  launch_tile_plan({0.f, f, (int)parts,
                     rest < 0 ? nullptr : TILE_FORMS + rest,
                     (int)(rest < 0 ? cols : to)},
                    c.data_ptr(), a, w, (int)end);

@@ -2,7 +2,8 @@
 import pytest
 import torch
 
-FORMS = [(8, 8), (6, 8), (8, 6), (6, 6), (8, 4), (4, 4)]
+FORMS = [(8, 8), (6, 8), (8, 6), (6, 6), (8, 4), (4, 4), (2, 4), (2, 8)]
+STAGES = [2, 2, 2, 3, 3, 4, 6, 4]       # the fewest of a part
 PLAIN, PARTS, GLU = 0, 1, 2
 
 
@@ -43,10 +44,10 @@ def test_forms(form, m, n, k):
     x, w, full, sums = _operands(m, n, k)
     wm, wn = FORMS[form]
     for end in (PLAIN, PARTS, GLU):
-        if end == GLU and wn % 4:
+        if (end == GLU and wn % 4) or k // 64 < STAGES[form]:
             continue
         for parts in (1, 2, 3) if end == PARTS else (1,):
-            if k // 64 // parts < 4:
+            if k // 64 // parts < max(4, STAGES[form]):
                 continue
             got = ops._hip.tile_form(x, w, end, form, parts, -1, 0)
             assert _near(got, end, full, sums), (end, parts)
@@ -67,8 +68,9 @@ def test_many_tiles_a_workgroup():
     """More tiles than workgroups, of a few stages each: loads run several
     tiles ahead."""
     from rbg_amd import ops
-    x, w, full, sums = _operands(2100, 9280, 256)
+    operands = {k: _operands(2100, 9280, k) for k in (256, 384)}
     for form in range(len(FORMS)):
+        x, w, full, sums = operands[384 if STAGES[form] > 4 else 256]
         for end in (PLAIN, GLU):
             if end == GLU and FORMS[form][1] % 4:
                 continue
@@ -79,6 +81,7 @@ def test_many_tiles_a_workgroup():
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [
     (65, 2048, 12288), (128, 4096, 12288), (129, 2048, 3584),
+    (65, 2048, 4096), (97, 5120, 3584), (128, 3072, 8192), (70, 12288, 4096),
     (256, 6144, 4096), (257, 2048, 5120), (999, 3136, 5120),
     (1000, 6144, 4096), (1500, 14336, 3584), (2048, 4096, 8192)])
 def test_parts_route(m, n, k):
@@ -94,6 +97,8 @@ def test_parts_route(m, n, k):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [
+    (5, 16448, 2048), (33, 26624, 2048), (41, 28672, 2048), (64, 32832, 2048),
+    (16, 18432, 4160), (63, 36864, 4096),
     (65, 24576, 1024), (128, 28672, 1088), (129, 8192, 2048),
     (256, 18432, 2048), (385, 28672, 1024), (1000, 11264, 2048),
     (2048, 28672, 1024)])
@@ -130,7 +135,8 @@ def test_rules_hand_over_what_it_takes():
                          4097, 8192):
                 for i, rule in enumerate((_tile, _tile_glu)):
                     if rule(rows, n, k):
-                        assert rows > 64 and n % 64 == 0 and k % 64 == 0
+                        assert rows > (64, 4)[i]
+                        assert n % 64 == 0 and k % 64 == 0
                         assert k >= 256
                         taken[i] += 1
     assert min(taken) > 50
