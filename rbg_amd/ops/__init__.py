@@ -180,6 +180,13 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return linear(x, w).float()
 
 
+def _tile_fits(rows: int, n: int, k: int) -> bool:
+    """Sizes that the GEMM of prompts has numbers for: offsets within W's halves of
+    32 bits, 2^24 tiles (hip/tile_bindings.h check_tile refuses others)."""
+    return ((n // 2 + 256) * k < 2 ** 31 and rows < 2 ** 24 and
+            -(-rows // 128) * -(-n // 128) < 2 ** 24)
+
+
 def _tile(rows: int, n: int, k: int) -> bool:
     """Does the GEMM of prompts (hip/tile_gemm.hip) take a [rows, k] x [n, k]
     product whose reader adds up parts, rather than the decode GEMM or
@@ -200,7 +207,8 @@ def _tile(rows: int, n: int, k: int) -> bool:
     rows the library's tiles are as full (8192 rows: 6144 x 4096 276 / 293, 4096 x
     14336 615 / 644), and wide matrices give it enough of them (16384 x 4096: 2048
     rows 243 / 256)."""
-    if k < 3584 or k % 64 or n % 64 or not 2048 <= n <= 14336:
+    if (k < 3584 or k % 64 or n % 64 or not 2048 <= n <= 14336 or
+            not _tile_fits(rows, n, k)):
         return False
     if rows <= 128:
         if n >= 12288:
@@ -298,7 +306,8 @@ def _tile_glu(rows: int, n: int, k: int) -> bool:
     5120: 199 / 217; 14336 x 4096: 53 / 53).  From 65 rows where tiles of 128 x 128
     nearly fill the chip once (28672 x 4096: 65 rows 56 / 45, 128 rows 58 / 51;
     not 51200 x 5120, 128 rows 120 / 128, nor 14336 x 4096, 65 rows 34 / 37)."""
-    if k < 1024 or k % 64 or n % 64 or n < 8192 or k > n:
+    if (k < 1024 or k % 64 or n % 64 or n < 8192 or k > n or
+            not _tile_fits(rows, n, k)):
         return False
     if rows <= 64:
         return _tile_few(rows, n, k)

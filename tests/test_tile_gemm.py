@@ -140,3 +140,19 @@ def test_rules_hand_over_what_it_takes():
                         assert k >= 256
                         taken[i] += 1
     assert min(taken) > 50
+
+
+@pytest.mark.parametrize("rows,n,k,fewer", [
+    (130, 65536, 65536, (130, 65536, 65024)),
+    (129, 131072, 32768, (129, 131072, 32512)),
+    (200, 14336, 289280, (200, 14336, 289216)),
+    (4096, 2048, 1677824, (4096, 2048, 1677696)),
+    (2 ** 24, 8192, 1024, (2 ** 24 - 1, 8192, 1024)),
+    (2 ** 24 - 1, 16384, 1024, (2 ** 23, 16384, 1024))])
+def test_rules_leave_what_it_refuses(rows, n, k, fewer):
+    """Beyond its 32-bit offsets and numbers of tiles a product stays with the
+    library, on both ways to it; a little below it is taken."""
+    from rbg_amd import ops
+    assert not ops._tile(rows, n, k) and not ops._tile_glu(rows, n, k)
+    assert not {2, 4} & set(ops.prompt_routes(rows, ((n, k),) * 4))
+    assert ops._tile(*fewer) or ops._tile_glu(*fewer)
