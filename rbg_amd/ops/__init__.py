@@ -95,6 +95,7 @@ def _on_gpu(t: torch.Tensor) -> bool:
     return t.is_cuda
 
 
+# 0: products go to hipBLASLt, not to the hand-written GEMMs
 SKINNY_GEMM = int(__import__("os").environ.get("RBG_SKINNY_GEMM", "1"))
 
 
@@ -225,7 +226,7 @@ def _tile(rows: int, n: int, k: int) -> bool:
 
 
 def _takes_tile(x: torch.Tensor, w: torch.Tensor, rule) -> bool:
-    return (_on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
+    return (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
             x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and
             x.shape[1] == w.shape[1] and
             rule(x.shape[0], w.shape[0], x.shape[1]) and _plain(x, w))
@@ -343,21 +344,26 @@ def place_inputs(fields, tables, new_fields, new_tables) -> None:
 
 
 @functools.lru_cache(maxsize=1024)
-def prompt_routes(rows: int, shapes: Tuple[Tuple[int, int], ...]
-                  ) -> Tuple[int, ...]:
-    """What linear_parts and linear_swiglu (the third) take for products of that
-    many rows and weights of ``shapes``, as numbers of bindings.cpp's Route."""
+def _own_routes(rows: int, shapes: Tuple[Tuple[int, int], ...]
+                ) -> Tuple[int, ...]:
     def parts(n, k):
         if rows > 64 and _tile(rows, n, k):
             return 2
-        return 1 if SKINNY_GEMM and _skinny(rows, n, k, True) else 0
+        return 1 if _skinny(rows, n, k, True) else 0
 
     def glu(n, k):
         if _tile_glu(rows, n, k):
             return 4
-        return 3 if SKINNY_GEMM and _glu(rows, n, k) else parts(n, k)
+        return 3 if _glu(rows, n, k) else parts(n, k)
     return tuple((glu if i == 2 else parts)(n, k)
                  for i, (n, k) in enumerate(shapes))
+
+
+def prompt_routes(rows: int, shapes: Tuple[Tuple[int, int], ...]
+                  ) -> Tuple[int, ...]:
+    """What linear_parts and linear_swiglu (the third) take for products of that
+    many rows and weights of ``shapes``, as numbers of bindings.cpp's Route."""
+    return _own_routes(rows, shapes) if SKINNY_GEMM else (0,) * len(shapes)
 
 
 def prompt_layer(*args):

@@ -156,3 +156,24 @@ def test_rules_leave_what_it_refuses(rows, n, k, fewer):
     assert not ops._tile(rows, n, k) and not ops._tile_glu(rows, n, k)
     assert not {2, 4} & set(ops.prompt_routes(rows, ((n, k),) * 4))
     assert ops._tile(*fewer) or ops._tile_glu(*fewer)
+
+
+def test_switched_off_everything_is_the_librarys(monkeypatch):
+    """Also after the same sizes were asked for with the switch on."""
+    from rbg_amd import ops
+
+    class Rows(torch.Tensor):
+        is_cuda = True
+    for rows, n, k in ((300, 16384, 2048), (2048, 4096, 14336), (64, 4096, 4096)):
+        x, w = (torch.zeros(1, dtype=torch.bfloat16).expand(m, k)
+                .as_subclass(Rows) for m in (rows, n))
+        monkeypatch.setattr(ops, "_plain", lambda *a: True)
+        monkeypatch.setattr(ops, "SKINNY_GEMM", 1)
+        rules = ops._tile, ops._tile_glu
+        assert any(ops._takes_tile(x, w, r) for r in rules) or \
+            ops._takes_skinny(x, w, parts=True)
+        assert any(ops.prompt_routes(rows, ((n, k),) * 4))
+        monkeypatch.setattr(ops, "SKINNY_GEMM", 0)
+        assert not any(ops._takes_tile(x, w, r) for r in rules)
+        assert not ops._takes_skinny(x, w, parts=True)
+        assert not any(ops.prompt_routes(rows, ((n, k),) * 4))
