@@ -43,9 +43,6 @@ class ForwardBatch:
     # cu_seqlens and cu_seqlens_k (None: the same) on the host
     cu_host: Optional[List[int]] = None
     cu_k_host: Optional[List[int]] = None
-    # who takes the products of a prompt's rows, where its layers are issued by
-    # one call each (ops.prompt_routes)
-    routes: Optional[tuple] = None
     _plans: Dict = field(default_factory=dict)
 
     def prefill_plan(self, heads: int, kv_heads: int):

@@ -22,7 +22,6 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-from torch.nn.modules.module import _has_any_global_hook
 
 from .. import ops
 from ..engine.batch import ForwardBatch
@@ -181,6 +180,17 @@ class LlamaAttention(nn.Module):
         T = residual.shape[0]
         key_cache = kv.key_cache(self.layer_idx)
         value_cache = kv.value_cache(self.layer_idx)
+        plan = None
+        if batch.mode == "prefill" and residual.is_cuda:
+            plan = batch.prefill_plan(self.heads, self.kv_heads)
+            if self.parts:
+                out = ops.prompt_attention_block(
+                    x, residual, norm, self.cfg.rms_eps, self.wqkv, self.wo,
+                    self.heads, self.q_norm, self.k_norm, key_cache,
+                    value_cache, cos_sin, batch.positions, batch.slot_mapping,
+                    self.scale, plan, batch.kv_gather_slots)
+                if out is not None:
+                    return out, residual
         # (Qwen: per-head norms,) RoPE and the paged KV write in one kernel,
         # which also adds up what a split GEMM left
         qkv, residual = ops.norm_heads(
@@ -194,9 +204,6 @@ class LlamaAttention(nn.Module):
         v = qkv[:, self.q_out + self.kv_out:]
         q3 = q.view(T, self.heads, self.head_dim)
         if batch.mode == "prefill":
-            plan = None
-            if q3.is_cuda:
-                plan = batch.prefill_plan(self.heads, self.kv_heads)
             if batch.kv_gather_slots is not None:
                 # behind a past: all rows, the new ones too, from the pages
                 o = ops.prefill_attention(
@@ -243,6 +250,11 @@ class LlamaMLP(nn.Module):
     def forward(self, x: torch.Tensor, residual: torch.Tensor,
                 norm: torch.Tensor, eps: float):
         """Of the norm of residual + x; and that sum."""
+        if self.parts:
+            out = ops.swiglu_block(x, residual, norm, eps, self.w_gate_up,
+                                   self.w_down)
+            if out is not None:
+                return out, residual
         h, residual = ops.norm_swiglu(x, residual, norm, eps, self.w_gate_up)
         if self.parts:
             return ops.linear_parts(h, self.w_down), residual
@@ -271,33 +283,10 @@ class LlamaLayer(nn.Module):
                 cos_sin: torch.Tensor):
         if residual is None:
             x, residual = None, x       # nothing to add yet
-        if batch.routes is not None:
-            out = self.issue(x, residual, batch, kv, cos_sin)
-            if out:
-                return out
         h, residual = self.attn(x, residual, self.input_norm, batch, kv,
                                 cos_sin)
         h, residual = self.mlp(h, residual, self.post_norm, self.eps)
         return h, residual
-
-
-    def issue(self, x: Optional[torch.Tensor], residual: torch.Tensor,
-              batch: ForwardBatch, kv: PagedKVCache, cos_sin: torch.Tensor):
-        """forward of a prompt's rows in one native call; None where parts of
-        the layer are hooked, whose calls would be missed."""
-        attn, mlp = self.attn, self.mlp
-        if (attn._forward_hooks or attn._forward_pre_hooks or
-                mlp._forward_hooks or mlp._forward_pre_hooks or
-                _has_any_global_hook()):
-            return None
-        plan = batch.prefill_plan(attn.heads, attn.kv_heads)
-        return ops.prompt_layer(
-            x, residual, self.input_norm, self.post_norm, self.eps, attn.wqkv,
-            attn.wo, mlp.w_gate_up, mlp.w_down, batch.routes, attn.heads,
-            attn.q_norm, attn.k_norm, kv.key_cache(attn.layer_idx),
-            kv.value_cache(attn.layer_idx), cos_sin, batch.positions,
-            batch.slot_mapping, attn.scale, plan.blocks, plan.lens, plan.items,
-            plan.joins, plan.parts, batch.kv_gather_slots)
 
 
 class LlamaForCausalLM(nn.Module):
@@ -393,30 +382,11 @@ class LlamaForCausalLM(nn.Module):
             assert hidden is not None, "non-first PP stage needs hidden"
             x = hidden.clone()      # the layers add to it in place
         residual = None
-        batch.routes = self.routes(x, batch, kv)
         for layer in self.layers:
             x, residual = layer(x, residual, batch, kv, self.cos_sin)
         if not self.pp.last:
             return x + residual
         return ops.add_rmsnorm(x, residual, self.final_norm, self.cfg.rms_eps)
-
-    def routes(self, x: torch.Tensor, batch: ForwardBatch, kv: PagedKVCache):
-        """Of a prompt whose layers one call each can issue.  Up to four rows
-        take norm and product in one launch, ranks exchange rows between
-        launches."""
-        page = kv.page_size
-        if (batch.mode != "prefill" or not x.is_cuda or x.shape[0] <= 4 or
-                self.tp.size > 1 or self.pp.size > 1 or
-                batch.cu_host is None or self.cfg.head_dim != 128 or
-                ops.PREFILL_SWZ < 16 or x.shape[1] % 8 or
-                (batch.kv_gather_slots is not None and page & (page - 1))):
-            return None
-        attn, mlp = self.layers[0].attn, self.layers[0].mlp
-        if attn.heads // attn.kv_heads > 128:
-            return None
-        return ops.prompt_routes(x.shape[0], tuple(
-            tuple(w.shape)
-            for w in (attn.wqkv, attn.wo, mlp.w_gate_up, mlp.w_down)))
 
     @torch.inference_mode()
     def logits(self, hidden: torch.Tensor,

@@ -343,32 +343,55 @@ def place_inputs(fields, tables, new_fields, new_tables) -> None:
     tables[:n, :used].copy_(new_tables)
 
 
+def _route(rows: int, n: int, k: int, glu: bool) -> int:
+    if glu and _tile_glu(rows, n, k):
+        return 4
+    if glu and _glu(rows, n, k):
+        return 3
+    if rows > 64 and _tile(rows, n, k):
+        return 2
+    return 1 if _skinny(rows, n, k, True) else 0
+
+
 @functools.lru_cache(maxsize=1024)
-def _own_routes(rows: int, shapes: Tuple[Tuple[int, int], ...]
-                ) -> Tuple[int, ...]:
-    def parts(n, k):
-        if rows > 64 and _tile(rows, n, k):
-            return 2
-        return 1 if _skinny(rows, n, k, True) else 0
-
-    def glu(n, k):
-        if _tile_glu(rows, n, k):
-            return 4
-        return 3 if _glu(rows, n, k) else parts(n, k)
-    return tuple((glu if i == 2 else parts)(n, k)
-                 for i, (n, k) in enumerate(shapes))
+def _own_routes(rows: int, first, second, glu: bool) -> Tuple[int, int]:
+    return _route(rows, *first, glu), _route(rows, *second, False)
 
 
-def prompt_routes(rows: int, shapes: Tuple[Tuple[int, int], ...]
-                  ) -> Tuple[int, ...]:
-    """What linear_parts and linear_swiglu (the third) take for products of that
-    many rows and weights of ``shapes``, as numbers of bindings.cpp's Route."""
-    return _own_routes(rows, shapes) if SKINNY_GEMM else (0,) * len(shapes)
+def block_routes(rows: int, first, second, glu: bool) -> Tuple[int, int]:
+    """What linear_parts, or linear_swiglu for the first, takes for products of
+    that many rows and weights of these two shapes, as numbers of bindings.cpp's
+    Route."""
+    return (_own_routes(rows, first, second, glu) if SKINNY_GEMM
+            else (0, 0))
 
 
-def prompt_layer(*args):
-    """bindings.cpp prompt_layer; an empty list where it does not take the call."""
-    return _require_hip().prompt_layer(*args)
+def prompt_attention_block(src, residual, weight, eps: float, wqkv, wo,
+                           heads: int, q_norm, k_norm, key_cache, value_cache,
+                           cos_sin, positions, slot_mapping, scale: float,
+                           plan, slots=None) -> Optional[torch.Tensor]:
+    """norm_heads, prefill_attention by ``plan`` and linear_parts in one native
+    call, which adds to ``residual`` in place; None, and nothing done, for what
+    it does not take."""
+    if not _on_gpu(residual) or plan is None or PREFILL_SWZ < 16:
+        return None
+    return _require_hip().prompt_attention_block(
+        src, residual, weight, eps, wqkv, wo,
+        block_routes(residual.shape[0], wqkv.shape, wo.shape, False), heads,
+        q_norm, k_norm, key_cache, value_cache, cos_sin, positions,
+        slot_mapping, scale, plan.blocks, plan.lens, plan.items, plan.joins,
+        plan.parts, slots)
+
+
+def swiglu_block(src, residual, weight, eps: float, w_gate_up,
+                 w_down) -> Optional[torch.Tensor]:
+    """norm_swiglu and linear_parts in one native call, which adds to
+    ``residual`` in place; None, and nothing done, for what it does not take."""
+    if not _on_gpu(residual):
+        return None
+    return _require_hip().swiglu_block(
+        src, residual, weight, eps, w_gate_up, w_down,
+        block_routes(residual.shape[0], w_gate_up.shape, w_down.shape, True))
 
 
 def embed_rows(ids: torch.Tensor, table: torch.Tensor) -> torch.Tensor:

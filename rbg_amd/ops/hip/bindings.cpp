@@ -549,7 +549,7 @@ torch::Tensor prefill_flash(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   return out;
 }
 
-// Who takes a product of a prompt's rows (ops.prompt_routes).
+// Who takes a product of many rows (ops.block_routes).
 enum Route { BY_LIBRARY, BY_SKINNY, BY_TILE, GLU_BY_SKINNY, GLU_BY_TILE };
 
 static torch::Tensor routed(const torch::Tensor& x, const torch::Tensor& w,
@@ -575,34 +575,48 @@ static torch::Tensor prompt_norm(const c10::optional<torch::Tensor>& src,
   return *src;
 }
 
-// A Llama layer on the rows of prompts: the launches of its parts' operations
-// (models/llama.py), issued by one call.  Short prompts waited for the host: 37
-// tokens of 2048 wide are 62 launches, whose kernels take 400 us and which took 576
-// to issue, 412 so.  routes: of wqkv, wo, w_gate_up and w_down.  Returns the layer's result for the next norm to add, and the
-// residual, which is changed in place; nothing, and does nothing, for weights
-// that only the library takes.
-std::vector<torch::Tensor> prompt_layer(
+// Rows that the blocks below take.  Up to four take norm and product in one
+// launch, by norm_rows.
+static bool block_rows(const torch::Tensor& residual) {
+  return residual.is_cuda() && residual.dim() == 2 && residual.size(0) > 4 &&
+         residual.size(1) % 8 == 0 && !at::GradMode::is_enabled();
+}
+
+// Weights that not only the library takes.
+static bool block_weight(const torch::Tensor& w) {
+  return w.is_cuda() && w.is_contiguous() && w.dim() == 2 &&
+         w.scalar_type() == torch::kBFloat16 &&
+         (reinterpret_cast<uintptr_t>(w.data_ptr()) & 15) == 0;
+}
+
+// The two blocks of a Llama layer on many rows: the launches of their operations
+// (models/llama.py), issued by one call each.  Short prompts wait for the host: 37
+// tokens of 2048 wide are 61 launches in six layers, whose kernels take 400 us and
+// which take 600 to issue, 478 so; a step among others takes 442.  (A whole layer
+// by one call 425, but hooked, replaced or substituted parts of it were passed by.)
+// Routes: of the products with the two weights.  Both return the block's result
+// for the next norm to add, and add to the residual in place; none, and nothing
+// is done, for what only the operations by themselves take.
+c10::optional<torch::Tensor> prompt_attention_block(
     c10::optional<torch::Tensor> src, torch::Tensor residual,
-    torch::Tensor input_norm, torch::Tensor post_norm, double eps,
-    torch::Tensor wqkv, torch::Tensor wo, torch::Tensor w_gate_up,
-    torch::Tensor w_down, std::vector<int64_t> routes, int64_t heads,
+    torch::Tensor norm, double eps, torch::Tensor wqkv, torch::Tensor wo,
+    std::pair<int64_t, int64_t> routes, int64_t heads,
     c10::optional<torch::Tensor> q_norm, c10::optional<torch::Tensor> k_norm,
     torch::Tensor key_cache, torch::Tensor value_cache, torch::Tensor cos_sin,
     torch::Tensor positions, torch::Tensor slot_mapping, double scale,
     torch::Tensor block_info, torch::Tensor seq_lens,
     c10::optional<torch::Tensor> items, c10::optional<torch::Tensor> joins,
     int64_t parts, c10::optional<torch::Tensor> gather_slots) {
-  TORCH_CHECK(routes.size() == 4, "a route per product");
-  for (const auto& w : {wqkv, wo, w_gate_up, w_down})
-    if (!w.is_cuda() || !w.is_contiguous() || w.dim() != 2 ||
-        w.scalar_type() != torch::kBFloat16 ||
-        (reinterpret_cast<uintptr_t>(w.data_ptr()) & 15))
-      return {};
   const int64_t rows = residual.size(0), kvh = key_cache.size(1);
-  auto x = prompt_norm(src, residual, input_norm, eps);
-  auto qkv = rope_heads(routed(x, wqkv, routes[0]), heads, q_norm, k_norm, eps,
-                        key_cache, value_cache, cos_sin, positions,
-                        slot_mapping);
+  const int64_t page = key_cache.size(2);
+  if (!block_rows(residual) || !block_weight(wqkv) || !block_weight(wo) ||
+      key_cache.size(3) != 128 || heads % kvh || heads / kvh > 128 ||
+      (gather_slots && (page & (page - 1))))
+    return c10::nullopt;
+  auto qkv = rope_heads(
+      routed(prompt_norm(src, residual, norm, eps), wqkv, routes.first), heads,
+      q_norm, k_norm, eps, key_cache, value_cache, cos_sin, positions,
+      slot_mapping);
   const auto part = [&](int64_t from, int64_t n) {
     return qkv.narrow(1, from * 128, n * 128).view({rows, n, 128});
   };
@@ -612,11 +626,21 @@ std::vector<torch::Tensor> prompt_layer(
                          gather_slots ? value_cache : part(heads + kvh, kvh),
                          block_info, seq_lens, scale, gather_slots, items,
                          joins, parts);
-  x = routed(o.view({rows, heads * 128}), wo, routes[1]);
-  x = prompt_norm(x, residual, post_norm, eps);
-  x = routed(x, w_gate_up, routes[2]);
-  if (routes[2] != GLU_BY_SKINNY && routes[2] != GLU_BY_TILE) x = silu_mul(x);
-  return {routed(x, w_down, routes[3]), residual};
+  return routed(o.view({rows, heads * 128}), wo, routes.second);
+}
+
+c10::optional<torch::Tensor> swiglu_block(
+    c10::optional<torch::Tensor> src, torch::Tensor residual,
+    torch::Tensor norm, double eps, torch::Tensor w_gate_up,
+    torch::Tensor w_down, std::pair<int64_t, int64_t> routes) {
+  if (!block_rows(residual) || !block_weight(w_gate_up) ||
+      !block_weight(w_down))
+    return c10::nullopt;
+  auto x = routed(prompt_norm(src, residual, norm, eps), w_gate_up,
+                  routes.first);
+  if (routes.first != GLU_BY_SKINNY && routes.first != GLU_BY_TILE)
+    x = silu_mul(x);
+  return routed(x, w_down, routes.second);
 }
 
 torch::Tensor mfma_probe(torch::Tensor a, torch::Tensor b, int64_t a_split,
@@ -792,7 +816,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("block_tables"), py::arg("context_lens"), py::arg("scale"),
         py::arg("num_splits"), py::arg("wide"), py::arg("span") = 128,
         py::arg("tickets") = c10::nullopt);
-  m.def("prompt_layer", &prompt_layer, "a Llama layer on rows of prompts");
+  m.def("prompt_attention_block", &prompt_attention_block,
+        "norm, attention and output product of prompts");
+  m.def("swiglu_block", &swiglu_block, "norm and gated MLP of many rows");
   m.def("place_inputs", &place_inputs, "a decode step's inputs to their place");
   m.def("prefill_attention", &prefill_attention, "varlen causal flash prefill");
   m.def("prefill_flash", &prefill_flash, "causal attention of prompts",

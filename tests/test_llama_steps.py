@@ -7,6 +7,7 @@ import math
 import pytest
 import torch
 
+from rbg_amd import ops
 from rbg_amd.engine.config import EngineConfig, ModelConfig
 from rbg_amd.engine.engine import LLMEngine
 from rbg_amd.engine.kv_cache import BlockTable
@@ -230,38 +231,130 @@ def test_nothing_is_collected_in_a_capture(collects):
     assert seen == [False] and out.isfinite().all()
 
 
+class Prompts:
+    """Two sequences, of which a step takes a half."""
+
+    def __init__(self, norms, rows):
+        self.runner = ModelRunner(engine_config(norms, "cuda"))
+        spread_norms(self.runner.model)
+        gen = torch.Generator().manual_seed(rows)
+        self.seqs = []
+        for count in (rows - 2, 2):
+            seq = Sequence(torch.randint(0, 512, (2 * count,),
+                                         generator=gen).tolist())
+            seq.block_table = BlockTable(self.runner.cache)
+            seq.block_table.ensure(2 * count)
+            self.seqs.append(seq)
+
+    def step(self, half):
+        chunks = []
+        for s in self.seqs:
+            n = len(s.prompt_tokens) // 2
+            chunks.append((s, half * n, s.prompt_tokens[half * n:][:n]))
+        return self.runner.feed(chunks, [[0, len(c[2]) - 1] for c in chunks])
+
+
+def count_blocks(monkeypatch):
+    """(name, whether it took the call) of every native block."""
+    calls = []
+    for name in ("prompt_attention_block", "swiglu_block"):
+        def counted(*args, name=name, inner=getattr(ops, name)):
+            out = inner(*args)
+            calls.append((name, out is not None))
+            return out
+        monkeypatch.setattr(ops, name, counted)
+    return calls
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("norms", [False, True])
 @pytest.mark.parametrize("rows", [5, 37, 65, 300, 1100])
-def test_layers_issued_by_one_call(norms, rows, monkeypatch):
-    """The same launches as of a layer's parts, so the same bits: prompts, and
-    portions behind a past; a hooked part is called."""
-    runner = ModelRunner(engine_config(norms, "cuda"))
-    spread_norms(runner.model)
-    gen = torch.Generator().manual_seed(rows)
-    seqs = []
-    for count in (rows - 2, 2):
-        seqs.append(Sequence(torch.randint(0, 512, (2 * count,),
-                                           generator=gen).tolist()))
-        seqs[-1].block_table = BlockTable(runner.cache)
-        seqs[-1].block_table.ensure(2 * count)
-    seen = []
-
-    def step(half):
-        chunks = []
-        for s in seqs:
-            n = len(s.prompt_tokens) // 2
-            chunks.append((s, half * n, s.prompt_tokens[half * n:][:n]))
-        return runner.feed(chunks, [[0, len(c[2]) - 1] for c in chunks])
-    got = [step(0), step(1), runner.cache.kv.clone()]
-    assert seen == []
-    hook = runner.model.layers[1].mlp.register_forward_hook(
-        lambda *a: seen.append(1))
-    again = step(0)
-    hook.remove()
-    assert seen and torch.equal(again, got[0])
-    monkeypatch.setattr(type(runner.model), "routes", lambda *a: None)
-    runner.cache.kv.zero_()
-    want = [step(0), step(1), runner.cache.kv]
+def test_blocks_issued_by_one_call(norms, rows, monkeypatch):
+    """The same launches as of a block's parts, so the same bits: prompts, and
+    portions behind a past."""
+    prompts = Prompts(norms, rows)
+    layers = len(prompts.runner.model.layers)
+    calls = count_blocks(monkeypatch)
+    got = [prompts.step(0), prompts.step(1), prompts.runner.cache.kv.clone()]
+    for name in ("prompt_attention_block", "swiglu_block"):
+        assert calls.count((name, True)) == 2 * layers
+        monkeypatch.setattr(ops, name, lambda *a: None)
+    prompts.runner.cache.kv.zero_()
+    want = [prompts.step(0), prompts.step(1), prompts.runner.cache.kv]
+    assert len(calls) == 4 * layers
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+class Delegate(torch.nn.Module):
+    """In the place of a module, with its attributes."""
+
+    def __init__(self, inner, seen):
+        super().__init__()
+        self.inner, self.seen = inner, seen
+
+    def forward(self, *args):
+        self.seen.append("other module")
+        return self.inner(*args)
+
+    def __getattr__(self, name):
+        try:
+            return super().__getattr__(name)
+        except AttributeError:
+            return getattr(self.inner, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("part", ["attn", "mlp"])
+def test_changed_parts_of_layers_are_called(part, monkeypatch):
+    """Prompts go through a part whose forward is replaced or hooked, or that is
+    another module, and give the same bits."""
+    prompts = Prompts(False, 37)
+    model, seen = prompts.runner.model, []
+    want = prompts.step(0)
+
+    def noted(name, result=None):
+        def note(*args):
+            seen.append(name)
+            return result(*args) if result else None
+        return note
+    module = getattr(model.layers[1], part)
+    module.forward = noted("instance", module.forward)
+    assert torch.equal(prompts.step(0), want)
+    del module.forward
+    with monkeypatch.context() as m:
+        inner = type(module).forward
+        m.setattr(type(module), "forward", noted("class", inner))
+        assert torch.equal(prompts.step(0), want)
+    setattr(model.layers[1], part, Delegate(module, seen))
+    assert torch.equal(prompts.step(0), want)
+    setattr(model.layers[1], part, module)
+    for name, register in (
+            ("hook", module.register_forward_hook),
+            ("hook before", module.register_forward_pre_hook)):
+        handle = register(noted(name))
+        assert torch.equal(prompts.step(0), want)
+        handle.remove()
+    handle = torch.nn.modules.module.register_module_forward_hook(
+        lambda m, *a: seen.append("any hook") if m is module else None)
+    assert torch.equal(prompts.step(0), want)
+    handle.remove()
+    assert seen == ["instance"] + ["class"] * len(model.layers) + [
+        "other module", "hook", "hook before", "any hook"]
+
+
+@pytest.mark.gpu
+def test_layers_of_other_widths(monkeypatch):
+    """A layer's products go by its own weights, not by the first layer's."""
+    prompts = Prompts(False, 300)
+    mlp = prompts.runner.model.layers[1].mlp
+    gate, up = mlp.w_gate_up.chunk(2)
+    with torch.inference_mode():        # no multiple that the kernels take
+        mlp.w_gate_up = torch.nn.Parameter(
+            torch.cat([gate[:1000], up[:1000]]), requires_grad=False)
+        mlp.w_down = torch.nn.Parameter(mlp.w_down[:, :1000].contiguous(),
+                                        requires_grad=False)
+    got = prompts.step(0)
+    for name in ("prompt_attention_block", "swiglu_block"):
+        monkeypatch.setattr(ops, name, lambda *a: None)
+    assert torch.equal(prompts.step(0), got)

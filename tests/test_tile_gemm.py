@@ -154,7 +154,8 @@ def test_rules_leave_what_it_refuses(rows, n, k, fewer):
     library, on both ways to it; a little below it is taken."""
     from rbg_amd import ops
     assert not ops._tile(rows, n, k) and not ops._tile_glu(rows, n, k)
-    assert not {2, 4} & set(ops.prompt_routes(rows, ((n, k),) * 4))
+    for glu in (False, True):
+        assert not {2, 4} & set(ops.block_routes(rows, (n, k), (n, k), glu))
     assert ops._tile(*fewer) or ops._tile_glu(*fewer)
 
 
@@ -172,8 +173,8 @@ def test_switched_off_everything_is_the_librarys(monkeypatch):
         rules = ops._tile, ops._tile_glu
         assert any(ops._takes_tile(x, w, r) for r in rules) or \
             ops._takes_skinny(x, w, parts=True)
-        assert any(ops.prompt_routes(rows, ((n, k),) * 4))
+        assert any(ops.block_routes(rows, (n, k), (n, k), True))
         monkeypatch.setattr(ops, "SKINNY_GEMM", 0)
         assert not any(ops._takes_tile(x, w, r) for r in rules)
         assert not ops._takes_skinny(x, w, parts=True)
-        assert not any(ops.prompt_routes(rows, ((n, k),) * 4))
+        assert not any(ops.block_routes(rows, (n, k), (n, k), True))
