@@ -683,8 +683,9 @@ def test_swiglu_of_small_workgroups(rows, n, k):
 def test_decode_attention_tickets(group, lens, splits):
     """Parts added up by a sequence's last workgroup as by a launch of its own:
     one part, two, more than a round of loads, longer ones than the least, and a
-    longer single one where there are many; again and again with the same tickets,
-    and replayed.  The same f32 sums in another order: a rounding of the result
+    longer single one where there are many; again and again with the same tickets
+    and sums' memory, eagerly and replayed, with other queries, rows and order of
+    lengths each time, so that sums of a former time would show.  The same f32 sums in another order: a rounding of the result
     apart, 2^-8 of it, or of the values' size where they cancel."""
     from rbg_amd import ops
     dev = torch.device("cuda:0")
@@ -703,21 +704,32 @@ def test_decode_attention_tickets(group, lens, splits):
     def run(t):
         return ops.decode_attention(q, k, v, tables, lens, 0.2,
                                     num_splits=splits, variant=7, tickets=t)
-    want = run(None).float()
-    bound = want.abs() * 2 ** -7 + 2 ** -9
-    for _ in range(3):
-        got = run(tickets)
+
+    def others():
+        for t in (q, k, v):
+            t.copy_(torch.randn(t.shape, device=dev, generator=gen))
+        lens.copy_(lens[torch.randperm(n, device=dev, generator=gen)])
+
+    def check(got):
+        want = run(None).float()
+        bound = want.abs() * 2 ** -7 + 2 ** -9
         assert ((got.float() - want).abs() <= bound).all()
         assert not tickets.any()
+    for _ in range(3):
+        got = run(tickets)
+        check(got)
+        others()
     g = torch.cuda.CUDAGraph()
     with torch.inference_mode(), torch.cuda.graph(g):
         out = run(tickets)
-    for _ in range(3):
+    for _ in range(4):
+        others()
         with torch.inference_mode():
             out.zero_()
         g.replay()
         torch.cuda.synchronize()
-        assert torch.equal(out, got) and not tickets.any()
+        check(out)
+        assert torch.equal(out, run(tickets))
 
 
 @pytest.mark.gpu
