@@ -79,6 +79,50 @@ def test_many_tiles_a_workgroup():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form", [f for f in range(len(FORMS))
+                                  if FORMS[f][1] % 4 == 0])
+def test_silu_of_very_negative_gates(form):
+    """Sigmoids below the smallest normal f32 are not lost, as a large up value
+    makes their product with it an ordinary number; an exponential above f32's
+    range gives 0.  The gates are exact: 2^-8 for the result's rounding, and
+    |g| 2^-23 for the exponential's argument."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gates = torch.tensor([0., -1., -60., -87., -87.5, -88., -88.5, -100.],
+                         device=dev)
+    m, k, up = 70, 512, 2. ** 100
+    x = torch.ones(m, k, dtype=torch.bfloat16, device=dev)
+    w = torch.full((128, k), up / k, device=dev)
+    w[:64] = (gates / k).repeat(8)[:, None]
+    got = ops._hip.tile_form(x, w.bfloat16(), GLU, form, 1, -1, 0).double()
+    g = gates.double()
+    want = (g / (1 + (-g).exp()) * up).masked_fill(g < -88.7, 0).repeat(8)
+    assert ((got - want).abs() <= want.abs() * (2 ** -8 + 100 * 2 ** -22)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [f for f in range(len(FORMS))
+                                  if FORMS[f][1] % 4 == 0])
+def test_silu_of_very_negative_gates(form):
+    """Sigmoids below the smallest normal f32 are not lost, as a large up value
+    makes their product with it an ordinary number; an exponential above f32's
+    range gives 0.  The gates are exact: 2^-8 for the result's rounding, and
+    |g| 2^-22 for the exponential's argument."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gates = torch.tensor([0., -1., -60., -87., -87.5, -88., -88.5, -100.],
+                         device=dev)
+    m, k, up = 70, 512, 2. ** 100
+    x = torch.ones(m, k, dtype=torch.bfloat16, device=dev)
+    w = torch.full((128, k), up / k, device=dev)
+    w[:64] = (gates / k).repeat(8)[:, None]
+    got = ops._hip.tile_form(x, w.bfloat16(), GLU, form, 1, -1, 0).double()
+    g = gates.double()
+    want = (g / (1 + (-g).exp()) * up).masked_fill(g < -88.7, 0).repeat(8)
+    assert ((got - want).abs() <= want.abs() * (2 ** -8 + 100 * 2 ** -22)).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [
     (65, 2048, 12288), (128, 4096, 12288), (129, 2048, 3584),
     (65, 2048, 4096), (97, 5120, 3584), (128, 3072, 8192), (70, 12288, 4096),
