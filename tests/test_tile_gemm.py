@@ -126,6 +126,7 @@ def test_silu_of_very_negative_gates(form):
 @pytest.mark.parametrize("m,n,k", [
     (65, 2048, 12288), (128, 4096, 12288), (129, 2048, 3584),
     (65, 2048, 4096), (97, 5120, 3584), (128, 3072, 8192), (70, 12288, 4096),
+    (112, 12544, 5120), (66, 14336, 4608),
     (256, 6144, 4096), (257, 2048, 5120), (999, 3136, 5120),
     (1000, 6144, 4096), (1500, 14336, 3584), (2048, 4096, 8192)])
 def test_parts_route(m, n, k):
@@ -222,3 +223,11 @@ def test_switched_off_everything_is_the_librarys(monkeypatch):
         assert not any(ops._takes_tile(x, w, r) for r in rules)
         assert not ops._takes_skinny(x, w, parts=True)
         assert not any(ops.block_routes(rows, (n, k), (n, k), True))
+
+
+def test_wide_matrices_are_taken_with_any_k():
+    """65 to 128 rows: no window between the sizes of common models."""
+    from rbg_amd.ops import _tile
+    for rows in (65, 96, 97, 128):
+        for n in (12288, 13312, 14336):
+            assert all(_tile(rows, n, k) for k in range(3584, 12289, 64))
