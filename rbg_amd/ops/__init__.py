@@ -278,23 +278,24 @@ def _tile_few(rows: int, n: int, k: int) -> bool:
     """Does the GEMM of prompts take gate/up of 5 to 64 rows, in tiles of 64?  Its
     ring of weights in LDS is deeper than the decode GEMM's registers, but a CU has
     one tile at a time, so that it gains where there is about one for each.  Against
-    what is taken without it, over 16384 to 65536 columns, 2048, 4096, 5120 and 8192 k,
-    5 to 64 rows (us): to 20480 columns (18432 x 4096: 8 rows 39.6 / 31.3, 64 rows 43.1 /
-    36.6; 20480 x 8192: 16 rows 74.5 / 64.1), from there to 28672 for more rows (24576 x
-    4096: 48 rows 44.0 / 38.7, 16 rows 37.0 / 37.0; 28672 x 4096: 48 rows 45.4 / 43.1, 33
-    rows 43.0 / 43.0), and beyond 32768 with tiles of 256 (36864 x 2048: 5 rows 38.9 /
-    30.3; 45056 x 4096: 64 rows 93.7 / 70.3; 57344 x 8192: 16 rows 180 / 169, 64 rows 192 /
-    167; not 57344 x 4096, 8 rows 83.6 / 88.6).  Rows that are no multiple of 4 KB apart
-    the library reads better (40960 x 5120: 64 rows 95 / 101), but not where they are few
-    and it has few tiles (18432 x 5120: 16 rows 85 / 46, 32 rows 45 / 50)."""
+    what is taken without it, over 16896 to 73728 columns, 2048 to 8192 k, 5 to 64 rows
+    (us): to 20480 columns (18432 x 4096: 64 rows 43.1 / 36.6; 20480 x 8192: 16 rows 68.9
+    / 64.3), from there to 26624 for more rows (24576 x 4096: 48 rows 45.0 / 40.6, 16 rows
+    38.3 / 39.3; 28672 x 4096: 48 rows 46.3 / 46.5, x 8192 86.0 / 90.0), and beyond 32768
+    with tiles of 256, while one round holds them, 65536 columns (36864 x 2048: 5 rows
+    39.3 / 32.1; 45056 x 4096: 64 rows 88.3 / 73.3).  A full round leaves no CU to spare:
+    from 53248 columns only long k (57344 x 4096: 5 rows 81.8 / 85.5, x 6144 121 / 123, x
+    8192 178 / 166), for more rows from 6144 (33 rows 135 / 125; 65536 x 6144 141 / 140, x
+    4096 94 / 104).  Rows that are no multiple of 4 KB apart the library reads better
+    (40960 x 5120: 64 rows 95 / 101), but not where they are few and it has few tiles
+    (18432 x 5120: 16 rows 85 / 46, 32 rows 45 / 50; x 4608 and 7168 alike)."""
     if not 4 < rows <= 64 or k < 2048 or k > 8192 or n <= 16384:
         return False
     if k % 2048:
         return rows <= 16 and k >= 4096 and n <= 32768
     if n <= 32768:
-        return n <= 20480 or (n <= 28672 and
-                              rows > (32 if n <= 26624 else 40))
-    return n <= 53248 or (n <= 65536 and k == 8192)
+        return n <= (20480 if rows <= 32 else 26624)
+    return n <= 53248 or (n <= 65536 and k >= (8192 if rows <= 32 else 6144))
 
 
 def _tile_glu(rows: int, n: int, k: int) -> bool:

@@ -142,7 +142,7 @@ def test_parts_route(m, n, k):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [
-    (5, 16448, 2048), (33, 26624, 2048), (41, 28672, 2048), (64, 32832, 2048),
+    (5, 16448, 2048), (33, 26624, 2048), (33, 65536, 6144), (64, 32832, 2048),
     (16, 18432, 4160), (63, 36864, 4096),
     (65, 24576, 1024), (128, 28672, 1088), (129, 8192, 2048),
     (256, 18432, 2048), (385, 28672, 1024), (1000, 11264, 2048),
@@ -231,3 +231,19 @@ def test_wide_matrices_are_taken_with_any_k():
     for rows in (65, 96, 97, 128):
         for n in (12288, 13312, 14336):
             assert all(_tile(rows, n, k) for k in range(3584, 12289, 64))
+
+
+def test_few_rows_of_gate_up_by_bounds():
+    """Beyond a round's tiles but for a few, what is taken of some k and rows is
+    taken of longer k and more rows; what tiles of 128 columns would need more than
+    a round of is left."""
+    from rbg_amd.ops import _tile_few
+    for n in range(53312, 65537, 64):
+        taken = [[_tile_few(rows, n, k) for k in (2048, 4096, 6144, 8192)]
+                 for rows in (5, 32, 33, 64)]
+        assert all(row == sorted(row) for row in taken)
+        assert all(list(col) == sorted(col) for col in zip(*taken))
+        assert taken[0][3] and taken[2][2]
+    for n in (26688, 28672, 32768):
+        assert not any(_tile_few(rows, n, k) for rows in range(5, 65)
+                       for k in (2048, 4096, 6144, 8192))
