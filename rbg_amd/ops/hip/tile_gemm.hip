@@ -375,8 +375,8 @@ extern "C" int launch_tile_gemm(void* out, const void* a, const void* w, int M,
   TG_GO(6, 6, 3, 3, TILE_PARTS)
   TG_ENDS(8, 4, 3, 3)
   TG_ENDS(4, 4, 5, 4)
-  TG_ENDS(2, 4, 6, 6)
-  TG_ENDS(2, 8, 4, 4)
+  TG_GO(2, 4, 6, 6, TILE_GLU)
+  TG_GO(2, 8, 4, 4, TILE_GLU)
 #undef TG_ENDS
 #undef TG_GO
   return 0;

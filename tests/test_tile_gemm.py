@@ -7,6 +7,12 @@ STAGES = [2, 2, 2, 3, 3, 4, 6, 4]       # the fewest of a part
 PLAIN, PARTS, GLU = 0, 1, 2
 
 
+def _built(form, end):
+    """Tiles of 64 rows are for gate/up only."""
+    wm, wn = FORMS[form]
+    return wn % 4 == 0 if end == GLU else wm > 2
+
+
 def _operands(m, n, k):
     dev = torch.device("cuda:0")
     gen = torch.Generator(device=dev).manual_seed(m * 1000003 + n + k)
@@ -42,9 +48,8 @@ def test_forms(form, m, n, k):
     numbers of stages, parts of unequal length, several tiles a workgroup."""
     from rbg_amd import ops
     x, w, full, sums = _operands(m, n, k)
-    wm, wn = FORMS[form]
     for end in (PLAIN, PARTS, GLU):
-        if (end == GLU and wn % 4) or k // 64 < STAGES[form]:
+        if not _built(form, end) or k // 64 < STAGES[form]:
             continue
         for parts in (1, 2, 3) if end == PARTS else (1,):
             if k // 64 // parts < max(4, STAGES[form]):
@@ -72,7 +77,7 @@ def test_many_tiles_a_workgroup():
     for form in range(len(FORMS)):
         x, w, full, sums = operands[384 if STAGES[form] > 4 else 256]
         for end in (PLAIN, GLU):
-            if end == GLU and FORMS[form][1] % 4:
+            if not _built(form, end):
                 continue
             got = ops._hip.tile_form(x, w, end, form, 1, -1, 0)
             assert _near(got, end, full, sums), (form, end)
@@ -80,29 +85,7 @@ def test_many_tiles_a_workgroup():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", [f for f in range(len(FORMS))
-                                  if FORMS[f][1] % 4 == 0])
-def test_silu_of_very_negative_gates(form):
-    """Sigmoids below the smallest normal f32 are not lost, as a large up value
-    makes their product with it an ordinary number; an exponential above f32's
-    range gives 0.  The gates are exact: 2^-8 for the result's rounding, and
-    |g| 2^-23 for the exponential's argument."""
-    from rbg_amd import ops
-    dev = torch.device("cuda:0")
-    gates = torch.tensor([0., -1., -60., -87., -87.5, -88., -88.5, -100.],
-                         device=dev)
-    m, k, up = 70, 512, 2. ** 100
-    x = torch.ones(m, k, dtype=torch.bfloat16, device=dev)
-    w = torch.full((128, k), up / k, device=dev)
-    w[:64] = (gates / k).repeat(8)[:, None]
-    got = ops._hip.tile_form(x, w.bfloat16(), GLU, form, 1, -1, 0).double()
-    g = gates.double()
-    want = (g / (1 + (-g).exp()) * up).masked_fill(g < -88.7, 0).repeat(8)
-    assert ((got - want).abs() <= want.abs() * (2 ** -8 + 100 * 2 ** -22)).all()
-
-
-@pytest.mark.gpu
-@pytest.mark.parametrize("form", [f for f in range(len(FORMS))
-                                  if FORMS[f][1] % 4 == 0])
+                                  if _built(f, GLU)])
 def test_silu_of_very_negative_gates(form):
     """Sigmoids below the smallest normal f32 are not lost, as a large up value
     makes their product with it an ordinary number; an exponential above f32's
@@ -168,6 +151,11 @@ def test_refuses_what_it_cannot_take():
                 f(*bad)
     with pytest.raises(RuntimeError):       # parts of too few stages
         ops._hip.tile_form(x, w, PARTS, 5, 4, -1, 0)
+    for form in range(len(FORMS)):          # forms that are not built
+        for end in (PLAIN, PARTS, GLU):
+            if not _built(form, end):
+                with pytest.raises(RuntimeError):
+                    ops._hip.tile_form(x, w, end, form, 1, -1, 0)
 
 
 def test_rules_hand_over_what_it_takes():
