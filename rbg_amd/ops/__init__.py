@@ -300,9 +300,9 @@ def _tile_few(rows: int, n: int, k: int) -> bool:
 
 def _tile_glu(rows: int, n: int, k: int) -> bool:
     """Does it take a gate/up product, with silu?  Against the product and
-    silu_mul, or the decode GEMM (us): from 129 rows (28672 x 4096: 256 rows 74 /
-    64, 512 rows 113 / 105, 2048 rows 387 / 350, 8192 rows 1417 / 1341; 11264 x
-    2048: 256 rows 30 / 22, 2048 rows 95 / 82).  Not where parts of k, which silu
+    silu_mul, or the decode GEMM (us): from 129 rows (28672 x 4096: 256 rows 80 /
+    70, 512 rows 121 / 115, 2048 rows 396 / 365, 8192 rows 1382 / 1301; 11264 x
+    2048: 256 rows 31 / 24, 2048 rows 98 / 81).  Not where parts of k, which silu
     cannot have, fill the chip better (16384 x 4096: 176 rows 46 / 51; 12288 x
     6144: 640 rows 100 / 122; 8192 x 28672: 1200 rows 472 / 495), and around 320
     rows, a round and a quarter of its tiles, only of narrower matrices (51200 x
@@ -629,10 +629,10 @@ def _cut_prefill(tiles: np.ndarray, kv_heads: int):
 
     A CU's share holds whole blocks as far as they fit, and other blocks are cut
     to fill it.  Times in us are those of hip/prefill_flash.hip: a tile takes 1.2
-    by itself on a CU and 1.05 beside another; a part leaves 64 KB of sums, which
+    by itself on a CU and 1.0 where its CU has others too; a part leaves 64 KB of sums, which
     are written and read at 5 TB/s, and the launch that adds them up takes 5.
-    Whole blocks and cut ones, 32 heads of 8 (us): 40 rows after 9000 keys 165 / 28,
-    512 after 4000 88 / 60, 1500 after 9000 297 / 261.  Not cut: 2048 rows, whose
+    Whole blocks and cut ones, 32 heads of 8 (us): 40 rows after 9000 keys 140 / 27,
+    512 after 4000 79 / 55, 1500 after 9000 294 / 249.  Not cut: 2048 rows, whose
     longest workgroups run beside the shortest (51), nor more blocks than four a
     CU, which even out by themselves."""
     cus = max(1, 256 // kv_heads)           # of a key head

@@ -28,8 +28,7 @@ inline SkinnyPlan pick_skinny(int M, int N, int K) {
   // a few rows, where K is whole turns of that kernel (8 waves x 4 chunks of 64
   // in flight; in a part of one it loads the last chunk again, with K = 2560 8
   // times for 5 chunks), or short, where that costs less than a reduction (2048 x
-  // 5632, 1 row: 9.0 us against 9.7, 4 rows 10.1 against 10.0).  5120 x 25600
-  // takes 66 us against 50, most of it for 320 workgroups on 256 CUs.
+  // 5632, 1 row: 9.0 us against 9.7, 4 rows 10.1 against 10.0).
   if ((M <= 4 && K % 2048 == 0) || (M <= 2 && K <= 8192 && N <= 12288))
     return {0, 1};
   // up to 32 rows of a narrow matrix: workgroups of half the size, half again

@@ -26,7 +26,7 @@
 //    stage, needs registers that spill (640).
 //  * Blocks are cut by keys where whole ones would leave CUs idle (ops
 //    _cut_prefill), whose sums a second launch adds up: 1500 tokens after 9000
-//    297 -> 255 us, 512 after 4000 88 -> 60, 40 after 9000 165 -> 28.
+//    294 -> 249 us, 512 after 4000 79 -> 55, 40 after 9000 140 -> 27.
 #include <type_traits>
 
 #include "mfma_util.h"

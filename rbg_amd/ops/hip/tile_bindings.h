@@ -15,7 +15,7 @@ enum TileEnd { TILE_PLAIN, TILE_PARTS, TILE_GLU };
 
 // A tile of 32 wm rows and 32 wn rows of W and the time of a launch in us: fixed
 // + rounds * (round + stages * (step + busy * share of workgroups with work)) +
-// write * MB / 2 of the result.  Fitted to 300 to 1300 launches of each form, 65
+// write * MB of the result.  Fitted to 300 to 1300 launches of each form, 65
 // to 8192 rows, 1536 to 57344 columns, 2048 to 28672 k with cold weights (half of
 // them within 4 to 10%).  A stage takes longer where more CUs are busy, as the
 // chip lowers its clock.
@@ -59,8 +59,7 @@ inline float tile_time(const TileForm& f, int M, int cols, int K, int end,
   const long rounds = ((items + 7) / 8 + 31) / 32;
   const float stages = K / 64.f / parts;
   const float share = items / (256.f * rounds);
-  const float mb = 1e-6f * M * cols *
-                   (end == TILE_PARTS ? 4.f * parts : end == TILE_GLU ? 2 : 2);
+  const float mb = 1e-6f * M * cols * (end == TILE_PARTS ? 4.f * parts : 2.f);
   return f.fixed +
          rounds * (f.round + stages * (f.step + f.busy * share)) + f.write * mb;
 }
@@ -100,7 +99,7 @@ inline TilePlan pick_tile_parts(int M, int N, int K) {
     for (int parts : {2, 3, 4, 6, 8}) {
       const int tiles =
           ((M + 32 * f.wm - 1) / (32 * f.wm)) * ((N + 32 * f.wn - 1) / (32 * f.wn));
-      // one round, which also bounds the sums (80 MB)
+      // a round and a quarter at most, which also bounds the sums (84 MB)
       if (tiles * parts > 320 || K / 64 / parts < f.fill) break;
       const float time = tile_time(f, M, N, K, TILE_PARTS, parts) +
                          (4 * parts - 2) * 2e-7f * M * N;
