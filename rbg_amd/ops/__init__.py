@@ -199,8 +199,8 @@ def _tile(rows: int, n: int, k: int) -> bool:
     of matrices that give parts enough to do (6144 x 4096: 128 rows 26.3 / 24.0; 8192 x
     8192: 45.2 / 42.1; 4096 x 8192: 29.0 / 27.1, x 4096 21.3 / 22.0; 3072 x 8192 26.3 /
     23.7), from 65 rows of long rows (4096 x 14336: 128 rows 34 / 32; 5120 x 25600: 97
-    rows 71 / 61), of wide matrices (3584 to 10240 k, 258 points 0.95 of the time
-    without it, 7 of them slower by 2 to 5%: 12288 x 8192, 112 rows 64.2 / 56.5; 14336 x
+    rows 71 / 61), of wide matrices (3584 to 10240 k, 238 points 0.94 of the time
+    without it, 5 of them slower by 2 to 5%: 12288 x 8192, 112 rows 64.2 / 56.5; 14336 x
     5120 48.6 / 46.6; 12288 x 5120 42.8 / 44.3) and of 2048 columns (x 4096: 65 rows
     15.2 / 13.7, x 6144 15.7 / 17.1).  Not short k
     (2048 x 2048: 256 rows 10 / 11), and from 257 rows to 999 only k from 5120 on
