@@ -285,7 +285,7 @@ def _tile_few(rows: int, n: int, k: int) -> bool:
     with tiles of 256, while one round holds them, 65536 columns (36864 x 2048: 5 rows
     39.3 / 32.1; 45056 x 4096: 64 rows 88.3 / 73.3).  A full round leaves no CU to spare:
     from 53248 columns only long k (57344 x 4096: 5 rows 81.8 / 85.5, x 6144 121 / 123, x
-    8192 178 / 166), for more rows from 6144 (33 rows 135 / 125; 65536 x 6144 141 / 140, x
+    8192 178 / 166), for more rows from 6144 (33 rows 135 / 125; 65536 x 6144 143 / 142, x
     4096 94 / 104).  Rows that are no multiple of 4 KB apart the library reads better
     (40960 x 5120: 64 rows 95 / 101), but not where they are few and it has few tiles
     (18432 x 5120: 16 rows 85 / 46, 32 rows 45 / 50; x 4608 and 7168 alike)."""
