@@ -1,5 +1,12 @@
 // Common device helpers for the rbg_amd CDNA4 (gfx950) kernels.
 // Wave size is 64 everywhere; block sizes are multiples of 64.
+//
+// The first 14 words of a kernel's arguments are in scalar registers when its
+// waves start (setup.py); the others, those behind the first struct, and the grid's
+// and the workgroup's sizes are loads of 0.35 us.  So the kernels of decode steps,
+// of which dozens wait for one another, take first what their first loads need, and
+// get sizes as arguments (six layers, us: 1 sequence 2048 wide 264.7 -> 254.4, 1 of
+// 8b 654 -> 644, 7 of qwen 8b 733 -> 715, 45 of 8b 1122 -> 1109, 128 2026 -> 2017).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -65,31 +65,31 @@ DEV_INLINE f32x2 dp_shared(const float* from) {
 // of ragged lengths would leave XCDs idle (45 of up to 2500: 63 -> 68 us).
 template <int QPG, bool TOGETHER>
 __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
+    const int* __restrict__ lens,           // [seqs]
+    const int kv_heads, const int seqs, const int splits,
+    const int* __restrict__ tables,         // [seqs, max_pages]
+    const int max_pages, const int least, const int whole,
+    const __hip_bfloat16* __restrict__ q,   // [seqs, QH, DIM], rows q_stride
+    const int q_stride, const float scale,  // to the base of 2
+    const __hip_bfloat16* __restrict__ keys,    // [pages, KVH, PAGE, DIM]
+    const __hip_bfloat16* __restrict__ values,
     float* __restrict__ part_o,             // [splits, seqs, QH, DIM]
     float* __restrict__ part_ml,            // [splits, seqs, QH, 2]
     __hip_bfloat16* __restrict__ out,       // [seqs, QH, DIM]
-    const __hip_bfloat16* __restrict__ q,   // [seqs, QH, DIM], rows q_stride
-    const __hip_bfloat16* __restrict__ keys,    // [pages, KVH, PAGE, DIM]
-    const __hip_bfloat16* __restrict__ values,
-    const int* __restrict__ tables,         // [seqs, max_pages]
-    const int* __restrict__ lens,           // [seqs]
-    const float scale,                      // to the base of 2
-    const int kv_heads, const int max_pages, const int least,
-    const int whole, const int q_stride,
     int* __restrict__ tickets) {            // [seqs, KVH], or null
   int kvh = blockIdx.x, seq = blockIdx.y, split = blockIdx.z;
   if (TOGETHER) {
-    const int lin = kvh + kv_heads * (seq + gridDim.y * split);
-    const int pairs = gridDim.y * gridDim.z, group = lin / (8 * kv_heads);
+    const int lin = kvh + kv_heads * (seq + seqs * split);
+    const int pairs = seqs * splits, group = lin / (8 * kv_heads);
     const int in = lin % (8 * kv_heads);
     const bool whole = (group + 1) * 8 <= pairs;
     const int pair = group * 8 + (whole ? in % 8 : in / kv_heads);
     kvh = whole ? in / 8 : in % kv_heads;
-    seq = pair % gridDim.y;
-    split = pair / gridDim.y;
+    seq = pair % seqs;
+    split = pair / seqs;
   }
   const int ctx = lens[seq];
-  const int span = part_keys(ctx, least, whole, gridDim.z);
+  const int span = part_keys(ctx, least, whole, splits);
   const int begin = split * span, end = min(ctx, begin + span);
   if (begin >= ctx && split > 0) return;
   const int lane = threadIdx.x & 63;
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     if (ctx <= span) {        // no keys: 0; NaN stays
       out[row * DIM + d] = f2bf(total == 0.f ? 0.f : o / total);
     } else {
-      const size_t at_row = (size_t)split * gridDim.y * heads + row;
+      const size_t at_row = (size_t)split * seqs * heads + row;
       // past the L2, which other XCDs' workgroups do not see
       dp_share(&part_o[at_row * DIM + d], o);
       if (d == 0) {
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __shared__ int taken;
   __syncthreads();
-  const int parts = min((ctx + span - 1) / span, (int)gridDim.z);
+  const int parts = min((ctx + span - 1) / span, splits);
   if (threadIdx.x == 0) {
     int* ticket = tickets + (size_t)seq * kv_heads + kvh;
     taken = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED,
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
   const int piece = threadIdx.x % PIECES, share = threadIdx.x / PIECES;
   const int h = piece / (DIM / 4), d = piece % (DIM / 4) * 4;
   const size_t row = (size_t)seq * heads + kvh * QPG + h;
-  const size_t step = (size_t)gridDim.y * heads;
+  const size_t step = (size_t)seqs * heads;
   float top = LOW, total = 0.f;
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
   for (int first = share; first < parts; first += 8 * SHARES) {
@@ -383,12 +383,11 @@ extern "C" void launch_decode_pages(
   const dim3 grid(kv_heads, seqs, splits), block(64 * WAVES);
 #define DP_LAUNCH(QPG, TOGETHER)                                           \
   decode_pages_kernel<QPG, TOGETHER><<<grid, block, 0, stream>>>(          \
-      (float*)part_o, (float*)part_ml, (__hip_bfloat16*)out,               \
-      (const __hip_bfloat16*)q, (const __hip_bfloat16*)keys,               \
-      (const __hip_bfloat16*)values, (const int*)tables, (const int*)lens, \
-      scale * 1.44269504088896f, kv_heads, max_pages, span, whole,        \
-      q_stride,                                                            \
-      (int*)tickets)
+      (const int*)lens, kv_heads, seqs, splits, (const int*)tables,        \
+      max_pages, span, whole, (const __hip_bfloat16*)q, q_stride,          \
+      scale * 1.44269504088896f, (const __hip_bfloat16*)keys,              \
+      (const __hip_bfloat16*)values, (float*)part_o, (float*)part_ml,      \
+      (__hip_bfloat16*)out, (int*)tickets)
 #define DP_GO(QPG)                                                         \
   do {                                                                     \
     if (seqs >= 96) DP_LAUNCH(QPG, true);                                  \

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(512) void embed_rows_kernel(
       reinterpret_cast<const uint4*>(table + (there ? id : 0) * width);
   uint4* dst = reinterpret_cast<uint4*>(out + (size_t)blockIdx.x * width);
   const uint4 none = {0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};
-  for (int i = threadIdx.x; i < width / 8; i += blockDim.x)
+  for (int i = threadIdx.x; i < width / 8; i += 512)
     dst[i] = there ? src[i] : none;
 }
 

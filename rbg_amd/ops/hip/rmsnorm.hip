@@ -17,8 +17,8 @@ __global__ void rmsnorm_kernel(__hip_bfloat16* __restrict__ out,      // [T,H]
                                const float eps, const int hidden) {
   const int row = blockIdx.x;
   const int tid = threadIdx.x;
-  const int nthreads = blockDim.x;
-  __shared__ float red[8];   // up to 8 waves
+  constexpr int nthreads = 256;
+  __shared__ float red[nthreads / 64];
   __shared__ float s_inv;
 
   __hip_bfloat16* in_row = input + (size_t)row * hidden;
@@ -84,12 +84,12 @@ __global__ void rmsnorm_kernel(__hip_bfloat16* __restrict__ out,      // [T,H]
 // kernel above, 3.0 of this one, 4.1 from 8 parts).
 template <bool PARTS>
 __global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(
-    __hip_bfloat16* __restrict__ out, const void* __restrict__ src,
-    __hip_bfloat16* __restrict__ residual,
-    const __hip_bfloat16* __restrict__ w, const float eps, const int parts,
-    const int rows, const int hidden) {
+    const void* __restrict__ src, __hip_bfloat16* __restrict__ residual,
+    const int parts, const int rows, const int hidden, const int threads,
+    const __hip_bfloat16* __restrict__ w, __hip_bfloat16* __restrict__ out,
+    const float eps) {
   constexpr int MOST = 4;         // pieces of 4 per thread: hidden <= 16384
-  const int row = blockIdx.x, tid = threadIdx.x, threads = blockDim.x;
+  const int row = blockIdx.x, tid = threadIdx.x;
   const size_t at = (size_t)row * hidden;
   __shared__ float red[16];
   union B4 { uint2 u; __hip_bfloat16 e[4]; };
@@ -152,14 +152,13 @@ void launch_add_rmsnorm_rows(void* out, const void* src, void* residual,
                              const void* weight, float eps, int parts,
                              int rows, int hidden, hipStream_t stream) {
   const int threads = min(1024, (hidden / 4 + 63) / 64 * 64);
-  if (parts)
-    add_rmsnorm_row_kernel<true><<<dim3(rows), dim3(threads), 0, stream>>>(
-        (__hip_bfloat16*)out, src, (__hip_bfloat16*)residual,
-        (const __hip_bfloat16*)weight, eps, parts, rows, hidden);
-  else
-    add_rmsnorm_row_kernel<false><<<dim3(rows), dim3(threads), 0, stream>>>(
-        (__hip_bfloat16*)out, src, (__hip_bfloat16*)residual,
-        (const __hip_bfloat16*)weight, eps, parts, rows, hidden);
+  auto go = [&](auto kernel) {
+    kernel<<<dim3(rows), dim3(threads), 0, stream>>>(
+        src, (__hip_bfloat16*)residual, parts, rows, hidden, threads,
+        (const __hip_bfloat16*)weight, (__hip_bfloat16*)out, eps);
+  };
+  if (parts) go(add_rmsnorm_row_kernel<true>);
+  else go(add_rmsnorm_row_kernel<false>);
 }
 
 void launch_rmsnorm(void* out, void* input, const void* weight, float eps,

@@ -94,16 +94,16 @@ __global__ void rope_store_kv_kernel(
 // with: 16-byte accesses, and a norm is three shuffles.
 template <bool PARTS, bool NORM>
 __global__ __launch_bounds__(256) void rope_heads_kernel(
-    __hip_bfloat16* __restrict__ q, __hip_bfloat16* __restrict__ k,
-    __hip_bfloat16* __restrict__ v, const float* __restrict__ sums,
-    const int parts, const __hip_bfloat16* __restrict__ q_norm,
-    const __hip_bfloat16* __restrict__ k_norm, const float eps,
-    __hip_bfloat16* __restrict__ key_cache,  // [pages, KVH, page, 128]
-    __hip_bfloat16* __restrict__ val_cache,
+    const float* __restrict__ sums, __hip_bfloat16* __restrict__ q,
+    const int parts, const int tokens, const int num_q_heads,
+    const int num_kv_heads, const int* __restrict__ positions,
     const float* __restrict__ cos_sin,       // [positions, 128] = cos | sin
-    const int* __restrict__ positions, const int* __restrict__ slot_mapping,
-    const int tokens, const int num_q_heads, const int num_kv_heads,
-    const int page_size, const int q_stride, const int kv_stride) {
+    const int q_stride, const int kv_stride, __hip_bfloat16* __restrict__ k,
+    __hip_bfloat16* __restrict__ v, const __hip_bfloat16* __restrict__ q_norm,
+    const __hip_bfloat16* __restrict__ k_norm, const float eps,
+    const int* __restrict__ slot_mapping, const int page_size,
+    __hip_bfloat16* __restrict__ key_cache,  // [pages, KVH, page, 128]
+    __hip_bfloat16* __restrict__ val_cache) {
   constexpr int D = 128;
   const int heads = num_q_heads + 2 * num_kv_heads;
   const int unit = blockIdx.x * 32 + (threadIdx.x >> 3);
@@ -214,12 +214,12 @@ void launch_rope_heads(void* q, void* k, void* v, const void* sums, int parts,
   const dim3 grid((units + 31) / 32), block(256);
 #define RH_GO(PARTS, NORM)                                                  \
   rope_heads_kernel<PARTS, NORM><<<grid, block, 0, stream>>>(               \
-      (__hip_bfloat16*)q, (__hip_bfloat16*)k, (__hip_bfloat16*)v,           \
-      (const float*)sums, parts, (const __hip_bfloat16*)q_norm,             \
-      (const __hip_bfloat16*)k_norm, eps, (__hip_bfloat16*)key_cache,       \
-      (__hip_bfloat16*)val_cache, (const float*)cos_sin,                    \
-      (const int*)positions, (const int*)slot_mapping, tokens, num_q_heads, \
-      num_kv_heads, page_size, q_stride, kv_stride)
+      (const float*)sums, (__hip_bfloat16*)q, parts, tokens, num_q_heads,   \
+      num_kv_heads, (const int*)positions, (const float*)cos_sin, q_stride, \
+      kv_stride, (__hip_bfloat16*)k, (__hip_bfloat16*)v,                    \
+      (const __hip_bfloat16*)q_norm, (const __hip_bfloat16*)k_norm, eps,    \
+      (const int*)slot_mapping, page_size, (__hip_bfloat16*)key_cache,      \
+      (__hip_bfloat16*)val_cache)
   if (parts && q_norm) RH_GO(true, true);
   else if (parts) RH_GO(true, false);
   else if (q_norm) RH_GO(false, true);

@@ -8,9 +8,9 @@ namespace {
 __global__ void silu_mul_kernel(__hip_bfloat16* __restrict__ out,   // [T, I]
                                 const __hip_bfloat16* __restrict__ x,  // [T, 2I]
                                 const int inter, const long total_vec) {
-  const long stride = (long)gridDim.x * blockDim.x;
+  const long stride = (long)gridDim.x * 256;
   const int nvec_row = inter / 8;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < total_vec;
+  for (long i = blockIdx.x * 256l + threadIdx.x; i < total_vec;
        i += stride) {
     const long row = i / nvec_row;
     const int col = (int)(i % nvec_row) * 8;
@@ -34,7 +34,7 @@ __global__ void silu_parts_kernel(__hip_bfloat16* __restrict__ out,  // [T, I]
                                   const float* __restrict__ x,
                                   const int parts, const int inter,
                                   const long total_vec) {
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+  const long i = blockIdx.x * 256l + threadIdx.x;
   if (i >= total_vec) return;
   const int nvec_row = inter / 4;
   const long row = i / nvec_row;

@@ -36,9 +36,9 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
     const __hip_bfloat16* __restrict__ a,   // [M, K]
     const __hip_bfloat16* __restrict__ w,   // [N, K]
     __hip_bfloat16* __restrict__ c,         // [M, N], GLU: [M, N / 2]
-    float* __restrict__ ws,                 // [gridDim.y, M, N] if > 1, or C
+    float* __restrict__ ws,                 // [splits, M, N] if > 1, or C
                                             // in f32 if c is null
-    const int M, const int N, const int K) {
+    const int M, const int N, const int K, const int splits) {
   constexpr int THREADS = 64 * NW, PITCH = KC + 8;   // + 8: no bank conflicts
   constexpr int PER = THREADS * 8 / KC;     // rows of A that one load covers
   constexpr int PIECES = (MT * 16 + PER - 1) / PER, ROWS = PIECES * PER;
@@ -52,8 +52,8 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
   const int col0 = (blockIdx.x * SIDE + wave % SIDE) * 16;
   const int row = min(col0, half - 16) + r + (wave / SIDE) * half;
   const int chunks = K / KC;
-  const int c0 = chunks * blockIdx.y / gridDim.y;
-  const int n = chunks * (blockIdx.y + 1) / gridDim.y - c0;
+  const int c0 = chunks * blockIdx.y / splits;
+  const int n = chunks * (blockIdx.y + 1) / splits - c0;
   const int first = ((blockIdx.x >> 3) + (blockIdx.x & 7) * (n >> 3)) % n;
   const __hip_bfloat16* wp = w + (size_t)row * K + c0 * KC + g * 8;
   const __hip_bfloat16* ap[PIECES];
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
       for (int q = 0; q < 4; ++q) {
         const int m = i * 16 + g * 4 + q;
         if (m >= M) continue;
-        if (gridDim.y > 1)
+        if (splits > 1)
           ws[((size_t)blockIdx.y * M + m) * N + col0 + r] = acc[i][q];
         else if (c)
           c[(size_t)m * N + col0 + r] = f2bf(acc[i][q]);
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
 __global__ void reduce_splits_kernel(const float* __restrict__ ws,
                                      __hip_bfloat16* __restrict__ c,
                                      const int splits, const long mn) {
-  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= mn) return;
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
@@ -187,7 +187,7 @@ void launch_tiles(__hip_bfloat16* c, float* ws, const __hip_bfloat16* a,
   const int cols = NW * (GLU ? 8 : 16), out = GLU ? N / 2 : N;
   skinny_gemm_kernel<MT, NW, GLU>
       <<<dim3((out + cols - 1) / cols, splits), dim3(64 * NW), 0, stream>>>(
-          a, w, c, ws, M, N, K);
+          a, w, c, ws, M, N, K, splits);
 }
 
 }  // namespace

@@ -70,11 +70,14 @@ struct RowsRope {
 // waits for it.  A launch of its own takes 2.6 us.
 template <int END, bool NORM, bool PAIR>
 __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
-    const __hip_bfloat16* __restrict__ a,   // [M, K]; NORM: src, may be null
     const __hip_bfloat16* __restrict__ w,   // [N, K]
+    const __hip_bfloat16* __restrict__ a,   // [M, K]; NORM: src, may be null
+    const int K, const int N, const int M,
+    const __hip_bfloat16* __restrict__ residual,    // NORM: RowsNorm
+    const __hip_bfloat16* __restrict__ norm_weight,
+    __hip_bfloat16* __restrict__ residual_out, const float eps,
     __hip_bfloat16* __restrict__ c,         // [M, N], GLU: [M, N / 2]
     float* __restrict__ wide,               // PLAIN: not null: C in f32
-    const int M, const int N, const int K, const RowsNorm norm,
     const RowsRope rope) {
   static_assert(!PAIR || (END == ROWS_PLAIN && !NORM), "plain products only");
   constexpr int WAVES = 8, STEP = PAIR ? 2 * ROWS_KC : ROWS_KC;
@@ -131,12 +134,12 @@ __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
     float ss[ROWS_MOST] = {};
     for (int i = threadIdx.x * 8; i < K; i += 512 * 8) {
       Bf16x8U g8;
-      g8.u = *reinterpret_cast<const uint4*>(norm.weight + i);
+      g8.u = *reinterpret_cast<const uint4*>(norm_weight + i);
 #pragma unroll
       for (int m = 0; m < ROWS_MOST; ++m) {
         if (m >= M) break;
         Bf16x8U x, res, o;
-        res.u = *reinterpret_cast<const uint4*>(norm.residual +
+        res.u = *reinterpret_cast<const uint4*>(residual +
                                                 (size_t)m * K + i);
         if (a) {
           x.u = *reinterpret_cast<const uint4*>(a + (size_t)m * K + i);
@@ -147,7 +150,7 @@ __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
             res.e[j] = f2bf(t);
           }
           if (blockIdx.x == 0)
-            *reinterpret_cast<uint4*>(norm.residual_out + (size_t)m * K + i) =
+            *reinterpret_cast<uint4*>(residual_out + (size_t)m * K + i) =
                 res.u;
         } else {
 #pragma unroll
@@ -214,7 +217,7 @@ __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
     float total = 0.f;
 #pragma unroll
     for (int k = 0; k < WAVES; ++k) total += squares[k][m];
-    factor = rsqrtf(total / K + norm.eps);
+    factor = rsqrtf(total / K + eps);
   }
   v *= factor;
   v2 *= factor;
@@ -257,7 +260,8 @@ void launch_skinny_rows(__hip_bfloat16* c, const __hip_bfloat16* a,
   const size_t rows = NORM ? (size_t)M * K * 2 : 0;
   skinny_rows_kernel<END, NORM, PAIR>
       <<<dim3(N / (PAIR ? 8 : 16)), dim3(512), rows > sums ? rows : sums,
-         stream>>>(a, w, c, wide, M, N, K, norm, rope);
+         stream>>>(w, a, K, N, M, norm.residual, norm.weight,
+                   norm.residual_out, norm.eps, c, wide, rope);
 }
 
 }  // namespace

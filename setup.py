@@ -21,9 +21,12 @@ from rbg_amd.utils.hip_build import HIP_SOURCES  # noqa: E402
 
 HIP_DIR = os.path.join("rbg_amd", "ops", "hip")
 
-# no packed-f32 VALU instructions: some of their forms are unreliable here
+# No packed-f32 VALU instructions: some of their forms are unreliable here.
+# Kernel arguments come in registers with the launch, the first 14 words of them
+# (common.h).
 NVCC_ARGS = ["-O3", "-std=c++17", "--offload-arch=gfx950",
-             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+             "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
 only = [n for n in os.environ.get("RBG_BUILD_EXT", "").split(",") if n]
 ext_modules = [
