@@ -191,6 +191,14 @@ class LlamaAttention(nn.Module):
                     self.scale, plan, batch.kv_gather_slots)
                 if out is not None:
                     return out, residual
+        if batch.mode != "prefill":
+            o, residual = ops.norm_decode(
+                x, residual, norm, self.cfg.rms_eps, self.wqkv, self.heads,
+                self.q_norm, self.k_norm, key_cache, value_cache, cos_sin,
+                batch.positions, batch.slot_mapping, batch.block_tables,
+                batch.context_lens, self.scale,
+                num_splits=batch.decode_num_splits, tickets=batch.tickets)
+            return self._out(o, T), residual
         # (Qwen: per-head norms,) RoPE and the paged KV write in one kernel,
         # which also adds up what a split GEMM left
         qkv, residual = ops.norm_heads(
@@ -203,27 +211,23 @@ class LlamaAttention(nn.Module):
         k = qkv[:, self.q_out:self.q_out + self.kv_out]
         v = qkv[:, self.q_out + self.kv_out:]
         q3 = q.view(T, self.heads, self.head_dim)
-        if batch.mode == "prefill":
-            if batch.kv_gather_slots is not None:
-                # behind a past: all rows, the new ones too, from the pages
-                o = ops.prefill_attention(
-                    q3, key_cache, value_cache, batch.cu_seqlens, self.scale,
-                    batch.cu_seqlens_k, plan, batch.kv_gather_slots)
-            else:
-                o = ops.prefill_attention(
-                    q3, k.view(T, self.kv_heads, self.head_dim),
-                    v.view(T, self.kv_heads, self.head_dim),
-                    batch.cu_seqlens, self.scale, plan=plan)
+        if batch.kv_gather_slots is not None:
+            # behind a past: all rows, the new ones too, from the pages
+            o = ops.prefill_attention(
+                q3, key_cache, value_cache, batch.cu_seqlens, self.scale,
+                batch.cu_seqlens_k, plan, batch.kv_gather_slots)
         else:
-            o = ops.decode_attention(q3, key_cache, value_cache,
-                                     batch.block_tables, batch.context_lens,
-                                     self.scale,
-                                     num_splits=batch.decode_num_splits,
-                                     tickets=batch.tickets)
-        o = o.view(T, self.q_out).contiguous()
+            o = ops.prefill_attention(
+                q3, k.view(T, self.kv_heads, self.head_dim),
+                v.view(T, self.kv_heads, self.head_dim),
+                batch.cu_seqlens, self.scale, plan=plan)
+        return self._out(o, T), residual
+
+    def _out(self, o: torch.Tensor, rows: int) -> torch.Tensor:
+        o = o.view(rows, self.q_out).contiguous()
         if self.parts:
-            return ops.linear_parts(o, self.wo), residual
-        return self.tp.all_reduce(ops.linear(o, self.wo)), residual
+            return ops.linear_parts(o, self.wo)
+        return self.tp.all_reduce(ops.linear(o, self.wo))
 
 
 class LlamaMLP(nn.Module):

@@ -491,6 +491,25 @@ def _normed(src, residual, weight, eps: float) -> torch.Tensor:
     return add_rmsnorm(src, residual, weight, eps)
 
 
+def _norm_project(src, residual, weight, eps: float, w, heads: int, q_norm,
+                  *store):
+    """The projection by ``w`` of the RMS norm of residual + src, the new residual,
+    and whether the projection's heads are rotated and stored already."""
+    # every workgroup norms the rows: 384 of them repay that for up to 16384
+    # values (us, norm + GEMM + rotation against one launch: 6144 x 4096, 1 row
+    # 19.3 / 13.7, 4 rows 20.2 / 15.2; 10240 x 8192, 2 rows 41.0 / 38.3, 4 rows
+    # 42.3 / 44.6)
+    if (_takes_rows(src, residual, w) and residual.numel() <= 16384 and
+            store[0].shape[3] == 128):
+        mod = _require_hip()
+        if q_norm is None:
+            return *mod.norm_rows(src, residual, weight, eps, w, 2, heads,
+                                  *store), True
+        return *mod.norm_rows(src, residual, weight, eps, w, 0), False
+    proj = linear_parts(_normed(src, residual, weight, eps), w)
+    return proj, residual, False
+
+
 def norm_heads(src, residual, weight, eps: float, w, heads: int, q_norm,
                k_norm, key_cache, value_cache, cos_sin, positions,
                slot_mapping):
@@ -498,20 +517,29 @@ def norm_heads(src, residual, weight, eps: float, w, heads: int, q_norm,
     (src: linear_parts' result, or None).  Returns the projection in bf16 and
     the new residual, perhaps in the old one's memory."""
     store = (key_cache, value_cache, cos_sin, positions, slot_mapping)
-    # every workgroup norms the rows: 384 of them repay that for up to 16384
-    # values (us, norm + GEMM + rotation against one launch: 6144 x 4096, 1 row
-    # 19.3 / 13.7, 4 rows 20.2 / 15.2; 10240 x 8192, 2 rows 41.0 / 38.3, 4 rows
-    # 42.3 / 44.6)
-    if (_takes_rows(src, residual, w) and residual.numel() <= 16384 and
-            key_cache.shape[3] == 128):
-        mod = _require_hip()
-        if q_norm is None:
-            return mod.norm_rows(src, residual, weight, eps, w, 2, heads,
-                                 *store)
-        proj, residual = mod.norm_rows(src, residual, weight, eps, w, 0)
-    else:
-        proj = linear_parts(_normed(src, residual, weight, eps), w)
-    return rope_heads(proj, heads, q_norm, k_norm, eps, *store), residual
+    proj, residual, stored = _norm_project(src, residual, weight, eps, w, heads,
+                                           q_norm, *store)
+    if not stored:
+        proj = rope_heads(proj, heads, q_norm, k_norm, eps, *store)
+    return proj, residual
+
+
+def norm_decode(src, residual, weight, eps: float, w, heads: int, q_norm,
+                k_norm, key_cache, value_cache, cos_sin, positions,
+                slot_mapping, block_tables, context_lens, scale: float,
+                num_splits: int = 0, tickets=None):
+    """decode_attention of norm_heads' queries, and the new residual."""
+    store = (key_cache, value_cache, cos_sin, positions, slot_mapping)
+    proj, residual, stored = _norm_project(src, residual, weight, eps, w, heads,
+                                           q_norm, *store)
+    if not stored:
+        return decode_heads(proj, heads, q_norm, k_norm, eps, *store,
+                            block_tables, context_lens, scale, num_splits,
+                            tickets), residual
+    q = proj[:, :heads * 128].view(-1, heads, 128)
+    return decode_attention(q, key_cache, value_cache, block_tables,
+                            context_lens, scale, num_splits,
+                            tickets=tickets), residual
 
 
 def norm_swiglu(src, residual, weight, eps: float, w):
@@ -609,6 +637,34 @@ def decode_attention(q, key_cache, value_cache, block_tables, context_lens,
             _decode_span(q.shape[0] * key_cache.shape[1])[0], tickets)
     return reference.decode_attention(q, key_cache, value_cache, block_tables,
                                       context_lens, scale)
+
+
+def decode_heads(proj, heads: int, q_norm, k_norm, eps: float, key_cache,
+                 value_cache, cos_sin, positions, slot_mapping, block_tables,
+                 context_lens, scale: float, num_splits: int = 0,
+                 tickets=None) -> torch.Tensor:
+    """decode_attention of rope_heads of one new token of every sequence, which
+    context_lens count and whose slot no other sequence reads.  One launch where
+    the attention has the kernel for pages of 16 (the rotation's own: 3 us)."""
+    dim, kvh = key_cache.shape[3], key_cache.shape[1]
+    if (_on_gpu(proj) and DECODE_VARIANT == 7 and dim == 128 and
+            key_cache.shape[2] == 16 and heads % kvh == 0 and
+            heads // kvh in (1, 2, 4, 8) and proj.is_contiguous() and
+            key_cache.is_contiguous() and value_cache.is_contiguous() and
+            block_tables.is_contiguous()):
+        rows = proj.shape[-2]
+        if num_splits <= 0:
+            num_splits = pick_decode_splits(rows, kvh,
+                                            block_tables.shape[1] * 16)
+        return _require_hip().decode_heads(
+            proj, heads, q_norm, k_norm, eps, key_cache, value_cache, cos_sin,
+            positions, slot_mapping, block_tables, context_lens, scale,
+            num_splits, _decode_span(rows * kvh)[0], tickets)
+    qkv = rope_heads(proj, heads, q_norm, k_norm, eps, key_cache, value_cache,
+                     cos_sin, positions, slot_mapping)
+    q = qkv[:, :heads * dim].view(-1, heads, dim)
+    return decode_attention(q, key_cache, value_cache, block_tables,
+                            context_lens, scale, num_splits, tickets=tickets)
 
 
 @dataclass

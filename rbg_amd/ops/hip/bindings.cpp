@@ -8,6 +8,7 @@
 #include <cstring>
 #include <vector>
 
+#include "decode_heads.h"
 #include "gemm_bindings.h"
 #include "tile_bindings.h"
 
@@ -36,9 +37,10 @@ void launch_decode_attention(void*, void*, void*, const void*, const void*,
                              const void*, const void*, const void*, float,
                              int, int, int, int, int, int, int, int,
                              hipStream_t);
-void launch_decode_pages(void*, void*, void*, const void*, const void*,
-                         const void*, const void*, const void*, float, int,
-                         int, int, int, int, int, int, void*, hipStream_t);
+void launch_decode_pages(void*, void*, void*, const void*, void*, void*,
+                         const void*, const void*, float, int, int, int, int,
+                         int, int, int, void*, const DecodeHeads*,
+                         hipStream_t);
 void launch_place_inputs(void*, const void*, int, void*, const void*, int, int,
                          int, int, hipStream_t);
 void launch_prefill_attention(void*, const void*, const void*, const void*,
@@ -431,7 +433,7 @@ torch::Tensor decode_attention(torch::Tensor q, torch::Tensor key_cache,
                         (float)scale, num_seqs, num_q_heads, num_kv_heads,
                         max_pages, (int)num_splits, (int)span,
                         (int)q.stride(0),
-                        tickets ? tickets->data_ptr() : nullptr,
+                        tickets ? tickets->data_ptr() : nullptr, nullptr,
                         current_stream());
     return out;
   }
@@ -441,6 +443,89 @@ torch::Tensor decode_attention(torch::Tensor q, torch::Tensor key_cache,
                           (float)scale, num_seqs, num_q_heads, num_kv_heads,
                           page_size, max_pages, (int)num_splits, (int)wide,
                           (int)q.stride(0), current_stream());
+  return out;
+}
+
+// rope_heads of one row a sequence and decode_attention by form 7 on pages of 16,
+// in one launch.  lens count the new token, whose slot no other sequence reads.
+torch::Tensor decode_heads(torch::Tensor proj, int64_t heads,
+                           c10::optional<torch::Tensor> q_norm,
+                           c10::optional<torch::Tensor> k_norm, double eps,
+                           torch::Tensor key_cache, torch::Tensor value_cache,
+                           torch::Tensor cos_sin, torch::Tensor positions,
+                           torch::Tensor slots, torch::Tensor block_tables,
+                           torch::Tensor lens, double scale, int64_t splits,
+                           int64_t span,
+                           c10::optional<torch::Tensor> tickets) {
+  const bool parted = proj.scalar_type() == torch::kFloat32;
+  TORCH_CHECK(proj.is_cuda() && proj.is_contiguous() &&
+              (parted ? proj.dim() == 3 && proj.size(0) >= 1
+                      : proj.dim() == 2 &&
+                            proj.scalar_type() == torch::kBFloat16),
+              "projection must be bf16 rows or f32 parts of them");
+  check_bf16_contig(key_cache, "key_cache");
+  check_bf16_contig(value_cache, "value_cache");
+  const int64_t seqs = proj.size(-2), width = proj.size(-1);
+  const int64_t kv_heads = key_cache.size(1), pages = block_tables.size(1);
+  TORCH_CHECK(key_cache.dim() == 4 && key_cache.size(2) == 16 &&
+              key_cache.size(3) == 128 && key_cache.size(0) >= 1 &&
+              value_cache.sizes() == key_cache.sizes(),
+              "pages of 16 keys of 128");
+  TORCH_CHECK(kv_heads >= 1 && width == (heads + 2 * kv_heads) * 128 &&
+              heads % kv_heads == 0, "heads of 128, q | k | v");
+  const int64_t group = heads / kv_heads;
+  TORCH_CHECK(group == 1 || group == 2 || group == 4 || group == 8,
+              "GQA group must be 1/2/4/8");
+  TORCH_CHECK(cos_sin.is_cuda() && cos_sin.scalar_type() == torch::kFloat32 &&
+              cos_sin.is_contiguous() && cos_sin.dim() == 2 &&
+              cos_sin.size(1) == 128, "cos_sin must be fp32 [positions, 128]");
+  for (const auto& t : {positions, slots, lens})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.numel() == seqs &&
+                t.scalar_type() == torch::kInt32, "an int32 per sequence");
+  TORCH_CHECK(block_tables.is_cuda() && block_tables.is_contiguous() &&
+              block_tables.dim() == 2 && block_tables.size(0) == seqs &&
+              pages >= 1 && block_tables.scalar_type() == torch::kInt32,
+              "int32 page tables");
+  TORCH_CHECK(q_norm.has_value() == k_norm.has_value(), "both norms or none");
+  for (const auto& n : {q_norm, k_norm})
+    if (n.has_value()) {
+      check_bf16_contig(*n, "norm");
+      TORCH_CHECK(n->numel() == 128, "norms of 128");
+    }
+  TORCH_CHECK(splits >= 1 && splits < 65536 && seqs < 65536 && span >= 1 &&
+              seqs * width < (1ll << 31), "parts");
+  if (tickets)
+    TORCH_CHECK(tickets->is_cuda() && tickets->is_contiguous() &&
+                tickets->scalar_type() == torch::kInt32 &&
+                tickets->numel() >= seqs * kv_heads,
+                "an int32 ticket per sequence and key head");
+  auto opts = proj.options().dtype(torch::kFloat32);
+  auto out = torch::empty({seqs, heads, 128},
+                          proj.options().dtype(torch::kBFloat16));
+  if (seqs == 0) return out;
+  torch::Tensor sums;           // of every part, then maximum and sum of each row
+  float *po = nullptr, *pml = nullptr;
+  if (splits > 1) {
+    const int64_t rows = splits * seqs * heads;
+    sums = torch::empty({rows * 130}, opts);
+    po = sums.data_ptr<float>();
+    pml = po + rows * 128;
+  }
+  const auto norm = [](const c10::optional<torch::Tensor>& t) -> const void* {
+    return t ? t->data_ptr() : nullptr;
+  };
+  const DecodeHeads in{parted ? proj.data_ptr<float>() : nullptr,
+                       positions.data_ptr<int>(), slots.data_ptr<int>(),
+                       cos_sin.data_ptr<float>(), norm(q_norm), norm(k_norm),
+                       (float)eps, parted ? (int)proj.size(0) : 0};
+  launch_decode_pages(out.data_ptr(), po, pml,
+                      parted ? nullptr : proj.data_ptr(),
+                      key_cache.data_ptr(), value_cache.data_ptr(),
+                      block_tables.data_ptr(), lens.data_ptr(), (float)scale,
+                      (int)seqs, (int)heads, (int)kv_heads, (int)pages,
+                      (int)splits, (int)span, (int)width,
+                      tickets ? tickets->data_ptr() : nullptr, &in,
+                      current_stream());
   return out;
 }
 
@@ -816,6 +901,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("block_tables"), py::arg("context_lens"), py::arg("scale"),
         py::arg("num_splits"), py::arg("wide"), py::arg("span") = 128,
         py::arg("tickets") = c10::nullopt);
+  m.def("decode_heads", &decode_heads, "rope_heads and decode_attention");
   m.def("prompt_attention_block", &prompt_attention_block,
         "norm, attention and output product of prompts");
   m.def("swiglu_block", &swiglu_block, "norm and gated MLP of many rows");

@@ -27,6 +27,7 @@
 //    stand behind the barrier after the ticket.  (Release and acquire fences write
 //    back and invalidate whole caches: six layers of 3 sequences of up to 15000
 //    tokens 871 -> 1715 us, 45 of up to 2500 1125 -> 1934.)
+#include "decode_heads.h"
 #include "decode_join.h"
 
 namespace {
@@ -63,7 +64,14 @@ DEV_INLINE f32x2 dp_shared(const float* from) {
 // XCD i % 8, which then translates an eighth of the pool's addresses (128
 // sequences of 2080 tokens, 8 heads: 198 -> 179 us, 6.1 TB/s).  A small batch
 // of ragged lengths would leave XCDs idle (45 of up to 2500: 63 -> 68 us).
-template <int QPG, bool TOGETHER>
+// PROJ: the heads come as the projection left them.  Every workgroup adds up,
+// norms and rotates its own queries, on the way to LDS, while its keys are on
+// theirs; the one with a sequence's last key does the new key and value too, stores
+// them, and puts them in place of what registers already hold of that row.  The
+// rotation's own launch was 3 us of a layer (six layers, us: 7 sequences of qwen 8b
+// 715 -> 700, 45 of 8b 1109 -> 1097, 64 of qwen 32b, four layers, 1282 -> 1275, 128 of
+// 8b 2017 -> 2014).
+template <int QPG, bool TOGETHER, bool PROJ>
 __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     const int* __restrict__ lens,           // [seqs]
     const int kv_heads, const int seqs, const int splits,
@@ -71,12 +79,13 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     const int max_pages, const int least, const int whole,
     const __hip_bfloat16* __restrict__ q,   // [seqs, QH, DIM], rows q_stride
     const int q_stride, const float scale,  // to the base of 2
-    const __hip_bfloat16* __restrict__ keys,    // [pages, KVH, PAGE, DIM]
-    const __hip_bfloat16* __restrict__ values,
+    __hip_bfloat16* keys,                   // [pages, KVH, PAGE, DIM]
+    __hip_bfloat16* values,
     float* __restrict__ part_o,             // [splits, seqs, QH, DIM]
     float* __restrict__ part_ml,            // [splits, seqs, QH, 2]
     __hip_bfloat16* __restrict__ out,       // [seqs, QH, DIM]
-    int* __restrict__ tickets) {            // [seqs, KVH], or null
+    int* __restrict__ tickets,              // [seqs, KVH], or null
+    const DecodeHeads proj) {
   int kvh = blockIdx.x, seq = blockIdx.y, split = blockIdx.z;
   if (TOGETHER) {
     const int lin = kvh + kv_heads * (seq + seqs * split);
@@ -99,12 +108,13 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
 
   __shared__ __align__(16) __hip_bfloat16 v_lds[WAVES][8 * VROW];
   __shared__ float sums[WAVES][QPG][2];
+  __shared__ __align__(16) __hip_bfloat16 heads_lds[PROJ ? QPG + 2 : 1][DIM];
   static_assert(sizeof(v_lds) >= WAVES * QPG * DIM * 4 &&
                     sizeof(v_lds) >= 64 * WAVES * 6 * 4, "merges fit");
 
   // the heads' queries as columns (QPG of 16), 4 pieces of 32 dims
   bf16x8 qf[4];
-  {
+  if (!PROJ) {
     const __hip_bfloat16* qp = q + (size_t)seq * q_stride +
                                (size_t)(kvh * QPG + min(c, QPG - 1)) * DIM;
 #pragma unroll
@@ -144,13 +154,132 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
   }
   int at = begin + wave * STEP;
   int page[2];                    // of the next step, known one step ahead
-  if (at < end) {
-    page[0] = DP_PAGE(at, 0);
-    page[1] = DP_PAGE(at, 1);
+  int fresh = -1;                 // PROJ: the new key, where this workgroup has it
+  if (!PROJ) {
+    if (at < end) {
+      page[0] = DP_PAGE(at, 0);
+      page[1] = DP_PAGE(at, 1);
+      DP_KEYS(page)
+      DP_VALUES(page)
+      page[0] = DP_PAGE(at + WAVES * STEP, 0);
+      page[1] = DP_PAGE(at + WAVES * STEP, 1);
+    }
+  } else {
+    // a wave has a head at a time, a lane two dims that rotate into one another;
+    // the last key's workgroup has the new ones too, of no keys the first
+    constexpr int MINE = (QPG + 2 + WAVES - 1) / WAVES, ROUND = 8;
+    const bool keeps = end == ctx || ctx <= 0;
+    const int units = keeps ? QPG + 2 : QPG;
+    const int parts = proj.parts, slot = proj.slots[seq];
+    if (ctx > 0) {
+      page[0] = DP_PAGE(at, 0);
+      page[1] = DP_PAGE(at, 1);
+      if (keeps && slot == table[(ctx - 1) / PAGE] * PAGE + (ctx - 1) % PAGE)
+        fresh = ctx - 1;
+    } else {
+      page[0] = page[1] = 0;
+    }
+    const float* cs = proj.cos_sin + (size_t)proj.positions[seq] * DIM;
+    const float co = cs[lane], si = cs[lane + 64];
+    const size_t step = (size_t)seqs * q_stride;
+    uint32_t raw[MINE][ROUND][2];
+    size_t from[MINE];
+#define DP_PART(n, i, s)    /* past the last part: that one, to no use */    \
+  do {                                                                     \
+    const float* part =                                                    \
+        proj.sums + (min(s, parts - 1) * step + from[n]);          \
+    raw[n][i][0] = __float_as_uint(part[lane]);                            \
+    raw[n][i][1] = __float_as_uint(part[lane + 64]);                       \
+  } while (0)
+#pragma unroll
+    for (int n = 0; n < MINE; ++n) {
+      const int u = min(wave + n * WAVES, units - 1);
+      const int head = u < QPG ? kvh * QPG + u
+                               : heads + (u - QPG) * kv_heads + kvh;
+      from[n] = (size_t)seq * q_stride + head * DIM;
+      if (parts) {
+#pragma unroll
+        for (int i = 0; i < ROUND; ++i) DP_PART(n, i, i);
+      } else {
+        const unsigned short* p = (const unsigned short*)q + from[n];
+        raw[n][0][0] = p[lane];
+        raw[n][0][1] = p[lane + 64];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // without a condition, which the sums' wait would have to take for none
     DP_KEYS(page)
     DP_VALUES(page)
-    page[0] = DP_PAGE(at + WAVES * STEP, 0);
-    page[1] = DP_PAGE(at + WAVES * STEP, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (ctx > 0) {
+      page[0] = DP_PAGE(at + WAVES * STEP, 0);
+      page[1] = DP_PAGE(at + WAVES * STEP, 1);
+    }
+#pragma unroll
+    for (int n = 0; n < MINE; ++n) {
+      const int u = wave + n * WAVES;
+      if (u >= units) break;
+      float x[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        x[h] = 0.f;
+        if (parts == 0) x[h] = __uint_as_float(raw[n][0][h] << 16);
+#pragma unroll
+        for (int i = 0; i < ROUND; ++i)
+          if (i < parts) x[h] += __uint_as_float(raw[n][i][h]);
+      }
+      for (int s = ROUND; s < parts; s += 2) {
+        DP_PART(n, 0, s);
+        DP_PART(n, 1, s + 1);
+        x[0] += __uint_as_float(raw[n][0][0]);
+        x[1] += __uint_as_float(raw[n][0][1]);
+        if (s + 1 < parts) {
+          x[0] += __uint_as_float(raw[n][1][0]);
+          x[1] += __uint_as_float(raw[n][1][1]);
+        }
+      }
+      const __hip_bfloat16* nw =
+          (const __hip_bfloat16*)(u < QPG ? proj.q_norm : proj.k_norm);
+      if (nw && u <= QPG) {
+        const float inv =
+            rsqrtf(wave_sum(x[0] * x[0] + x[1] * x[1]) / DIM + proj.eps);
+        x[0] *= inv * bf2f(nw[lane]);
+        x[1] *= inv * bf2f(nw[lane + 64]);
+      }
+      const bool turns = u <= QPG;
+      const __hip_bfloat16 o1 = f2bf(turns ? x[0] * co - x[1] * si : x[0]);
+      const __hip_bfloat16 o2 = f2bf(turns ? x[1] * co + x[0] * si : x[1]);
+      heads_lds[u][lane] = o1;
+      heads_lds[u][lane + 64] = o2;
+      if (u >= QPG && slot >= 0) {
+        __hip_bfloat16* dst = (u == QPG ? keys : values) +
+                              (size_t)(slot / PAGE) * page_size + head_at +
+                              slot % PAGE * DIM + lane;
+        dst[0] = o1;
+        dst[64] = o2;
+      }
+    }
+#undef DP_PART
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+      qf[d] = dp_frag(dp_load(&heads_lds[min(c, QPG - 1)][d * 32 + g * 8]));
+    // A step that is asked for from here on has the new row from memory: it stands
+    // behind the barrier, and the waves of a workgroup share their CU's cache.
+    if (fresh >= 0) {
+      const int in = fresh % PAGE;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        // past the last page it is that one: weights of 0 meet its values too
+        if (min(at / PAGE + p, last_page) != fresh / PAGE) continue;
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          if (in == c) kr[p][d] = dp_load(&heads_lds[QPG][d * 32 + g * 8]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (in == j * 4 + g) vr[p][j] = dp_load(&heads_lds[QPG + 1][c * 8]);
+      }
+    }
   }
   for (; at < end; at += WAVES * STEP) {
     const int later[2] = {DP_PAGE(at + 2 * WAVES * STEP, 0),
@@ -369,11 +498,14 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
 
 }  // namespace
 
+// heads_in: null where q is as attention takes it; else q, or its sums, are rows of
+// q | k | v heads as the projection left them
 extern "C" void launch_decode_pages(
-    void* out, void* part_o, void* part_ml, const void* q, const void* keys,
-    const void* values, const void* tables, const void* lens, float scale,
+    void* out, void* part_o, void* part_ml, const void* q, void* keys,
+    void* values, const void* tables, const void* lens, float scale,
     int seqs, int heads, int kv_heads, int max_pages, int splits, int span,
-    int q_stride, void* tickets, hipStream_t stream) {
+    int q_stride, void* tickets, const DecodeHeads* heads_in,
+    hipStream_t stream) {
   // in whole rounds of the waves
   span = max(1, (span + PART_ROUND - 1) / PART_ROUND) * PART_ROUND;
   // Where pairs of sequence and key head fill the chip three times, no part of a
@@ -381,17 +513,20 @@ extern "C" void launch_decode_pages(
   // 96 of up to 2500 106 -> 101; 64 of up to 4000 143 -> 146, so not for fewer).
   const int whole = seqs * kv_heads >= 768 ? span + span / 4 : span;
   const dim3 grid(kv_heads, seqs, splits), block(64 * WAVES);
-#define DP_LAUNCH(QPG, TOGETHER)                                           \
-  decode_pages_kernel<QPG, TOGETHER><<<grid, block, 0, stream>>>(          \
+#define DP_LAUNCH(QPG, TOGETHER, PROJ)                                     \
+  decode_pages_kernel<QPG, TOGETHER, PROJ><<<grid, block, 0, stream>>>(    \
       (const int*)lens, kv_heads, seqs, splits, (const int*)tables,        \
       max_pages, span, whole, (const __hip_bfloat16*)q, q_stride,          \
-      scale * 1.44269504088896f, (const __hip_bfloat16*)keys,              \
-      (const __hip_bfloat16*)values, (float*)part_o, (float*)part_ml,      \
-      (__hip_bfloat16*)out, (int*)tickets)
+      scale * 1.44269504088896f, (__hip_bfloat16*)keys,                    \
+      (__hip_bfloat16*)values, (float*)part_o, (float*)part_ml,            \
+      (__hip_bfloat16*)out, (int*)tickets,                                 \
+      heads_in ? *heads_in : DecodeHeads{})
 #define DP_GO(QPG)                                                         \
   do {                                                                     \
-    if (seqs >= 96) DP_LAUNCH(QPG, true);                                  \
-    else DP_LAUNCH(QPG, false);                                            \
+    if (seqs >= 96 && heads_in) DP_LAUNCH(QPG, true, true);                \
+    else if (seqs >= 96) DP_LAUNCH(QPG, true, false);                      \
+    else if (heads_in) DP_LAUNCH(QPG, false, true);                        \
+    else DP_LAUNCH(QPG, false, false);                                     \
   } while (0)
   switch (heads / kv_heads) {
     case 1: DP_GO(1); break;

@@ -99,7 +99,7 @@ HIP_SOURCES = {
 }
 
 HIP_HEADERS = {
-    "_hip_ops": ["common.h", "decode_join.h", "gemm_bindings.h", "mfma_util.h",
+    "_hip_ops": ["common.h", "decode_heads.h", "decode_join.h", "gemm_bindings.h", "mfma_util.h",
                  "skinny_rows.h", "tile_bindings.h"],
     "_hip_mix": ["act.h", "act_kinds.h", "bind_util.h", "common.h",
                  "delta_scan.h", "embed_bindings.h", "gemm_bindings.h",

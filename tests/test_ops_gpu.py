@@ -988,6 +988,58 @@ def test_decode_parts_of_any_page(variant, page, splits):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,kvh,parts,norms", [
+    (8, 8, 0, False), (4, 2, 1, True), (32, 8, 5, False), (32, 8, 9, True),
+    (64, 8, 8, True), (16, 2, 13, False)])
+@pytest.mark.parametrize("splits,span,many", [(1, 256, 1), (5, 256, 1),
+                                              (17, 128, 1), (4, 512, 10)])
+def test_decode_takes_raw_heads(heads, kvh, parts, norms, splits, span, many):
+    """The rotation, the store and the attention in one launch as in two: new keys
+    in the first step of a wave and behind it, first, last and only ones of a part,
+    in a row that held no numbers; rows that are not stored, or elsewhere; no keys."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    lens = [1, 2, 17, 32, 33, 128, 129, 160, 255, 256, 257, 513, 2048, 2100, 700,
+            701, 5] * many
+    kc, vc, tables, ctx = _paged(dev, lens, kvh, 4096)
+    n, width = len(lens), (heads + 2 * kvh) * 128
+    at = (ctx - 1).long()
+    slots = (tables.gather(1, at[:, None] // 16)[:, 0] * 16 + at % 16).int()
+    for c in (kc, vc):
+        c[slots.long() // 16, :, slots.long() % 16] = math.nan
+    kc[slots[14] // 16, :, slots[14] % 16] = 0.5    # not stored: the old row counts
+    vc[slots[14] // 16, :, slots[14] % 16] = 0.25
+    slots[14] = -1
+    ctx[16] = 0                                     # stored, not read
+    gen = torch.Generator(device=dev).manual_seed(7)
+    proj = torch.randn(max(1, parts), n, width, device=dev, generator=gen)
+    if parts == 0:
+        proj = proj[0].bfloat16()
+    pos = torch.randint(0, 4096, (n,), device=dev, generator=gen).int()
+    table = ops.build_cos_sin_table(128, 4096, 10000.0, device=dev)
+    nw = [torch.randn(128, device=dev, generator=gen).bfloat16()
+          if norms else None for _ in range(2)]
+    other = [kc.clone(), vc.clone()]
+    qkv = ops.rope_heads(proj.clone(), heads, *nw, 1e-6, *other, table, pos, slots)
+    q = qkv[:, :heads * 128].view(n, heads, 128)
+    want = ops._hip.decode_attention(q, *other, tables, ctx, 0.09, splits, 7, span)
+    tickets = torch.zeros(n * kvh, dtype=torch.int32, device=dev)
+    for t in (None, tickets):
+        mine = [kc.clone(), vc.clone()]
+        got = ops._hip.decode_heads(proj, heads, *nw, 1e-6, *mine, table, pos,
+                                    slots, tables, ctx, 0.09, splits, span, t)
+        assert not tickets.any()
+        for a, b in zip(mine, other):
+            # the last bit of a value, for another order of a norm's sum
+            err = (a.float() - b.float()).abs()
+            assert (err.nan_to_num() <= b.float().abs().nan_to_num() * 2 ** -7
+                    ).all() and torch.equal(a.isnan(), b.isnan())
+        assert got.isfinite().all()
+        err = (got.float() - want.float()).norm() / want.float().norm()
+        assert err <= 2 ** -8       # of queries' and keys' last bits
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("splits", [1, 4, 12])
 @pytest.mark.parametrize("bad", [math.nan, math.inf])
 def test_decode_shows_broken_rows(splits, bad):
