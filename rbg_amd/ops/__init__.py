@@ -160,9 +160,29 @@ def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
                  (x.requires_grad or w.requires_grad)))
 
 
+def _stream(rows: int, n: int, k: int) -> bool:
+    """Does the GEMM of up to 4 rows (hip/stream_rows.hip) take a [rows, k] x [n, k]
+    product?  Of 268 of 1024 to 128256 columns and 1024 to 25600 k, 1 to 4 rows with
+    cold weights, it takes 0.84 of the time of what is taken without it, and of 10 of
+    them 0.2 to 3% more.  Not the widest of 2048 k, which the decode GEMM takes as one
+    turn (us, 1 row: 128256 x 2048 84.6 / 90.6, 65536 x 2048 44.9 / 46.3, 49152 x 2048
+    33.5 / 33.8, 65536 x 1024 27.4 / 22.5)."""
+    return (1 <= rows <= 4 and n >= 1024 and n % 32 == 0 and k >= 1024 and
+            k % 256 == 0 and (n <= 49152 or k > 2048 or k == 1024))
+
+
+def _takes_stream(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (SKINNY_GEMM and _hip is not None and _on_gpu(x) and x.dim() == 2 and
+            w.dim() == 2 and x.dtype == torch.bfloat16 and
+            w.dtype == torch.bfloat16 and x.shape[1] == w.shape[1] and
+            _stream(x.shape[0], w.shape[0], x.shape[1]) and _plain(x, w))
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """Projection GEMM: decode shapes take the hand-written kernel,
+    """Projection GEMM: decode shapes take the hand-written kernels,
     prefill-sized ones the library."""
+    if _takes_stream(x, w):
+        return _hip.stream_linear(x.contiguous(), w)
     if _takes_skinny(x, w):
         # one of these is there whatever the model
         return require("_hip_ops", "_hip_mix", "_hip_gated", "_hip_moe",
@@ -174,6 +194,8 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear(x, w).float(): the decode GEMM stores its rounded results so (a
     launch of 2 to 4 us less)."""
+    if _takes_stream(x, w):
+        return _hip.stream_linear(x.contiguous(), w, 1)
     if _takes_skinny(x, w):
         return require("_hip_ops", "_hip_mix", "_hip_gated", "_hip_moe",
                        "_hip_hyper").skinny_gemm(
@@ -234,8 +256,15 @@ def _takes_tile(x: torch.Tensor, w: torch.Tensor, rule) -> bool:
 
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """linear for a reader that adds up: where the GEMM splits k, the f32 sums
-    [parts, T, N] before their reduction, else [T, N] in x's dtype."""
+    """linear for a reader that adds up: where the GEMM splits k, or perhaps has few
+    rows, f32 sums [parts, T, N] before their reduction, else [T, N] in x's dtype."""
+    if _takes_stream(x, w):
+        # in bf16, which the next norm reads in half the time (3 sequences of up to
+        # 15000 tokens, six layers: 814 us, of sums 852), where the decode GEMM has
+        # them so; the others keep their f32
+        rows, k = x.shape
+        once = k % 2048 == 0 or rows <= 2 and k <= 8192 and w.shape[0] <= 12288
+        return _hip.stream_linear(x.contiguous(), w, 0 if once else 2)
     if x.shape[0] > 64 and _takes_tile(x, w, _tile):
         return _require_hip().tile_parts(x.contiguous(), w)
     if _takes_skinny(x, w, parts=True):
@@ -323,6 +352,8 @@ def _tile_glu(rows: int, n: int, k: int) -> bool:
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T), w = [Wg; Wu]."""
+    if _takes_stream(x, w):
+        return _hip.stream_swiglu(x.contiguous(), w)
     if x.shape[0] > 4 and _takes_tile(x, w, _tile_glu):
         return _require_hip().tile_swiglu(x.contiguous(), w)
     if (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
@@ -474,15 +505,19 @@ def rope_heads(proj, heads: int, q_norm, k_norm, eps: float, key_cache,
     return proj
 
 
-def _takes_rows(src, residual: torch.Tensor, w: torch.Tensor) -> bool:
-    """Can norm and GEMM be one launch (hip/skinny_rows.h)?  The shapes that its
-    kernel without a norm takes, in bf16 without parts, whose normed rows are at
-    most 64 KB, as every workgroup keeps them in LDS."""
-    return (_takes_skinny(residual, w) and residual.shape[0] <= 4 and
-            residual.numel() <= 32768 and
-            residual.shape[1] % 2048 == 0 and residual.is_contiguous() and
-            (src is None or (src.dtype == torch.bfloat16 and
-                             src.is_contiguous())))
+def _takes_rows(src, residual: torch.Tensor, weight: torch.Tensor,
+                w: torch.Tensor) -> bool:
+    """Can norm and GEMM of up to 4 rows be one launch (hip/stream_rows.hip)?  Its
+    waves hold an eighth of k of the rows, a sixteenth above 5120, in registers.  Of 184
+    shapes of 1536 to 12288 columns and 1024 to 8192 k it takes 0.76 of the time of what
+    was taken before, with silu of 4096 to 57344 columns 0.83 of 192; slower by 0.2 to
+    2.5% are ten of 6144 k, by 5% 8192 x 6144 of one row."""
+    return (_takes_stream(residual, w) and residual.shape[1] <= 8192 and
+            residual.is_contiguous() and weight.data_ptr() % 16 == 0 and
+            (src is None or (src.numel() == residual.numel() and
+                             src.dtype in (torch.bfloat16, torch.float32) and
+                             src.is_contiguous() and
+                             src.data_ptr() % 16 == 0)))
 
 
 def _normed(src, residual, weight, eps: float) -> torch.Tensor:
@@ -491,23 +526,12 @@ def _normed(src, residual, weight, eps: float) -> torch.Tensor:
     return add_rmsnorm(src, residual, weight, eps)
 
 
-def _norm_project(src, residual, weight, eps: float, w, heads: int, q_norm,
-                  *store):
-    """The projection by ``w`` of the RMS norm of residual + src, the new residual,
-    and whether the projection's heads are rotated and stored already."""
-    # every workgroup norms the rows: 384 of them repay that for up to 16384
-    # values (us, norm + GEMM + rotation against one launch: 6144 x 4096, 1 row
-    # 19.3 / 13.7, 4 rows 20.2 / 15.2; 10240 x 8192, 2 rows 41.0 / 38.3, 4 rows
-    # 42.3 / 44.6)
-    if (_takes_rows(src, residual, w) and residual.numel() <= 16384 and
-            store[0].shape[3] == 128):
-        mod = _require_hip()
-        if q_norm is None:
-            return *mod.norm_rows(src, residual, weight, eps, w, 2, heads,
-                                  *store), True
-        return *mod.norm_rows(src, residual, weight, eps, w, 0), False
-    proj = linear_parts(_normed(src, residual, weight, eps), w)
-    return proj, residual, False
+def _norm_project(src, residual, weight, eps: float, w):
+    """The projection by ``w`` of the RMS norm of residual + src, and the new
+    residual, perhaps in the old one's memory."""
+    if _takes_rows(src, residual, weight, w):
+        return _require_hip().norm_rows(src, residual, weight, eps, w, 2)
+    return linear_parts(_normed(src, residual, weight, eps), w), residual
 
 
 def norm_heads(src, residual, weight, eps: float, w, heads: int, q_norm,
@@ -516,12 +540,9 @@ def norm_heads(src, residual, weight, eps: float, w, heads: int, q_norm,
     """rope_heads of the projection by ``w`` of the RMS norm of residual + src
     (src: linear_parts' result, or None).  Returns the projection in bf16 and
     the new residual, perhaps in the old one's memory."""
-    store = (key_cache, value_cache, cos_sin, positions, slot_mapping)
-    proj, residual, stored = _norm_project(src, residual, weight, eps, w, heads,
-                                           q_norm, *store)
-    if not stored:
-        proj = rope_heads(proj, heads, q_norm, k_norm, eps, *store)
-    return proj, residual
+    proj, residual = _norm_project(src, residual, weight, eps, w)
+    return rope_heads(proj, heads, q_norm, k_norm, eps, key_cache, value_cache,
+                      cos_sin, positions, slot_mapping), residual
 
 
 def norm_decode(src, residual, weight, eps: float, w, heads: int, q_norm,
@@ -529,25 +550,21 @@ def norm_decode(src, residual, weight, eps: float, w, heads: int, q_norm,
                 slot_mapping, block_tables, context_lens, scale: float,
                 num_splits: int = 0, tickets=None):
     """decode_attention of norm_heads' queries, and the new residual."""
-    store = (key_cache, value_cache, cos_sin, positions, slot_mapping)
-    proj, residual, stored = _norm_project(src, residual, weight, eps, w, heads,
-                                           q_norm, *store)
-    if not stored:
-        return decode_heads(proj, heads, q_norm, k_norm, eps, *store,
-                            block_tables, context_lens, scale, num_splits,
-                            tickets), residual
-    q = proj[:, :heads * 128].view(-1, heads, 128)
-    return decode_attention(q, key_cache, value_cache, block_tables,
-                            context_lens, scale, num_splits,
-                            tickets=tickets), residual
+    proj, residual = _norm_project(src, residual, weight, eps, w)
+    return decode_heads(proj, heads, q_norm, k_norm, eps, key_cache,
+                        value_cache, cos_sin, positions, slot_mapping,
+                        block_tables, context_lens, scale, num_splits,
+                        tickets), residual
 
 
 def norm_swiglu(src, residual, weight, eps: float, w):
     """linear_swiglu of the RMS norm of residual + src, and the new residual."""
-    # 1792 workgroups repay it for one row only (28672 x 4096: 1 row 45.2 / 43.3,
-    # 2 rows 44.0 / 47.2)
-    if (_takes_rows(src, residual, w) and residual.shape[0] == 1 and
-            w.shape[0] % 64 == 0):
+    # of more rows than one where the norm does not cost more than its launch
+    # (hip/stream_rows.hip launch_norm_rows)
+    rows, k = residual.shape
+    if _takes_rows(src, residual, weight, w) and (
+            rows == 1 or (src is None or src.dtype == torch.bfloat16) and
+            (rows == 2 or k <= 4096)):
         return _require_hip().norm_rows(src, residual, weight, eps, w, 1)
     return linear_swiglu(_normed(src, residual, weight, eps), w), residual
 

@@ -22,10 +22,6 @@ void launch_rope_heads(void*, void*, void*, const void*, int, const void*,
                        const void*, float, void*, void*, const void*,
                        const void*, const void*, int, int, int, int, int, int,
                        hipStream_t);
-void launch_norm_rows(void*, const void*, const void*, void*, const void*,
-                      float, const void*, int, int, int, int, const void*,
-                      const void*, const void*, void*, void*, int, int, int,
-                      hipStream_t);
 void launch_embed_rows(void*, const void*, const void*, long, int, int,
                        hipStream_t);
 void launch_silu_parts(void*, const void*, int, int, int, hipStream_t);
@@ -41,6 +37,11 @@ void launch_decode_pages(void*, void*, void*, const void*, void*, void*,
                          const void*, const void*, float, int, int, int, int,
                          int, int, int, void*, const DecodeHeads*,
                          hipStream_t);
+bool launch_norm_rows(void*, void*, const void*, int, const void*, void*,
+                      const void*, float, const void*, int, int, int, int,
+                      hipStream_t);
+bool launch_stream_rows(void*, void*, int, const void*, const void*, int, int,
+                        int, int, hipStream_t);
 void launch_place_inputs(void*, const void*, int, void*, const void*, int, int,
                          int, int, hipStream_t);
 void launch_prefill_attention(void*, const void*, const void*, const void*,
@@ -307,59 +308,74 @@ torch::Tensor rope_heads(torch::Tensor proj, int64_t num_q_heads,
   return out;
 }
 
-// Up to 4 rows: the RMS norm of residual + src (src may be missing), a GEMM and
-// its end in one launch: nothing (0), silu(gate) * up (1), or rotation and
-// paged store of fused heads (2, as rope_heads).  Returns the product and the
-// new residual, which is another tensor unless src is missing.
-std::vector<torch::Tensor> norm_rows(
-    c10::optional<torch::Tensor> src, torch::Tensor residual,
-    torch::Tensor norm_weight, double eps, torch::Tensor w, int64_t end,
-    int64_t heads, c10::optional<torch::Tensor> key_cache,
-    c10::optional<torch::Tensor> value_cache,
-    c10::optional<torch::Tensor> cos_sin,
-    c10::optional<torch::Tensor> positions,
-    c10::optional<torch::Tensor> slots) {
+// silu(a Wg^T) * (a Wu^T) of up to 4 rows, w = [Wg; Wu]
+torch::Tensor stream_swiglu(torch::Tensor a, torch::Tensor w) {
+  check_skinny(a, w);
+  const int64_t M = a.size(0), K = a.size(1), N = w.size(0);
+  auto c = torch::empty({M, N / 2}, a.options());
+  TORCH_CHECK(launch_stream_rows(c.data_ptr(), nullptr, 0, a.data_ptr(),
+                                 w.data_ptr(), (int)M, (int)N, (int)K, 1,
+                                 current_stream()),
+              "at most 4 rows");
+  return c;
+}
+
+// Up to 4 rows: the RMS norm of residual + src (bf16, or f32 sums [1, M, K] of
+// stream_linear; it may be missing), a GEMM and its end in one launch: the product in
+// bf16 (0), silu(gate) * up (1; perhaps behind a launch of the norm's own), or the
+// product's f32 sums [1, M, N] (2).  Returns that and the new residual, which is another tensor unless src is missing.
+std::vector<torch::Tensor> norm_rows(c10::optional<torch::Tensor> src,
+                                     torch::Tensor residual,
+                                     torch::Tensor norm_weight, double eps,
+                                     torch::Tensor w, int64_t end) {
   check_skinny(residual, w);
   check_bf16_contig(norm_weight, "norm weight");
   const int64_t M = residual.size(0), K = residual.size(1), N = w.size(0);
-  TORCH_CHECK(M <= 4 && M * K <= 32768, "at most 4 rows, 64 KB of them");
   TORCH_CHECK(norm_weight.numel() == K, "norm weight of K");
   TORCH_CHECK(end >= 0 && end <= 2, "unknown end");
-  if (src.has_value()) {
-    check_bf16_contig(*src, "src");
-    TORCH_CHECK(src->sizes() == residual.sizes(), "src like residual");
+  const bool sums = src && src->scalar_type() == torch::kFloat32;
+  if (src) {
+    TORCH_CHECK(src->is_cuda() && src->is_contiguous() &&
+                src->numel() == residual.numel() && src->size(-1) == K &&
+                (sums || src->scalar_type() == torch::kBFloat16),
+                "src like residual, or f32 sums");
   }
-  int64_t kv_heads = 0, page_size = 1;
-  if (end == 2) {
-    TORCH_CHECK(key_cache && value_cache && cos_sin && positions && slots,
-                "the rotation's inputs");
-    check_bf16_contig(*key_cache, "key_cache");
-    check_bf16_contig(*value_cache, "value_cache");
-    kv_heads = key_cache->size(1);
-    page_size = key_cache->size(2);
-    TORCH_CHECK(key_cache->size(3) == 128 &&
-                value_cache->sizes() == key_cache->sizes() &&
-                N == (heads + 2 * kv_heads) * 128, "heads of 128, q | k | v");
-    TORCH_CHECK(cos_sin->scalar_type() == torch::kFloat32 &&
-                cos_sin->is_contiguous() && cos_sin->size(1) == 128,
-                "cos_sin must be fp32 [positions, 128]");
-    for (const auto& t : {*positions, *slots})
-      TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kInt32 &&
-                  t.is_contiguous() && t.numel() == M,
-                  "an int32 position and slot per row");
+  if (end == 1 && M > 1 && (sums || (M > 2 && K > 4096))) {
+    auto next = src ? residual.clone() : residual;
+    return {stream_swiglu(src ? add_rmsnorm(*src, next, norm_weight, eps)
+                              : rmsnorm(residual, norm_weight, eps), w),
+            next};
   }
-  auto out = torch::empty({M, end == 1 ? N / 2 : N}, residual.options());
+  const auto f32 = residual.options().dtype(torch::kFloat32);
+  auto out = end == 2 ? torch::empty({1, M, N}, f32)
+                      : torch::empty({M, end == 1 ? N / 2 : N},
+                                     residual.options());
   auto next = src ? torch::empty_like(residual) : residual;
-  const auto ptr = [](const c10::optional<torch::Tensor>& t) -> void* {
-    return t ? t->data_ptr() : nullptr;
-  };
-  launch_norm_rows(out.data_ptr(), ptr(src), residual.data_ptr(),
-                   next.data_ptr(), norm_weight.data_ptr(), (float)eps,
-                   w.data_ptr(), (int)M, (int)N, (int)K, (int)end,
-                   ptr(cos_sin), ptr(positions), ptr(slots), ptr(key_cache),
-                   ptr(value_cache), (int)heads, (int)kv_heads,
-                   (int)page_size, current_stream());
+  TORCH_CHECK(launch_norm_rows(end == 2 ? nullptr : out.data_ptr(),
+                               end == 2 ? out.data_ptr() : nullptr,
+                               src ? src->data_ptr() : nullptr, sums,
+                               residual.data_ptr(), next.data_ptr(),
+                               norm_weight.data_ptr(), (float)eps, w.data_ptr(),
+                               (int)M, (int)N, (int)K, end == 1,
+                               current_stream()),
+              "at most 4 rows of 1024 to 8192");
   return {out, next};
+}
+
+// a W^T of up to 4 rows, in bf16 (0), in bf16's values as f32 (1), or its f32 sums as
+// one part [1, M, N] (2)
+torch::Tensor stream_linear(torch::Tensor a, torch::Tensor w, int64_t end) {
+  check_skinny(a, w);
+  const int64_t M = a.size(0), K = a.size(1), N = w.size(0);
+  TORCH_CHECK(end >= 0 && end <= 2, "unknown end");
+  auto c = torch::empty({M, N}, end ? a.options().dtype(torch::kFloat32)
+                                    : a.options());
+  TORCH_CHECK(launch_stream_rows(end ? nullptr : c.data_ptr(),
+                                 end ? c.data_ptr() : nullptr, end == 1,
+                                 a.data_ptr(), w.data_ptr(), (int)M, (int)N,
+                                 (int)K, 0, current_stream()),
+              "at most 4 rows");
+  return end == 2 ? c.unsqueeze(0) : c;
 }
 
 // fields and tables [rows, width]: a captured step's inputs, from new ones, whose
@@ -923,13 +939,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_swiglu", &tile_swiglu, "gate/up GEMM of a prompt with silu");
   m.def("tile_parts", &tile_parts, "GEMM of a prompt, perhaps as parts' sums");
   m.def("tile_form", &tile_form, "one form of these");
-  m.def("norm_rows", &norm_rows, "norm, GEMM of a few rows and its end",
-        py::arg("src"), py::arg("residual"), py::arg("norm_weight"),
-        py::arg("eps"), py::arg("w"), py::arg("end"), py::arg("heads") = 0,
-        py::arg("key_cache") = c10::nullopt,
-        py::arg("value_cache") = c10::nullopt,
-        py::arg("cos_sin") = c10::nullopt, py::arg("positions") = c10::nullopt,
-        py::arg("slots") = c10::nullopt);
+  m.def("norm_rows", &norm_rows, "norm, GEMM of a few rows and its end");
+  m.def("stream_swiglu", &stream_swiglu, "gate/up GEMM of a few rows with silu");
+  m.def("stream_linear", &stream_linear, "GEMM of a few rows",
+        py::arg("a"), py::arg("w"), py::arg("end") = 0);
   m.def("add_rmsnorm", &add_rmsnorm, "residual += x; its RMS norm");
   m.def("rope_heads", &rope_heads, "head norms, RoPE, paged store");
   // gil_scoped_release on the IPC/copy entry points: mapping or launching

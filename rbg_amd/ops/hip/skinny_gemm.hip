@@ -217,14 +217,14 @@ extern "C" void launch_skinny_gemm(void* c, void* ws, const void* a,
   launch_tiles<MT, 4, true>(cp, wsp, ap, wp, M, N, K, 1, stream)
   if (waves == 0) {             // the kernel of a few rows
     if (glu)
-      launch_skinny_rows<ROWS_GLU, false>(cp, ap, wp, M, N, K, {}, {}, stream);
+      launch_skinny_rows<true>(cp, ap, wp, M, N, K, stream);
     else if ((N <= 2048 && K >= 4096) ||
              (M == 1 && N > 4096 && N <= 6144 && K >= 8192))
-      launch_skinny_rows<ROWS_PLAIN, false, true>(cp, ap, wp, M, N, K, {}, {},
-                                                  stream, cp ? nullptr : wsp);
+      launch_skinny_rows<false, true>(cp, ap, wp, M, N, K, stream,
+                                      cp ? nullptr : wsp);
     else
-      launch_skinny_rows<ROWS_PLAIN, false>(cp, ap, wp, M, N, K, {}, {},
-                                            stream, cp ? nullptr : wsp);
+      launch_skinny_rows<false>(cp, ap, wp, M, N, K, stream,
+                                cp ? nullptr : wsp);
   } else if (mt <= 1 && waves == 4) SG_GO(1, 4);
   else if (mt <= 2 && waves == 4) SG_GO(2, 4);
   else if (mt <= 1) SG_GO(1, 8);

@@ -1,5 +1,4 @@
-// Decode GEMM of a few rows, C[M,N] = A[M,K] x W[N,K]^T, M <= 4, with what
-// stands before and after it in a layer.
+// Decode GEMM of a few rows, C[M,N] = A[M,K] x W[N,K]^T, M <= 4.
 #pragma once
 #include "common.h"
 
@@ -27,79 +26,37 @@ DEV_INLINE int sg_turn(int c, int first, int n) {
 
 constexpr int ROWS_KC = 64, ROWS_DEPTH = 4, ROWS_MOST = 4;
 
-// what becomes of the product
-enum RowsEnd {
-  ROWS_PLAIN,     // C
-  ROWS_GLU,       // W's halves are gate and up: silu(gate) * up, [M, N / 2]
-  ROWS_ROPE,      // C = q | k | v heads of 128: q and k rotated, k and v also
-                  // to the pages
-};
-
-// A = RMS norm of src + residual, which is written to residual_out
-struct RowsNorm {
-  const __hip_bfloat16* residual;       // [M, K]
-  const __hip_bfloat16* weight;         // [K]
-  __hip_bfloat16* residual_out;         // not residual: others still read it
-  float eps;
-};
-
-struct RowsRope {
-  const float* cos_sin;                 // [positions, 128] = cos | sin
-  const int* positions;                 // [M]
-  const int* slots;                     // [M], -1: not stored
-  __hip_bfloat16* keys;                 // [pages, KVH, page_size, 128]
-  __hip_bfloat16* values;
-  int heads, kv_heads, page_size;
-};
-
 // 8 waves share one 16-row tile of W and take its K in turns, without a
 // barrier until their sums meet in LDS, and without splits whose sums another
 // launch would add.  4096 x 4096, one row: 8.5 us against 10.5 of
 // skinny_gemm_kernel with its reduction.  Its time grows with the rows, since
 // every workgroup reads all of A (28672 x 4096: 1 row 41.8 us, 4 rows 44.3).
-// GLU and ROPE: the tile is 8 rows of W and the 8 that they meet, N / 2 or 64
-// further on.
+// GLU: W's halves are gate and up, the tile is 8 rows of each: silu(gate) * up.
 // PAIR: the tile is 8 rows of W, whose k are taken two chunks at a time, so that
 // twice as many workgroups are half as long.  For matrices whose tiles of 16 rows
 // leave half of the chip or more idle, with long k (1 row: 1024 x 4096 8.0 -> 6.1
 // us, 2048 x 5632 10.6 -> 9.8, x 14336 19.6 -> 15.8, x 2048 6.1 -> 6.5; 4 rows: 2048
 // x 4096 8.9 -> 8.4), and where they fill it one and a half times (1 row of 5120 x
 // 8192 24.1 -> 19.5, of 6144 x 25600 69 -> 58; 4 rows 25.4 -> 25.1, 74 -> 78).
-// NORM: every workgroup forms A for itself, in LDS, while its first weights are
-// on their way; the row's 1 / rms is a factor of the result, so that nothing
-// waits for it.  A launch of its own takes 2.6 us.
-template <int END, bool NORM, bool PAIR>
+template <bool GLU, bool PAIR>
 __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
     const __hip_bfloat16* __restrict__ w,   // [N, K]
-    const __hip_bfloat16* __restrict__ a,   // [M, K]; NORM: src, may be null
+    const __hip_bfloat16* __restrict__ a,   // [M, K]
     const int K, const int N, const int M,
-    const __hip_bfloat16* __restrict__ residual,    // NORM: RowsNorm
-    const __hip_bfloat16* __restrict__ norm_weight,
-    __hip_bfloat16* __restrict__ residual_out, const float eps,
     __hip_bfloat16* __restrict__ c,         // [M, N], GLU: [M, N / 2]
-    float* __restrict__ wide,               // PLAIN: not null: C in f32
-    const RowsRope rope) {
-  static_assert(!PAIR || (END == ROWS_PLAIN && !NORM), "plain products only");
+    float* __restrict__ wide) {             // not null: C in f32, not GLU
+  static_assert(!PAIR || !GLU, "plain products only");
   constexpr int WAVES = 8, STEP = PAIR ? 2 * ROWS_KC : ROWS_KC;
-  extern __shared__ __align__(16) char rows_lds[];
-  __shared__ float squares[WAVES][ROWS_MOST];
-  __hip_bfloat16* al = (__hip_bfloat16*)rows_lds;         // NORM: [M, K]
+  __shared__ __align__(16) float red[WAVES * 16 * ROWS_MOST];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
-  const int apart = END == ROWS_GLU ? N / 2 : 64;
-  const int col0 = PAIR ? blockIdx.x * 8
-                   : END == ROWS_PLAIN ? blockIdx.x * 16
-                   : END == ROWS_GLU ? blockIdx.x * 8
-                                     : (blockIdx.x >> 3) * 128 +
-                                           (blockIdx.x & 7) * 8;
+  const int col0 = blockIdx.x * (PAIR || GLU ? 8 : 16);
   const int row = PAIR ? col0 + (r & 7)
-                  : END == ROWS_PLAIN ? col0 + r
-                                      : col0 + (r & 7) + (r >> 3) * apart;
+                  : GLU ? col0 + (r & 7) + (r >> 3) * (N / 2) : col0 + r;
   // PAIR: W's second 8 rows and A's second 4 stand for the first ones' next k
   const __hip_bfloat16* wp = w + (size_t)row * K + wave * STEP + g * 8 +
                              (PAIR ? (r >> 3) * ROWS_KC : 0);
-  const __hip_bfloat16* ap = (NORM ? al : a) +
-                             (size_t)min(PAIR ? r & 3 : r, M - 1) * K +
+  const __hip_bfloat16* ap = a + (size_t)min(PAIR ? r & 3 : r, M - 1) * K +
                              wave * STEP + g * 8 +
                              (PAIR ? (r >> 2 & 1) * ROWS_KC : 0);
   const int n = (K / STEP - wave + WAVES - 1) / WAVES;
@@ -129,50 +86,6 @@ __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
 #pragma unroll
     for (int s = 0; s < ROWS_DEPTH; ++s) SR_WEIGHTS(s, min(s, n - 1));
   }
-  if (NORM) {
-    __builtin_amdgcn_sched_barrier(0);
-    float ss[ROWS_MOST] = {};
-    for (int i = threadIdx.x * 8; i < K; i += 512 * 8) {
-      Bf16x8U g8;
-      g8.u = *reinterpret_cast<const uint4*>(norm_weight + i);
-#pragma unroll
-      for (int m = 0; m < ROWS_MOST; ++m) {
-        if (m >= M) break;
-        Bf16x8U x, res, o;
-        res.u = *reinterpret_cast<const uint4*>(residual +
-                                                (size_t)m * K + i);
-        if (a) {
-          x.u = *reinterpret_cast<const uint4*>(a + (size_t)m * K + i);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float t = bf2f(x.e[j]) + bf2f(res.e[j]);
-            ss[m] += t * t;
-            res.e[j] = f2bf(t);
-          }
-          if (blockIdx.x == 0)
-            *reinterpret_cast<uint4*>(residual_out + (size_t)m * K + i) =
-                res.u;
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float t = bf2f(res.e[j]);
-            ss[m] += t * t;
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          o.e[j] = f2bf(bf2f(res.e[j]) * bf2f(g8.e[j]));
-        *reinterpret_cast<uint4*>(al + (size_t)m * K + i) = o.u;
-      }
-    }
-#pragma unroll
-    for (int m = 0; m < ROWS_MOST; ++m) {
-      if (m >= M) break;
-      ss[m] = wave_sum(ss[m]);
-      if (lane == 0) squares[wave][m] = ss[m];
-    }
-    __syncthreads();
-  }
   if (n > 0) {
 #pragma unroll
     for (int s = 0; s < ROWS_DEPTH; ++s) SR_ROWS(s, min(s, n - 1));
@@ -196,72 +109,32 @@ __global__ __launch_bounds__(512, 2) void skinny_rows_kernel(
 
   // lane l, register q: row 4 * (l >> 4) + q of A, row l & 15 of the tile; only
   // the first ROWS_MOST rows are there, the first 16 lanes'
-  if (NORM) __syncthreads();                // A is read
-  float* red = (float*)rows_lds;            // [WAVES][16 columns][ROWS_MOST]
   if (PAIR ? g == r >> 3 : g == 0)
     *reinterpret_cast<f32x4*>(red + (wave * 16 + r) * ROWS_MOST) = acc;
   __syncthreads();
   const int e = threadIdx.x;
   if (e >= 16 * ROWS_MOST) return;
   const int col = e / ROWS_MOST, m = e % ROWS_MOST;
-  if (m >= M || ((PAIR || END != ROWS_PLAIN) && col >= 8)) return;
-  float v = 0.f, v2 = 0.f, factor = 1.f;
+  if (m >= M || ((PAIR || GLU) && col >= 8)) return;
+  float v = 0.f, v2 = 0.f;
 #pragma unroll
   for (int k = 0; k < WAVES; ++k) {
     v += red[k * 16 * ROWS_MOST + e];
-    if (PAIR || END != ROWS_PLAIN)
-      v2 += red[k * 16 * ROWS_MOST + e + 8 * ROWS_MOST];
+    if (PAIR || GLU) v2 += red[k * 16 * ROWS_MOST + e + 8 * ROWS_MOST];
   }
   if (PAIR) v += v2;
-  if (NORM) {
-    float total = 0.f;
-#pragma unroll
-    for (int k = 0; k < WAVES; ++k) total += squares[k][m];
-    factor = rsqrtf(total / K + eps);
-  }
-  v *= factor;
-  v2 *= factor;
-  if (END == ROWS_PLAIN) {
-    if (wide) wide[(size_t)m * N + col0 + col] = bf2f(f2bf(v));
-    else c[(size_t)m * N + col0 + col] = f2bf(v);
-  } else if (END == ROWS_GLU) {
-    c[(size_t)m * (N / 2) + col0 + col] = f2bf(silu(v) * v2);
-  } else {
-    const int head = col0 / 128, d = col0 % 128 + col;
-    const bool is_v = head >= rope.heads + rope.kv_heads;
-    if (!is_v) {
-      const float* cs = rope.cos_sin + (size_t)rope.positions[m] * 128 + d;
-      const float co = cs[0], si = cs[64], x1 = v, x2 = v2;
-      v = x1 * co - x2 * si;
-      v2 = x2 * co + x1 * si;
-    }
-    const __hip_bfloat16 o1 = f2bf(v), o2 = f2bf(v2);
-    c[(size_t)m * N + col0 + col] = o1;
-    c[(size_t)m * N + col0 + col + 64] = o2;
-    const int kvh = head - rope.heads - (is_v ? rope.kv_heads : 0);
-    const int slot = rope.slots[m];
-    if (kvh >= 0 && slot >= 0) {
-      __hip_bfloat16* dst =
-          (is_v ? rope.values : rope.keys) +
-          (((size_t)(slot / rope.page_size) * rope.kv_heads + kvh) *
-               rope.page_size + slot % rope.page_size) * 128 + d;
-      dst[0] = o1;
-      dst[64] = o2;
-    }
-  }
+  if (GLU) c[(size_t)m * (N / 2) + col0 + col] = f2bf(silu(v) * v2);
+  else if (wide) wide[(size_t)m * N + col0 + col] = bf2f(f2bf(v));
+  else c[(size_t)m * N + col0 + col] = f2bf(v);
 }
 
-template <int END, bool NORM, bool PAIR = false>
+template <bool GLU, bool PAIR = false>
 void launch_skinny_rows(__hip_bfloat16* c, const __hip_bfloat16* a,
                         const __hip_bfloat16* w, int M, int N, int K,
-                        const RowsNorm& norm, const RowsRope& rope,
                         hipStream_t stream, float* wide = nullptr) {
-  const size_t sums = 8 * 16 * ROWS_MOST * sizeof(float);
-  const size_t rows = NORM ? (size_t)M * K * 2 : 0;
-  skinny_rows_kernel<END, NORM, PAIR>
-      <<<dim3(N / (PAIR ? 8 : 16)), dim3(512), rows > sums ? rows : sums,
-         stream>>>(w, a, K, N, M, norm.residual, norm.weight,
-                   norm.residual_out, norm.eps, c, wide, rope);
+  skinny_rows_kernel<GLU, PAIR>
+      <<<dim3(N / (PAIR ? 8 : 16)), dim3(512), 0, stream>>>(w, a, K, N, M, c,
+                                                           wide);
 }
 
 }  // namespace

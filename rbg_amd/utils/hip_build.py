@@ -29,7 +29,6 @@ HIP_SOURCES = {
     "_hip_ops": [
         "attn_decode.hip",
         "decode_pages.hip",
-        "decode_rows.hip",
         "embed_rows.hip",
         "attn_prefill.hip",
         "prefill_flash.hip",
@@ -39,6 +38,7 @@ HIP_SOURCES = {
         "rope_kv.hip",
         "silu_mul.hip",
         "skinny_gemm.hip",
+        "stream_rows.hip",
         "tile_gemm.hip",
         "kv_peer_copy.hip",
         "allreduce.hip",

@@ -879,6 +879,63 @@ def test_norm_rows(rows, k, first):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 2, 3, 4])
+@pytest.mark.parametrize("n", [1024, 1056, 3104, 16416])
+@pytest.mark.parametrize("k", [1024, 1280, 2304, 3072, 4096, 5120, 5376, 8192,
+                               16640])
+def test_stream_rows(rows, n, k):
+    """Products of up to four rows against float64: waves with and without a last
+    segment, workgroups with and without a last group, long rows, 512 k at a time and
+    256; plain, in f32, after a norm and with silu.  Bounds as in test_norm_rows; plain
+    ones half a unit of bf16's last place, 2^-8 of a value, and of f32 sums 1e-4, the
+    root of k units of 2^-24 of values of 1 and what is rounded on the way."""
+    from rbg_amd import ops
+    if n * k > 3e7 and rows != 3:
+        pytest.skip("large once")
+    assert ops._stream(rows, n, k)
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(rows * 100000 + n + k)
+    def rnd(*shape):
+        return torch.randn(*shape, device=dev, generator=gen).bfloat16()
+    x, w = rnd(rows, k), (rnd(n, k).float() / k ** 0.5).bfloat16()
+    w[n - 1, k - 1] = math.inf              # in the last piece, that others repeat
+    x[0, k - 1] = 1.0
+    want = x.double() @ w.double().t().contiguous()
+    got = ops.linear(x, w)
+    assert got[0, n - 1] == math.inf
+    err = (got.double() - want)[:, :n - 1].abs()
+    assert (err <= want[:, :n - 1].abs() * 2 ** -8 + 1e-4).all()
+    sums = ops._hip.stream_linear(x, w, 2)
+    assert sums.shape == (1, rows, n) and sums.dtype == torch.float32
+    parts = ops.linear_parts(x, w)
+    assert torch.equal(parts, got if parts.dim() == 2 else sums)
+    assert ((sums[0].double() - want)[:, :n - 1].abs() <= 1e-4).all()
+    assert torch.equal(sums[0].bfloat16(), got)
+    assert torch.equal(ops.linear_f32(x, w), got.float())
+    if k > 8192:
+        return
+    w[n - 1, k - 1] = 1.0
+    res, nw = rnd(rows, k) * 3, rnd(k)
+    for src in (x, torch.randn(1, rows, k, device=dev, generator=gen), None):
+        total = res.double() + (0 if src is None else src.double().view(rows, k))
+        h = total * torch.rsqrt(total.square().mean(-1, keepdim=True) + 1e-5) * \
+            nw.double()
+        full = h @ w.double().t().contiguous()
+        old = res.clone()
+        assert ops._takes_rows(src, res, nw, w)
+        out, new = ops._norm_project(src, res, nw, 1e-5, w)
+        assert out.shape == (1, rows, n) and torch.equal(res, old)
+        assert torch.equal(out[0].bfloat16(),
+                           ops._hip.norm_rows(src, res, nw, 1e-5, w, 0)[0])
+        assert ((new.double() - total).abs() <= total.abs() * 2 ** -8).all()
+        assert (out.double() - full).norm() <= 2 ** -7 * full.norm()
+        want = torch.nn.functional.silu(full[:, :n // 2]) * full[:, n // 2:]
+        out, new2 = ops.norm_swiglu(src, res, nw, 1e-5, w)
+        assert torch.equal(new2, new)
+        assert (out.double() - want).norm() <= 2 ** -7 * want.norm()
+
+
+@pytest.mark.gpu
 def test_linear_takes_what_the_library_takes():
     """Transposed and misaligned operands and gradients, at a shape that the
     decode GEMM would take otherwise."""
