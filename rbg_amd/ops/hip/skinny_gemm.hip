@@ -18,8 +18,17 @@
 //    rows: 75 -> 64 us),
 //  * two lines of a row at a time, not one (57344 x 8192, 1 row: 189 -> 169),
 //  * workgroups begin at different places of K.  All rows of A and W are K
-//    apart, so workgroups in step ask the same few L2 channels (128 rows: 78
-//    -> 75 us).
+//    apart, so workgroups in step ask the same few channels.  The eight
+//    workgroups that begin on the eight XCDs together begin at the same k; the
+//    next eight one chunk of 256 bytes later, whose A is then still in L2, or
+//    two where rows are 8 or 16 KB apart, so that one chunk does not leave the
+//    channel.  With the XCDs spread over K as well rows of a multiple of 16 KB
+//    met again: 57344 x 8192, 32 rows 183 -> 165 us; 16384 x 16384, 7 rows 123
+//    -> 89; 28672 x 4096, 45 rows 44.1 -> 43.2.  One chunk or two: 28672 x 4096
+//    44.0 / 43.2, 8192 x 8192 in 4 parts 27.0 / 24.2, but 16384 x 2048 19.7 /
+//    20.4 and, 128 rows of A, whose panel then leaves the L2s, 106496 x 16384
+//    808 / 840.  Short parts of rows of 32 KB have too few places for that and
+//    stay spread: 4096 x 16384 in 8, 45 rows 26.0, two chunks 28.3.
 #include "skinny_rows.h"
 
 namespace {
@@ -54,7 +63,13 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
   const int chunks = K / KC;
   const int c0 = chunks * blockIdx.y / splits;
   const int n = chunks * (blockIdx.y + 1) / splits - c0;
-  const int first = ((blockIdx.x >> 3) + (blockIdx.x & 7) * (n >> 3)) % n;
+  // where a workgroup begins (see above)
+  const int octet = blockIdx.x >> 3;
+  const bool two = K % 8192 == 0 ? splits > 1 || MT <= 4 || K == 8192
+                                 : splits == 1 && K % 4096 == 0;
+  const bool spread = K % 8192 == 0 && K > 8192 && splits > 1 && n <= 32;
+  const int first = (spread ? octet + (int)(blockIdx.x & 7) * (n >> 3)
+                            : two ? octet * 2 : octet) % n;
   const __hip_bfloat16* wp = w + (size_t)row * K + c0 * KC + g * 8;
   const __hip_bfloat16* ap[PIECES];
 #pragma unroll
