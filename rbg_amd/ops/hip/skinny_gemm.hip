@@ -3,14 +3,20 @@
 // matrix and C[M,N/2] = silu(A Wg^T) * (A Wu^T).
 //
 // Bound: the weights, read once from HBM.  A plain read reaches 6.1-6.3 TB/s
-// here, so 28672 x 4096 takes 38 us at best; up to 16 rows take 40 of them,
-// 64 take 46 and 128 take 58, whose A panels pass the L2s as often as the
+// here, so 28672 x 4096 takes 38 us at best; up to 16 rows take 38 of them,
+// 64 take 41 and 128 take 58, whose A panels pass the L2s as often as the
 // weights do.
 //
-// Weights go from global memory straight into MFMA operand registers: a lane
-// of v_mfma_f32_16x16x32_bf16 holds 8 consecutive k of one row, so a wave's
-// load covers 64 bytes of 16 rows, the next one the other half of the lines.
-// What made the difference, at 28672 x 4096:
+// A lane of v_mfma_f32_16x16x32_bf16 holds 8 consecutive k of one row, and the
+// lanes beside it other rows.  Loads in that order touch 16 lines for every 16
+// lanes, which a CU does at 27 bytes a ns where 256 neighbouring bytes of a row
+// give 38, so up to 96 rows a wave loads its chunk as 256 bytes of 4 rows at a
+// time and turns it through 4 KB of LDS of its own, without a barrier (28672 x
+// 4096: 7 rows of 24576 36.3 -> 33.9 us, 45 rows 43.1 -> 40.3, 64 rows 44.8 ->
+// 40.7; 5120 x 25600 in 6 parts, 64 rows 54.9 -> 50.0, 96 rows 62.0 -> 56.3;
+// 10240 x 5120 25.2 -> 23.0).  With 128 rows LDS is as busy as the loads, and
+// the turn gains nothing (4096 x 4096 in 8: 14.8, turned 15.2).
+// What else made the difference, at 28672 x 4096:
 //  * plain loads, not non-temporal ones, which send both halves of a line to
 //    L2 and back as requests of their own (16 rows: 48 -> 42 us),
 //  * loads pinned where they are issued: the compiler otherwise moves A's to
@@ -33,14 +39,14 @@
 
 namespace {
 
-constexpr int KC = 128;           // k per chunk
+constexpr int KC = 128;           // k per chunk: 4 loads of 16 rows
 constexpr int DEPTH = 2;          // chunks of weights in flight per wave
 
-// NW waves of 16 rows of W each share MT * 16 rows of A through LDS, a chunk
-// at a time, two buffers, one barrier a chunk.  blockIdx.y: a part of K, whose
-// sums go to ws in f32.  GLU: half of the waves hold the gate's rows, the
+// NW waves of T * 16 rows of W each share MT * 16 rows of A through LDS, a
+// chunk at a time, two buffers, one barrier a chunk.  blockIdx.y: a part of K,
+// whose sums go to ws in f32.  GLU: half of the waves hold the gate's rows, the
 // others the same rows of the up matrix, and meet in LDS.
-template <int MT, int NW, bool GLU>
+template <int MT, int NW, bool GLU, int T>
 __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
     const __hip_bfloat16* __restrict__ a,   // [M, K]
     const __hip_bfloat16* __restrict__ w,   // [N, K]
@@ -58,8 +64,8 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
   // columns of this wave; beyond the last it reads the last ones again
   const int half = GLU ? N / 2 : N;
   constexpr int SIDE = GLU ? NW / 2 : NW;
-  const int col0 = (blockIdx.x * SIDE + wave % SIDE) * 16;
-  const int row = min(col0, half - 16) + r + (wave / SIDE) * half;
+  const int col0 = (blockIdx.x * SIDE + wave % SIDE) * 16 * T;
+  const int row = min(col0, half - 16 * T) + (wave / SIDE) * half;
   const int chunks = K / KC;
   const int c0 = chunks * blockIdx.y / splits;
   const int n = chunks * (blockIdx.y + 1) / splits - c0;
@@ -70,7 +76,15 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
   const bool spread = K % 8192 == 0 && K > 8192 && splits > 1 && n <= 32;
   const int first = (spread ? octet + (int)(blockIdx.x & 7) * (n >> 3)
                             : two ? octet * 2 : octet) % n;
-  const __hip_bfloat16* wp = w + (size_t)row * K + c0 * KC + g * 8;
+  // TURN: a load brings 256 bytes of rows g, 4 + g, ... and 4 KB are turned
+  constexpr bool TURN = MT <= 6;
+  static_assert(T == 1 || TURN, "more rows of a wave come in whole chunks");
+  const __hip_bfloat16* wp = w + (size_t)(row + (TURN ? g : r)) * K + c0 * KC +
+                             (TURN ? r : g) * 8;
+  const size_t hop = TURN ? (size_t)4 * K : 32;
+  constexpr int LOADS = T * KC / 32;
+  __shared__ __align__(16) __hip_bfloat16 turned[TURN ? NW * T * 16 * PITCH : 8];
+  __hip_bfloat16* own = turned + (TURN ? wave * T * 16 * PITCH : 0);
   const __hip_bfloat16* ap[PIECES];
 #pragma unroll
   for (int p = 0; p < PIECES; ++p)
@@ -81,15 +95,13 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
   buf[1] = buf[0] + ROWS * PITCH;
   const int put = (tid / (KC / 8)) * PITCH + (tid % (KC / 8)) * 8;
 
-  f32x4 acc[MT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i) acc[i] = {0.f, 0.f, 0.f, 0.f};
-  sg_u4 wr[DEPTH][KC / 32], ar[PIECES], a0[PIECES];
+  f32x4 acc[T][MT] = {};
+  sg_u4 wr[DEPTH][LOADS], ar[PIECES], a0[PIECES];
 #define SG_W(s, at)                                                        \
   do {                                                                     \
     const int off = sg_turn(at, first, n) * KC;                            \
-    _Pragma("unroll") for (int h = 0; h < KC / 32; ++h)                    \
-        wr[s][h] = sg_load(wp + off + h * 32);                             \
+    _Pragma("unroll") for (int h = 0; h < LOADS; ++h)                      \
+        wr[s][h] = sg_load(wp + off + h * hop);                            \
   } while (0)
 #define SG_A(regs, at)                                                     \
   do {                                                                     \
@@ -104,11 +116,26 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
   } while (0)
 #define SG_MATH(s, b)                                                      \
   do {                                                                     \
+    sg_u4 f[LOADS];                                                        \
+    if (TURN) {                                                            \
+      _Pragma("unroll") for (int h = 0; h < LOADS; ++h)                    \
+          *reinterpret_cast<sg_u4*>(own + (h * 4 + g) * PITCH + r * 8) =   \
+              wr[s][h];                                                    \
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");               \
+      __builtin_amdgcn_wave_barrier();                                     \
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");               \
+    }                                                                      \
+    _Pragma("unroll") for (int h = 0; h < LOADS; ++h)                      \
+        f[h] = TURN ? sg_load(own + (h / 4 * 16 + r) * PITCH +             \
+                              h % 4 * 32 + g * 8)                          \
+                    : wr[s][h];                                            \
     _Pragma("unroll") for (int h = 0; h < KC / 32; ++h)                    \
-    _Pragma("unroll") for (int i = 0; i < MT; ++i)                         \
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(                  \
-            sg_frag(sg_load((b) + (i * 16 + r) * PITCH + h * 32 + g * 8)), \
-            sg_frag(wr[s][h]), acc[i], 0, 0, 0);                           \
+    _Pragma("unroll") for (int i = 0; i < MT; ++i) {                       \
+      const sg_u4 x = sg_load((b) + (i * 16 + r) * PITCH + h * 32 + g * 8); \
+      _Pragma("unroll") for (int t = 0; t < T; ++t)                        \
+          acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(             \
+              sg_frag(x), sg_frag(f[t * (KC / 32) + h]), acc[t][i], 0, 0, 0); \
+    }                                                                      \
   } while (0)
 
   // everything that the first chunks need is asked for before any wait
@@ -146,37 +173,43 @@ __global__ __launch_bounds__(64 * NW, 2) void skinny_gemm_kernel(
 #undef SG_PUT
 #undef SG_MATH
 
-  // lane l, register q: row 4 * g + q of A's tile, column r of the wave's 16
+  // lane l, register q: row 4 * g + q of A's tile, column r of 16 of the wave's
   if (GLU) {
     float* meet = (float*)lds;
-    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-      *reinterpret_cast<f32x4*>(&meet[(wave * MT + i) * 256 + lane * 4]) =
-          acc[i];
-    __syncthreads();
-    for (int e = tid; e < SIDE * MT * 256; e += THREADS) {
-      const int i = (e >> 8) % MT, side = (e >> 8) / MT;
-      const int m = i * 16 + ((e >> 6) & 3) * 4 + (e & 3);
-      const int col = (blockIdx.x * SIDE + side) * 16 + ((e >> 2) & 15);
-      if (m < M && col < half)
-        c[(size_t)m * half + col] =
-            f2bf(silu(meet[e]) * meet[e + SIDE * MT * 256]);
+    for (int t = 0; t < T; ++t) {
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        *reinterpret_cast<f32x4*>(&meet[(wave * MT + i) * 256 + lane * 4]) =
+            acc[t][i];
+      __syncthreads();
+      for (int e = tid; e < SIDE * MT * 256; e += THREADS) {
+        const int i = (e >> 8) % MT, side = (e >> 8) / MT;
+        const int m = i * 16 + ((e >> 6) & 3) * 4 + (e & 3);
+        const int col = ((blockIdx.x * SIDE + side) * T + t) * 16 +
+                        ((e >> 2) & 15);
+        if (m < M && col < half)
+          c[(size_t)m * half + col] =
+              f2bf(silu(meet[e]) * meet[e + SIDE * MT * 256]);
+      }
     }
   } else if (col0 < N) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int t = 0; t < T; ++t)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int m = i * 16 + g * 4 + q;
-        if (m >= M) continue;
-        if (splits > 1)
-          ws[((size_t)blockIdx.y * M + m) * N + col0 + r] = acc[i][q];
-        else if (c)
-          c[(size_t)m * N + col0 + r] = f2bf(acc[i][q]);
-        else
-          ws[(size_t)m * N + col0 + r] = bf2f(f2bf(acc[i][q]));
-      }
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int m = i * 16 + g * 4 + q, col = col0 + t * 16 + r;
+          if (m >= M) continue;
+          if (splits > 1)
+            ws[((size_t)blockIdx.y * M + m) * N + col] = acc[t][i][q];
+          else if (c)
+            c[(size_t)m * N + col] = f2bf(acc[t][i][q]);
+          else
+            ws[(size_t)m * N + col] = bf2f(f2bf(acc[t][i][q]));
+        }
   }
 }
 
@@ -195,14 +228,32 @@ __global__ void reduce_splits_kernel(const float* __restrict__ ws,
   *reinterpret_cast<uint2*>(c + i) = o.u;
 }
 
-template <int MT, int NW, bool GLU>
+template <int MT, int NW, bool GLU, int T = 1>
 void launch_tiles(__hip_bfloat16* c, float* ws, const __hip_bfloat16* a,
                   const __hip_bfloat16* w, int M, int N, int K, int splits,
                   hipStream_t stream) {
-  const int cols = NW * (GLU ? 8 : 16), out = GLU ? N / 2 : N;
-  skinny_gemm_kernel<MT, NW, GLU>
+  const int cols = NW * T * (GLU ? 8 : 16), out = GLU ? N / 2 : N;
+  skinny_gemm_kernel<MT, NW, GLU, T>
       <<<dim3((out + cols - 1) / cols, splits), dim3(64 * NW), 0, stream>>>(
           a, w, c, ws, M, N, K, splits);
+}
+
+// Up to 64 rows: 32 rows of W a wave where that makes one round of the chip of
+// what would be one and a part.  A CU with two workgroups reads no faster than
+// with one, so that the others wait, and A passes L2 half as often (64 rows:
+// 51200 x 5120 108 -> 95 us, 45056 x 4096 77 -> 67, 36864 x 4096 75 -> 62; over
+// 2048 to 8192 k: to 40960 columns 0.76 to 0.91, to 53248 0.84 to 1.03, 57344
+// 0.90 to 1.05; 65536, two whole rounds, 0.92 to 1.07, 69632 1.09 to 1.22).
+template <int MT, bool GLU>
+void launch_wide(__hip_bfloat16* c, float* ws, const __hip_bfloat16* a,
+                 const __hip_bfloat16* w, int M, int N, int K, int splits,
+                 hipStream_t stream) {
+  if (MT <= 4 && splits == 1 && N > 32768 && N <= 57344 &&
+      (GLU ? N / 2 : N) % 32 == 0)
+    launch_tiles<MT, 8, GLU, MT <= 4 ? 2 : 1>(c, ws, a, w, M, N, K, splits,
+                                             stream);
+  else
+    launch_tiles<MT, 8, GLU>(c, ws, a, w, M, N, K, splits, stream);
 }
 
 }  // namespace
@@ -220,16 +271,15 @@ extern "C" void launch_skinny_gemm(void* c, void* ws, const void* a,
   __hip_bfloat16* cp = (__hip_bfloat16*)c;
   float* wsp = (float*)ws;
   const int mt = (M + 15) >> 4;
-#define SG_GO(MT, NW)                                                      \
+#define SG_GO(MT)                                                          \
   do {                                                                     \
     if (glu)                                                               \
-      launch_tiles<MT, NW, true>(cp, wsp, ap, wp, M, N, K, 1, stream);     \
+      launch_wide<MT, true>(cp, wsp, ap, wp, M, N, K, 1, stream);          \
     else                                                                   \
-      launch_tiles<MT, NW, false>(cp, wsp, ap, wp, M, N, K, splits,        \
-                                  stream);                                 \
+      launch_wide<MT, false>(cp, wsp, ap, wp, M, N, K, splits, stream);    \
   } while (0)
-#define SG_GLU(MT)                                                         \
-  launch_tiles<MT, 4, true>(cp, wsp, ap, wp, M, N, K, 1, stream)
+#define SG_HALF(MT, GLU)                                                   \
+  launch_tiles<MT, 4, GLU>(cp, wsp, ap, wp, M, N, K, GLU ? 1 : splits, stream)
   if (waves == 0) {             // the kernel of a few rows
     if (glu)
       launch_skinny_rows<true>(cp, ap, wp, M, N, K, stream);
@@ -240,22 +290,26 @@ extern "C" void launch_skinny_gemm(void* c, void* ws, const void* a,
     else
       launch_skinny_rows<false>(cp, ap, wp, M, N, K, stream,
                                 cp ? nullptr : wsp);
-  } else if (mt <= 1 && waves == 4) SG_GO(1, 4);
-  else if (mt <= 2 && waves == 4) SG_GO(2, 4);
-  else if (mt <= 1) SG_GO(1, 8);
-  else if (mt <= 2) SG_GO(2, 8);
-  else if (mt <= 3 && waves == 4 && glu) SG_GLU(3);
-  else if (mt <= 4 && waves == 4 && glu) SG_GLU(4);
-  else if (mt <= 3) SG_GO(3, 8);
-  else if (mt <= 4) SG_GO(4, 8);
-  else if (mt <= 6) SG_GO(6, 8);
-  else if (mt <= 8) SG_GO(8, 8);
+  } else if (mt <= 1 && waves == 4) {
+    if (glu) SG_HALF(1, true);
+    else SG_HALF(1, false);
+  } else if (mt <= 2 && waves == 4) {
+    if (glu) SG_HALF(2, true);
+    else SG_HALF(2, false);
+  } else if (mt <= 1) SG_GO(1);
+  else if (mt <= 2) SG_GO(2);
+  else if (mt <= 3 && waves == 4 && glu) SG_HALF(3, true);
+  else if (mt <= 4 && waves == 4 && glu) SG_HALF(4, true);
+  else if (mt <= 3) SG_GO(3);
+  else if (mt <= 4) SG_GO(4);
+  else if (mt <= 6) SG_GO(6);
+  else if (mt <= 8) SG_GO(8);
   else if (mt <= 12)
     launch_tiles<12, 8, false>(cp, wsp, ap, wp, M, N, K, splits, stream);
   else
     launch_tiles<16, 8, false>(cp, wsp, ap, wp, M, N, K, splits, stream);
 #undef SG_GO
-#undef SG_GLU
+#undef SG_HALF
 }
 
 extern "C" void launch_reduce_splits(void* c, const void* ws, int splits,

@@ -1241,6 +1241,34 @@ def test_skinny_gemm_forms(m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [5, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(32832, 768), (32864, 1280), (57344, 512),
+                                 (57376, 512)])
+def test_skinny_gemm_wide(m, n, k):
+    """32 rows of W a wave: from 32769 to 57344 columns, a last workgroup of a
+    few of them, halves of gate/up that are no multiple of 32, a result in f32.
+    The bounds of test_skinny_gemm_forms and test_linear_swiglu."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(m * 1000003 + n + k)
+    x = torch.randn(m, k, device=dev, generator=gen).bfloat16()
+    w = torch.randn(n, k, device=dev, generator=gen).bfloat16()
+    want = x.double() @ w.double().t().contiguous()
+    bound = want.abs() * 2 ** -8 + \
+        (x.double().abs() @ w.double().abs().t().contiguous()) * k * 2 ** -24
+    got = ops._hip.skinny_gemm(x, w)
+    assert ((got.double() - want).abs() <= bound).all()
+    assert torch.equal(ops._hip.skinny_gemm(x, w, wide=True), got.float())
+    w = (w.float() / k ** 0.5).bfloat16()
+    full = x.double() @ w.double().t().contiguous()
+    gate, up = full[:, :n // 2], full[:, n // 2:]
+    want = torch.nn.functional.silu(gate) * up
+    bound = 2 ** -7 * (gate.abs() + 1) * (up.abs() + 1)
+    got = ops._hip.skinny_swiglu(x, w)
+    assert ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [1, 2, 4, 5, 17, 32, 33, 64])
 @pytest.mark.parametrize("f,k", [(3584, 4096), (7168, 2048), (6176, 2560),
                                  (8160, 2048), (9216, 2560), (19456, 2048)])
