@@ -98,6 +98,39 @@ DEV_INLINE float block_sum(float x, float* scratch /* NW floats */) {
   return total;
 }
 
+// v += parts s to s + U - 1, in order; part s of piece i by load(s, i).  All loads
+// are on their way before the first is used.
+template <int U, int PIECES, typename Load>
+DEV_INLINE void add_round(f32x4 (&v)[PIECES], const int s, const Load& load) {
+  f32x4 x[U][PIECES];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) x[u][i] = load(s + u, i);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) v[i] += x[u][i];
+}
+
+template <int U, int PIECES, typename Load>
+DEV_INLINE void add_rest(f32x4 (&v)[PIECES], const int s, const int n,
+                         const Load& load) {
+  if (n - s == U) add_round<U>(v, s, load);
+  else if constexpr (U > 1) add_rest<U - 1>(v, s, n, load);
+}
+
+// v + the sums of n parts, U of them in flight and the rest in one round.  (A loop
+// unrolled 8 times takes what is left of n one by one, half a us each: the norm of 64
+// rows of 5120 took 6.5 us of 6 parts and 5.1 of 8, now 4.5 and 4.8.)
+template <int U, int PIECES, typename Load>
+DEV_INLINE void add_parts(f32x4 (&v)[PIECES], const int n, const Load load) {
+  int s = 0;
+#pragma unroll 1
+  for (; s + U <= n; s += U) add_round<U>(v, s, load);
+  if constexpr (U > 1) add_rest<U - 1>(v, s, n, load);
+}
+
 DEV_INLINE int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 #define HIP_KERNEL_CHECK()                                                    \

@@ -77,70 +77,100 @@ __global__ void rmsnorm_kernel(__hip_bfloat16* __restrict__ out,      // [T,H]
 
 // residual += src; returns its RMS norm: for decode batches.  src is a row of
 // bf16, or (PARTS) the f32 sums that the parts of a split GEMM left, [parts,
-// rows, hidden], whose own reduction launch this replaces (2 us or more).
+// rows, hidden], whose own reduction launch this replaces (2 us or more), or
+// (ALONE) there is none, and the residual stays as it is.
 // Bound by latency: a row is one workgroup, so it has as many threads as the
-// row has 8-byte pieces and every load of a thread is independent; the sums
-// stay in registers between the passes (4096 wide, 128 rows: 3.2 us of the
-// kernel above, 3.0 of this one, 4.1 from 8 parts).
-template <bool PARTS>
+// row has 8-byte pieces, to 1024; every load of a thread, the weight's as well, is
+// on its way before the first is used, and the sums stay in registers between the
+// passes.
+enum NormSource { NORM_ALONE, NORM_ROWS, NORM_PARTS };
+
+template <int SOURCE, int MOST, int U>
 __global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(
     const void* __restrict__ src, __hip_bfloat16* __restrict__ residual,
     const int parts, const int rows, const int hidden, const int threads,
     const __hip_bfloat16* __restrict__ w, __hip_bfloat16* __restrict__ out,
     const float eps) {
-  constexpr int MOST = 4;         // pieces of 4 per thread: hidden <= 16384
-  const int row = blockIdx.x, tid = threadIdx.x;
+  const int row = blockIdx.x, tid = threadIdx.x, waves = threads >> 6;
   const size_t at = (size_t)row * hidden;
-  __shared__ float red[16];
+  __shared__ __align__(16) float red[16];
   union B4 { uint2 u; __hip_bfloat16 e[4]; };
-  B4 sum[MOST];
+  B4 x[MOST], r[MOST], g[MOST], sum[MOST];
+  f32x4 v[MOST] = {};
+  int col[MOST];                  // beyond the row: its end again, to no use
+#pragma unroll
+  for (int i = 0; i < MOST; ++i) {
+    col[i] = min((i * threads + tid) * 4, hidden - 4);
+    r[i].u = *reinterpret_cast<const uint2*>(residual + at + col[i]);
+    if (SOURCE == NORM_ROWS)
+      x[i].u = *reinterpret_cast<const uint2*>(
+          (const __hip_bfloat16*)src + at + col[i]);
+    g[i].u = *reinterpret_cast<const uint2*>(w + col[i]);
+  }
+  if (tid < 16 && tid >= waves) red[tid] = 0.f;
+  if (SOURCE == NORM_PARTS)
+    add_parts<U>(v, parts, [&](int s, int i) {
+      return *reinterpret_cast<const f32x4*>(
+          (const float*)src + at + col[i] + (size_t)s * rows * hidden);
+    });
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < MOST; ++i) {
-    const int col = (i * threads + tid) * 4;
-    if (col < hidden) {
-      B4 r;
-      r.u = *reinterpret_cast<const uint2*>(residual + at + col);
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
-      if (PARTS) {
-        const float* p = (const float*)src + at + col;
-#pragma unroll 8
-        for (int s = 0; s < parts; ++s)
-          v += *reinterpret_cast<const f32x4*>(p + (size_t)s * rows * hidden);
-      } else {
-        B4 x;
-        x.u = *reinterpret_cast<const uint2*>(
-            (const __hip_bfloat16*)src + at + col);
+    const bool live = i * threads + tid < hidden >> 2;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = bf2f(x.e[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float t = v[j] + bf2f(r.e[j]);
-        sum[i].e[j] = f2bf(t);
-        ss += t * t;
-      }
-      *reinterpret_cast<uint2*>(residual + at + col) = sum[i].u;
+    for (int j = 0; j < 4; ++j) {
+      const float t = (SOURCE == NORM_ROWS ? bf2f(x[i].e[j]) : v[i][j]) +
+                      bf2f(r[i].e[j]);
+      sum[i].e[j] = f2bf(t);
+      ss += live ? t * t : 0.f;
     }
   }
   ss = wave_sum(ss);
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
   float total = 0.f;
-  for (int k = 0; k < threads >> 6; ++k) total += red[k];
+#pragma unroll
+  for (int k = 0; k < 16; k += 4) {
+    const f32x4 t = *reinterpret_cast<const f32x4*>(red + k);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) total += t[j];
+  }
   const float inv = rsqrtf(total / hidden + eps);
 #pragma unroll
   for (int i = 0; i < MOST; ++i) {
-    const int col = (i * threads + tid) * 4;
-    if (col < hidden) {
-      B4 g, o;
-      g.u = *reinterpret_cast<const uint2*>(w + col);
+    if (i * threads + tid < hidden >> 2) {
+      B4 o;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        o.e[j] = f2bf(bf2f(sum[i].e[j]) * inv * bf2f(g.e[j]));
-      *reinterpret_cast<uint2*>(out + at + col) = o.u;
+        o.e[j] = f2bf(bf2f(sum[i].e[j]) * inv * bf2f(g[i].e[j]));
+      *reinterpret_cast<uint2*>(out + at + col[i]) = o.u;
+      if (SOURCE != NORM_ALONE)
+        *reinterpret_cast<uint2*>(residual + at + col[i]) = sum[i].u;
     }
   }
+}
+
+template <int SOURCE>
+void norm_rows(void* out, const void* src, void* residual, const void* weight,
+               float eps, int parts, int rows, int hidden, hipStream_t stream) {
+  auto go = [&](auto kernel, int most) {
+    const int threads = (hidden / 4 + 64 * most - 1) / (64 * most) * 64;
+    kernel<<<dim3(rows), dim3(threads), 0, stream>>>(
+        src, (__hip_bfloat16*)residual, parts, rows, hidden, threads,
+        (const __hip_bfloat16*)weight, (__hip_bfloat16*)out, eps);
+  };
+  constexpr bool PARTS = SOURCE == NORM_PARTS;
+  // many rows hide the loads' latency by themselves, and fit in fewer registers
+  const bool many = PARTS && rows > 256;
+  if (hidden <= 4096) go(add_rmsnorm_row_kernel<SOURCE, 1, PARTS ? 8 : 1>, 1);
+  else if (hidden <= 8192 && many)
+    go(add_rmsnorm_row_kernel<SOURCE, 2, PARTS ? 2 : 1>, 2);
+  else if (hidden <= 8192)
+    go(add_rmsnorm_row_kernel<SOURCE, 2, PARTS ? 8 : 1>, 2);
+  else if (hidden <= 12288 && !many)
+    go(add_rmsnorm_row_kernel<SOURCE, 3, PARTS ? 6 : 1>, 3);
+  else
+    go(add_rmsnorm_row_kernel<SOURCE, 4, PARTS ? 2 : 1>, 4);
 }
 
 }  // namespace
@@ -151,18 +181,21 @@ extern "C" {
 void launch_add_rmsnorm_rows(void* out, const void* src, void* residual,
                              const void* weight, float eps, int parts,
                              int rows, int hidden, hipStream_t stream) {
-  const int threads = min(1024, (hidden / 4 + 63) / 64 * 64);
-  auto go = [&](auto kernel) {
-    kernel<<<dim3(rows), dim3(threads), 0, stream>>>(
-        src, (__hip_bfloat16*)residual, parts, rows, hidden, threads,
-        (const __hip_bfloat16*)weight, (__hip_bfloat16*)out, eps);
-  };
-  if (parts) go(add_rmsnorm_row_kernel<true>);
-  else go(add_rmsnorm_row_kernel<false>);
+  if (parts)
+    norm_rows<NORM_PARTS>(out, src, residual, weight, eps, parts, rows, hidden,
+                          stream);
+  else
+    norm_rows<NORM_ROWS>(out, src, residual, weight, eps, 0, rows, hidden,
+                         stream);
 }
 
 void launch_rmsnorm(void* out, void* input, const void* weight, float eps,
                     int tokens, int hidden, hipStream_t stream) {
+  if (tokens <= 256 && hidden >= 256 && hidden <= 16384) {
+    norm_rows<NORM_ALONE>(out, nullptr, input, weight, eps, 0, tokens, hidden,
+                          stream);
+    return;
+  }
   dim3 grid(tokens), block(256);
   hipLaunchKernelGGL(rmsnorm_kernel<false>, grid, block, 0, stream,
                      (__hip_bfloat16*)out, (__hip_bfloat16*)input,

@@ -122,17 +122,15 @@ __global__ __launch_bounds__(256) void rope_heads_kernel(
   if (PARTS) {
     const float* p = sums + ((size_t)token * heads + head) * D + d;
     const size_t step = (size_t)tokens * heads * D;
-    f32x4 t[2][2] = {};
-#pragma unroll 8
-    for (int s = 0; s < parts; ++s)
-#pragma unroll
-      for (int h = 0; h < 4; ++h)
-        t[h >> 1][h & 1] += *reinterpret_cast<const f32x4*>(
-            p + s * step + (h >> 1) * 64 + (h & 1) * 4);
+    f32x4 t[4] = {};
+    add_parts<8>(t, parts, [&](int s, int h) {
+      return *reinterpret_cast<const f32x4*>(p + s * step + (h >> 1) * 64 +
+                                             (h & 1) * 4);
+    });
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[h][j] = t[h][j >> 2][j & 3];
+      for (int j = 0; j < 8; ++j) x[h][j] = t[h * 2 + (j >> 2)][j & 3];
   } else {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {

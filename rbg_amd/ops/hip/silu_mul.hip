@@ -41,16 +41,14 @@ __global__ void silu_parts_kernel(__hip_bfloat16* __restrict__ out,  // [T, I]
   const int col = (int)(i % nvec_row) * 4;
   const float* p = x + row * 2 * inter + col;
   const size_t step = (size_t)total_vec * 8;
-  f32x4 g = {0.f, 0.f, 0.f, 0.f}, u = g;
-#pragma unroll 4
-  for (int s = 0; s < parts; ++s) {
-    g += *reinterpret_cast<const f32x4*>(p + s * step);
-    u += *reinterpret_cast<const f32x4*>(p + s * step + inter);
-  }
+  f32x4 v[2] = {};                // gate, up
+  add_parts<8>(v, parts, [&](int s, int i) {
+    return *reinterpret_cast<const f32x4*>(p + s * step + i * inter);
+  });
   union { __hip_bfloat16 e[4]; uint2 u; } o;
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    o.e[j] = f2bf(g[j] / (1.f + __expf(-g[j])) * u[j]);
+    o.e[j] = f2bf(v[0][j] / (1.f + __expf(-v[0][j])) * v[1][j]);
   *reinterpret_cast<uint2*>(out + row * inter + col) = o.u;
 }
 

@@ -218,13 +218,13 @@ __global__ void reduce_splits_kernel(const float* __restrict__ ws,
                                      const int splits, const long mn) {
   const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= mn) return;
-  f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-  for (int s = 0; s < splits; ++s)
-    v += *reinterpret_cast<const f32x4*>(ws + (size_t)s * mn + i);
+  f32x4 v[1] = {};
+  add_parts<8>(v, splits, [&](int s, int) {
+    return *reinterpret_cast<const f32x4*>(ws + (size_t)s * mn + i);
+  });
   union { __hip_bfloat16 e[4]; uint2 u; } o;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) o.e[j] = f2bf(v[j]);
+  for (int j = 0; j < 4; ++j) o.e[j] = f2bf(v[0][j]);
   *reinterpret_cast<uint2*>(c + i) = o.u;
 }
 

@@ -1241,6 +1241,40 @@ def test_skinny_gemm_forms(m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 7, 257])
+@pytest.mark.parametrize("hidden", [4, 256, 4096, 4100, 8192, 8196, 12288, 12292,
+                                    16384])
+def test_norm_of_rows(rows, hidden):
+    """Every number of pieces that a thread holds, rows that end within one, and
+    numbers of parts around what is in flight.  The sum is rounded to bf16 (2^-8 of
+    it); the norm reads what was rounded and is rounded itself, from squares whose
+    sum is off by 2^-8 at most where each is."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(rows + hidden)
+    res = torch.randn(rows, hidden, device=dev, generator=gen).bfloat16()
+    w = torch.randn(hidden, device=dev, generator=gen).bfloat16()
+
+    def normed(t):
+        return t * (t.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * w.double()
+    if hidden % 8 == 0:
+        want = normed(res.double())
+        assert ((ops.rmsnorm(res, w, 1e-5).double() - want).abs()
+                <= want.abs() * 2 ** -8 + 1e-6).all()
+    for parts in (0, 1, 2, 3, 5, 7, 8, 9, 16):
+        src = torch.randn(parts or 1, rows, hidden, device=dev, generator=gen)
+        src = src if parts else src[0].bfloat16()
+        total = (src.double().sum(0) if parts else src.double()) + res.double()
+        got = res.clone()
+        out = ops._hip.add_rmsnorm(src, got, w, 1e-5)
+        assert ((got.double() - total).abs() <= total.abs() * 2 ** -8 + 1e-5).all()
+        want = normed(total)
+        # the residual's rounding is not in the norm's sum of squares
+        assert ((out.double() - want).abs()
+                <= want.abs() * 2 ** -7 + 1e-4 * w.double().abs() + 1e-5).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [5, 32, 33, 64])
 @pytest.mark.parametrize("n,k", [(32832, 768), (32864, 1280), (57344, 512),
                                  (57376, 512)])
