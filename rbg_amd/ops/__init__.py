@@ -106,41 +106,56 @@ def _skinny(rows: int, n: int, k: int, parts: bool = False) -> bool:
     whole range with cold weights (us, own / library): the library is uneven.
 
     Up to 10240 columns, as it splits k and the library does not: long ones at
-    any decode batch (4096 x 4096: 128 rows 19.5 / 24.4, 129 rows 22.1 / 22.1;
-    4096 x 14336: 192 rows 48 / 103, 256 rows 63 / 62; 5120 x 25600: 256 rows
-    121 / 261), short ones for few rows (4096 x 2048: 32 rows 9.8 / 11.9, 64
-    rows 13.1 / 12.4; 1024 x 4096: 64 rows 10.3 / 12.1, 128 rows 14.6 / 9.4).
+    any decode batch (4096 x 4096: 96 rows 19 / 25, 129 rows 22.1 / 22.1;
+    4096 x 14336: 192 rows 47 / 103, 256 rows 63 / 62; 5120 x 25600: 256 rows
+    121 / 261), short ones for few rows (4096 x 2048: 32 rows 11.3 / 13.6, 64
+    rows 15.3 / 14.5; 1024 x 4096: 64 rows 12.2 / 14.7, 128 rows 16.5 / 12.0).
 
-    Beyond, a few rows by the form for them (12288 x 8192: 4 rows 37 / 40,
-    28672 x 4096: 42 / 60), and short k up to 16 rows (18432 x 2560: 16 rows
-    26 / 55, 17 rows 25 / 23).  To 12288 columns its workgroups fill only two
-    thirds of the chip (12288 x 8192: 16 rows 43 / 40).
-
-    Wide ones up to 64 rows where rows of W are a multiple of 4 KB apart: the
-    library reads those at 4.6 TB/s and others at 5.8, and this kernel, whose
-    workgroups begin at different k, both at 5.3 to 6; the form of a few rows
-    loads more than once where k is no multiple of 2048 (28672 x 4096: 64 rows
-    47 / 52, 128 rows 60 / 54; 1 row of 51200 x 4096 72 / 91, x 5120 98 / 91).
-    Not where there is a round of workgroups and a small rest (40960 x 4096: 64
-    rows 82 / 78), nor near 16384 x 8192, where the library is good (14336 x
-    8192: 16 rows 50 / 45, 64 rows 57 / 48)."""
+    Beyond, up to 64 rows where its workgroups fill the chip: from 16384 columns
+    (24576 x 3072: 5 rows 28 / 51, 64 rows 35 / 38; 32768 x 5120: 48 rows 66 / 87,
+    64 rows 68 / 70; 36864 x 4096: 68 / 73 and 80 / 82; 65536 x 4096: 92 / 124 and
+    103 / 136), except between its whole rounds for rows that are no multiple of 4
+    KB apart or long, which the library reads as well (36864 x 3072: 16 rows 52 /
+    53, 48 rows 61 / 56; 49152 x 5120: 32 rows 105 / 98; 49152 x 8192: 5 rows 148 /
+    172, 32 rows 165 / 156).  Of fewer columns two thirds of the chip are enough for
+    short k (12288 x 1536: 48 rows 16.2 / 16.9, 64 rows 17.7 / 17.0; x 4096: 64 rows
+    28.7 / 28.9; not x 5120: 16 rows 30.7 / 29.2).  From 65 rows the library's tiles
+    are as good (24576 x 2048: 64 rows 24.7 / 30.0, 96 rows 30 / 32, 128 rows 36 /
+    34)."""
     if rows < 1 or n % 32 or k % 512:
         return False
     if n <= 10240:
         if k <= 2048:
-            return rows <= (64 if parts else 32)
+            return rows <= (64 if parts or k <= 1024 and n >= 8192 else 32)
         if n <= 2048 and not parts:
             return rows <= min(256, k // 64)
         return rows <= (256 if k > 16384 else 192 if k >= 12288 else 128)
-    if rows <= 4 and k % 2048 == 0 or rows <= 16 and n <= 24576 and k <= 4096:
-        return True
-    if n <= 12288:
-        return (16 < rows <= 256 if k > 16384 else
-                rows <= 64 and k <= 4096 if parts else
-                rows <= 32 and k <= 2048)
-    return (rows <= 64 and k % 2048 == 0 and
-            not (32768 < n < 49152 and k > 2048) and
-            not (n <= 16384 and 6144 < k < 12288))
+    if rows <= 4:
+        return k % 2048 == 0 or n <= 24576 and k <= 4096
+    if n <= 12288 and k > 16384:
+        return 16 < rows <= 256
+    if rows > 64:
+        return False
+    if n < 16384 and k <= 6144:
+        return (k <= 1024 or k % 2048 == 0 and (n > 12288 or k <= 4096) or
+                k <= 4096 and (rows <= 48 or parts and n <= 12288))
+    if n < 16384 or k > 8192:
+        return (k % 2048 == 0 and not 32768 < n < 49152 and
+                (n > 16384 or k >= 12288))
+    if n >= 65536:
+        return _after_rounds(rows, n, k)
+    return not (32768 < n < 65536 and rows > 16 and
+                (k > 2560 if k % 2048 else k > 6144 and n <= 53248))
+
+
+def _after_rounds(rows: int, n: int, k: int) -> bool:
+    """The decode GEMM from 65536 columns and to 8192 k, where its workgroups make
+    whole rounds and a part of one (of the library's time: 4096 and 6144 k 0.83 to 1;
+    73728 x 5120: 32 rows 0.90, 64 rows 1.14; 77824 x 8192: 16 rows 0.89, 32 rows 1.07;
+    98304 x 8192 0.74 to 0.89)."""
+    if k <= 6144:
+        return k <= 4096 or k % 2048 == 0 or rows <= 32 or n >= 77824
+    return n >= 90112 or rows <= 16 and n >= 77824
 
 
 def _takes_skinny(x: torch.Tensor, w: torch.Tensor,
@@ -275,53 +290,52 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def _glu(rows: int, n: int, k: int) -> bool:
     """Does a gate/up product apply silu in the decode GEMM, which then
-    cannot split k?  Where its workgroups fill the chip all the same (us,
-    against the product, by linear_parts or the library, and silu_mul): up to
-    64 rows of a wide matrix (28672 x 4096: 64 rows 47 / 55; 18432 x 2560: 16
-    rows 26 / 57; not 38912 x 4096, a round and a small rest: 16 rows 76 / 72),
-    32 rows to 16384 columns (14336 x 4096: 32 rows 27 / 29, 64 rows 42 / 30;
-    not x 8192: 16 rows 60 / 48), and narrow ones of short k (7168 x 2048: 16
-    rows 13.1 / 15.4, x 4096 23.9 / 18.4; 11264 x 2048: 32 rows 14.1 / 17.5, 37
-    rows 16.8 / 18.5; 16384 x 2048, 64 rows 19.4 / 21.3; 4096 x 1024, 48 rows 8.6 /
-    9.8, but 8192 x 2048 15.6 / 14.5, 12288 x 3072 25.1 / 25.1;
-    12288 x 4096: 16 rows 25.6 / 29.5, x 5120: 32 rows 33.6 / 29.7).  The form
-    of a few rows splits k within a workgroup (7168 x 8192: 4 rows 25 / 27)."""
-    if rows < 1 or n % 64 or k % 512:
+    cannot split k?  Where its workgroups fill the chip all the same.  Against the
+    product, by linear_parts or the library or in tiles, and silu_mul, at 1500
+    shapes of 5 to 64 rows, 4096 to 131072 columns and 1024 to 10240 k (us): any
+    from 11264 or 16384 columns (24576 x 4096: 5 rows 33.4 / 34.8, 64 rows 37.6 /
+    38.8; 51200 x 5120 95 / 102), fewer of short k (4096 x 1024: 5 rows 7.2 / 8.7; 8192 x
+    2048, 48 rows 13.0 / 13.1; 11264 x 4096: 32 rows even, 64 rows 9% more; 13312 x
+    8192: 16 rows 0.96, 64 rows 1.07), 0.83 to 1.0 of the time but 5% more between
+    those lines.  Not long k of 32769 to 40959 (36864 x 10240: 16 rows 1.07, 45056
+    0.96).
+
+    Up to 4 rows what the GEMM for them leaves: k below 1024, few columns."""
+    if rows < 1 or n % 64 or k % 256 or k < 512:
         return False
-    if rows <= 4 and k % 2048 == 0:
+    if rows <= 4:
+        return k % 512 == 0 and (k % 2048 == 0 or n <= 24576 and k <= (
+            8192 if rows <= 2 and n <= 12288 else 1536))
+    if rows > 64:
+        return False
+    if n < 4096:
+        return k <= (1536 if rows <= 32 else 1024)
+    if k <= 2048:
         return True
-    if 32 < rows <= 64 and n <= 16384:
-        return k <= 1024 or n >= 10240 and k <= 2048
-    if n <= 12288:
-        return (rows <= 2 and k <= 8192 or rows <= 32 and
-                (k <= (1536 if n <= 4096 else 2048) or
-                 n >= 10240 and k <= 4096))
-    if rows <= 16 and n <= 24576 and k <= 4096:
-        return True
-    return (k % 2048 == 0 and rows <= (32 if n <= 16384 else 64) and
-            not (32768 < n < 49152 and k > 2048) and
-            not (n <= 16384 and 6144 < k < 12288))
+    if n < 16384:
+        few = rows <= 32
+        return n >= 11264 and (k <= (4096 if few else 3072) or
+                               few and n >= 13312 and k <= 8192)
+    if k > 8192:
+        return (n >= 18432 and not 32768 < n < 40960 and
+                (n <= 65536 or k % 2048 == 0))
+    return n < 65536 or _after_rounds(rows, n, k)
 
 
 def _tile_few(rows: int, n: int, k: int) -> bool:
-    """Does the GEMM of prompts take gate/up of 5 to 64 rows, in tiles of 64?  Its
-    ring of weights in LDS is deeper than the decode GEMM's registers, but a CU has
-    one tile at a time, so that it gains where there is about one for each.  Against
-    what is taken without it, over 16896 to 73728 columns, 2048 to 8192 k, 5 to 64 rows
-    (us): to 20480 columns (18432 x 4096: 64 rows 43.1 / 36.6; 20480 x 8192: 16 rows 68.9
-    / 64.3), from there to 26624 for more rows (24576 x 4096: 48 rows 45.0 / 40.6, 16 rows
-    38.3 / 39.3; 28672 x 4096: 48 rows 46.3 / 46.5, x 8192 86.0 / 90.0), and beyond 32768
-    with tiles of 256, while one round holds them, 65536 columns (36864 x 2048: 5 rows
-    39.3 / 32.1; 45056 x 4096: 64 rows 88.3 / 73.3).  A full round leaves no CU to spare:
-    from 53248 columns only long k (57344 x 4096: 5 rows 81.8 / 85.5, x 6144 121 / 123, x
-    8192 178 / 166), for more rows from 6144 (33 rows 135 / 125; 65536 x 6144 143 / 142, x
-    4096 94 / 104).  Rows that are no multiple of 4 KB apart the library reads better
-    (40960 x 5120: 64 rows 95 / 101), but not where they are few and it has few tiles
-    (18432 x 5120: 16 rows 85 / 46, 32 rows 45 / 50; x 4608 and 7168 alike)."""
+    """Does the GEMM of prompts take gate/up of 5 to 64 rows, in tiles of 64?  Asked
+    after the decode GEMM (_glu), which reads its weights as well and leaves k that is
+    no multiple of 256.  There it takes 0.3 to 1.0 of the library and silu_mul over 16640
+    to 57344 columns, 2112 to 7232 k (us: 16640 x 4160: 5 rows 0.38, 64 rows 0.81; 36864 x
+    6080: 5 rows 1.01, 48 rows 0.87).  Of multiples of 2048, where a CU has about one
+    tile: to 20480 columns, from there to 26624 for more rows, and beyond 32768 with
+    tiles of 256, while one round holds them, 65536 columns (45056 x 4096: 64 rows 88 /
+    70); a full round leaves no CU to spare, and from 53248 columns only long k gain, for
+    more rows from 6144."""
     if not 4 < rows <= 64 or k < 2048 or k > 8192 or n <= 16384:
         return False
     if k % 2048:
-        return rows <= 16 and k >= 4096 and n <= 32768
+        return k % 256 > 0
     if n <= 32768:
         return n <= (20480 if rows <= 32 else 26624)
     return n <= 53248 or (n <= 65536 and k >= (8192 if rows <= 32 else 6144))
@@ -354,13 +368,10 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T), w = [Wg; Wu]."""
     if _takes_stream(x, w):
         return _hip.stream_swiglu(x.contiguous(), w)
+    if _takes_tile(x, w, _glu):
+        return _require_hip().skinny_swiglu(x.contiguous(), w)
     if x.shape[0] > 4 and _takes_tile(x, w, _tile_glu):
         return _require_hip().tile_swiglu(x.contiguous(), w)
-    if (SKINNY_GEMM and _on_gpu(x) and x.dim() == 2 and w.dim() == 2 and
-            x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and
-            _glu(x.shape[0], w.shape[0], x.shape[1]) and _plain(x, w)):
-        return _require_hip().skinny_swiglu(
-            x if x.is_contiguous() else x.contiguous(), w)
     return silu_mul(linear_parts(x, w))
 
 
@@ -377,10 +388,10 @@ def place_inputs(fields, tables, new_fields, new_tables) -> None:
 
 
 def _route(rows: int, n: int, k: int, glu: bool) -> int:
-    if glu and _tile_glu(rows, n, k):
-        return 4
     if glu and _glu(rows, n, k):
         return 3
+    if glu and _tile_glu(rows, n, k):
+        return 4
     if rows > 64 and _tile(rows, n, k):
         return 2
     return 1 if _skinny(rows, n, k, True) else 0

@@ -31,18 +31,29 @@ inline SkinnyPlan pick_skinny(int M, int N, int K) {
   // 5632, 1 row: 9.0 us against 9.7, 4 rows 10.1 against 10.0).
   if ((M <= 4 && K % 2048 == 0) || (M <= 2 && K <= 8192 && N <= 12288))
     return {0, 1};
-  // up to 32 rows of a narrow matrix: workgroups of half the size, half again
-  // as many as fit at once (6144 x 4096, one row: 13.2 us against 14.2; above
-  // 32 rows A's copies cost more, 14336 x 4096, 64 rows: 30.1 against 26.7)
-  if (M <= 32 && N <= 8192) {
-    const int tiles = (N + 63) / 64;
-    return {4, std::max(1, std::min({768 / tiles, K / 256, 8}))};
-  }
-  // one workgroup of 8 waves per CU, all of them at once: the last of 1.5 or
-  // 2.5 rounds is lost (10240 x 8192, 64 rows: 3 splits = 240 workgroups 38 us,
-  // 4 splits 48, 6 splits 40)
-  const int tiles = (N + 127) / 128;
-  return {8, std::max(1, std::min({256 / tiles, K / 256, 16}))};
+  // One round of workgroups, the last of 1.5 or 2.5 is lost (10240 x 8192, 64 rows:
+  // 3 parts = 240 workgroups 38 us, 4 parts 48, 6 parts 40).  Of those the form in
+  // which a CU has the least to read, as it reads about as fast with four waves as with
+  // eight, and between nearly equal ones that with fewer parts, which are written and
+  // read again.  Of all forms at 774 shapes of 5 to 128 rows, 1024 to 10240 columns and
+  // 1024 to 25600 k, the parts' reader at 4 TB/s, it takes 0.6% more than the best one;
+  // up to three workgroups of four waves on a CU took 8% (7 rows: 4096 x 12288 19.0, 4
+  // parts 18.3; 6144 x 4096 10.9, 11.0; 32 rows of 8192 x 2048 1.35 of the best).
+  SkinnyPlan best{8, 1};
+  float least = 1e30f;
+  for (int waves = M <= 32 ? 4 : 8; waves <= 8; waves += 4)
+    for (int splits : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16}) {
+      if (splits > std::max(1, K / 256) ||
+          (N + 16 * waves - 1) / (16 * waves) * splits > 256)
+        break;
+      const float t = (K / 128 + splits - 1) / splits * waves +
+                      splits * (1.f + 0.02f * M);
+      if (t < least) {
+        least = t;
+        best = {waves, splits};
+      }
+    }
+  return best;
 }
 
 // The same for a product whose parts a launch of its own adds up, which a few

@@ -82,7 +82,8 @@ __global__ void rmsnorm_kernel(__hip_bfloat16* __restrict__ out,      // [T,H]
 // Bound by latency: a row is one workgroup, so it has as many threads as the
 // row has 8-byte pieces, to 1024; every load of a thread, the weight's as well, is
 // on its way before the first is used, and the sums stay in registers between the
-// passes.
+// passes (4096 wide: 8 rows 2.5 us alone, 3.4 from 8 parts, where loads after the
+// barrier and pieces in turn took 2.9 and 3.8; 128 rows 2.6, 5.3, before 3.0, 5.7).
 enum NormSource { NORM_ALONE, NORM_ROWS, NORM_PARTS };
 
 template <int SOURCE, int MOST, int U>

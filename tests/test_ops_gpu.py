@@ -1241,6 +1241,26 @@ def test_skinny_gemm_forms(m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [5, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(4096, 768), (8192, 1280), (11264, 2816),
+                                 (16448, 2304), (66048, 768), (16448, 2112)])
+def test_swiglu_of_odd_lengths(m, n, k):
+    """Gate/up of k that are no multiple of 512, or of 256, on whichever way; the bound
+    of test_linear_swiglu."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(m * 7 + n + k)
+    x = torch.randn(m, k, device=dev, generator=gen).bfloat16()
+    w = (torch.randn(n, k, device=dev, generator=gen) / k ** 0.5).bfloat16()
+    full = x.double() @ w.double().t().contiguous()
+    gate, up = full[:, :n // 2], full[:, n // 2:]
+    want = torch.nn.functional.silu(gate) * up
+    bound = 2 ** -7 * (gate.abs() + 1) * (up.abs() + 1)
+    assert ((ops.linear_swiglu(x, w).double() - want).abs() <= bound).all()
+    assert ops._glu(m, n, k) or ops._tile_few(m, n, k) or k == 2816 and m > 32
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 7, 257])
 @pytest.mark.parametrize("hidden", [4, 256, 4096, 4100, 8192, 8196, 12288, 12292,
                                     16384])
