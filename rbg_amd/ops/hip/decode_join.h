@@ -19,6 +19,50 @@ DEV_INLINE int part_keys(int ctx, int least, int whole, int splits) {
   return (ctx + all - 1) / all * PART_ROUND;
 }
 
+// Sums, or the largest, of a lane's value and those of the lanes below; of none 0.
+template <bool MAX>
+DEV_INLINE int up_to_lane(int x) {
+#define DJ_STEP(ctrl, rows)                                                \
+  do {                                                                     \
+    const int y = __builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xf, false); \
+    x = MAX ? max(x, y) : x + y;                                           \
+  } while (0)
+  DJ_STEP(0x111, 0xf);            // by 1, 2, 4 and 8 lanes of a row of 16
+  DJ_STEP(0x112, 0xf);
+  DJ_STEP(0x114, 0xf);
+  DJ_STEP(0x118, 0xf);
+  DJ_STEP(0x142, 0xa);            // a row's last to the next, 31 to the upper half
+  DJ_STEP(0x143, 0xc);
+#undef DJ_STEP
+  return x;
+}
+
+// Keys of a part where the sequences of a batch, at most 64, share `slots`
+// workgroups a key head: as few as leave none over, but not below `least`, nor so
+// few that a sequence has more than `splits` parts.  n: lane i has the length of
+// sequence i, others 0.  `parts` are the lane's, one where it has no keys, and
+// `upto` those of all sequences to it.
+DEV_INLINE int even_keys(const int n, const int seqs, const int slots,
+                         const int least, const int splits, int* parts,
+                         int* upto) {
+  const int lane = threadIdx.x & 63;
+  const int rounds = (max(n, 0) + PART_ROUND - 1) / PART_ROUND;
+  const int longest = __builtin_amdgcn_readlane(up_to_lane<true>(rounds), 63);
+  int span = least / PART_ROUND;
+  *parts = lane < seqs;
+  *upto = min(lane + 1, seqs);
+  if (longest <= span) return least;
+  const int all = __builtin_amdgcn_readlane(up_to_lane<false>(rounds), 63);
+  span = max(span, max((all + slots - 1) / slots,
+                       (longest + splits - 1) / splits));
+  for (;; span += max(1, span / 8)) {
+    *parts = lane < seqs ? max(1, (rounds + span - 1) / span) : 0;
+    *upto = up_to_lane<false>(*parts);
+    if (span >= longest || __builtin_amdgcn_readlane(*upto, 63) <= slots)
+      return span * PART_ROUND;
+  }
+}
+
 // A workgroup per query head adds the parts' sums, in shares that meet in LDS.
 // Bound by latency: the loads of a round of 8 parts are independent (one load
 // after another took 9-10 us for 16 parts of one sequence).  Of more than 8

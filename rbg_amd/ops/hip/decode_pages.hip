@@ -17,6 +17,13 @@
 //    lengths fills the chip as a regular one does; longer ones only where the
 //    grid has too few for the sequence.  The grid is fixed when a step is
 //    captured; workgroups past the end of their sequence leave at once.
+//    Few sequences share one workgroup a CU: every wave reads all lengths, takes
+//    the shortest parts that leave none over, and finds its own among those that
+//    have keys.  A CU with two workgroups takes twice as long as the others, and
+//    with fixed parts, and workgroups without keys between them, some had two: 7 of
+//    300 to 3000 tokens 19.6 -> 16.0 us, 3 of 10500 to 15000 38.1 -> 33.7, 20 of 400
+//    to 6000 61 -> 56, 16 of 4000 to 16000 138 -> 128, 30 of 400 to 4000 with 2 key
+//    heads 25.0 -> 19.2; but 7 of 100 7.3 -> 7.6.
 //  * With a ticket per (sequence, key head), which the caller keeps and which is
 //    0 between launches, the last workgroup of a sequence adds up what its parts
 //    left: no launch of its own, which costs 1 to 3 us (1 sequence of 100 keys
@@ -77,6 +84,7 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     const int kv_heads, const int seqs, const int splits,
     const int* __restrict__ tables,         // [seqs, max_pages]
     const int max_pages, const int least, const int whole,
+    const int slots,                        // a key head's workgroups, or 0
     const __hip_bfloat16* __restrict__ q,   // [seqs, QH, DIM], rows q_stride
     const int q_stride, const float scale,  // to the base of 2
     __hip_bfloat16* keys,                   // [pages, KVH, PAGE, DIM]
@@ -97,8 +105,21 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     seq = pair % seqs;
     split = pair / seqs;
   }
-  const int ctx = lens[seq];
-  const int span = part_keys(ctx, least, whole, splits);
+  int ctx, span;
+  if (!TOGETHER && slots) {
+    const int in = threadIdx.x & 63;
+    const int n = in < seqs ? lens[in] : 0;
+    int parts, upto;
+    span = even_keys(n, seqs, slots, least, splits, &parts, &upto);
+    const uint64_t later = __ballot(upto > (int)blockIdx.y);
+    if (!later) return;
+    seq = __builtin_ctzll(later);
+    ctx = __builtin_amdgcn_readlane(n, seq);
+    split = blockIdx.y - __builtin_amdgcn_readlane(upto - parts, seq);
+  } else {
+    ctx = lens[seq];
+    span = part_keys(ctx, least, whole, splits);
+  }
   const int begin = split * span, end = min(ctx, begin + span);
   if (begin >= ctx && split > 0) return;
   const int lane = threadIdx.x & 63;
@@ -512,11 +533,21 @@ extern "C" void launch_decode_pages(
   // few keys beside one of many (128 sequences of 2080 and 8 heads 181 -> 171 us,
   // 96 of up to 2500 106 -> 101; 64 of up to 4000 143 -> 146, so not for fewer).
   const int whole = seqs * kv_heads >= 768 ? span + span / 4 : span;
-  const dim3 grid(kv_heads, seqs, splits), block(64 * WAVES);
+  // Up to as many sequences as a key head has CUs: one workgroup for every CU, dealt
+  // out by the lengths, which a wave sees at once (comment above).  More sequences
+  // leave two or three on a CU either way, and no order of parts of 512 to 2048 keys
+  // was better (45 of up to 2500 60 to 67 us).  Of one sequence parts of `span` keys
+  // come to the same.
+  const int cus = 256 / kv_heads;
+  const int slots =
+      tickets && splits > 1 && seqs > 1 && seqs <= min(cus, 64) ? cus : 0;
+  const dim3 grid(kv_heads, slots ? slots : seqs, slots ? 1 : splits);
+  const dim3 block(64 * WAVES);
 #define DP_LAUNCH(QPG, TOGETHER, PROJ)                                     \
   decode_pages_kernel<QPG, TOGETHER, PROJ><<<grid, block, 0, stream>>>(    \
       (const int*)lens, kv_heads, seqs, splits, (const int*)tables,        \
-      max_pages, span, whole, (const __hip_bfloat16*)q, q_stride,          \
+      max_pages, slots ? min(span, 256) : span, whole, slots,              \
+      (const __hip_bfloat16*)q, q_stride,                                  \
       scale * 1.44269504088896f, (__hip_bfloat16*)keys,                    \
       (__hip_bfloat16*)values, (float*)part_o, (float*)part_ml,            \
       (__hip_bfloat16*)out, (int*)tickets,                                 \

@@ -1241,6 +1241,42 @@ def test_skinny_gemm_forms(m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,kvh", [(4, 4), (8, 2), (32, 8), (16, 16)])
+@pytest.mark.parametrize("lens", [
+    [0, 700], [1, 128, 129, 256, 257], [9000, 40, 3000], [2049] * 16,
+    [100 + 37 * i for i in range(31)], [0] * 15 + [5000], list(range(64)),
+    [1500, 30] * 32])
+@pytest.mark.parametrize("splits", [2, 7, 32])
+def test_decode_shares_out_lengths(heads, kvh, lens, splits):
+    """Workgroups dealt out by the lengths, which a call with tickets takes for up to
+    256 / kvh sequences, against parts of a fixed length and their own join: weights
+    round to bf16 after other maxima (2^-9 of them each), results to bf16.  Twice, as
+    the tickets are zeros again."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(sum(lens) + kvh)
+    pages = sum((n + 15) // 16 for n in lens) + 1
+    kc, vc = (torch.randn(pages, kvh, 16, 128, device=dev, generator=gen).bfloat16()
+              for _ in "kv")
+    most = max((n + 15) // 16 for n in lens) + 3
+    table = torch.zeros(len(lens), most, dtype=torch.int32)
+    order, at = torch.randperm(pages - 1) + 1, 0
+    for i, n in enumerate(lens):
+        table[i, :(n + 15) // 16] = order[at:at + (n + 15) // 16]
+        at += (n + 15) // 16
+    q = torch.randn(len(lens), heads, 128, device=dev, generator=gen).bfloat16()
+    ctx = torch.tensor(lens, dtype=torch.int32, device=dev)
+    tickets = torch.zeros(len(lens) * kvh, dtype=torch.int32, device=dev)
+    args = q, kc, vc, table.to(dev), ctx, 0.09, splits
+    want = ops.decode_attention(*args).double()
+    bound = want.abs() * 2 ** -8 + vc.double().abs().max() * 2 ** -8
+    for _ in range(2):
+        got = ops.decode_attention(*args, tickets=tickets).double()
+        assert ((got - want).abs() <= bound).all()
+        assert not tickets.any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [5, 32, 33, 64])
 @pytest.mark.parametrize("n,k", [(4096, 768), (8192, 1280), (11264, 2816),
                                  (16448, 2304), (66048, 768), (16448, 2112)])
