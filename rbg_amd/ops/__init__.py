@@ -208,14 +208,32 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """linear(x, w).float(): the decode GEMM stores its rounded results so (a
-    launch of 2 to 4 us less)."""
+    launch of 2 to 4 us less), the GEMM of prompts its sums."""
     if _takes_stream(x, w):
         return _hip.stream_linear(x.contiguous(), w, 1)
     if _takes_skinny(x, w):
         return require("_hip_ops", "_hip_mix", "_hip_gated", "_hip_moe",
                        "_hip_hyper").skinny_gemm(
             x if x.is_contiguous() else x.contiguous(), w, wide=True)
+    if _hip is not None and _takes_tile(x, w, _tile_f32):
+        return _hip.tile_f32(x.contiguous(), w)
     return linear(x, w).float()
+
+
+def _tile_f32(rows: int, n: int, k: int) -> bool:
+    """Does the GEMM of prompts take a product in f32, rather than hipBLASLt and a
+    conversion (a launch and its result once more)?  From 65 rows, where the decode GEMM
+    ends, of wide matrices, as for fewer columns it would have to split k.  Own /
+    library over 16384 to 128256 columns, 2048 to 12288 k (us): 128 rows of 32768 x 4096
+    65 / 73, 32768 x 8192 117 / 142, 128256 x 4096 241 / 269, 65536 x 8192 even, of 16384
+    x 4096 48 / 41, of 32768 x 12288 187 / 184; k that is no multiple of 2048 only below
+    4096 (32768 x 3072: 48 / 54; 24576 x 5120: 73 / 70).  From 129 rows of the widest
+    (65536 x 5120: 129 rows 155 / 174, 192 rows 164 / 162; 32768 x 4096: 80 / 75)."""
+    if k < 1024 or k > 8192 or k % 64 or n % 64 or not _tile_fits(rows, n, k):
+        return False
+    if rows <= 128:
+        return rows > 64 and n >= 24576 and (k % 2048 == 0 or k <= 4096)
+    return rows <= 256 and n >= 49152 and k <= 6144
 
 
 def _tile_fits(rows: int, n: int, k: int) -> bool:

@@ -938,6 +938,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_swiglu", &skinny_swiglu, "decode gate/up GEMM with silu");
   m.def("tile_swiglu", &tile_swiglu, "gate/up GEMM of a prompt with silu");
   m.def("tile_parts", &tile_parts, "GEMM of a prompt, perhaps as parts' sums");
+  m.def("tile_f32", &tile_f32, "GEMM of a prompt with its result in f32");
   m.def("tile_form", &tile_form, "one form of these");
   m.def("norm_rows", &norm_rows, "norm, GEMM of a few rows and its end");
   m.def("stream_swiglu", &stream_swiglu, "gate/up GEMM of a few rows with silu");

@@ -170,6 +170,20 @@ inline torch::Tensor tile_parts(torch::Tensor a, torch::Tensor w) {
   return c;
 }
 
+// a W^T in f32.
+inline torch::Tensor tile_f32(torch::Tensor a, torch::Tensor w) {
+  check_tile(a, w);
+  const int M = a.size(0), N = w.size(0), K = a.size(1);
+  auto c = torch::empty({M, N}, a.options().dtype(torch::kFloat32));
+  TilePlan best{1e30f, nullptr, 1, nullptr, N};
+  for (const TileForm& f : TILE_FORMS) {
+    const float time = tile_time(f, M, N, K, TILE_PARTS, 1);
+    if (K / 64 >= f.fill && time < best.time) best = {time, &f, 1, nullptr, N};
+  }
+  launch_tile_plan(best, c.data_ptr(), a, w, TILE_PARTS);
+  return c;
+}
+
 // One form of the above, for tests: its number (TILE_FEW's after the others), the
 // parts, and for a second form the column that it begins at.
 inline torch::Tensor tile_form(torch::Tensor a, torch::Tensor w, int64_t end,

@@ -138,6 +138,20 @@ def test_swiglu_route(m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(65, 24576, 1024), (128, 24640, 2048),
+                                   (100, 32768, 1088), (129, 49152, 1024),
+                                   (256, 49216, 1024)])
+def test_f32_route(m, n, k):
+    from rbg_amd import ops
+    assert ops._tile_f32(m, n, k)
+    x, w, full, sums = _operands(m, n, k)
+    got = ops.linear_f32(x, w)
+    assert got.dtype == torch.float32 and got.shape == (m, n)
+    assert ((got.double() - full).abs() <= sums).all()
+    assert not ops._tile_f32(64, n, k) and not ops._tile_f32(257, n, k)
+
+
+@pytest.mark.gpu
 def test_refuses_what_it_cannot_take():
     from rbg_amd import ops
     dev = torch.device("cuda:0")
