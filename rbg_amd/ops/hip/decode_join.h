@@ -37,21 +37,29 @@ DEV_INLINE int up_to_lane(int x) {
   return x;
 }
 
+// Rounds of a part below which there is none: up to three are one part; a sequence
+// has as many as its join reads at once, `joins`, or 512 keys each (one of 300 / 1000 /
+// 2048 / 4000 / 8000 keys, 4 query heads, us: parts of 128 7.8 / 8.1 / 9.1 / 12.2 /
+// 19.9, of 256 8.6 / 9.2 / 9.6 / 10.4 / 14.3, of 512 7.1 / 11.7 / 12.2 / 12.2 / 13.1).
+DEV_INLINE int least_rounds(int longest, int joins) {
+  return longest <= 3 ? 3 : min(4, (longest + joins - 1) / joins);
+}
+
 // Keys of a part where the sequences of a batch, at most 64, share `slots`
-// workgroups a key head: as few as leave none over, but not below `least`, nor so
+// workgroups a key head: as few as leave none over, but not below the above, nor so
 // few that a sequence has more than `splits` parts.  n: lane i has the length of
 // sequence i, others 0.  `parts` are the lane's, one where it has no keys, and
 // `upto` those of all sequences to it.
 DEV_INLINE int even_keys(const int n, const int seqs, const int slots,
-                         const int least, const int splits, int* parts,
+                         const int joins, const int splits, int* parts,
                          int* upto) {
   const int lane = threadIdx.x & 63;
   const int rounds = (max(n, 0) + PART_ROUND - 1) / PART_ROUND;
   const int longest = __builtin_amdgcn_readlane(up_to_lane<true>(rounds), 63);
-  int span = least / PART_ROUND;
+  int span = least_rounds(longest, joins);
   *parts = lane < seqs;
   *upto = min(lane + 1, seqs);
-  if (longest <= span) return least;
+  if (longest <= span) return span * PART_ROUND;
   const int all = __builtin_amdgcn_readlane(up_to_lane<false>(rounds), 63);
   span = max(span, max((all + slots - 1) / slots,
                        (longest + splits - 1) / splits));
@@ -61,6 +69,15 @@ DEV_INLINE int even_keys(const int n, const int seqs, const int slots,
     if (span >= longest || __builtin_amdgcn_readlane(*upto, 63) <= slots)
       return span * PART_ROUND;
   }
+}
+
+// The same of one sequence.
+DEV_INLINE int even_keys(const int ctx, const int slots, const int joins,
+                         const int splits) {
+  const int rounds = (max(ctx, 0) + PART_ROUND - 1) / PART_ROUND;
+  const int most = min(slots, splits);
+  return max(least_rounds(rounds, joins), (rounds + most - 1) / most) *
+         PART_ROUND;
 }
 
 // A workgroup per query head adds the parts' sums, in shares that meet in LDS.

@@ -23,7 +23,7 @@
 //    with fixed parts, and workgroups without keys between them, some had two: 7 of
 //    300 to 3000 tokens 19.6 -> 16.0 us, 3 of 10500 to 15000 38.1 -> 33.7, 20 of 400
 //    to 6000 61 -> 56, 16 of 4000 to 16000 138 -> 128, 30 of 400 to 4000 with 2 key
-//    heads 25.0 -> 19.2; but 7 of 100 7.3 -> 7.6.
+//    heads 25.0 -> 19.2, one of 1000 9.2 -> 8.1; but 7 of 100 7.3 -> 7.6.
 //  * With a ticket per (sequence, key head), which the caller keeps and which is
 //    0 between launches, the last workgroup of a sequence adds up what its parts
 //    left: no launch of its own, which costs 1 to 3 us (1 sequence of 100 keys
@@ -106,11 +106,17 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     split = pair / seqs;
   }
   int ctx, span;
-  if (!TOGETHER && slots) {
+  constexpr int JOINS = 64 * WAVES / (QPG * DIM / 4) * 8;    // parts of a round
+  if (!TOGETHER && slots && seqs == 1) {
+    ctx = lens[0];
+    span = even_keys(ctx, slots, JOINS, splits);
+    split = blockIdx.y;
+    seq = 0;
+  } else if (!TOGETHER && slots) {
     const int in = threadIdx.x & 63;
     const int n = in < seqs ? lens[in] : 0;
     int parts, upto;
-    span = even_keys(n, seqs, slots, least, splits, &parts, &upto);
+    span = even_keys(n, seqs, slots, JOINS, splits, &parts, &upto);
     const uint64_t later = __ballot(upto > (int)blockIdx.y);
     if (!later) return;
     seq = __builtin_ctzll(later);
@@ -536,17 +542,16 @@ extern "C" void launch_decode_pages(
   // Up to as many sequences as a key head has CUs: one workgroup for every CU, dealt
   // out by the lengths, which a wave sees at once (comment above).  More sequences
   // leave two or three on a CU either way, and no order of parts of 512 to 2048 keys
-  // was better (45 of up to 2500 60 to 67 us).  Of one sequence parts of `span` keys
-  // come to the same.
+  // was better (45 of up to 2500 60 to 67 us).
   const int cus = 256 / kv_heads;
-  const int slots =
-      tickets && splits > 1 && seqs > 1 && seqs <= min(cus, 64) ? cus : 0;
+  const int slots = tickets && splits > 1 && seqs <= min(cus, 64)
+                        ? min(cus, seqs * splits) : 0;
   const dim3 grid(kv_heads, slots ? slots : seqs, slots ? 1 : splits);
   const dim3 block(64 * WAVES);
 #define DP_LAUNCH(QPG, TOGETHER, PROJ)                                     \
   decode_pages_kernel<QPG, TOGETHER, PROJ><<<grid, block, 0, stream>>>(    \
       (const int*)lens, kv_heads, seqs, splits, (const int*)tables,        \
-      max_pages, slots ? min(span, 256) : span, whole, slots,              \
+      max_pages, span, whole, slots,                                       \
       (const __hip_bfloat16*)q, q_stride,                                  \
       scale * 1.44269504088896f, (__hip_bfloat16*)keys,                    \
       (__hip_bfloat16*)values, (float*)part_o, (float*)part_ml,            \

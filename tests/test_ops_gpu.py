@@ -1245,7 +1245,7 @@ def test_skinny_gemm_forms(m, n, k):
 @pytest.mark.parametrize("lens", [
     [0, 700], [1, 128, 129, 256, 257], [9000, 40, 3000], [2049] * 16,
     [100 + 37 * i for i in range(31)], [0] * 15 + [5000], list(range(64)),
-    [1500, 30] * 32])
+    [1500, 30] * 32, [0], [384], [385], [2049], [16000]])
 @pytest.mark.parametrize("splits", [2, 7, 32])
 def test_decode_shares_out_lengths(heads, kvh, lens, splits):
     """Workgroups dealt out by the lengths, which a call with tickets takes for up to
