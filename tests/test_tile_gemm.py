@@ -189,6 +189,26 @@ def test_rules_hand_over_what_it_takes():
     assert min(taken) > 50
 
 
+def test_rules_of_f32_and_few_rows_hand_over_what_is_taken():
+    """Sizes that the tiles, and the decode GEMM with silu, refuse go elsewhere."""
+    from rbg_amd.ops import _glu, _tile_f32, _tile_few, _tile_fits
+    taken = [0, 0]
+    for n in (64, 4096, 4128, 16448, 24576, 24608, 49152, 65536, 128256, 131072):
+        for k in (64, 512, 768, 1000, 1088, 2048, 2112, 2304, 5120, 8192, 8256,
+                  16384):
+            for rows in (0, 1, 4, 5, 16, 17, 33, 64, 65, 128, 129, 256, 257):
+                if _tile_f32(rows, n, k):
+                    assert 64 < rows <= 256 and n % 64 == 0 and k % 64 == 0
+                    assert k >= 512 and _tile_fits(rows, n, k)
+                    taken[0] += 1
+                if _glu(rows, n, k):
+                    assert 1 <= rows <= 64 and n % 64 == 0 and k % 256 == 0
+                    taken[1] += 1
+                if _tile_few(rows, n, k):
+                    assert 4 < rows <= 64 and k >= 1024
+    assert min(taken) > 30
+
+
 @pytest.mark.parametrize("rows,n,k,fewer", [
     (130, 65536, 65536, (130, 65536, 65024)),
     (129, 131072, 32768, (129, 131072, 32512)),
