@@ -606,8 +606,8 @@ def _decode_span(pairs: int) -> Tuple[int, int]:
     19.7 / 29.8; 128 pairs of up to 2048 31 / 26 / 24 / 29; 360 pairs of up to
     2500 63 / 59 / 58 / 68; 512 pairs of up to 2048, 8 query heads each, 98 / 89 /
     84 / 76; 1024 pairs of 2080 224 / 191 / 177 / 174).  With
-    tickets and no more sequences than CUs for a key head the kernel finds the parts
-    by the lengths, at most this many of a sequence (hip/decode_join.h)."""
+    tickets and no more sequences than 64 and than CUs for a key head the kernel finds
+    the parts by the lengths, at most this many of a sequence (hip/decode_join.h)."""
     if pairs <= 64:
         return 256, 32
     if pairs <= 96:

@@ -45,30 +45,61 @@ DEV_INLINE int least_rounds(int longest, int joins) {
   return longest <= 3 ? 3 : min(4, (longest + joins - 1) / joins);
 }
 
+// ceil(x / y), exact for x + y to 2^21 (the quotient of x + y - 1/2 is 1/(2y) away from whole
+// numbers, and off by 2^-22 of itself at most): a division of whole numbers is 0.15 us
+// of a search for parts, which has several.
+DEV_INLINE int over(int x, int y) {
+  return (int)(((float)(x + y) - 0.5f) * __builtin_amdgcn_rcpf((float)y));
+}
+
 // Keys of a part where the sequences of a batch, at most 64, share `slots`
-// workgroups a key head: as few as leave none over, but not below the above, nor so
-// few that a sequence has more than `splits` parts.  n: lane i has the length of
-// sequence i, others 0.  `parts` are the lane's, one where it has no keys, and
-// `upto` those of all sequences to it.
+// workgroups a key head: as few as leave none over, or a sixteenth more, but not below
+// the above, nor so few that a sequence has more than `splits` parts.  Sequences that
+// use up the slots, and rows that stand for none, leave no cut for a long one: two
+// workgroups a slot then (`most`), if that saves more than a fifth of the keys of a
+// slot; a CU whose others have ended reads up to 2.5 times faster, so that less is no
+// gain (8 key heads, us, one a slot / two: 31 of 500 and one of 16000 181 / 42, 17 of
+// 8000 in 24 rows 119 / 105, 9 of 15000 in 16 118 / 101, 20 of 400 to 6000 in 24 63 /
+// 59, 32 of 200 to 2500 42 / 44, 24 of 8000 131 / 153; with three a slot as with two, to
+// 2%).  n: lane i has the length of sequence i, others 0.  `parts` are the lane's, one
+// where it has no keys, and `upto` those of all sequences to it.
 DEV_INLINE int even_keys(const int n, const int seqs, const int slots,
-                         const int joins, const int splits, int* parts,
-                         int* upto) {
+                         const int most, const int joins, const int splits,
+                         int* parts, int* upto) {
   const int lane = threadIdx.x & 63;
   const int rounds = (max(n, 0) + PART_ROUND - 1) / PART_ROUND;
   const int longest = __builtin_amdgcn_readlane(up_to_lane<true>(rounds), 63);
-  int span = least_rounds(longest, joins);
+  const int least = least_rounds(longest, joins);
   *parts = lane < seqs;
   *upto = min(lane + 1, seqs);
-  if (longest <= span) return span * PART_ROUND;
+  if (longest <= least) return least * PART_ROUND;
   const int all = __builtin_amdgcn_readlane(up_to_lane<false>(rounds), 63);
-  span = max(span, max((all + slots - 1) / slots,
-                       (longest + splits - 1) / splits));
-  for (;; span += max(1, span / 8)) {
-    *parts = lane < seqs ? max(1, (rounds + span - 1) / span) : 0;
+  const int from = max(least, over(longest, splits));
+  const auto fit = [&](int span, int places) {
+    *parts = lane < seqs ? max(1, over(rounds, span)) : 0;
     *upto = up_to_lane<false>(*parts);
-    if (span >= longest || __builtin_amdgcn_readlane(*upto, 63) <= slots)
-      return span * PART_ROUND;
+    return __builtin_amdgcn_readlane(*upto, 63) <= places;
+  };
+  const auto shortest = [&](int places) {
+    int low = max(from, over(all, places));
+    if (fit(low, places)) return low;
+    // a sequence has less than one part above its share
+    int high = places > seqs ? min(longest, over(all, places - seqs)) : longest;
+    while (high - low > max(1, low / 16)) {
+      const int mid = (low + high) / 2;
+      if (fit(mid, places)) high = mid;
+      else low = mid;
+    }
+    fit(high, places);
+    return high;
+  };
+  int span = shortest(slots);
+  if (most > 1 && span * slots > all + all / 2) {
+    const int two = shortest(2 * slots);
+    if (two * 5 < span * 2) span = two;
+    else fit(span, slots);
   }
+  return span * PART_ROUND;
 }
 
 // The same of one sequence.

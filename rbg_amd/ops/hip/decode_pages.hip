@@ -17,13 +17,16 @@
 //    lengths fills the chip as a regular one does; longer ones only where the
 //    grid has too few for the sequence.  The grid is fixed when a step is
 //    captured; workgroups past the end of their sequence leave at once.
-//    Few sequences share one workgroup a CU: every wave reads all lengths, takes
-//    the shortest parts that leave none over, and finds its own among those that
-//    have keys.  A CU with two workgroups takes twice as long as the others, and
-//    with fixed parts, and workgroups without keys between them, some had two: 7 of
-//    300 to 3000 tokens 19.6 -> 16.0 us, 3 of 10500 to 15000 38.1 -> 33.7, 20 of 400
-//    to 6000 61 -> 56, 16 of 4000 to 16000 138 -> 128, 30 of 400 to 4000 with 2 key
-//    heads 25.0 -> 19.2, one of 1000 9.2 -> 8.1; but 7 of 100 7.3 -> 7.6.
+//    Few sequences share one workgroup a CU, or two (even_keys): every wave reads all
+//    lengths, takes the shortest parts that leave none over, and finds its own among
+//    those that have keys.  A CU with two workgroups takes twice as long as the others,
+//    and with fixed parts, and workgroups without keys between them, some had two: 7 of
+//    300 to 3000 tokens 19.4 -> 14.9 us, 3 of 10500 to 15000 43 -> 33, 20 of 400 to
+//    6000 in 24 rows 60 -> 59, 16 of 4000 to 16000 138 -> 123, 31 of 500 and one of
+//    16000 81 -> 42, 30 of 400 to 4000 with 2 key heads 26 -> 18.  Over 70 batches it
+//    takes 0.85 of the time of fixed parts; eight take longer: six 0.2 to 0.9 us, for
+//    the search (7 of 100 6.0 -> 6.2), 11 of 300 to 6000 with 16 key heads 60.0 ->
+//    63.4, 25 of up to 4800 with two query heads a key head 60.2 -> 63.2.
 //  * With a ticket per (sequence, key head), which the caller keeps and which is
 //    0 between launches, the last workgroup of a sequence adds up what its parts
 //    left: no launch of its own, which costs 1 to 3 us (1 sequence of 100 keys
@@ -82,6 +85,7 @@ template <int QPG, bool TOGETHER, bool PROJ>
 __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     const int* __restrict__ lens,           // [seqs]
     const int kv_heads, const int seqs, const int splits,
+    const int most,                         // workgroups of a slot, below
     const int* __restrict__ tables,         // [seqs, max_pages]
     const int max_pages, const int least, const int whole,
     const int slots,                        // a key head's workgroups, or 0
@@ -116,7 +120,7 @@ __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     const int in = threadIdx.x & 63;
     const int n = in < seqs ? lens[in] : 0;
     int parts, upto;
-    span = even_keys(n, seqs, slots, JOINS, splits, &parts, &upto);
+    span = even_keys(n, seqs, slots, most, JOINS, splits, &parts, &upto);
     const uint64_t later = __ballot(upto > (int)blockIdx.y);
     if (!later) return;
     seq = __builtin_ctzll(later);
@@ -539,18 +543,23 @@ extern "C" void launch_decode_pages(
   // few keys beside one of many (128 sequences of 2080 and 8 heads 181 -> 171 us,
   // 96 of up to 2500 106 -> 101; 64 of up to 4000 143 -> 146, so not for fewer).
   const int whole = seqs * kv_heads >= 768 ? span + span / 4 : span;
-  // Up to as many sequences as a key head has CUs: one workgroup for every CU, dealt
-  // out by the lengths, which a wave sees at once (comment above).  More sequences
-  // leave two or three on a CU either way, and no order of parts of 512 to 2048 keys
-  // was better (45 of up to 2500 60 to 67 us).
+  // Up to as many sequences as a key head has CUs, and 64, whose lengths a wave sees
+  // at once: workgroups are dealt out by the lengths, one for every CU (comment above).
+  // More sequences leave two or three on a CU either way, and no order of parts of 512
+  // to 2048 keys was better (45 of up to 2500 60 to 67 us).
   const int cus = 256 / kv_heads;
-  const int slots = tickets && splits > 1 && seqs <= min(cus, 64)
+  const int slots = tickets && splits > 1 && seqs <= min(cus, 64) &&
+                            (int64_t)seqs * max_pages < 1 << 23   // even_keys
                         ? min(cus, seqs * splits) : 0;
-  const dim3 grid(kv_heads, slots ? slots : seqs, slots ? 1 : splits);
+  // a second one where sequences may use up the first (even_keys); it costs a batch
+  // that does not take it up to 0.3 us
+  const int most = seqs * 4 <= cus ? 1 : 2;
+  const dim3 grid(kv_heads, slots ? min(slots * most, seqs * splits) : seqs,
+                  slots ? 1 : splits);
   const dim3 block(64 * WAVES);
 #define DP_LAUNCH(QPG, TOGETHER, PROJ)                                     \
   decode_pages_kernel<QPG, TOGETHER, PROJ><<<grid, block, 0, stream>>>(    \
-      (const int*)lens, kv_heads, seqs, splits, (const int*)tables,        \
+      (const int*)lens, kv_heads, seqs, splits, most, (const int*)tables,  \
       max_pages, span, whole, slots,                                       \
       (const __hip_bfloat16*)q, q_stride,                                  \
       scale * 1.44269504088896f, (__hip_bfloat16*)keys,                    \

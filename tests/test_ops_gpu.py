@@ -1245,11 +1245,14 @@ def test_skinny_gemm_forms(m, n, k):
 @pytest.mark.parametrize("lens", [
     [0, 700], [1, 128, 129, 256, 257], [9000, 40, 3000], [2049] * 16,
     [100 + 37 * i for i in range(31)], [0] * 15 + [5000], list(range(64)),
-    [1500, 30] * 32, [0], [384], [385], [2049], [16000]])
+    [1500, 30] * 32, [0], [384], [385], [2049], [16000],
+    [500] * 31 + [16000], [5874 - 199 * i for i in range(28)] + [1] * 4,
+    [8000] * 17 + [1] * 7, [15000] * 9 + [1] * 7, [300] * 64 + [3000]])
 @pytest.mark.parametrize("splits", [2, 7, 32])
 def test_decode_shares_out_lengths(heads, kvh, lens, splits):
     """Workgroups dealt out by the lengths, which a call with tickets takes for up to
-    256 / kvh sequences, against parts of a fixed length and their own join: weights
+    256 / kvh sequences and 64, two for each of these where sequences or rows without
+    any leave none over, against parts of a fixed length and their own join: weights
     round to bf16 after other maxima (2^-9 of them each), results to bf16.  Twice, as
     the tickets are zeros again."""
     from rbg_amd import ops
@@ -1274,6 +1277,31 @@ def test_decode_shares_out_lengths(heads, kvh, lens, splits):
         got = ops.decode_attention(*args, tickets=tickets).double()
         assert ((got - want).abs() <= bound).all()
         assert not tickets.any()
+
+
+@pytest.mark.gpu
+def test_decode_cuts_one_long_among_many():
+    """As many sequences as a key head has CUs: the long one is cut all the same.  The
+    call with tickets takes about half of the time of fixed parts and their join; 2.2
+    times of it with the long one whole."""
+    from rbg_amd import ops
+    dev = torch.device("cuda:0")
+    kc, vc, tables, ctx = _paged(dev, [500] * 31 + [16000], 8, 16384)
+    q = torch.randn(32, 32, 128, device=dev).bfloat16()
+    tickets = torch.zeros(32 * 8, dtype=torch.int32, device=dev)
+
+    def least(**kw):
+        times = []
+        for _ in range(20):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in "be")
+            begin.record()
+            for _ in range(10):
+                ops.decode_attention(q, kc, vc, tables, ctx, 0.09, 8, **kw)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+    assert least(tickets=tickets) < 1.2 * least()
 
 
 @pytest.mark.gpu
