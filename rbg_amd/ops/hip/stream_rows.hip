@@ -95,9 +95,19 @@ struct Turn {
                          sg_u4 (&out)[SEG]) const {
 #pragma unroll
     for (int l = 0; l < SEG; ++l) *reinterpret_cast<sg_u4*>(lds + put[l]) = in[l];
+    meet();
 #pragma unroll
     for (int s = 0; s < SEG; ++s)
       out[s] = *reinterpret_cast<const sg_u4*>(lds + get + s * 256);
+    meet();                       // the next turn's stores stay behind these loads
+  }
+  // What lanes stored is there for the others of the wave: no instruction, but a bound
+  // on the compiler's order (644 shapes 0.99 to 1.0 of the time without; 12288 x 7168
+  // with a norm, 1 row 34.3 -> 31.0 us, 4096 x 7168, 4 rows 14.7 -> 15.1).
+  DEV_INLINE static void meet() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
   }
 };
 
@@ -397,11 +407,13 @@ __global__ __launch_bounds__(512, 2) void stream_kernel(
 // many workgroups are better, of more rows few (10240 x 8192, 1280 / 256, us: 1 row 29.6
 // / 30.4, 4 rows 39.1 / 31.5; with silu 28672 x 4096, 3584 / 1792 / 896 / 256: 1 row 38.9
 // / 40.0 / 40.7 / 41.3, 2 rows 43.1 / 40.0 / 41.4 / 41.3, 4 rows - / 42.1 / 42.0 / 42.1).
-constexpr int norm_stream_ahead(bool glu, int rows, int waves, int seg) {
+// Of one row and few k two groups ahead, but where a workgroup has no more than two (us,
+// one / two: 3072 x 1024 4.5 / 4.0, x 2048 5.3 / 5.0, but 4096 x 2048 5.6 / 5.8).
+constexpr int norm_stream_ahead(bool glu, int rows, int waves, int seg, bool many) {
   if (glu && rows == 1) return waves == 16 || seg > 4 ? 2 : 1;
   if (waves == 16) return seg < 4 ? 2 : 1;
   if (glu) return seg <= 4 ? 2 : 1;
-  if (rows == 1) return seg <= 2 ? 1 : 2;
+  if (rows == 1) return seg <= 2 && many ? 1 : 2;
   return seg <= 2 ? 4 : seg == 3 ? 3 : 2;
 }
 
@@ -425,8 +437,11 @@ bool launch_norm_stream(__hip_bfloat16* c, float* wide, const void* src,
   const int lds =
       WAVES * (Turn<SEG>::BYTES + groups * 16 * (int)sizeof(float));
   const auto kernel =
-      norm_stream_kernel<GLU, SUMS, ROWS, WAVES, SEG,
-                         norm_stream_ahead(GLU, ROWS, WAVES, SEG)>;
+      units > 768
+          ? norm_stream_kernel<GLU, SUMS, ROWS, WAVES, SEG,
+                               norm_stream_ahead(GLU, ROWS, WAVES, SEG, true)>
+          : norm_stream_kernel<GLU, SUMS, ROWS, WAVES, SEG,
+                               norm_stream_ahead(GLU, ROWS, WAVES, SEG, false)>;
   if (lds > 64 * 1024 &&
       hipFuncSetAttribute((const void*)kernel,
                           hipFuncAttributeMaxDynamicSharedMemorySize,
