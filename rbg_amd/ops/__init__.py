@@ -590,11 +590,11 @@ def norm_swiglu(src, residual, weight, eps: float, w):
     """linear_swiglu of the RMS norm of residual + src, and the new residual."""
     # of more rows than one where the norm does not cost more than its launch
     # (hip/stream_rows.hip launch_norm_rows)
-    rows, k = residual.shape
-    if _takes_rows(src, residual, weight, w) and (
-            rows == 1 or (src is None or src.dtype == torch.bfloat16) and
-            (rows == 2 or k <= 4096)):
-        return _require_hip().norm_rows(src, residual, weight, eps, w, 1)
+    if _takes_rows(src, residual, weight, w):
+        rows, k = residual.shape
+        if rows == 1 or (src is None or src.dtype == torch.bfloat16) and (
+                rows == 2 or k <= 4096):
+            return _require_hip().norm_rows(src, residual, weight, eps, w, 1)
     return linear_swiglu(_normed(src, residual, weight, eps), w), residual
 
 
