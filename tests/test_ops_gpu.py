@@ -935,25 +935,6 @@ def test_stream_rows(rows, n, k):
         assert (out.double() - want).norm() <= 2 ** -7 * want.norm()
 
 
-@pytest.mark.parametrize("shape", [(64,), (3, 64), (2, 3, 64), (0, 64)])
-def test_norm_swiglu_of_any_rows(shape):
-    """Rows in any number of dimensions, as the norm and the product take them; within
-    2^-6 of the values' scale, as both and silu round to bf16."""
-    from rbg_amd import ops
-    gen = torch.Generator().manual_seed(len(shape))
-    src, res = (torch.randn(shape, generator=gen).bfloat16() for _ in "sr")
-    nw = torch.randn(64, generator=gen).bfloat16()
-    w = (torch.randn(96, 64, generator=gen) / 8).bfloat16()
-    total = src.double() + res.double()
-    h = total * (total.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * nw.double()
-    gate, up = (h @ w.double().t()).chunk(2, -1)
-    got, new = ops.norm_swiglu(src, res.clone(), nw, 1e-5, w)
-    assert got.shape == (*shape[:-1], 48) and new.shape == shape
-    bound = 2 ** -6 * (gate.abs() + 1) * (up.abs() + 1)
-    want = torch.nn.functional.silu(gate) * up
-    assert ((got.double() - want).abs() <= bound).all()
-
-
 @pytest.mark.gpu
 def test_linear_takes_what_the_library_takes():
     """Transposed and misaligned operands and gradients, at a shape that the

@@ -189,6 +189,25 @@ def test_rules_hand_over_what_it_takes():
     assert min(taken) > 50
 
 
+@pytest.mark.parametrize("shape", [(64,), (3, 64), (2, 3, 64), (0, 64)])
+def test_norm_swiglu_of_any_rows(shape):
+    """Rows in any number of dimensions, as the norm and the product take them; within
+    2^-6 of the values' scale, as both and silu round to bf16."""
+    from rbg_amd import ops
+    gen = torch.Generator().manual_seed(len(shape))
+    src, res = (torch.randn(shape, generator=gen).bfloat16() for _ in "sr")
+    nw = torch.randn(64, generator=gen).bfloat16()
+    w = (torch.randn(96, 64, generator=gen) / 8).bfloat16()
+    total = src.double() + res.double()
+    h = total * (total.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * nw.double()
+    gate, up = (h @ w.double().t()).chunk(2, -1)
+    got, new = ops.norm_swiglu(src, res.clone(), nw, 1e-5, w)
+    assert got.shape == (*shape[:-1], 48) and new.shape == shape
+    bound = 2 ** -6 * (gate.abs() + 1) * (up.abs() + 1)
+    want = torch.nn.functional.silu(gate) * up
+    assert ((got.double() - want).abs() <= bound).all()
+
+
 def test_rules_of_f32_and_few_rows_hand_over_what_is_taken():
     """Sizes that the tiles, and the decode GEMM with silu, refuse go elsewhere."""
     from rbg_amd.ops import _glu, _tile_f32, _tile_few, _tile_fits
