@@ -496,10 +496,13 @@ torch::Tensor decode_heads(torch::Tensor proj, int64_t heads,
               cos_sin.is_contiguous() && cos_sin.dim() == 2 &&
               cos_sin.size(1) == 128, "cos_sin must be fp32 [positions, 128]");
   for (const auto& t : {positions, slots, lens})
-    TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.numel() == seqs &&
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
                 t.scalar_type() == torch::kInt32, "an int32 per sequence");
+  // lengths and tables may be those of a larger batch, as decode_attention takes them
+  TORCH_CHECK(positions.numel() == seqs && slots.numel() == seqs &&
+              lens.numel() >= seqs, "a position, slot and length per sequence");
   TORCH_CHECK(block_tables.is_cuda() && block_tables.is_contiguous() &&
-              block_tables.dim() == 2 && block_tables.size(0) == seqs &&
+              block_tables.dim() == 2 && block_tables.size(0) >= seqs &&
               pages >= 1 && block_tables.scalar_type() == torch::kInt32,
               "int32 page tables");
   TORCH_CHECK(q_norm.has_value() == k_norm.has_value(), "both norms or none");

@@ -1083,8 +1083,12 @@ def test_decode_takes_raw_heads(heads, kvh, parts, norms, splits, span, many):
     tickets = torch.zeros(n * kvh, dtype=torch.int32, device=dev)
     for t in (None, tickets):
         mine = [kc.clone(), vc.clone()]
+        # with tickets: lengths and tables of a batch that has more rows
+        more = [] if t is None else [tables[:1], ctx[:1]]
         got = ops._hip.decode_heads(proj, heads, *nw, 1e-6, *mine, table, pos,
-                                    slots, tables, ctx, 0.09, splits, span, t)
+                                    slots, torch.cat([tables, *more[:1]]),
+                                    torch.cat([ctx, *more[1:]]), 0.09, splits, span,
+                                    t)
         assert not tickets.any()
         for a, b in zip(mine, other):
             # the last bit of a value, for another order of a norm's sum
