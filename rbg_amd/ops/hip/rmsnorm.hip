@@ -151,6 +151,64 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(
   }
 }
 
+// The same of parts for many long rows, which fill the chip only while two workgroups
+// of 1024 threads have room on a CU: a piece of the row after another, its residual
+// written before the next, the weight read when all are there.  (us, above / this: 300
+// rows of 5120 in 4 parts 9.1 / 9.8, of 8192 in 4 13.7 / 12.8, of 12288 in 3 18.2 /
+// 15.6, of 16384 in 4 27.2 / 23.6; 600 of 10240 in 2 19.8 / 19.5, of 8192 in 4 22.4 /
+// 24.8; 2048 of 10240 in 2 54.9 / 52.3; 256 of 13696 in 6 20.5 / 22.6.)
+__global__ __launch_bounds__(1024, 8) void add_rmsnorm_pieces_kernel(
+    const float* __restrict__ src, __hip_bfloat16* __restrict__ residual,
+    const int parts, const int rows, const int hidden, const int threads,
+    const __hip_bfloat16* __restrict__ w, __hip_bfloat16* __restrict__ out,
+    const float eps) {
+  constexpr int MOST = 4;
+  const int tid = threadIdx.x;
+  const size_t at = (size_t)blockIdx.x * hidden;
+  __shared__ float red[16];
+  union B4 { uint2 u; __hip_bfloat16 e[4]; };
+  B4 sum[MOST];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < MOST; ++i) {
+    const int col = (i * threads + tid) * 4;
+    if (col < hidden) {
+      B4 r;
+      r.u = *reinterpret_cast<const uint2*>(residual + at + col);
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+      for (int s = 0; s < parts; ++s)
+        v += *reinterpret_cast<const f32x4*>(src + at + col +
+                                             (size_t)s * rows * hidden);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float t = v[j] + bf2f(r.e[j]);
+        sum[i].e[j] = f2bf(t);
+        ss += t * t;
+      }
+      *reinterpret_cast<uint2*>(residual + at + col) = sum[i].u;
+    }
+  }
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  float total = 0.f;
+  for (int k = 0; k < threads >> 6; ++k) total += red[k];
+  const float inv = rsqrtf(total / hidden + eps);
+#pragma unroll
+  for (int i = 0; i < MOST; ++i) {
+    const int col = (i * threads + tid) * 4;
+    if (col < hidden) {
+      B4 g, o;
+      g.u = *reinterpret_cast<const uint2*>(w + col);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        o.e[j] = f2bf(bf2f(sum[i].e[j]) * inv * bf2f(g.e[j]));
+      *reinterpret_cast<uint2*>(out + at + col) = o.u;
+    }
+  }
+}
+
 template <int SOURCE>
 void norm_rows(void* out, const void* src, void* residual, const void* weight,
                float eps, int parts, int rows, int hidden, hipStream_t stream) {
@@ -161,14 +219,24 @@ void norm_rows(void* out, const void* src, void* residual, const void* weight,
         (const __hip_bfloat16*)weight, (__hip_bfloat16*)out, eps);
   };
   constexpr bool PARTS = SOURCE == NORM_PARTS;
-  // many rows hide the loads' latency by themselves, and fit in fewer registers
-  const bool many = PARTS && rows > 256;
-  if (hidden <= 4096) go(add_rmsnorm_row_kernel<SOURCE, 1, PARTS ? 8 : 1>, 1);
-  else if (hidden <= 8192 && many)
+  if (PARTS && rows > 256 && hidden > 4096 && (hidden > 8192 || rows <= 512)) {
+    const int threads = std::min(1024, (hidden / 4 + 63) / 64 * 64);
+    add_rmsnorm_pieces_kernel<<<dim3(rows), dim3(threads), 0, stream>>>(
+        (const float*)src, (__hip_bfloat16*)residual, parts, rows, hidden,
+        threads, (const __hip_bfloat16*)weight, (__hip_bfloat16*)out, eps);
+    return;
+  }
+  // a few loads on their way are enough, or better, where a second round of workgroups
+  // has only some (300 rows of 4096 in 6 parts 10.1 -> 9.2 us; 600 in 4 12.0 -> 13.4)
+  if (hidden <= 4096 && rows > 256 && rows <= 512)
+    go(add_rmsnorm_row_kernel<SOURCE, 1, 1>, 1);
+  else if (hidden <= 4096)
+    go(add_rmsnorm_row_kernel<SOURCE, 1, PARTS ? 8 : 1>, 1);
+  else if (hidden <= 8192 && PARTS && rows > 512)
     go(add_rmsnorm_row_kernel<SOURCE, 2, PARTS ? 2 : 1>, 2);
   else if (hidden <= 8192)
     go(add_rmsnorm_row_kernel<SOURCE, 2, PARTS ? 8 : 1>, 2);
-  else if (hidden <= 12288 && !many)
+  else if (hidden <= 12288)
     go(add_rmsnorm_row_kernel<SOURCE, 3, PARTS ? 6 : 1>, 3);
   else
     go(add_rmsnorm_row_kernel<SOURCE, 4, PARTS ? 2 : 1>, 4);

@@ -30,6 +30,7 @@ __global__ void silu_mul_kernel(__hip_bfloat16* __restrict__ out,   // [T, I]
 // The same of the f32 sums [parts, T, 2I] that a split GEMM left, for decode
 // batches: the reduction's launch (2 us) and its result's way through memory
 // are saved.
+template <int U>
 __global__ void silu_parts_kernel(__hip_bfloat16* __restrict__ out,  // [T, I]
                                   const float* __restrict__ x,
                                   const int parts, const int inter,
@@ -42,7 +43,7 @@ __global__ void silu_parts_kernel(__hip_bfloat16* __restrict__ out,  // [T, I]
   const float* p = x + row * 2 * inter + col;
   const size_t step = (size_t)total_vec * 8;
   f32x4 v[2] = {};                // gate, up
-  add_parts<8>(v, parts, [&](int s, int i) {
+  add_parts<U>(v, parts, [&](int s, int i) {
     return *reinterpret_cast<const f32x4*>(p + s * step + i * inter);
   });
   union { __hip_bfloat16 e[4]; uint2 u; } o;
@@ -59,8 +60,14 @@ extern "C" {
 void launch_silu_parts(void* out, const void* x, int parts, int tokens,
                        int inter, hipStream_t stream) {
   const long vecs = (long)tokens * (inter / 4);
-  silu_parts_kernel<<<dim3((vecs + 255) / 256), dim3(256), 0, stream>>>(
-      (__hip_bfloat16*)out, (const float*)x, parts, inter, vecs);
+  auto go = [&](auto kernel) {
+    kernel<<<dim3((vecs + 255) / 256), dim3(256), 0, stream>>>(
+        (__hip_bfloat16*)out, (const float*)x, parts, inter, vecs);
+  };
+  // parts on their way: eight, but two where there are many threads (16 rows of 10240
+  // in 6 parts 3.2 / 3.6 us; 200 of 13696 in 2 7.0 / 6.4, 600 of 5120 in 2 7.5 / 6.9)
+  if (vecs <= 1 << 17) go(silu_parts_kernel<8>);
+  else go(silu_parts_kernel<2>);
 }
 
 void launch_silu_mul(void* out, const void* x, int tokens, int inter,

@@ -1329,7 +1329,7 @@ def test_swiglu_of_odd_lengths(m, n, k):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows", [1, 7, 257])
+@pytest.mark.parametrize("rows", [1, 7, 256, 257, 512, 513])
 @pytest.mark.parametrize("hidden", [4, 256, 4096, 4100, 8192, 8196, 12288, 12292,
                                     16384])
 def test_norm_of_rows(rows, hidden):
