@@ -92,7 +92,11 @@ __global__ void rope_store_kv_kernel(
 // reduction nor copies and norms of the slices are launches of their own.
 // Eight lanes hold a head, each 8 neighbouring dims and the 8 they rotate
 // with: 16-byte accesses, and a norm is three shuffles.
-template <bool PARTS, bool NORM>
+// PARTS: those on their way at a time, of few heads eight, of more one, as there are
+// threads enough in fewer registers (us, a loop unrolled eight times / eight / one: 32 + 8
+// heads, 64 rows of 8 parts 4.8 / 4.2 / -, 1024 of 2 13.7 / 15.0 / 13.2, 2048 of 2 25.0 /
+// 26.7 / 24.7; 64 + 8 heads, 1024 of 2 20.5 / 23.7 / 20.0; of 984 sizes 0.94).
+template <int PARTS, bool NORM>
 __global__ __launch_bounds__(256) void rope_heads_kernel(
     const float* __restrict__ sums, __hip_bfloat16* __restrict__ q,
     const int parts, const int tokens, const int num_q_heads,
@@ -119,11 +123,11 @@ __global__ __launch_bounds__(256) void rope_heads_kernel(
            : (is_v ? v : k) + (size_t)token * kv_stride + kvh * D;
   const int d = lane * 8;
   float x[2][8];
-  if (PARTS) {
+  if constexpr (PARTS > 0) {
     const float* p = sums + ((size_t)token * heads + head) * D + d;
     const size_t step = (size_t)tokens * heads * D;
     f32x4 t[4] = {};
-    add_parts<8>(t, parts, [&](int s, int h) {
+    add_parts<PARTS>(t, parts, [&](int s, int h) {
       return *reinterpret_cast<const f32x4*>(p + s * step + (h >> 1) * 64 +
                                              (h & 1) * 4);
     });
@@ -218,10 +222,13 @@ void launch_rope_heads(void* q, void* k, void* v, const void* sums, int parts,
       (const __hip_bfloat16*)q_norm, (const __hip_bfloat16*)k_norm, eps,    \
       (const int*)slot_mapping, page_size, (__hip_bfloat16*)key_cache,      \
       (__hip_bfloat16*)val_cache)
-  if (parts && q_norm) RH_GO(true, true);
-  else if (parts) RH_GO(true, false);
-  else if (q_norm) RH_GO(false, true);
-  else RH_GO(false, false);
+  const bool many = units > 4096;
+  if (parts && many && q_norm) RH_GO(1, true);
+  else if (parts && many) RH_GO(1, false);
+  else if (parts && q_norm) RH_GO(8, true);
+  else if (parts) RH_GO(8, false);
+  else if (q_norm) RH_GO(0, true);
+  else RH_GO(0, false);
 #undef RH_GO
 }
 

@@ -512,7 +512,7 @@ def test_add_rmsnorm_rows(parts, rows, hidden):
 @pytest.mark.parametrize("parts", [0, 1, 6])
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("tokens,heads,kvh", [(1, 2, 1), (5, 32, 8),
-                                              (37, 6, 3)])
+                                              (37, 6, 3), (87, 32, 8)])
 def test_rope_heads(parts, norm, tokens, heads, kvh):
     """Head norms, rotation and store from bf16 rows (in place) and from the
     sums of a split GEMM, with a skipped slot; one rounding of the result."""
@@ -521,7 +521,7 @@ def test_rope_heads(parts, norm, tokens, heads, kvh):
     gen = torch.Generator(device=dev).manual_seed(tokens * 100 + parts)
     def rnd(*shape):
         return torch.randn(*shape, device=dev, generator=gen)
-    width, pages = (heads + 2 * kvh) * 128, 4
+    width, pages = (heads + 2 * kvh) * 128, max(4, tokens // 8)
     proj = (rnd(parts, tokens, width) if parts
             else rnd(tokens, width).bfloat16())
     x = (proj.double().sum(0) if parts else proj.double()).view(
