@@ -134,7 +134,7 @@ def _skinny(rows: int, n: int, k: int, parts: bool = False) -> bool:
         return k % 2048 == 0 or n <= 24576 and k <= 4096
     if n <= 12288 and k > 16384:
         return 16 < rows <= 256
-    if rows > 64:
+    if rows > 64 or _uneven(rows, n, k, parts):
         return False
     if n < 16384 and k <= 6144:
         return (k <= 1024 or k % 2048 == 0 and (n > 12288 or k <= 4096) or
@@ -146,6 +146,31 @@ def _skinny(rows: int, n: int, k: int, parts: bool = False) -> bool:
         return _after_rounds(rows, n, k)
     return not (32768 < n < 65536 and rows > 16 and
                 (k > 2560 if k % 2048 else k > 6144 and n <= 53248))
+
+
+def _uneven(rows: int, n: int, k: int, parts: bool) -> bool:
+    """Widths that _skinny gives away: a little above whole rounds of the decode GEMM's
+    workgroups, 32768 columns or with 32 rows of W a wave 65536 (own / library, us: 33152
+    x 4096, 48 rows 82.7 / 75.0, 32 rows even; 66048 x 3584, 64 rows 118 / 110, x 2560 56
+    rows 0.84; 102400 x 7168, 48 rows 312 / 270, 56 rows 0.94), 50304 to 52224, whose
+    second round is half full (x 5120: 5 rows 104 / 96, 16 rows 0.93; x 7168: 16 rows 141 /
+    131), and short ones where the library's tiles of 64 rows fill the chip (13696 x 1024,
+    64 rows 12.3 / 10.3; 15232 x 1536, 48 rows 15.5 / 14.7; 22016 x 7168, 24 rows 66 /
+    63)."""
+    if n < 16384:
+        return not parts and (rows > 56 if k <= 1024 else
+                              rows > 32 and k < 2048)
+    if 20480 < n < 24576:
+        return rows > 16 and k % 2048 > 0 and k > 6144
+    if 32768 < n < 36864 and rows > 40:
+        return 2048 < k <= 4096
+    if 40960 < n < 54272 and rows <= 16:
+        return k % 2048 > 0 and k > 4096 and (rows <= 8 or k > 6144)
+    if 65536 < n < 73728:
+        return k % 4096 > 0 and k > 2048 and (
+            rows > 56 or rows > 32 and 2560 < k < 4096)
+    return (98304 < n < 110592 and rows > 32 and rows % 16 == 0 and
+            k > (6144 if rows > 48 else 4096))
 
 
 def _after_rounds(rows: int, n: int, k: int) -> bool:
@@ -227,13 +252,27 @@ def _tile_f32(rows: int, n: int, k: int) -> bool:
     library over 16384 to 128256 columns, 2048 to 12288 k (us): 128 rows of 32768 x 4096
     65 / 73, 32768 x 8192 117 / 142, 128256 x 4096 241 / 269, 65536 x 8192 even, of 16384
     x 4096 48 / 41, of 32768 x 12288 187 / 184; k that is no multiple of 2048 only below
-    4096 (32768 x 3072: 48 / 54; 24576 x 5120: 73 / 70).  From 129 rows of the widest
-    (65536 x 5120: 129 rows 155 / 174, 192 rows 164 / 162; 32768 x 4096: 80 / 75)."""
+    4096 (32768 x 3072: 48 / 54; 24576 x 5120: 73 / 70).  Not where its tiles begin a
+    round that the library's do not (34048 x 1536: 128 rows 44.4 / 37.7; 50304 x 3584 102 /
+    94, but x 2048 0.85; 66048 x 4096: 128 rows 166 / 157, 72 rows 0.95; 102400 x 2560: 80
+    rows 143 / 131, 72 rows 0.86).  From 129 rows of the widest (65536 x 5120: 129 rows
+    155 / 174, 192 rows 164 / 162; 32768 x 4096: 80 / 75)."""
     if k < 1024 or k > 8192 or k % 64 or n % 64 or not _tile_fits(rows, n, k):
         return False
-    if rows <= 128:
-        return rows > 64 and n >= 24576 and (k % 2048 == 0 or k <= 4096)
-    return rows <= 256 and n >= 49152 and k <= 6144
+    if rows > 128:
+        return rows <= 256 and n >= 49152 and k <= 6144
+    if rows <= 64 or n < 24576:
+        return False
+    if k < 2048:
+        return not 32768 < n < 41984
+    fourth = rows >= 80 and 98304 < n < 126976
+    if k % 2048:
+        return k <= 4096 and not (49152 < n < 65536 or fourth or
+                                  rows > 112 and 65536 < n < 71680)
+    if rows > 112 and (32768 < n < 36864 and k == 4096 or
+                       65536 < n < 71680 and k > 2048):
+        return False
+    return k <= 4096 or not fourth
 
 
 def _tile_fits(rows: int, n: int, k: int) -> bool:

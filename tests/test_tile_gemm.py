@@ -228,6 +228,29 @@ def test_rules_of_f32_and_few_rows_hand_over_what_is_taken():
     assert min(taken) > 30
 
 
+@pytest.mark.parametrize("rows,n,k,taken", [
+    (48, 33152, 4096, False), (32, 33152, 4096, True), (48, 36864, 4096, True),
+    (5, 50304, 5120, False), (16, 50304, 5120, True), (16, 50304, 7168, False),
+    (5, 54272, 5120, True), (64, 66048, 3584, False), (56, 66048, 2560, True),
+    (48, 102400, 7168, False), (56, 102400, 7168, True), (64, 13696, 1024, False),
+    (24, 22016, 7168, False), (16, 22016, 7168, True)])
+def test_decode_gemm_between_rounds(rows, n, k, taken):
+    """Widths a little above whole rounds of workgroups, which are the library's, and
+    their neighbours."""
+    from rbg_amd import ops
+    assert ops._skinny(rows, n, k) == taken
+
+
+@pytest.mark.parametrize("rows,n,k,taken", [
+    (128, 34048, 1536, False), (128, 41984, 1536, True), (128, 34048, 2048, True),
+    (128, 50304, 3584, False), (128, 50304, 2048, True), (128, 49152, 3584, True),
+    (128, 66048, 4096, False), (72, 66048, 4096, True), (80, 102400, 2560, False),
+    (72, 102400, 2560, True), (128, 102400, 8192, False), (128, 128256, 8192, True)])
+def test_f32_tiles_between_rounds(rows, n, k, taken):
+    from rbg_amd import ops
+    assert ops._tile_f32(rows, n, k) == taken
+
+
 @pytest.mark.parametrize("rows,n,k,fewer", [
     (130, 65536, 65536, (130, 65536, 65024)),
     (129, 131072, 32768, (129, 131072, 32512)),
