@@ -382,20 +382,18 @@ def _glu(rows: int, n: int, k: int) -> bool:
 def _tile_few(rows: int, n: int, k: int) -> bool:
     """Does the GEMM of prompts take gate/up of 5 to 64 rows, in tiles of 64?  Asked
     after the decode GEMM (_glu), which reads its weights as well and leaves k that is
-    no multiple of 256.  There it takes 0.3 to 1.0 of the library and silu_mul over 16640
-    to 57344 columns, 2112 to 7232 k (us: 16640 x 4160: 5 rows 0.38, 64 rows 0.81; 36864 x
-    6080: 5 rows 1.01, 48 rows 0.87).  Of multiples of 2048, where a CU has about one
-    tile: to 20480 columns, from there to 26624 for more rows, and beyond 32768 with
-    tiles of 256, while one round holds them, 65536 columns (45056 x 4096: 64 rows 88 /
-    70); a full round leaves no CU to spare, and from 53248 columns only long k gain, for
-    more rows from 6144."""
+    no multiple of 256, and 65536 x 8192, where both and the library are even.  Of odd k
+    it takes 0.3 to 1.0 of the library and silu_mul over 16640 to 57344 columns, 2112 to
+    7232 k (us: 16640 x 4160: 5 rows 0.38, 64 rows 0.81; 36864 x 6080: 5 rows 1.01, 48
+    rows 0.87), 0.5 to 1.04 to 98304 columns, but of long k up to 32 rows only (73728 x
+    8000: 32 rows 271 / 370, 48 rows 273 / 232); not beyond (131072 x 4160: 5 rows 216 /
+    184)."""
     if not 4 < rows <= 64 or k < 2048 or k > 8192 or n <= 16384:
         return False
-    if k % 2048:
-        return k % 256 > 0
-    if n <= 32768:
-        return n <= (20480 if rows <= 32 else 26624)
-    return n <= 53248 or (n <= 65536 and k >= (8192 if rows <= 32 else 6144))
+    if k % 2048 == 0:       # a CU has about one tile; of these _glu leaves one size
+        return n <= 26624 or 32768 < n <= 65536
+    return k % 256 > 0 and (n <= 57344 or
+                            n <= 98304 and (k <= 7232 or rows <= 32))
 
 
 def _tile_glu(rows: int, n: int, k: int) -> bool:

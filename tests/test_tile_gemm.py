@@ -127,12 +127,18 @@ def test_parts_route(m, n, k):
 @pytest.mark.parametrize("m,n,k", [
     (5, 16448, 2048), (33, 26624, 2048), (33, 65536, 6144), (64, 32832, 2048),
     (16, 18432, 4160), (63, 36864, 4096),
+    (64, 16448, 2112), (33, 32768, 2112), (5, 32832, 2112), (33, 36864, 4160),
+    (64, 57408, 2112), (17, 65536, 8192),
     (65, 24576, 1024), (128, 28672, 1088), (129, 8192, 2048),
     (256, 18432, 2048), (385, 28672, 1024), (1000, 11264, 2048),
     (2048, 28672, 1024)])
 def test_swiglu_route(m, n, k):
+    """In tiles, but for what the decode GEMM is asked for first: few rows of k that is
+    a multiple of 2048, below 65536 columns or 8192 k."""
     from rbg_amd import ops
     assert ops._tile_glu(m, n, k)
+    first = m <= 64 and k % 2048 == 0 and n * k < 2 ** 29
+    assert ops.block_routes(m, (n, k), (n, k), True)[0] == (3 if first else 4)
     x, w, full, sums = _operands(m, n, k)
     assert _near(ops.linear_swiglu(x, w), GLU, full, sums)
 
@@ -226,6 +232,27 @@ def test_rules_of_f32_and_few_rows_hand_over_what_is_taken():
                 if _tile_few(rows, n, k):
                     assert 4 < rows <= 64 and k >= 1024
     assert min(taken) > 30
+
+
+def test_gate_up_of_few_rows_goes_where_the_rules_say():
+    """The decode GEMM is asked first, and leaves the tiles k that is no multiple of 256
+    and one size of those that are."""
+    from rbg_amd.ops import _glu, _own_routes, _tile_few
+    left = set()
+    for n in range(16448, 131073, 1216):
+        for k in (2048, 2112, 2304, 4096, 4160, 6144, 7232, 7296, 8192, 8256):
+            for rows in (4, 5, 32, 33, 64, 65):
+                route = _own_routes(rows, (n, k), (n, k), True)[0]
+                assert (route == 3) == _glu(rows, n, k)
+                if rows <= 64:
+                    assert (route == 4) == (_tile_few(rows, n, k) and
+                                            not _glu(rows, n, k))
+                    if route == 4:
+                        left.add(k % 256)
+                        assert n <= (98304 if k <= 7232 or rows <= 32 else 57344)
+    assert left == {7296 % 256, 64}
+    assert _own_routes(48, (65536, 8192), (65536, 8192), True)[0] == 4
+    assert all(_glu(rows, n, 8192) for rows in (5, 64) for n in (32768, 65472))
 
 
 @pytest.mark.parametrize("rows,n,k,taken", [
