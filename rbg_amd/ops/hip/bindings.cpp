@@ -322,8 +322,10 @@ torch::Tensor stream_swiglu(torch::Tensor a, torch::Tensor w) {
 
 // Up to 4 rows: the RMS norm of residual + src (bf16, or f32 sums [1, M, K] of
 // stream_linear; it may be missing), a GEMM and its end in one launch: the product in
-// bf16 (0), silu(gate) * up (1; perhaps behind a launch of the norm's own), or the
-// product's f32 sums [1, M, N] (2).  Returns that and the new residual, which is another tensor unless src is missing.
+// bf16 (0, which the models leave for 2), silu(gate) * up (1; what launch_norm_rows
+// refuses behind a launch of the norm's own, which ops.norm_swiglu does in place), or
+// the product's f32 sums [1, M, N] (2).  Returns that and the new residual, which is
+// another tensor unless src is missing.
 std::vector<torch::Tensor> norm_rows(c10::optional<torch::Tensor> src,
                                      torch::Tensor residual,
                                      torch::Tensor norm_weight, double eps,

@@ -31,6 +31,9 @@ constexpr int ROWS_KC = 64, ROWS_DEPTH = 4, ROWS_MOST = 4;
 // launch would add.  4096 x 4096, one row: 8.5 us against 10.5 of
 // skinny_gemm_kernel with its reduction.  Its time grows with the rows, since
 // every workgroup reads all of A (28672 x 4096: 1 row 41.8 us, 4 rows 44.3).
+// Where stream_rows.hip is linked it takes what has 1024 columns and k or more, but
+// the widest of 2048 k (ops._stream); this takes the others, and all of them in a
+// process with an extension of another family alone.
 // GLU: W's halves are gate and up, the tile is 8 rows of each: silu(gate) * up.
 // PAIR: the tile is 8 rows of W, whose k are taken two chunks at a time, so that
 // twice as many workgroups are half as long.  For matrices whose tiles of 16 rows
