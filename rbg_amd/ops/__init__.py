@@ -203,8 +203,8 @@ def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
 def _stream(rows: int, n: int, k: int) -> bool:
     """Does the GEMM of up to 4 rows (hip/stream_rows.hip) take a [rows, k] x [n, k]
     product?  Of 268 of 1024 to 128256 columns and 1024 to 25600 k, 1 to 4 rows with
-    cold weights, it takes 0.84 of the time of what is taken without it, and of 10 of
-    them 0.2 to 3% more.  Not the widest of 2048 k, which the decode GEMM takes as one
+    cold weights, it takes 0.82 of the time of what is taken without it, and of 7 of
+    them, of 25600 k, 0.2 to 3% more.  Not the widest of 2048 k, which the decode GEMM takes as one
     turn (us, 1 row: 128256 x 2048 84.6 / 90.6, 65536 x 2048 44.9 / 46.3, 49152 x 2048
     33.5 / 33.8, 65536 x 1024 27.4 / 22.5)."""
     return (1 <= rows <= 4 and n >= 1024 and n % 32 == 0 and k >= 1024 and
@@ -575,9 +575,9 @@ def _takes_rows(src, residual: torch.Tensor, weight: torch.Tensor,
                 w: torch.Tensor) -> bool:
     """Can norm and GEMM of up to 4 rows be one launch (hip/stream_rows.hip)?  Its
     waves hold an eighth of k of the rows, a sixteenth above 5120, in registers.  Of 184
-    shapes of 1536 to 12288 columns and 1024 to 8192 k it takes 0.76 of the time of what
-    was taken before, with silu of 4096 to 57344 columns 0.83 of 192; slower by 0.2 to
-    2.5% are ten of 6144 k, by 5% 8192 x 6144 of one row."""
+    shapes of 1536 to 12288 columns and 1024 to 8192 k it takes 0.74 of the time of what
+    was taken before, with silu of 4096 to 57344 columns 0.81 of 192; slower by 1 to
+    1.5% are two of 6144 k, with silu."""
     return (_takes_stream(residual, w) and residual.shape[1] <= 8192 and
             residual.is_contiguous() and weight.data_ptr() % 16 == 0 and
             (src is None or (src.numel() == residual.numel() and

@@ -408,10 +408,12 @@ __global__ __launch_bounds__(512, 2) void stream_kernel(
 // / 30.4, 4 rows 39.1 / 31.5; with silu 28672 x 4096, 3584 / 1792 / 896 / 256: 1 row 38.9
 // / 40.0 / 40.7 / 41.3, 2 rows 43.1 / 40.0 / 41.4 / 41.3, 4 rows - / 42.1 / 42.0 / 42.1).
 // Of one row and few k two groups ahead, but where a workgroup has no more than two (us,
-// one / two: 3072 x 1024 4.5 / 4.0, x 2048 5.3 / 5.0, but 4096 x 2048 5.6 / 5.8).
+// one / two: 3072 x 1024 4.5 / 4.0, x 2048 5.3 / 5.0, but 4096 x 2048 5.6 / 5.8), of many
+// k one (8192 x 6144 19.3 / 21.3, 4 rows 21.7 / 21.2; 51200 x 5632 with silu, 2 rows 108
+// / 102).
 constexpr int norm_stream_ahead(bool glu, int rows, int waves, int seg, bool many) {
   if (glu && rows == 1) return waves == 16 || seg > 4 ? 2 : 1;
-  if (waves == 16) return seg < 4 ? 2 : 1;
+  if (waves == 16) return seg < 4 && (glu || rows > 1) ? 2 : 1;
   if (glu) return seg <= 4 ? 2 : 1;
   if (rows == 1) return seg <= 2 && many ? 1 : 2;
   return seg <= 2 ? 4 : seg == 3 ? 3 : 2;
