@@ -80,7 +80,10 @@ DEV_INLINE f32x2 dp_shared(const float* from) {
 // them, and puts them in place of what registers already hold of that row.  The
 // rotation's own launch was 3 us of a layer (six layers, us: 7 sequences of qwen 8b
 // 715 -> 700, 45 of 8b 1109 -> 1097, 64 of qwen 32b, four layers, 1282 -> 1275, 128 of
-// 8b 2017 -> 2014).
+// 8b 2017 -> 2014).  With the parts by the lengths 80 batches of 1 to 256 sequences,
+// from bf16 and 1, 5 and 12 parts, take 0.77 of the time of rotation and fixed parts, 25
+// of up to 4800 and 11 of 300 to 6000 of the above 1 to 3% more or less, and 256 of 40
+// tokens 1.0 to 1.07, as each has a workgroup's start.
 template <int QPG, bool TOGETHER, bool PROJ>
 __global__ __launch_bounds__(64 * WAVES, 3) void decode_pages_kernel(
     const int* __restrict__ lens,           // [seqs]
