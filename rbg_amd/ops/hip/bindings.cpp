@@ -1052,6 +1052,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_parts", &tile_parts, "GEMM of a prompt, perhaps as parts' sums");
   m.def("tile_f32", &tile_f32, "GEMM of a prompt with its result in f32");
   m.def("tile_form", &tile_form, "one form of these");
+  m.def("tile_split", &tile_split, "the parts of tile_parts");
   m.def("norm_rows", &norm_rows, "norm, GEMM of a few rows and its end");
   m.def("stream_swiglu", &stream_swiglu, "gate/up GEMM of a few rows with silu");
   m.def("stream_linear", &stream_linear, "GEMM of a few rows",

@@ -101,12 +101,22 @@ inline TilePlan pick_tile(int M, int N, int K, int end) {
 }
 
 // Parts of K whose f32 sums a reader adds up, where that is faster with what it reads
-// more than bf16, at 4 TB/s.  A short k of many rows stays whole, as the library's is:
-// parts would gain 3 us of 35 at most (4096 x 4096, 384 rows 30 / 27, 640 rows 38 / 35,
-// 1024 rows 43 / 44; 6144 x 4096, 320 rows 36 / 33, 640 rows 46.5 / 44.5).
+// more than bf16, at 4 TB/s.  A k below 4736 of more than 256 rows stays whole: it
+// stands in for a rounded product of the library, and is rounded as that is.  In parts
+// it would be sooner (us with the norm, library / whole / parts: 4096 x 4096, 288 rows
+// 29.4 / 28 / 24.4, 384 rows 29.6 / 33 / 27.2; 6144 x 4096, 384 rows 42 / 41 / 35), and
+// ops._tile leaves the library the sizes at which the whole tiles are the slower ones.
 inline TilePlan pick_tile_parts(int M, int N, int K) {
   TilePlan best = pick_tile(M, N, K, TILE_PLAIN);
-  if (M > 256 && K < 5120) return best;
+  if (M > 256 && K < 4736) return best;
+  // Where both are within 10% the reader gets the f32 sums, not a rounded product.  Of
+  // results up to 5.25 M the model has parts of a long k too slow (whole / parts, us:
+  // 288 x 10240 x 5120 59.0 / 53.4, 384 65.0 / 56.9; 800 x 6144 x 5120 67.9 / 61.6; of 82
+  // sizes that this line and the one above split 0.91 of the time, 974 x 4416 x 4800
+  // 49.9 / 55.8), not of larger ones (704 x 10240 x 8192 112 / 115, 768 112 / 119) nor
+  // of a short k (88 x 12096 x 1024 14.9 / 16.1).
+  float least = best.time;
+  if (K >= 3584 && (long)M * N <= 5250000) least *= 1.1f;
   for (const TileForm& f : TILE_FORMS)
     for (int parts : {2, 3, 4, 5, 6, 8, 10, 12}) {
       const int tiles =
@@ -116,9 +126,19 @@ inline TilePlan pick_tile_parts(int M, int N, int K) {
       if (tiles * parts > 256 || !tile_takes(f, K / parts, TILE_PARTS)) break;
       const float time = tile_time(f, M, N, K, TILE_PARTS, parts) +
                          (4 * parts - 2) * 2.5e-7f * M * N;
-      if (time < best.time) best = {time, &f, parts, nullptr, N};
+      if (time < least) {
+        least = time;
+        best = {time, &f, parts, nullptr, N};
+      }
     }
   return best;
+}
+
+// The parts of tile_parts, for tests.
+inline int64_t tile_split(int64_t M, int64_t N, int64_t K) {
+  TORCH_CHECK(M >= 1 && N >= 64 && K >= 256 && M < (1 << 24) && N < (1 << 24) &&
+              K < (1 << 24), "sizes");
+  return pick_tile_parts((int)M, (int)N, (int)K).parts;
 }
 
 inline void check_tile(const torch::Tensor& a, const torch::Tensor& w) {

@@ -404,3 +404,16 @@ def test_rules_by_the_result():
     assert _tile(200, 2048, 2112) and not _tile(200, 2048, 2048)
     assert not _tile_glu(320, 36864, 5120) and not _tile_glu(384, 24576, 5120)
     assert not _tile_glu(300, 4096, 8192) and _tile_glu(2100, 4096, 8192)
+
+
+@pytest.mark.parametrize("rows,n,k", [
+    (163, 13312, 3584), (191, 14336, 4096), (257, 10880, 5376), (300, 13824, 5120),
+    (313, 12288, 5120), (450, 9216, 5120), (600, 7168, 5120), (786, 6464, 16896),
+    (797, 6528, 13824), (800, 5120, 5120), (800, 6144, 5120), (1050, 4096, 4992),
+    (1112, 4608, 5504)])
+def test_sums_of_these_are_not_rounded(rows, n, k):
+    """A reader that adds up gets these products in f32 parts."""
+    from rbg_amd import ops
+    if ops._hip is None:
+        pytest.skip("extension not built")
+    assert ops._tile(rows, n, k) and ops._hip.tile_split(rows, n, k) > 1
