@@ -385,17 +385,23 @@ def _tile_few(rows: int, n: int, k: int) -> bool:
 
 
 def _tile_glu(rows: int, n: int, k: int) -> bool:
-    """Does it take a gate/up product, with silu?  Against the product by linear_parts or
-    the library and silu_mul, over 4400 shapes of 65 to 9500 rows, 2048 to 65536 columns
-    and 1024 to 28672 k: 0.75 to 0.9 of the time to 2048 k and 0.9 to 0.95 of the longer,
-    where its tiles fill the chip (us: 28672 x 4096: 300 rows 82 / 72, 640 rows 147 / 127,
-    2048 rows 381 / 342; 11264 x 2048: 96 rows 21.1 / 18.4, 1600 rows 95 / 68), which by the
-    size of the result they have to do the more the longer k is, as parts of k, which
-    silu cannot have, do then (4096 x 8192: 320 rows 1.8 times, 1500 rows 1.1; 8192 x
-    28672: 1200 rows 472 / 495).  Wide matrices are a round of tiles of any rows (28672 x
-    4096: 65 rows 56 / 45), but for a part of a second one (36864 x 8192: 320 rows 1.09;
-    24576 x 5120: 192 rows 1.14).  The rule takes 0.6% more than the faster of each, and
-    more than 8% of 111."""
+    """Does it take a gate/up product, with silu?  Against what linear_swiglu would take
+    instead, over 4400 shapes of 65 to 9500 rows, 2048 to 65536 columns and 1024 to 28672
+    k: 0.75 to 0.9 of the time to 2048 k and 0.9 to 0.95 of the longer, where its tiles
+    fill the chip (us: 28672 x 4096: 300 rows 82 / 72, 640 rows 147 / 127, 2048 rows 381 /
+    342; 11264 x 2048: 96 rows 21.1 / 18.4, 1600 rows 95 / 68), which by the size of the
+    result they have to do the more the longer k is.
+
+    Instead of it stand, to 16384 columns, the parts of linear_parts, which silu cannot
+    have here and which fill the chip with a small result (4096 x 8192: 320 rows 1.8 times,
+    1500 rows 1.1); they keep f32 too, up to sizes that the rule knows.  Of more columns
+    it is the library and silu_mul, which round gate and up to bf16.  What is taken there
+    by its range is 0.94 of that time over 97 sizes where the result alone would not tell
+    (24576 x 4096: 65 rows 54.8 / 44.9, 80 rows 54.6 / 45.9, 96 rows 51.6 / 47.5; 23552 x
+    16512: 623 rows 0.58) and up to 1.15 for some of long k (36480 x 8704: 256 rows 1.11;
+    32704 x 12608: 170 rows 1.15).  Left to the library are a part of a second round
+    (36864 x 8192: 320 rows 1.09) and few rows of the widest (51200 x 5120: 65 to 99 rows
+    117 / 127)."""
     if (k < 1024 or k % 64 or n < 2048 or n % 64 or
             not _tile_fits(rows, n, k)):
         return False
@@ -403,6 +409,17 @@ def _tile_glu(rows: int, n: int, k: int) -> bool:
         return _tile_few(rows, n, k)
     if k <= 1536:
         return True
+    if n > 16384:
+        if k <= n and (24576 <= n <= 32768 if rows <= 128 else
+                       not 256 < rows <= 384):
+            return True
+    elif k <= n:        # where linear_parts has no sums, but one rounded product
+        if n > 12288 and rows > 256 and (
+                k < 4736 or (rows > 512 or k < 10240) and
+                rows * n > (6_300_000 if k >= 8192 else 5_500_000)):
+            return True
+        if n >= 8192 and rows > 128 and k < 3584 and rows * n > 1_590_000:
+            return True
     if 24576 < n <= 32768 and k <= 8192 or n > 49152 and k > 6144:
         return True
     if k > 4096 and (20480 < n <= 24576 and rows <= 384 or

@@ -417,3 +417,46 @@ def test_sums_of_these_are_not_rounded(rows, n, k):
     if ops._hip is None:
         pytest.skip("extension not built")
     assert ops._tile(rows, n, k) and ops._hip.tile_split(rows, n, k) > 1
+
+
+def _in_f32_all_along(rows, n, k):
+    """Sizes of more than 64 rows whose gate and up silu has always had unrounded."""
+    if n < 8192 or k > n or k < 1024 or k % 64 or n % 64 or rows <= 64:
+        return False
+    if rows <= 128:
+        return 24576 <= n <= 32768
+    if k >= 3584 and n <= (16384 if rows <= 256 else 12288) and rows < 1000:
+        return False
+    return rows <= 256 or rows > 384 or n <= 16384
+
+
+def test_gate_up_is_not_rounded_before_silu():
+    """They go to the tiles with silu, or where the parts that linear_parts makes are
+    sooner, to those."""
+    from rbg_amd import ops
+    if ops._hip is None:
+        pytest.skip("extension not built")
+    seen = [0, 0]
+    for n in (*range(8192, 16385, 320), *range(16448, 65537, 2048), 24576, 28672,
+              51200, 57344):
+        for k in (*range(1024, 6000, 192), *range(6144, 20000, 1024), 8704):
+            for rows in (65, 80, 99, 128, 129, 160, 200, 256, 257, 300, 384, 385,
+                         450, 490, 512, 513, 600, 999, 1000, 2048):
+                if _in_f32_all_along(rows, n, k) and ops._tile_fits(rows, n, k):
+                    fused = ops._tile_glu(rows, n, k)
+                    seen[fused] += 1
+                    assert fused or (ops._route(rows, n, k, True) == 2 and
+                                     ops._hip.tile_split(rows, n, k) > 1), \
+                        (rows, n, k)
+    assert min(seen) > 1000
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [
+    (65, 24576, 4096), (99, 24576, 4096), (200, 22528, 5120), (155, 38912, 2112),
+    (600, 12800, 8192), (210, 8192, 3008), (440, 14080, 9728), (330, 14336, 4608)])
+def test_swiglu_by_unrounded_gates(m, n, k):
+    from rbg_amd import ops
+    assert ops.block_routes(m, (n, k), (n, k), True)[0] == (2 if m == 440 else 4)
+    x, w, full, sums = _operands(m, n, k)
+    assert _near(ops.linear_swiglu(x, w), GLU, full, sums)
