@@ -293,19 +293,39 @@ def _tile(rows: int, n: int, k: int) -> bool:
     4096: 1200 rows 55 / 47; 8192 x 28672: 400 rows 420 / 200).  The rule takes 0.5%
     more than the faster one of each.  Left to the others is a short k of a small result,
     which the library's smaller tiles end sooner (2048 x 2048: 200 rows 12.8 / 13.1, 640
-    rows 17.2 / 16.5; 3072 x 2048: 150 rows 13.0 / 14.9, 704 rows 21 / 19; 1400 x 2560:
-    300 rows 14.2 / 19), of up to 256 rows only if it is a multiple of 128 (1984 x 6144:
-    113 rows 23 / 16) or below 1536; and rows longer than the norm takes sums of.  Of
-    more rows than 256 k below 5120 is not split, which costs a few sizes something
-    (6144 x 4096: 270 rows 34 / 39, 320 rows 35.5 / 34.4; 4096 x 4096: 384 rows 1.06, 320
-    and 448 rows 0.9)."""
+    rows 17.2 / 16.5; 3072 x 2048: 150 rows 13.0 / 14.9, 704 rows 21 / 19; 1408 x 2560:
+    300 rows 14.2 / 19.0), of up to 256 rows only if it is a multiple of 128 (1984 x 6144:
+    113 rows 23 / 16) or below 1536; rows longer than the norm takes sums of; and what
+    _whole_sooner says."""
     if (rows <= 64 or k < 1024 or k % 64 or not 1024 <= n <= 16384 or
             n % 64 or not _tile_fits(rows, n, k)):
         return False
-    if rows > 256 and k < 5120:     # whole: tile_bindings.h pick_tile_parts
-        return rows * n > 1_000_000
+    if rows > 256 and k < 5120:
+        return rows * n > 1_000_000 and not _whole_sooner(rows, n, k)
     return (k > 2048 or k > 1536 and k % 128 > 0 or n > 8192 or
             rows * n > 1_200_000)
+
+
+def _whole_sooner(rows: int, n: int, k: int) -> bool:
+    """Is the library sooner than the tiles, of more than 256 rows and a k that those do
+    not split (hip/tile_bindings.h pick_tile_parts)?  Over 3200 sizes of 257 to 1000 rows,
+    2048 to 16384 columns and 2304 to 4608 k, with the norm, the tiles take 0.93 of its
+    time and more of it where its own make whole rounds (library / tiles, us): to 288 rows
+    of 5632 to 6400 columns 1.07 to 1.22 times (6144 x 4096: 257 rows 33.0 / 37.7, 288
+    rows 34.0 / 40.1, 289 rows 34.5 / 33.7) and of 8704 to 10752 1.00 to 1.08; of 321 to
+    384 rows, 3328 to 4096 columns 0.98 to 1.14 (4096 x 4096: 336 rows 28.7 / 30.0, 384
+    rows 29.6 / 33.0, 385 rows 30.2 / 27.9) and more than 10752 columns 1.02 to 1.13
+    (12288 x 4096: 300 rows 63 / 57, 380 rows 62 / 67); of 513 to 576 rows, 3328 to 3584
+    and 8704 to 10752 columns 1.00 to 1.16.  A k between multiples of 128 slows the
+    library down (3840 x 4160: 365 rows 0.79)."""
+    if k >= 4736 or k <= 2048 or k % 128:
+        return False
+    if rows <= 288:
+        return 5376 < n <= 6400 or k >= 2560 and 8448 < n <= 10752
+    if 320 < rows <= 384:
+        return 10752 < n < 16384 or k >= 3072 and 3200 < n <= 4096
+    return k >= 2560 and 512 < rows <= 576 and (3200 < n <= 3584 or
+                                                8448 < n <= 10752)
 
 
 def _takes_tile(x: torch.Tensor, w: torch.Tensor, rule) -> bool:

@@ -460,3 +460,18 @@ def test_swiglu_by_unrounded_gates(m, n, k):
     assert ops.block_routes(m, (n, k), (n, k), True)[0] == (2 if m == 440 else 4)
     x, w, full, sums = _operands(m, n, k)
     assert _near(ops.linear_swiglu(x, w), GLU, full, sums)
+
+
+@pytest.mark.parametrize("n,k,rows,taken", [
+    (6144, 4096, (257, 270, 288), False), (6144, 4096, (256, 289, 300, 320), True),
+    (6144, 2304, (264,), False), (6144, 4736, (270,), True), (5376, 4096, (270,), True),
+    (6464, 4096, (270,), True), (10240, 4096, (257, 288), False),
+    (10240, 4096, (289, 512), True), (4096, 4096, (321, 384), False),
+    (4096, 4096, (320, 385), True), (3840, 4160, (365,), True),
+    (12288, 4096, (321, 384), False), (12288, 4096, (320, 385), True),
+    (3584, 4096, (513, 576), False), (9728, 4608, (513, 576), False),
+    (9728, 4608, (512, 577), True)])
+def test_whole_products_that_the_library_ends_sooner(n, k, rows, taken):
+    """Of more than 256 rows and a k that is not split."""
+    from rbg_amd import ops
+    assert all(ops._tile(m, n, k) == taken for m in rows)
