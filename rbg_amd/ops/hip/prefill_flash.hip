@@ -469,6 +469,10 @@ __global__ __launch_bounds__(THREADS, 2) void prefill_flash_kernel(
                               (c & 3) * 256 + (((n * 2 + h) ^ (c & 15)) * 16)) =
         pf_u4{x[0], y[0], x[1], y[1]};
   }
+  // lanes read what others of the wave wrote: in that order for the compiler too
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const int row = j * 4 + (lane >> 4), r = wave * 32 + row, token = token_of(r);
