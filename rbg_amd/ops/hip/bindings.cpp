@@ -176,14 +176,35 @@ torch::Tensor embed_rows(torch::Tensor ids, torch::Tensor table) {
   return out;
 }
 
+// Is this memory of the host what host_read.h takes it for?
+static bool fine_grained(const torch::Tensor& host) {
+  unsigned flags = 0;
+  if (hipHostGetFlags(&flags, host.data_ptr()) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return !(flags & hipHostMallocNonCoherent);
+}
+
+// Pinned memory as a kernel may read it: itself, or its copy on the GPU.
+static torch::Tensor for_kernels(const torch::Tensor& host, torch::Device device) {
+  return fine_grained(host) ? host : host.to(device, /*non_blocking=*/true);
+}
+
 // Memory of the host that a kernel on the current stream has read: torch gives it to
-// nobody else before the stream has come so far.
-static void read_by_stream(const torch::Tensor& host) {
+// nobody else before the stream has come so far, if it is of torch's allocator.
+static bool held_for_stream(const torch::Tensor& host) {
   const auto stream = at::hip::getCurrentHIPStream();
-  at::getHostAllocator(at::kCUDA)->record_event(
+  return at::getHostAllocator(at::kCUDA)->record_event(
       host.data_ptr(), host.storage().data_ptr().get_context(),
       c10::Stream(c10::Stream::UNSAFE,
                   c10::Device(c10::kCUDA, stream.device_index()), stream.id()));
+}
+
+static void read_by_stream(const torch::Tensor& host) {
+  if (!held_for_stream(host))
+    TORCH_CHECK(hipStreamSynchronize(current_stream()) == hipSuccess,
+                "waiting for a read of the host's memory");
 }
 
 // Rows of x that the host names, below 0 from its end.
@@ -199,7 +220,8 @@ torch::Tensor rows_at(torch::Tensor x, const std::vector<int64_t>& rows) {
   if (n == 0) return out;
   auto host = torch::empty({n}, torch::dtype(torch::kInt64).pinned_memory(true));
   std::copy(rows.begin(), rows.end(), host.data_ptr<int64_t>());
-  launch_embed_rows(out.data_ptr(), x.data_ptr(), host.data_ptr(), all,
+  const auto from = for_kernels(host, x.device());
+  launch_embed_rows(out.data_ptr(), x.data_ptr(), from.data_ptr(), all,
                     (int)x.size(1), (int)n, true, current_stream());
   read_by_stream(host);
   return out;
@@ -454,6 +476,8 @@ void place_host_inputs(torch::Tensor fields, torch::Tensor tables,
   char* at = (char*)host.data_ptr();
   if (head) std::memcpy(at, new_fields.data_ptr(), head);
   if (rest) std::memcpy(at + head, new_tables.data_ptr(), rest);
+  const auto from = for_kernels(host, fields.device());
+  at = (char*)from.data_ptr();
   launch_place_inputs(fields.data_ptr(), at, (int)fields.numel(),
                       tables.data_ptr(), at + head, (int)tables.size(0),
                       (int)tables.size(1), (int)new_tables.size(0),
@@ -1027,6 +1051,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("tickets") = c10::nullopt);
   m.def("rows_at", &rows_at, "rows that the host names");
   m.def("place_host_inputs", &place_host_inputs, "place_inputs from the host");
+  m.def("host_memory", [](torch::Tensor host) {
+    return std::make_tuple(fine_grained(host), held_for_stream(host));
+  }, "whether kernels read it as it is, and torch keeps it for them");
   m.def("prefill_plan", &prefill_plan, "prompt attention's workgroups",
         py::call_guard<py::gil_scoped_release>());
   m.def("decode_heads", &decode_heads, "rope_heads and decode_attention");

@@ -1564,3 +1564,17 @@ def test_embed_rows(rows, width, count):
         got = ops.embed_rows(ids, table)
         assert got[2:5].isnan().all()
         assert torch.equal(got[5:].cpu(), want[5:])
+
+
+@pytest.mark.gpu
+def test_host_memory_that_kernels_read():
+    """Pinned memory is fine-grained, and kept by torch's allocator until the stream has
+    read it; of other memory neither is taken for granted, and no error is left."""
+    from rbg_amd import ops
+    for _ in range(3):
+        pinned = torch.empty(4096, dtype=torch.uint8, pin_memory=True)
+        assert ops._hip.host_memory(pinned) == (True, True)
+        assert ops._hip.host_memory(torch.empty(4096, dtype=torch.uint8)) == \
+            (False, False)
+    torch.ones(8, device="cuda:0").add_(1)
+    torch.cuda.synchronize()
