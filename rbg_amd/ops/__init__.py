@@ -460,11 +460,8 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def place_inputs(fields, tables, new_fields, new_tables) -> None:
-    """A captured decode step's inputs from new ones: ``fields``, and ``tables``
-    [rows, width] with page 0 beyond ``new_tables`` [seqs, used]."""
-    if _on_gpu(fields) and _hip is not None:
-        _hip.place_inputs(fields, tables, new_fields, new_tables)
-        return
+    """A captured decode step's inputs from new ones on its device: ``fields``, and
+    ``tables`` [rows, width] with page 0 beyond ``new_tables`` [seqs, used]."""
     n, used = new_tables.shape
     fields.copy_(new_fields)
     tables.zero_()

@@ -45,7 +45,7 @@ bool launch_norm_rows(void*, void*, const void*, int, const void*, void*,
 bool launch_stream_rows(void*, void*, int, const void*, const void*, int, int,
                         int, int, hipStream_t);
 void launch_place_inputs(void*, const void*, int, void*, const void*, int, int,
-                         int, int, bool, hipStream_t);
+                         int, int, hipStream_t);
 void launch_prefill_attention(void*, const void*, const void*, const void*,
                               const void*, const void*, float, int, int, int,
                               int, int, int, hipStream_t);
@@ -433,42 +433,24 @@ torch::Tensor stream_linear(torch::Tensor a, torch::Tensor w, int64_t end) {
   return end == 2 ? c.unsqueeze(0) : c;
 }
 
-static void check_inputs(const torch::Tensor& fields, const torch::Tensor& tables,
-                         const torch::Tensor& new_fields,
-                         const torch::Tensor& new_tables, bool host) {
+// fields and tables [rows, width]: a captured step's inputs, from new ones of the host,
+// whose tables are [seqs, used].  The kernel reads pinned memory, whose pages the GPU
+// maps.
+void place_host_inputs(torch::Tensor fields, torch::Tensor tables,
+                       torch::Tensor new_fields, torch::Tensor new_tables) {
   for (const auto& t : {fields, new_fields})
     TORCH_CHECK(t.is_contiguous() && t.scalar_type() == torch::kInt64,
                 "fields: int64");
   for (const auto& t : {tables, new_tables})
     TORCH_CHECK(t.is_contiguous() && t.dim() == 2 &&
                 t.scalar_type() == torch::kInt32, "tables: int32");
-  TORCH_CHECK(fields.is_cuda() && tables.is_cuda(), "inputs on GPU");
-  for (const auto& t : {new_fields, new_tables})
-    TORCH_CHECK(host ? t.is_cpu() : t.is_cuda(), "new ones on ",
-                host ? "the host" : "GPU");
+  TORCH_CHECK(fields.is_cuda() && tables.is_cuda() && new_fields.is_cpu() &&
+              new_tables.is_cpu(), "inputs on GPU, new ones on the host");
   TORCH_CHECK(fields.numel() == new_fields.numel() &&
               new_tables.size(0) <= tables.size(0) &&
               new_tables.size(1) <= tables.size(1), "sizes disagree");
   TORCH_CHECK(fields.numel() < (1 << 30) && tables.numel() < (1 << 30),
               "too many");
-}
-
-// fields and tables [rows, width]: a captured step's inputs, from new ones, whose
-// tables are [seqs, used]
-void place_inputs(torch::Tensor fields, torch::Tensor tables,
-                  torch::Tensor new_fields, torch::Tensor new_tables) {
-  check_inputs(fields, tables, new_fields, new_tables, false);
-  launch_place_inputs(fields.data_ptr(), new_fields.data_ptr(),
-                      (int)fields.numel(), tables.data_ptr(),
-                      new_tables.data_ptr(), (int)tables.size(0),
-                      (int)tables.size(1), (int)new_tables.size(0),
-                      (int)new_tables.size(1), false, current_stream());
-}
-
-// The same from the host: the kernel reads pinned memory, whose pages the GPU maps.
-void place_host_inputs(torch::Tensor fields, torch::Tensor tables,
-                       torch::Tensor new_fields, torch::Tensor new_tables) {
-  check_inputs(fields, tables, new_fields, new_tables, true);
   const size_t head = new_fields.nbytes(), rest = new_tables.nbytes();
   if (head + rest == 0 && tables.numel() == 0) return;
   auto host = torch::empty({(int64_t)std::max<size_t>(head + rest, 16)},
@@ -481,7 +463,7 @@ void place_host_inputs(torch::Tensor fields, torch::Tensor tables,
   launch_place_inputs(fields.data_ptr(), at, (int)fields.numel(),
                       tables.data_ptr(), at + head, (int)tables.size(0),
                       (int)tables.size(1), (int)new_tables.size(0),
-                      (int)new_tables.size(1), true, current_stream());
+                      (int)new_tables.size(1), current_stream());
   read_by_stream(host);
 }
 
@@ -1050,7 +1032,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("num_splits"), py::arg("wide"), py::arg("span") = 128,
         py::arg("tickets") = c10::nullopt);
   m.def("rows_at", &rows_at, "rows that the host names");
-  m.def("place_host_inputs", &place_host_inputs, "place_inputs from the host");
+  m.def("place_host_inputs", &place_host_inputs, "a decode step's inputs to their place");
   m.def("host_memory", [](torch::Tensor host) {
     return std::make_tuple(fine_grained(host), held_for_stream(host));
   }, "whether kernels read it as it is, and torch keeps it for them");
@@ -1060,7 +1042,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("prompt_attention_block", &prompt_attention_block,
         "norm, attention and output product of prompts");
   m.def("swiglu_block", &swiglu_block, "norm and gated MLP of many rows");
-  m.def("place_inputs", &place_inputs, "a decode step's inputs to their place");
   m.def("prefill_attention", &prefill_attention, "varlen causal flash prefill");
   m.def("prefill_flash", &prefill_flash, "causal attention of prompts",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("block_info"),

@@ -9,8 +9,7 @@
 
 namespace {
 
-// HOST: the new ones are in the host's memory
-template <bool HOST>
+// the new ones are in the host's memory
 __global__ __launch_bounds__(256) void place_inputs_kernel(
     long* __restrict__ fields, const long* __restrict__ new_fields,
     const int count, int* __restrict__ tables,     // [rows, width]
@@ -19,10 +18,9 @@ __global__ __launch_bounds__(256) void place_inputs_kernel(
   const int at = blockIdx.x * 256 + threadIdx.x;
   const int row = at / width, col = at % width;
   const bool held = row < seqs && col < used;
-  if (at < count) fields[at] = HOST ? host_read(new_fields + at) : new_fields[at];
+  if (at < count) fields[at] = host_read(new_fields + at);
   if (at >= rows * width) return;
-  const int* from = new_tables + row * used + col;
-  tables[at] = !held ? 0 : HOST ? host_read(from) : *from;
+  tables[at] = held ? host_read(new_tables + row * used + col) : 0;
 }
 
 }  // namespace
@@ -30,16 +28,11 @@ __global__ __launch_bounds__(256) void place_inputs_kernel(
 extern "C" void launch_place_inputs(void* fields, const void* new_fields,
                                     int count, void* tables,
                                     const void* new_tables, int rows,
-                                    int width, int seqs, int used, bool host,
+                                    int width, int seqs, int used,
                                     hipStream_t stream) {
   const int most = max(count, rows * width);
   if (most == 0) return;
-#define PI_GO(HOST)                                                        \
-  place_inputs_kernel<HOST><<<dim3((most + 255) / 256), dim3(256), 0,      \
-                              stream>>>(                                   \
-      (long*)fields, (const long*)new_fields, count, (int*)tables,         \
-      (const int*)new_tables, rows, max(width, 1), seqs, used)
-  if (host) PI_GO(true);
-  else PI_GO(false);
-#undef PI_GO
+  place_inputs_kernel<<<dim3((most + 255) / 256), dim3(256), 0, stream>>>(
+      (long*)fields, (const long*)new_fields, count, (int*)tables,
+      (const int*)new_tables, rows, max(width, 1), seqs, used);
 }
