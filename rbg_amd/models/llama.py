@@ -393,10 +393,7 @@ class LlamaForCausalLM(nn.Module):
         return ops.add_rmsnorm(x, residual, self.final_norm, self.cfg.rms_eps)
 
     @torch.inference_mode()
-    def logits(self, hidden: torch.Tensor,
-               gather_idx: Optional[torch.Tensor] = None) -> torch.Tensor:
-        if gather_idx is not None:
-            hidden = hidden[gather_idx.long()]
+    def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         return ops.linear_f32(hidden, self.lm_head)
 
     def reload_weights(self, seed: int) -> None:

@@ -202,6 +202,5 @@ class NotadraForCausalLM(StreamForCausalLM):
                                  self.cfg.rms_eps, self.dtype)
 
     @torch.inference_mode()
-    def logits(self, hidden: torch.Tensor,
-               gather_idx: Optional[torch.Tensor] = None) -> torch.Tensor:
-        return super().logits(hidden, gather_idx).mul_(self.cfg.logit_scale)
+    def logits(self, hidden: torch.Tensor) -> torch.Tensor:
+        return super().logits(hidden).mul_(self.cfg.logit_scale)

@@ -131,10 +131,7 @@ class StreamForCausalLM(nn.Module):
         return self.final(x, pending)
 
     @torch.inference_mode()
-    def logits(self, hidden: torch.Tensor,
-               gather_idx: Optional[torch.Tensor] = None) -> torch.Tensor:
-        if gather_idx is not None:
-            hidden = hidden[gather_idx.long()]
+    def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         return torch.nn.functional.linear(hidden, self.lm_head).float()
 
     def reload_weights(self, seed: int) -> None:
