@@ -475,3 +475,36 @@ def test_whole_products_that_the_library_ends_sooner(n, k, rows, taken):
     """Of more than 256 rows and a k that is not split."""
     from rbg_amd import ops
     assert all(ops._tile(m, n, k) == taken for m in rows)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form,stages,silu", MORE_FORMS)
+def test_more_forms_for_the_rest(form, stages, silu):
+    """Beginning at a column between, and before another form's columns."""
+    from rbg_amd import ops
+    x, w, full, sums = _operands(500, 2048, 512)
+    for end in (PLAIN, GLU) if silu else (PLAIN,):
+        for first, rest, to in ((0, form, 256), (0, form, 768), (form, 5, 512)):
+            got = ops._hip.tile_form(x, w, end, first, 1, rest, to)
+            assert _near(got, end, full, sums), (end, first, rest, to)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form,stages,silu", MORE_FORMS)
+def test_more_forms_many_tiles_a_workgroup(form, stages, silu):
+    """As test_many_tiles_a_workgroup, with the fewest stages that they take, and sums
+    of one part and of several."""
+    from rbg_amd import ops
+    x, w, full, sums = _operands(2100, 9280, 64 * max(stages, 4))
+    for end in (PLAIN, PARTS, GLU) if silu else (PLAIN, PARTS):
+        got = ops._hip.tile_form(x, w, end, form, 1, -1, 0)
+        assert _near(got, end, full, sums), end
+    x, w, full, sums = _operands(2100, 2112, 64 * stages * 4)
+    got = ops._hip.tile_form(x, w, PARTS, form, 4, -1, 0)
+    assert _near(got, PARTS, full, sums)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [f for f, _, silu in MORE_FORMS if silu])
+def test_more_forms_of_very_negative_gates(form):
+    test_silu_of_very_negative_gates(form)
