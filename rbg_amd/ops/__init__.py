@@ -249,14 +249,17 @@ def _tile_f32(rows: int, n: int, k: int) -> bool:
     """Does the GEMM of prompts take a product in f32, rather than hipBLASLt and a
     conversion (a launch and its result once more)?  From 65 rows, where the decode GEMM
     ends, of wide matrices, as for fewer columns it would have to split k.  Own /
-    library over 16384 to 128256 columns, 2048 to 12288 k (us): 128 rows of 32768 x 4096
-    65 / 73, 32768 x 8192 117 / 142, 128256 x 4096 241 / 269, 65536 x 8192 even, of 16384
-    x 4096 48 / 41, of 32768 x 12288 187 / 184; k that is no multiple of 2048 only below
-    4096 (32768 x 3072: 48 / 54; 24576 x 5120: 73 / 70).  Not where its tiles begin a
-    round that the library's do not (34048 x 1536: 128 rows 44.4 / 37.7; 50304 x 3584 102 /
-    94, but x 2048 0.85; 66048 x 4096: 128 rows 166 / 157, 72 rows 0.95; 102400 x 2560: 80
-    rows 143 / 131, 72 rows 0.86).  From 129 rows of the widest (65536 x 5120: 129 rows
-    155 / 174, 192 rows 164 / 162; 32768 x 4096: 80 / 75)."""
+    library, in us, over 2030 sizes of 65 to 256 rows, 16384 to 128256 columns and 1024 to
+    10240 k: what the rule takes 0.85 of the time (128 rows of 32768 x 4096 67.6 / 71.8,
+    32768 x 8192 120 / 151, 128256 x 4096 220 / 268, 65536 x 8192 224 / 234; 129 rows of
+    65536 x 5120 150 / 170, 192 rows even), 18 of 1148 slower by 3 to 6% (49152 x 2560: 80
+    rows 71.0 / 67.7).  The lines lie where they were drawn for stores that took up
+    to 5 us a tile longer: not k that is no multiple of 2048 from 4096 on (24576 x 5120:
+    128 rows 78.3 / 75.2), nor where its tiles begin a round that the library's do not
+    (66048 x 4096: 128 rows 166 / 161, 80 rows 146 / 158; 102400 x 2560: 80 rows 144 /
+    135).  Of what they leave to the library it would now take 0.92 of the time on
+    average, by 0.68 to 1.37 (34048 x 1536: 129 rows 36 / 53; 16384 x 4096: 128 rows 41 /
+    45)."""
     if k < 1024 or k > 8192 or k % 64 or n % 64 or not _tile_fits(rows, n, k):
         return False
     if rows > 128:
@@ -290,8 +293,8 @@ def _tile(rows: int, n: int, k: int) -> bool:
     columns and 1024 to 28672 k, with the norm that reads the sums, it takes 0.6 to 0.8
     of the better of both from 8192 k, 0.85 to 0.95 of shorter (us: 5120 x 8192: 200 rows
     55 / 36; 2048 x 5632: 128 rows 18.5 / 15.9; 6144 x 4096: 704 rows 57 / 45; 4096 x
-    4096: 1200 rows 55 / 47; 8192 x 28672: 400 rows 420 / 200).  The rule takes 0.5%
-    more than the faster one of each.  Left to the others is a short k of a small result,
+    4096: 1200 rows 55 / 47; 8192 x 28672: 400 rows 420 / 200).  The rule takes 0.4%
+    more than the fastest of each.  Left to the others is a short k of a small result,
     which the library's smaller tiles end sooner (2048 x 2048: 200 rows 12.8 / 13.1, 640
     rows 17.2 / 16.5; 3072 x 2048: 150 rows 13.0 / 14.9, 704 rows 21 / 19; 1408 x 2560:
     300 rows 14.2 / 19.0), of up to 256 rows only if it is a multiple of 128 (1984 x 6144:
@@ -315,9 +318,10 @@ def _whole_sooner(rows: int, n: int, k: int) -> bool:
     rows 34.0 / 40.1, 289 rows 34.5 / 33.7) and of 8704 to 10752 1.00 to 1.08; of 321 to
     384 rows, 3328 to 4096 columns 0.98 to 1.14 (4096 x 4096: 336 rows 28.7 / 30.0, 384
     rows 29.6 / 33.0, 385 rows 30.2 / 27.9) and more than 10752 columns 1.02 to 1.13
-    (12288 x 4096: 300 rows 63 / 57, 380 rows 62 / 67); of 513 to 576 rows, 3328 to 3584
-    and 8704 to 10752 columns 1.00 to 1.16.  A k between multiples of 128 slows the
-    library down (3840 x 4160: 365 rows 0.79)."""
+    (12288 x 4096: 300 rows 63 / 57, 380 rows 62 / 67; 16384 themselves stay with the
+    tiles at 1.04 to 1.10, so that of them rows once taken stay taken); of 513 to 576
+    rows, 3328 to 3584 and 8704 to 10752 columns 1.00 to 1.16.  A k between multiples of
+    128 slows the library down (3840 x 4160: 365 rows 0.79)."""
     if k >= 4736 or k <= 2048 or k % 128:
         return False
     if rows <= 288:
@@ -893,8 +897,10 @@ def _turn_round(order: np.ndarray, kv_heads: int) -> np.ndarray:
 
 def prefill_plan(cu, cu_k, heads: int, kv_heads: int, device) -> PrefillPlan:
     """``cu`` and ``cu_k``: where each sequence's query and kv rows begin, on
-    the host."""
-    if torch.device(device).type == "cuda":     # the same, native (hip/prefill_plan.h)
+    the host.  For a GPU by hip/prefill_plan.h; what follows below, with _cut_prefill and
+    _turn_round, states its steps and reasons, is its oracle in the tests, number by
+    number, and plans for other devices.  A change to one is a change to both."""
+    if torch.device(device).type == "cuda":
         return PrefillPlan(*_require_hip().prefill_plan(
             *(x if isinstance(x, list) else np.asarray(x).tolist()
               for x in (cu, cu_k)), heads, kv_heads, torch.device(device)))

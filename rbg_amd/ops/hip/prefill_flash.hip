@@ -9,7 +9,9 @@
 // TFLOP/s.  So nothing is computed in the loop that can be kept: a lane's offsets, which
 // change for the last tile only, took 12 instructions a tile, of pages, then in 64 bits,
 // 48 (us: 8192 tokens 526 -> 518, 4 of 2048 160 -> 158.6, 1500 after 9000 in pages 254
-// -> 248).
+// -> 248).  Cards differ by a tenth, and figures are of one card each: this kernel and
+// the one before queries passed LDS and offsets were kept, in turn on a third, 8192
+// tokens 541 -> 530, 4 of 2048 169 -> 164, 1500 after 9000 261 -> 252.
 // A workgroup is 4 waves of 32 query rows each; tiles of 64 keys pass LDS in two
 // stages, one barrier a tile.
 //  * The rows of a workgroup are 128 / group tokens with all the query heads
@@ -35,7 +37,8 @@
 //    in one piece.  From and to registers as the products have them every lane of an
 //    instruction was in another line, of which a CU takes one a cycle: 1.9 us of a
 //    workgroup (64 sequences of 64 tokens, 32 heads of 8, 30.3 -> 24.0 us; 23 of 40 to
-//    854 104 -> 95; 37 tokens of 16 heads 7.4 -> 6.7; 8192 594 -> 590).
+//    854 104 -> 95; 37 tokens of 16 heads 7.4 -> 6.7; 8192, on the slowest card, 594 ->
+//    590).
 //  * Blocks are cut by keys where whole ones would leave CUs idle (ops
 //    _cut_prefill), whose sums a second launch adds up: 1500 tokens after 9000
 //    294 -> 249 us, 512 after 4000 79 -> 55, 40 after 9000 140 -> 27.

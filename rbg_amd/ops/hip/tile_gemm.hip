@@ -23,8 +23,10 @@
 //    with silu 1318 -> 1258 us, 2048 rows 361 -> 342; in parts 128 x 4096 x 4096 14.8 ->
 //    13.5, 256 x 4096 x 4096 22.1 -> 19.8; 1500 x 4096 x 4096 52.7 -> 51.5.
 // It gains on the library by what the library does not do: silu in the product
-// (8192 x 28672 x 4096 with silu 1301 us / 1382), parts of a long k (2048 x 4096
-// x 14336 182 / 214 with the norm that adds them up), and tiles by the shape.
+// (8192 x 28672 x 4096 with silu 1327 us, the library and silu_mul 1463, both on a card
+// that is slower than that of the figures above; 2048 rows 371 / 412), parts of a long k
+// (2048 x 4096 x 14336 201 / 244 with the norm that adds them up), and tiles by the
+// shape.
 #include <algorithm>
 #include <type_traits>
 #include <utility>
